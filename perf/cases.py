@@ -19,11 +19,12 @@ import math
 
 import numpy as np
 import torch
+import torch.utils.checkpoint
 
 from alpha2_amd import FastHipBackend, HipBackend, SeededRng
 from alpha2_amd.autograd import Tape
 from alpha2_amd.fused import FusedTrainer
-from alpha2_amd.model import ModelConfig, ffn_dim, gptForward, initGPT
+from alpha2_amd.model import ModelConfig, collectParamEntries, ffn_dim, gptForward, initGPT
 from alpha2_amd.sample import SampleConfig, sampleTokens
 from alpha2_amd.train import DataLoader, TrainConfig, Trainer, zipfBatches
 
@@ -320,3 +321,126 @@ def prepare(case, seed):
 
 def run(state):
     return state.go()
+
+
+# ---------------------------------------------------------------------------------------------- the same passes in 64 bits
+def _act64(case, h, p):
+    """h: pre-activation (swiglu: gate and up); p(name): a parameter of the layer's MLP."""
+    F, act = torch.nn.functional, case["act"]
+    if act == "swiglu":
+        return F.silu(h[0]) * h[1]
+    if act == "silu":
+        return F.silu(h)
+    if act == "universal":
+        return F.silu(h) * p("act_gate") + h * p("act_skip")
+    gelu = F.gelu(h, approximate="tanh")
+    if act == "kan_spline":
+        return F.silu(h) * p("kan_c0") + F.relu(h) * p("kan_c1") + gelu * p("kan_c2") + h * p("kan_c3") + h * h * p("kan_c4")
+    return gelu
+
+
+def _block64(case, p, x):
+    F, (B, T, C), H = torch.nn.functional, x.shape, case["heads"]
+    D, cap = C // H, 30.0 if case["cap"] < 0 else case["cap"]
+    qkv = F.layer_norm(x, (C,), p("ln1.weight"), p("ln1.bias"), 1e-5) @ p("attn.wqkv").t()
+    if case["attention"] == "heads":
+        q, k, v = (t.reshape(B, T, H, D).transpose(1, 2).contiguous() for t in qkv.split(C, 2))
+    else:                                                       # the rows of a matrix re-read as slabs, no head transpose
+        q, k, v = (t.reshape(B, H, T, D) for t in qkv.split(C, 2))
+    s = q @ k.transpose(2, 3).contiguous() / math.sqrt(D)
+    if cap > 0:
+        s = cap * torch.tanh(s / cap)
+    s = s.masked_fill(torch.ones(T, T, dtype=torch.bool, device=x.device).triu(1), -math.inf)
+    x = x + (torch.softmax(s, 3) @ v).transpose(1, 2).reshape(B, T, C) @ p("attn.wo").t()
+    y = F.layer_norm(x, (C,), p("ln2.weight"), p("ln2.bias"), 1e-5)
+    if case["act"] == "swiglu":
+        return x + _act64(case, (y @ p("mlp.fc_gate").t(), y @ p("mlp.fc_up").t()), None) @ p("mlp.fc_proj").t()
+    return x + _act64(case, y @ p("mlp.fc1").t(), lambda n: p("mlp." + n)) @ p("mlp.fc2").t()
+
+
+def _logits64(case, w, ids):
+    x = w["wte"][ids] + w["wpe"][: ids.shape[1]]
+    for l in range(case["layers"]):
+        block = lambda x, l=l: _block64(case, lambda n: w["layer.%d.%s" % (l, n)], x)
+        x = torch.utils.checkpoint.checkpoint(block, x, use_reentrant=False) if torch.is_grad_enabled() else block(x)
+    return torch.nn.functional.layer_norm(x, (case["width"],), w["lnF.weight"], w["lnF.bias"], 1e-5) @ w["lmHead"].t()
+
+
+def _loss64(logits, targets):
+    return torch.nn.functional.cross_entropy(logits.reshape(-1, logits.shape[-1]), targets.reshape(-1))
+
+
+def _ids(t):
+    return torch.from_numpy(np.array(t.data, dtype=np.int64).reshape(t.shape)).cuda()
+
+
+def _step64(case, seed, w):
+    tc, names = _train_config(case), list(w)
+    bare = {"wte", "wpe"} | {n for n in names if ".ln" in n or n.startswith("lnF")}                 # not decayed
+    for t in w.values():
+        t.requires_grad_(True)
+    loss = 0.0
+    for x, y in _batches(case, seed)[: case["accum"]]:
+        part = _loss64(_logits64(case, w, _ids(x)), _ids(y))
+        part.backward()
+        loss += float(part.detach()) / case["accum"]
+        del part
+    norm = math.sqrt(sum(float((t.grad ** 2).sum()) for t in w.values())) / case["accum"]
+    scale = min(1.0, tc.gradClip / norm) / case["accum"]
+    low = tc.lr / 10                                            # the first step of the warm-up
+    lr = low + (tc.lr - low) / min(2000, tc.iters // 5)
+    grads, moments, after = {n: t.grad for n, t in w.items()}, {}, {}
+    for n, t in w.items():
+        t, g = t.detach(), grads[n] * scale
+        if case["optimizer"] == "sgd":
+            after[n] = t - lr * g
+            continue
+        decayed = t if n in bare else t * (1 - lr * tc.weightDecay)
+        if case["optimizer"] == "lion":
+            moments[n], after[n] = (1 - tc.beta2) * g, decayed - lr * torch.sign(g)
+        else:
+            moments[n], after[n] = (1 - tc.beta1) * g, decayed - lr * g / (g.abs() + tc.eps)
+    if case["how"] == "fused":                                  # one arena: decayed, then not; every tensor from a multiple of 64 on
+        order = [n for n in names if n not in bare] + [n for n in names if n in bare]
+        flat = lambda d: torch.cat([torch.nn.functional.pad(d[n].reshape(-1), (0, -d[n].numel() % 64)) for n in order])
+        return {"loss": torch.tensor([loss], dtype=torch.float64), "weights": flat(after), "gradients": flat(grads)}
+    matrices = [n for n in names if w[n].ndim == 2 and w[n].shape[0] > 1]
+    return {"loss": loss, "norm": norm, "moments": {n: moments[n] for n in matrices if moments},
+            "weights": {n: after[n] for n in matrices if not moments or not n.startswith("layer.")}}
+
+
+def _sample64(case, seed, w):
+    rng = SeededRng(seed % (1 << 30) + 3)
+    tokens = [int(t) for t in np.floor(rng.fillUniform(case["prompt"]) * case["vocab"])]
+    rng = SeededRng(seed % (1 << 30) + 5)
+    for _ in range(case["new"]):
+        row = _logits64(case, w, torch.tensor([tokens], device="cuda"))[0, -1]
+        if case["temperature"] <= 0:
+            tokens.append(int(row.argmax()))
+            continue
+        row = row / case["temperature"]
+        if case["vocab"] > 40:
+            row = row.masked_fill(row < row.topk(40).values[-1], -math.inf)
+        at = int((torch.softmax(row, 0).cumsum(0) <= rng.next()).sum())
+        tokens.append(at if at < case["vocab"] else 0)
+    return {"tokens": np.array(tokens, dtype=np.int32), "logits": _logits64(case, w, torch.tensor([tokens], device="cuda"))}
+
+
+def exact(case, seed):
+    """What the first run(prepare(case, seed)) returns, in 64 bits; None where masks of the library's own generator are in it."""
+    if case["dropout"] > 0:
+        return None
+    w = {n: torch.from_numpy(v.data.data.reshape(v.data.shape)).cuda().double() for n, v in collectParamEntries(initGPT(_config(case), None, _Normal(seed)))}
+    if case["do"] == "step":
+        return _step64(case, seed, w)
+    with torch.no_grad():
+        if case["do"] == "sample":
+            w["lmHead"] *= 5.0
+            return _sample64(case, seed, w)
+        length, T = case["batch"] * (case["tokens"] + 1) * 8, case["tokens"]
+        (x, _), = zipfBatches(seed % (1 << 30) + 1, 1, 1, length, case["vocab"])
+        corpus, rng = _ids(x).reshape(-1), SeededRng(seed % (1 << 30) + 7)
+        starts = [math.floor(rng.next() * (length - T)) for _ in range(case["batch"])]
+        cut = lambda by: torch.stack([corpus[s + by: s + by + T] for s in starts])
+        logits = _logits64(case, w, cut(0))
+        return {"loss": float(_loss64(logits, cut(1))) if case["do"] == "eval" else 0.0, "logits": logits}
