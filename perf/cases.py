@@ -156,9 +156,10 @@ def tolerance(case):
     function op by op, two steps: gradients 3e-7 .. 8e-7, single values 1e-4 of a tensor's rms; an update whose sign is decided
     by a gradient of the size of that rounding moves one weight by twice the learning rate, 6e-3 of a weight's rms.  bf16: the
     hand-scheduled step against the op-by-op one, which round in other places: gradients 1e-3 .. 5e-3, rows of the token
-    embedding that few tokens reach up to 0.5 of the tensor's rms; logits against fp32 1e-2."""
+    embedding that few tokens reach up to 0.5 of the tensor's rms; logits against fp32 1e-2.  fp32 with a vocabulary of 50304: the
+head's gradient, 16384 terms summed one after the other, is 6.7e-5 from the 64-bit one where the other gradients are 1e-6."""
     if case["how"] == "f32":
-        return {"rel": 1e-5, "max": 1e-2}
+        return {"rel": 3e-4 if case["do"] == "step" and case["vocab"] > 8192 else 1e-5, "max": 1e-2}
     return {"rel": 2e-2, "max": 0.9}
 
 
