@@ -1,5 +1,5 @@
 // GEMM on the gfx950 matrix cores.
-//   fp32 (parity mode): v_mfma_f32_32x32x2_f32, 128x128x16 LDS tiles, 4 waves (2x2) of 64x64.
+//   fp32 (parity mode): operands cut into three bf16 parts each, six bf16 products (gemm_f32.hip).
 //   bf16 (fast mode)  : v_mfma_f32_32x32x16_bf16, BMxBNx32 LDS tiles double-buffered, fp32 accumulate.
 // All three operand layouts the training step needs are handled (NN: dX = G W, NT: Y = X W^T,
 // TN: dW = G^T X).  Epilogues fuse GELU (+ saved pre-activation), the residual add, gradient
@@ -12,119 +12,6 @@
 using namespace ah;
 
 namespace {
-
-// ================================================================ fp32 MFMA kernel
-// LDS tiles are k-major: As[k][m], Bs[k][n]; a lane of the 32x32x2 MFMA reads As[2*kk + lane/32][m0 + lane%32].
-constexpr int F_BM = 128, F_BN = 128, F_BK = 16, F_PAD = 4;
-
-// Load a [rows x F_BK] tile of an operand into registers (2 float4 per thread).
-//   KCONTIG = true : memory is [row][k] (k contiguous), thread -> (row = t/4 + 64*i, kq = t%4)
-//   KCONTIG = false: memory is [k][row] (row contiguous), thread -> (k = t/32 + 8*i, r4 = t%32)
-template <bool KCONTIG>
-__device__ __forceinline__ void f32_load_tile(const float *__restrict__ base, int64_t ld, int row0, int k0, int rows, int K,
-                                              bool vec, float4 (&v)[2]) {
-  int t = threadIdx.x;
-#pragma unroll
-  for (int i = 0; i < 2; i++) {
-    int r, k;
-    if (KCONTIG) { r = row0 + (t >> 2) + 64 * i; k = k0 + (t & 3) * 4; }
-    else { k = k0 + (t >> 5) + 8 * i; r = row0 + (t & 31) * 4; }
-    float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (KCONTIG) {
-      if (r < rows) {
-        const float *p = base + (int64_t)r * ld + k;
-        if (vec && k + 3 < K) x = *reinterpret_cast<const float4 *>(p);
-        else { if (k < K) x.x = p[0]; if (k + 1 < K) x.y = p[1]; if (k + 2 < K) x.z = p[2]; if (k + 3 < K) x.w = p[3]; }
-      }
-    } else {
-      if (k < K) {
-        const float *p = base + (int64_t)k * ld + r;
-        if (vec && r + 3 < rows) x = *reinterpret_cast<const float4 *>(p);
-        else { if (r < rows) x.x = p[0]; if (r + 1 < rows) x.y = p[1]; if (r + 2 < rows) x.z = p[2]; if (r + 3 < rows) x.w = p[3]; }
-      }
-    }
-    v[i] = x;
-  }
-}
-template <bool KCONTIG>
-__device__ __forceinline__ void f32_store_tile(float (*s)[F_BM + F_PAD], const float4 (&v)[2]) {
-  int t = threadIdx.x;
-#pragma unroll
-  for (int i = 0; i < 2; i++) {
-    if (KCONTIG) {
-      int r = (t >> 2) + 64 * i, k = (t & 3) * 4;
-      s[k + 0][r] = v[i].x; s[k + 1][r] = v[i].y; s[k + 2][r] = v[i].z; s[k + 3][r] = v[i].w;
-    } else {
-      int k = (t >> 5) + 8 * i, r = (t & 31) * 4;
-      *reinterpret_cast<float4 *>(&s[k][r]) = v[i];
-    }
-  }
-}
-
-template <int LAYOUT, int EPI, class OUT>
-__global__ __launch_bounds__(256) void k_gemm_f32(GemmArgs g, int vec_a, int vec_b, int vec_c) {
-  __shared__ __attribute__((aligned(16))) float As[2][F_BK][F_BM + F_PAD];
-  __shared__ __attribute__((aligned(16))) float Bs[2][F_BK][F_BN + F_PAD];
-  constexpr bool A_KC = (LAYOUT != AH_GEMM_TN);     // A is [M][K] except for TN ([K][M])
-  constexpr bool B_KC = (LAYOUT == AH_GEMM_NT);     // B is [N][K] only for NT
-  int bz = blockIdx.z;
-  const float *A = (const float *)g.a + (int64_t)bz * g.sa;
-  const float *B = (const float *)g.b + (int64_t)bz * g.sb;
-  int64_t cbase = (int64_t)bz * g.sc;
-  int m0 = blockIdx.y * F_BM, n0 = blockIdx.x * F_BN;
-  int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
-  int lr = lane & 31, lk = lane >> 5;
-
-  f32x16 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; i++)
-#pragma unroll
-    for (int j = 0; j < 2; j++)
-#pragma unroll
-      for (int e = 0; e < 16; e++) acc[i][j][e] = 0.f;
-
-  float4 ra[2], rb[2];
-  int nt = (g.K + F_BK - 1) / F_BK;
-  f32_load_tile<A_KC>(A, g.lda, m0, 0, g.M, g.K, vec_a, ra);
-  f32_load_tile<B_KC>(B, g.ldb, n0, 0, g.N, g.K, vec_b, rb);
-  f32_store_tile<A_KC>(As[0], ra);
-  f32_store_tile<B_KC>(Bs[0], rb);
-  __syncthreads();
-  for (int t = 0; t < nt; t++) {
-    int cur = t & 1;
-    if (t + 1 < nt) {
-      f32_load_tile<A_KC>(A, g.lda, m0, (t + 1) * F_BK, g.M, g.K, vec_a, ra);
-      f32_load_tile<B_KC>(B, g.ldb, n0, (t + 1) * F_BK, g.N, g.K, vec_b, rb);
-    }
-#pragma unroll
-    for (int kk = 0; kk < F_BK / 2; kk++) {
-      float a0 = As[cur][2 * kk + lk][wm + lr], a1 = As[cur][2 * kk + lk][wm + 32 + lr];
-      float b0 = Bs[cur][2 * kk + lk][wn + lr], b1 = Bs[cur][2 * kk + lk][wn + 32 + lr];
-      // operands swapped: the accumulator holds C^T tiles (rows = n, columns = m)
-      acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(b0, a0, acc[0][0], 0, 0, 0);
-      acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(b1, a0, acc[0][1], 0, 0, 0);
-      acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(b0, a1, acc[1][0], 0, 0, 0);
-      acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(b1, a1, acc[1][1], 0, 0, 0);
-    }
-    if (t + 1 < nt) {
-      f32_store_tile<A_KC>(As[cur ^ 1], ra);
-      f32_store_tile<B_KC>(Bs[cur ^ 1], rb);
-    }
-    __syncthreads();
-  }
-  // accumulator element e of a (transposed) 32x32 tile: n = 8*(e/4) + 4*(lane/32) + e%4, m = lane%32
-#pragma unroll
-  for (int i = 0; i < 2; i++)
-#pragma unroll
-    for (int j = 0; j < 2; j++)
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        int row = m0 + wm + 32 * i + lr;
-        int col = n0 + wn + 32 * j + 8 * q + 4 * lk;
-        epilogue4<EPI, OUT>(g, cbase, row, col, acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3], vec_c);
-      }
-}
 
 // ================================================================ bf16 MFMA kernel (NT operands)
 // Both operands are [rows][K] with K contiguous.  LDS tiles are [rows][BK] with an 80-byte row pitch
@@ -270,29 +157,6 @@ int32_t run_bf16_nt(const GemmArgs &ga, int batch, int out_dtype, int vec_c) {
     case AH_EPI_GELU_GRAD: return launch_bf16_nt_t<128, 128, 2, 2, AH_EPI_GELU_GRAD, uint16_t>(ga, batch, vec_c);
     case AH_EPI_MUL_AUX: return launch_bf16_nt_t<128, 128, 2, 2, AH_EPI_MUL_AUX, uint16_t>(ga, batch, vec_c);
     default: return launch_bf16_nt_t<128, 128, 2, 2, AH_EPI_GELU_BWD, uint16_t>(ga, batch, vec_c);
-  }
-}
-
-template <int LAYOUT, int EPI, class OUT>
-int32_t launch_f32_t(const GemmArgs &ga, int batch, int vec_a, int vec_b, int vec_c) {
-  dim3 grid((unsigned)cdiv(ga.N, F_BN), (unsigned)cdiv(ga.M, F_BM), (unsigned)batch);
-  note_gemm_kernel("k_gemm_f32<%d, %d, %s>", LAYOUT, EPI, sizeof(OUT) == 4 ? "float" : "unsigned short");
-  note_gemm_split(1);
-  ah::launch_kernel((k_gemm_f32<LAYOUT, EPI, OUT>), grid, dim3(256), 0, ga, vec_a, vec_b, vec_c);
-  AH_LAUNCH_CHECK();
-  return AH_OK;
-}
-template <int LAYOUT>
-int32_t launch_f32(const GemmArgs &ga, int batch, int out_dtype, int vec_a, int vec_b, int vec_c) {
-  switch (ga.epi) {
-    case AH_EPI_NONE: return out_dtype == AH_F32 ? launch_f32_t<LAYOUT, AH_EPI_NONE, float>(ga, batch, vec_a, vec_b, vec_c)
-                                                 : launch_f32_t<LAYOUT, AH_EPI_NONE, uint16_t>(ga, batch, vec_a, vec_b, vec_c);
-    case AH_EPI_ACCUM: return launch_f32_t<LAYOUT, AH_EPI_ACCUM, float>(ga, batch, vec_a, vec_b, vec_c);
-    case AH_EPI_GELU: return launch_f32_t<LAYOUT, AH_EPI_GELU, float>(ga, batch, vec_a, vec_b, vec_c);
-    case AH_EPI_RESIDUAL: return launch_f32_t<LAYOUT, AH_EPI_RESIDUAL, float>(ga, batch, vec_a, vec_b, vec_c);
-    case AH_EPI_GELU_GRAD: return launch_f32_t<LAYOUT, AH_EPI_GELU_GRAD, float>(ga, batch, vec_a, vec_b, vec_c);
-    case AH_EPI_MUL_AUX: return launch_f32_t<LAYOUT, AH_EPI_MUL_AUX, float>(ga, batch, vec_a, vec_b, vec_c);
-    default: return launch_f32_t<LAYOUT, AH_EPI_GELU_BWD, float>(ga, batch, vec_a, vec_b, vec_c);
   }
 }
 
@@ -696,40 +560,7 @@ int32_t ah_gemm(const AhGemm *p) {
   if (q.in_dtype == AH_F32) {
     int vec_a = aligned16(q.a) && (q.lda % 4 == 0) && (q.stride_a % 4 == 0);
     int vec_b = aligned16(q.b) && (q.ldb % 4 == 0) && (q.stride_b % 4 == 0);
-    auto run_f32 = [&](const GemmArgs &g, int nb, int vc) -> int32_t {
-      switch (q.layout) {
-        case AH_GEMM_NN: return launch_f32<AH_GEMM_NN>(g, nb, q.out_dtype, vec_a, vec_b, vc);
-        case AH_GEMM_NT: return launch_f32<AH_GEMM_NT>(g, nb, q.out_dtype, vec_a, vec_b, vc);
-        default: return launch_f32<AH_GEMM_TN>(g, nb, q.out_dtype, vec_a, vec_b, vc);
-      }
-    };
-    // Split-K for a long contraction with too few output tiles to fill the chip (weight gradients: K = tokens): the
-    // slices run as batch entries of the same kernel (batch strides step along K) into a workspace [slices][M][N], which
-    // is then summed in fixed order.
-    int64_t tiles = cdiv(q.m, F_BM) * cdiv(q.n, F_BN);
-    if (batch == 1 && q.out_dtype == AH_F32 && (q.epilogue == AH_EPI_NONE || q.epilogue == AH_EPI_ACCUM) && tiles < num_cus() && q.k >= 2048 &&
-        (q.m * q.n) % 4 == 0 && q.n % 4 == 0 && vec_c) {
-      int s = (int)cdiv(2ll * num_cus(), tiles);
-      if (s > 32) s = 32;
-      while (s > 1 && (q.k % (s * 4) != 0 || q.k / s < 512)) s--;
-      if (s > 1) {
-        ah_ptr ws = 0;
-        int32_t rc = ah_alloc((uint64_t)s * q.m * q.n * 4, &ws);
-        if (rc) return rc;
-        GemmArgs gs = ga;
-        int64_t ks = q.k / s;
-        gs.K = (int)ks; gs.ksplit = (int)ks;
-        gs.sa = q.layout == AH_GEMM_TN ? ks * q.lda : ks;
-        gs.sb = q.layout == AH_GEMM_NT ? ks : ks * q.ldb;
-        gs.c = dp<void>(ws); gs.ldc = q.n; gs.sc = q.m * q.n; gs.epi = AH_EPI_NONE;
-        rc = run_f32(gs, s, 1);
-        if (rc == AH_OK) rc = ah::splitk_reduce(dp<const float>(ws), (float *)ga.c, s, ga.M, ga.N, ga.ldc, q.epilogue == AH_EPI_ACCUM);
-        note_gemm_split(s);
-        int32_t rf = ah_free(ws);
-        return rc ? rc : rf;
-      }
-    }
-    return run_f32(ga, batch, vec_c);
+    return ah::gemm_f32(ga, q.layout, batch, q.out_dtype, vec_a, vec_b, vec_c);
   }
 
   AH_ARG(q.k % 8 == 0, "ah_gemm: bf16 contraction length %lld must be a multiple of 8", (long long)q.k);

@@ -27,7 +27,7 @@ struct GemmArgs {
   int64_t lda, ldb, ldc;
   int64_t sa, sb, sc;  // batch strides (elements)
   int epi;
-  int ksplit, nsplit;  // split-K (bf16 direct kernel only): K elements per split, number of splits (1 = off)
+  int ksplit, nsplit;  // split-K (bf16 direct kernel, fp32 tiles): K elements per split, number of splits (1 = off)
   float *sumsq;        // grouped launches that also sum the squares of what they store: the block's four slots (one per wave)
   // Planes (the large-tile bf16 kernel with a k-contiguous A only; off by default).  C: columns [p n, (p + 1) n) with
   // n = c_plane_n live c_plane_adj ELEMENTS further per p than in one [M, ldc] matrix.  A: k-tiles [p t, (p + 1) t) with
@@ -279,6 +279,8 @@ __device__ __forceinline__ void store_tiles(const GemmArgs &g, int64_t cbase, in
 }
 
 
+// gemm_f32.hip: fp32 operands; vec_a / vec_b / vec_c: the rows of that matrix are 16-byte aligned (vec_c: of aux too)
+int32_t gemm_f32(const GemmArgs &ga, int layout, int batch, int out_dtype, int vec_a, int vec_b, int vec_c);
 // gemm_bf16.hip
 int32_t gemm_bf16_direct(const GemmArgs &ga, int layout, int batch, int out_dtype);
 bool gemm_bf16_takes_large_tile(const GemmArgs &ga, int layout);       // would gemm_bf16_direct run it on the 256-row tile kernel (batch 1)

@@ -865,6 +865,64 @@ def test_gemm_f32_long_contraction_split_k(B, M, K, N):
     assert np.max(np.abs(c.data.reshape(M, N) - (want + c0))) <= 2e-6 * K ** 0.5 * scale
 
 
+def _gemm_f32(B, layout, a, b, c0=None, pad=(0, 0, 0)):
+    """One fp32 product through ah_gemm on buffers whose rows are `pad` elements longer than they need to be; returns [M, N]."""
+    import ctypes
+    from alpha2_amd import _ffi as ffi
+    (M, K), N = a.shape, b.shape[1]
+    wide = lambda x, n: np.ascontiguousarray(np.pad(x, ((0, 0), (0, n)), constant_values=np.nan))
+    A, Bm, c = wide(a.T if layout == ffi.GEMM_TN else a, pad[0]), wide(b.T if layout == ffi.GEMM_NT else b, pad[1]), wide(np.zeros((M, N), np.float32) if c0 is None else c0, pad[2])
+    ta, tb, tc = dev(B, A), dev(B, Bm), dev(B, c)
+    g = ffi.AhGemm(layout, ffi.F32, ffi.F32, ffi.EPI_NONE if c0 is None else ffi.EPI_ACCUM, M, N, K, A.shape[1], Bm.shape[1], c.shape[1], 1, 0, 0, 0,
+                   B._ptr(ta), B._ptr(tb), B._ptr(tc), 0)
+    ffi.check(B.lib.ah_gemm(ctypes.byref(g)))
+    B._dirty(tc)
+    out = tc.data.reshape(c.shape)
+    assert np.isnan(out[:, N:]).all()                           # nothing written beside the result
+    return out[:, :N]
+
+
+# sizes one off the tiles (32, 64, 128, 256), contractions one off the 16 of a step, with and without slices, and each kernel of the dispatch
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (33, 31, 17), (64, 64, 16), (65, 129, 15), (127, 260, 1000), (384, 128, 1030), (700, 256, 4750), (1100, 520, 33),
+                                   (2100, 1300, 130), (4097, 640, 64), (8200, 3100, 50)])
+@pytest.mark.parametrize("pad", [(0, 0, 0), (1, 3, 2), (4, 8, 4)])
+def test_gemm_f32_edges_of_tiles_slices_and_strides(B, M, N, K, pad):
+    """Every layout against a float64 product.  Bound: the six partial products of a step of 16 are rounded into the sum one after
+    the other (0.375 K roundings, at most one more per slice, wave or partial product), and what the split leaves out is 2^-24 of a term."""
+    from alpha2_amd import _ffi as ffi
+    g = np.random.default_rng(M + N + K)
+    a, b = g.standard_normal((M, K), dtype=np.float32), g.standard_normal((K, N), dtype=np.float32)
+    want, size = a.astype(np.float64) @ b.astype(np.float64), np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
+    bound = (6 * -(-K // 16) + 40) * 2.0 ** -24 * size
+    for layout in (ffi.GEMM_NN, ffi.GEMM_NT, ffi.GEMM_TN):
+        assert np.all(np.abs(_gemm_f32(B, layout, a, b, pad=pad) - want) <= bound), (layout, B.lastGemmKernel())
+    c0 = g.standard_normal((M, N), dtype=np.float32)
+    got = _gemm_f32(B, ffi.GEMM_TN, a, b, c0, pad)
+    assert np.all(np.abs(got - (want + c0)) <= bound + 2.0 ** -23 * np.abs(want + c0)), B.lastGemmKernel()
+
+
+@pytest.mark.parametrize("M,N,K", [(40, 40, 40), (500, 300, 512), (300, 2000, 36), (4000, 1200, 64)])
+def test_gemm_f32_with_numbers_the_split_cannot_hold(B, M, N, K):
+    """Infinities, NaNs and numbers above the largest bf16 (3.39e38): the result is the fp32 product's, entry by entry, also in the
+    tiles' other rows; numbers down to 1e-30 lose nothing."""
+    from alpha2_amd import _ffi as ffi
+    g = np.random.default_rng(K)
+    a, b = g.standard_normal((M, K), dtype=np.float32), np.abs(g.standard_normal((K, N), dtype=np.float32)) + np.float32(0.1)
+    a[3, 5], a[7, 1], a[M - 1, 0] = np.inf, np.nan, -np.inf
+    a[9] = 0.0
+    a[9, 2] = np.float32(3.4e38)                                # times b < 1: finite
+    b[2] = np.float32(0.25)
+    a[11] *= np.float32(1e-30)
+    with np.errstate(invalid="ignore", over="ignore"):
+        want, size = a.astype(np.float64) @ b.astype(np.float64), np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
+    fin = np.isfinite(want)
+    assert not fin[3].any() and not fin[7].any() and fin[9].all()
+    for layout in (ffi.GEMM_NN, ffi.GEMM_NT, ffi.GEMM_TN):
+        got = _gemm_f32(B, layout, a, b)
+        assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[np.isinf(want)], want[np.isinf(want)].astype(np.float32)), layout
+        assert np.all(np.abs(got[fin] - want[fin]) <= (K + 40) * 2.0 ** -24 * size[fin]), layout      # (K roundings where the fp32 instruction ran)
+
+
 def test_gemm_f32_batched_and_broadcast(B):
     a, b = rs.randn(2, 3, 40, 16).astype(np.float32), rs.randn(2, 3, 16, 24).astype(np.float32)
     assert_close(B.matmul(dev(B, a), dev(B, b)).data, O.matmul(orc(a), orc(b)).data)
