@@ -238,7 +238,7 @@ int32_t launch(const GemmArgs &ga, int batch, int out_dtype) {
 // Large outputs go to the kernel fed by global->LDS loads (gemm_bf16_dma.inc): half the L2 traffic and a third of the
 // LDS traffic per flop of the 128x128 tile.  It holds one block per CU, so what matters is how evenly the tiles fill
 // whole rounds of CUs: take 256 x 256, 256 x 192 or 256 x 128 tiles, whichever wastes least of its last round, and keep the
-// 128x128 tile of this file (two blocks per CU, finer grain) when neither fills 70 %.  Returns the tile width, 0 = the
+// tiles of this file (two blocks per CU, finer grain) when none fills 70 % and they need no second round.  Returns the tile width, 0 = the
 // 128x128 kernel.  A product with planes only gets tile widths that divide a plane of C, and always gets one.
 int pick_large_tile(const GemmArgs &ga, int batch, bool akm, bool bkm) {
   if (!(ga.M >= 256 && ga.N >= 128 && ga.ldc < (1 << 22))) return 0;      // (its epilogue addresses 128 rows of C with 31-bit byte offsets)
@@ -255,7 +255,10 @@ int pick_large_tile(const GemmArgs &ga, int batch, bool akm, bool bkm) {
   int bn = f256 >= f192 && f256 >= f128 ? 256 : f192 >= f128 ? 192 : 128;
   const double best = bn == 256 ? f256 : bn == 192 ? f192 : f128;
   if (ga.c_plane_n > 0 || ga.a_plane_adj != 0) return best > 0.0 ? bn : 0;      // planes exist on this kernel only: taken however few tiles there are
-  return best >= 0.7 ? bn : 0;
+  // More 128 x 128 tiles than CUs: some CUs run two of them, and the launch takes as long as they do; then the large tiles are faster
+  // however unevenly they fill their last round (us, 128 x 128 / chosen: 8192 x 768 x 3072 NN 63 / 48, 16384 x 384 x 384 14.6 / 11.2,
+  // 11000 x 768 x 3072 NT 94 / 65, 2304 x 2304 x 1024 TN 31 / 23, 4352 x 1024 x 1024 NT 24 / 21).
+  return best >= 0.7 || cdiv(ga.M, 128) * cdiv(ga.N, 128) * per > cus ? bn : 0;
 }
 
 template <bool AKM, bool BKM>
@@ -263,6 +266,14 @@ int32_t run(const GemmArgs &ga, int batch, int out_dtype) {
   const int bn = pick_large_tile(ga, batch, AKM, BKM);
   if (bn) return AKM ? gemm_bf16_dma_tn(ga, batch, out_dtype, bn) : BKM ? gemm_bf16_dma_nn(ga, batch, out_dtype, bn) : gemm_bf16_dma_nt(ga, batch, out_dtype, bn);
   if (ga.c_plane_n > 0 || ga.a_plane_adj != 0) return fail(AH_ERR_UNSUPPORTED, "ah_gemm_planes: this shape does not run on the large-tile kernel");
+  // An output with too few 128 x 128 tiles to give every CU one runs a CU per tile at the latency of its k-tiles, whatever the tile's
+  // size: smaller tiles, as long as there is at most one to a CU, are as many times more CUs at work, and shorter k-tiles.  Measured
+  // (us, 128 x 128 / 64 x 128 / 64 x 64): 128 x 384 x 128 5.6 / 4.1 / 3.4, 777 x 768 x 768 11.5 / 7.7 / 6.0, 777 x 768 x 3072 31.3 / 20.7 /
+  // 19.8, 2048 x 1024 x 4096 (256 tiles of 64 x 128, 512 of 64 x 64) 44.2 / 32.6 / 35.0; beyond one tile to a CU: 777 x 3072 x 768
+  // 13.5 / 14.2 / 13.3, 10240 x 384 x 1536 21.9 / 22.5 / 26.3.  The sums are the same, bit for bit.
+  const int64_t per = (int64_t)batch * ga.nsplit * cdiv(ga.M, 64);
+  if (per * cdiv(ga.N, 64) <= num_cus()) return launch<64, 64, 2, 2, AKM, BKM>(ga, batch, out_dtype);
+  if (per * cdiv(ga.N, 128) <= num_cus()) return launch<64, 128, 2, 2, AKM, BKM>(ga, batch, out_dtype);
   return launch<128, 128, 2, 2, AKM, BKM>(ga, batch, out_dtype);
 }
 

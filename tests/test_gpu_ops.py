@@ -1191,6 +1191,29 @@ def test_gemm_layouts_epilogues_dtypes(B, in_bf16, out_bf16, M, N, K):
         assert B.lib.ah_gemm(C.byref(g)) == 5 and b"not provided" in B.lib.ah_last_error()
 
 
+# one, some and all of a tile's rows; the last shape with at most one 64-wide (64 x 128) tile to a CU and the first beyond it; more
+# 128-wide tiles than CUs, whose large tiles do not fill a round
+@pytest.mark.parametrize("M,N,K,kernel", [(8, 8, 64, "<64, 64"), (72, 136, 64, "<64, 64"), (1024, 1024, 128, "<64, 64"), (1032, 1024, 128, "<64, 128"),
+                                          (2048, 1024, 192, "<64, 128"), (2056, 1024, 64, "<128, 128"), (4232, 1024, 128, "_dma<")])
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
+def test_gemm_bf16_tile_by_the_number_of_tiles(B, M, N, K, kernel, layout):
+    """Against a float64 product of the same bf16 operands; the f32 sum of K exact products is off by at most K 2^-24 of the sum of
+    their sizes, the bf16 result by 2^-9 of itself more."""
+    import ctypes
+    from alpha2_amd import _ffi as ffi
+    L = {"nn": ffi.GEMM_NN, "nt": ffi.GEMM_NT, "tn": ffi.GEMM_TN}[layout]
+    g = np.random.default_rng(M + K)
+    a, b = _bf16_round(g.standard_normal((M, K), dtype=np.float32))[0], _bf16_round(g.standard_normal((K, N), dtype=np.float32))[0]
+    A, Bm = np.ascontiguousarray(a.T if L == ffi.GEMM_TN else a), np.ascontiguousarray(b.T if L == ffi.GEMM_NT else b)
+    ta, tb = B.castStore(dev(B, A), "bf16"), B.castStore(dev(B, Bm), "bf16")
+    tc = B._new((M, N), "f32", "bf16")
+    q = ffi.AhGemm(L, ffi.BF16, ffi.BF16, ffi.EPI_NONE, M, N, K, A.shape[1], Bm.shape[1], N, 1, 0, 0, 0, B._ptr(ta), B._ptr(tb), B._ptr(tc), 0)
+    ffi.check(B.lib.ah_gemm(ctypes.byref(q)))
+    assert kernel in B.lastGemmKernel()[0], B.lastGemmKernel()
+    want, size = a.astype(np.float64) @ b.astype(np.float64), np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
+    assert np.all(np.abs(tc.data.reshape(M, N) - want) <= 2.0 ** -8 * np.abs(want) + K * 2.0 ** -24 * size)
+
+
 def test_gemm_bf16_split_k_weight_gradient(B):
     """dW = G^T X with a long token axis and few output tiles takes the split-K path (slices of the token axis into a
     workspace, summed in a fixed order by a second kernel)."""
