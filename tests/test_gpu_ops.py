@@ -481,6 +481,48 @@ def test_data_movement_bit_exact(B):
     assert_close(B.castDtype(h, "f32").data, a.reshape(-1).astype(np.float16).astype(np.float32), rel=0)
 
 
+@pytest.mark.parametrize("write", ["addInplace", "scaleInplace", "sgdStep", "data", "raw view"])
+@pytest.mark.parametrize("side", ["original", "clone"])
+def test_clone_shares_its_block_until_either_side_is_written(B, write, side):
+    """Whatever writes one side in place leaves the other as it was; views go on naming what their own side holds; the block lives
+    as long as one of the two does."""
+    a = rs.randn(6, 20).astype(np.float32)
+    x = dev(B, a)
+    B._ptr(x)
+    y, live = B.clone(x), B._stats().live_allocs
+    z = B.clone(B.reshape(y, (20, 6)))
+    assert B._ptr(y) == B._ptr(x) == B._ptr(z) and B._stats().live_allocs == live
+    w, other = (x, y) if side == "original" else (y, x)
+    view = B.reshape(w, (120,))
+    if write == "addInplace":
+        B.addInplace(w, B.clone(other))                         # the addend shares the block that is left
+        want = a + a
+    elif write == "scaleInplace":
+        B.scaleInplace(w, 0.5)
+        want = a * np.float32(0.5)
+    elif write == "sgdStep":
+        B.sgdStep(w, other, 0.25)
+        want = a - np.float32(0.25) * a
+    elif write == "data":
+        w.data = np.arange(120, dtype=np.float32)
+        B._ptr(w)
+        want = np.arange(120, dtype=np.float32)
+    else:
+        B.scaleInplace(view, 2.0)
+        want = a * np.float32(2.0)
+        B._dirty(w)
+    view._host_valid = False
+    want = want.reshape(-1)
+    assert np.array_equal(w.data, want) and np.array_equal(view.data, want)
+    B.releaseGpuTensor(w), B.releaseGpuTensor(view)
+    assert np.array_equal(other.data, a.reshape(-1)) and np.array_equal(z.data, a.reshape(-1))
+    B.releaseGpuTensor(other)
+    z._host_valid = False
+    assert np.array_equal(z.data, a.reshape(-1))                # the last of the block's owners
+    part = B.clone(B._view(z, (3, 6), 24))                      # a piece of a buffer is copied
+    assert B._ptr(part) != B._ptr(z) and np.array_equal(part.data, a.reshape(-1)[6:24])
+
+
 def test_embedding_fwd_bwd(B):
     V, D = 257, 48
     w = rs.randn(V, D).astype(np.float32)
