@@ -121,6 +121,127 @@ __global__ __launch_bounds__(256) void k_flash_fwd_f32(FlashArgs a) {
   }
 }
 
+// The same for few blocks of 128 queries: a block owns 32 query rows and its W waves share the keys, wave w taking the tiles
+// w, w + W, ... with a running max / sum / output of its own; the W of them are joined in LDS at the end, in the order of the waves.
+// K and V go from memory straight into the operand registers: the contraction over features may take them in any order as long as
+// both operands do, so half lane/32 owns the features (D/2)*half .. and reads 16 bytes of its key's row at a time; a V operand is 32
+// features of one key side by side.  No LDS and no barrier before the join.
+// What bounded the kernel above there is its serial chain: a tile is 4096 cycles of matrix instructions at D = 64 after two barriers
+// and an unhidden load, T / 32 tiles one after the other on a few CUs.
+template <int D, int W>
+__global__ __launch_bounds__(64 * W) void k_flash_fwd_f32_keys(FlashArgs a) {
+  constexpr int DB = D / 32, H4 = D / 8;
+  __shared__ float4 part[W * 4 * 64];
+  __shared__ float Ms[W * 32], Lsum[W * 32];
+  int bh, xblk;
+  flash_block(bh, xblk, flash_head_group(a.T, D, 4));
+  xblk = gridDim.x - 1 - xblk;                                     // longest (latest) query blocks are scheduled first
+  const int b = bh / a.H, h = bh % a.H;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 31, lk = lane >> 5;
+  const int q0 = xblk * 32, qi = q0 + lr;
+  const float *Q = (const float *)a.q + b * a.q_sb + h * a.q_sh;
+  const float *K = (const float *)a.k + b * a.k_sb + h * a.k_sh;
+  const float *V = (const float *)a.v + b * a.v_sb + h * a.v_sh;
+  const float inv_cap = a.cap > 0.f ? 1.0f / a.cap : 0.f;
+  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+  // 4 H4 features of a row, those of this half
+  auto row = [&](const float *p, float mul, float4 (&r)[H4]) {
+#pragma unroll
+    for (int i = 0; i < H4; i++) {
+      const int d = lk * (D / 2) + 4 * i;
+      r[i] = d < a.hd ? *reinterpret_cast<const float4 *>(p + d) : zero;
+      r[i].x *= mul; r[i].y *= mul; r[i].z *= mul; r[i].w *= mul;
+    }
+  };
+  float4 q[H4], k[H4];
+  row(Q + (int64_t)min(qi, a.T - 1) * a.q_st, a.scale, q);         // rows past the end repeat the last one: not stored, masked as keys
+
+  f32x16 o[DB];
+#pragma unroll
+  for (int d = 0; d < DB; d++)
+#pragma unroll
+    for (int e = 0; e < 16; e++) o[d][e] = 0.f;
+  float m = -INFINITY, l = 0.f;
+  for (int kv0 = wave * 32; kv0 <= q0; kv0 += W * 32) {
+    row(K + (int64_t)min(kv0 + lr, a.T - 1) * a.k_st, 1.0f, k);
+    float v[DB][16];
+#pragma unroll
+    for (int d = 0; d < DB; d++)
+#pragma unroll
+      for (int e = 0; e < 16; e++) {
+        const int kv = min(kv0 + 8 * (e >> 2) + 4 * lk + (e & 3), a.T - 1);
+        v[d][e] = 32 * d + lr < a.hd ? V[(int64_t)kv * a.v_st + 32 * d + lr] : 0.f;
+      }
+    f32x16 s;
+#pragma unroll
+    for (int e = 0; e < 16; e++) s[e] = 0.f;
+#pragma unroll
+    for (int i = 0; i < H4; i++) {
+      s = __builtin_amdgcn_mfma_f32_32x32x2f32(k[i].x, q[i].x, s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_32x32x2f32(k[i].y, q[i].y, s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_32x32x2f32(k[i].z, q[i].z, s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_32x32x2f32(k[i].w, q[i].w, s, 0, 0, 0);
+    }
+    float tmax = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+      const int kv = kv0 + 8 * (e >> 2) + 4 * lk + (e & 3);
+      float x = softcap_fwd(s[e], a.cap, inv_cap);
+      x = (kv > qi || kv >= a.T) ? -INFINITY : x;
+      s[e] = x;
+      tmax = fmaxf(tmax, x);
+    }
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+    const float m_new = fmaxf(m, tmax), m_use = m_new == -INFINITY ? 0.f : m_new;
+    const float alpha = expf(m - m_use);
+    float psum = 0.f;
+#pragma unroll
+    for (int e = 0; e < 16; e++) { const float p = expf(s[e] - m_use); s[e] = p; psum += p; }
+    psum += __shfl_xor(psum, 32, 64);
+    l = l * alpha + psum;
+    m = m_new;
+#pragma unroll
+    for (int d = 0; d < DB; d++)
+#pragma unroll
+      for (int e = 0; e < 16; e++) o[d][e] *= alpha;
+#pragma unroll
+    for (int d = 0; d < DB; d++)
+#pragma unroll
+      for (int e = 0; e < 16; e++) o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[d][e], s[e], o[d], 0, 0, 0);
+  }
+
+  if (lk == 0) { Ms[wave * 32 + lr] = m; Lsum[wave * 32 + lr] = l; }
+  __syncthreads();
+  float top = -INFINITY;
+#pragma unroll
+  for (int w = 0; w < W; w++) top = fmaxf(top, Ms[w * 32 + lr]);
+  const float use = top == -INFINITY ? 0.f : top;
+  float total = 0.f;
+#pragma unroll
+  for (int w = 0; w < W; w++) total += Lsum[w * 32 + lr] * expf(Ms[w * 32 + lr] - use);
+  const float factor = expf(m - use) * (total > 0.f ? 1.0f / total : 0.f);
+  if (wave == 0 && lk == 0 && qi < a.T) a.lse[((int64_t)b * a.H + h) * a.T + qi] = top + logf(total);
+  // 8 threads to a row: piece ch of its 32 features is the accumulator quarter ch / 2 of half ch % 2
+  const int r = threadIdx.x >> 3, ch = threadIdx.x & 7;
+#pragma unroll
+  for (int d = 0; d < DB; d++) {
+    if (d) __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      part[(wave * 4 + j) * 64 + lane] = make_float4(o[d][4 * j] * factor, o[d][4 * j + 1] * factor, o[d][4 * j + 2] * factor, o[d][4 * j + 3] * factor);
+    __syncthreads();
+    if (threadIdx.x < 256 && q0 + r < a.T && 32 * d + 4 * ch < a.hd) {
+      float4 sum = part[(ch >> 1) * 64 + 32 * (ch & 1) + r];
+#pragma unroll
+      for (int w = 1; w < W; w++) {
+        const float4 x = part[(w * 4 + (ch >> 1)) * 64 + 32 * (ch & 1) + r];
+        sum.x += x.x; sum.y += x.y; sum.z += x.z; sum.w += x.w;
+      }
+      *reinterpret_cast<float4 *>((float *)a.o + b * a.o_sb + h * a.o_sh + (int64_t)(q0 + r) * a.o_st + 32 * d + 4 * ch) = sum;
+    }
+  }
+}
+
 // delta[b,h,t] = sum_d dO[t,d] * O[t,d]
 template <int D>
 __global__ void k_flash_delta_f32(FlashArgs a) {
@@ -326,6 +447,20 @@ int32_t check(const AhFlash *f, bool bwd, FlashArgs &a) {
 
 template <int D>
 int32_t run_fwd(const FlashArgs &a) {
+  if constexpr (D <= 64) {
+    // Blocks of 128 queries until there is one for every CU; before that the keys go to 8 waves where that gives each at least one
+    // tile, or where all workgroups run at once.  us, 128-query blocks / keys among waves, soft cap on:
+    //   D = 64, 12 heads: T = 64 16 / 16, T = 256 46 / 23, T = 500 88 / 36, T = 1024 172 / 95; T = 1024 24 heads 176 / 122, 32 heads 178 / 157;
+    //   160 heads x T = 100 26 / 42;  D = 32, 8 heads: T = 32 7.9 / 10, T = 128 17 / 11, T = 256 32 / 14
+    // Larger heads keep the one kernel: there a call over many heads and calls over each alone give the same bits.
+    constexpr int W = 8;
+    const int64_t heads = (int64_t)a.B * a.H, blocks = cdiv(a.T, 32) * heads;
+    if (a.T > 64 && cdiv(a.T, WAVES * 32) * heads <= num_cus() && (a.T >= W * 32 || blocks <= num_cus())) {
+      ah::launch_kernel((k_flash_fwd_f32_keys<D, W>), dim3((unsigned)cdiv(a.T, 32), (unsigned)heads), dim3(64 * W), 0, a);
+      AH_LAUNCH_CHECK();
+      return AH_OK;
+    }
+  }
   dim3 grid((unsigned)cdiv(a.T, WAVES * 32), (unsigned)(a.B * a.H));
   ah::launch_kernel(k_flash_fwd_f32<D>, grid, dim3(256), 0, a);
   AH_LAUNCH_CHECK();

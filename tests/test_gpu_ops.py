@@ -1676,6 +1676,24 @@ def test_flash_attention_heads_are_independent_of_how_blocks_are_dealt_out(B, st
             assert np.array_equal(a[h], b_), (h, what)
 
 
+@pytest.mark.parametrize("BH,T,D,cap", [(1, 31, 32, 30.0), (3, 33, 64, 0.0), (12, 256, 64, 30.0), (2, 257, 64, 30.0), (2, 545, 64, 0.0), (1, 300, 40, 30.0),
+                                        (2, 161, 128, 30.0), (256, 128, 32, 30.0), (257, 128, 32, 30.0), (129, 130, 64, 30.0), (2, 2050, 32, 0.0)])
+def test_flash_attention_f32_forward_with_keys_shared_by_waves(B, BH, T, D, cap):
+    """Where one key tile, W of them and one more end, and both sides of the grid size from which blocks of 128 queries are taken.
+    A sum of T fp32 products rounds by at most T 2^-24 of its terms' sizes, 2^-24 sqrt(T) at random: 16 times that, and 1e-5 at most."""
+    q, k, v = (rs.randn(BH, T, D).astype(np.float32) for _ in range(3))
+    r = B.flashAttention(dev(B, q), dev(B, k), dev(B, v), T, 1 / math.sqrt(D), cap)
+    for h in {0, BH // 2, BH - 1}:
+        s = q[h].astype(np.float64) @ k[h].astype(np.float64).T / math.sqrt(D)
+        s = cap * np.tanh(s / cap) if cap > 0 else s
+        s = np.where(np.tril(np.ones((T, T), bool)), s, -np.inf)
+        m = s.max(1, keepdims=True)
+        e = np.exp(s - m)
+        rel = min(1e-5, 16 * 2.0 ** -24 * math.sqrt(max(T, D)))
+        assert_close(np.asarray(r["output"].data).reshape(BH, T, D)[h], e @ v[h].astype(np.float64) / e.sum(1, keepdims=True), rel=rel, what="O")
+        assert_close(np.asarray(r["lse"].data).reshape(BH, T)[h], (m + np.log(e.sum(1, keepdims=True)))[:, 0], rel=rel, what="LSE")
+
+
 @pytest.mark.parametrize("T", [256, 1024, 2048])
 @pytest.mark.parametrize("cap", [0.0, 30.0])
 def test_flash_attention_microbench_shapes(B, bwd_variant, T, cap):
