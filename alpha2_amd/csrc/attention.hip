@@ -4,7 +4,7 @@
 //   s = scale * q.k;  s = cap * tanh(s / cap) when cap > 0;  keys after the query are masked;
 //   P = softmax(s);  O = P V;  LSE = max + log(sum exp).
 //
-// fp32 path: v_mfma_f32_32x32x2_f32.  One wave owns 32 query rows (forward, dQ) or 32 key rows (dK/dV)
+// fp32 path: v_mfma_f32_32x32x2_f32 (backward up to head size 64: bf16 matrix instructions on three parts, below).  One wave owns 32 query rows (forward, dQ) or 32 key rows (dK/dV)
 // and the products are arranged so that the owned index is the accumulator COLUMN (= lane % 32):
 //   forward / dQ : S^T[kv, q] = K Q^T, so a lane holds 16 kv entries of one query row and the running
 //                  max / sum / rescale are per-lane scalars (one cross-half shuffle per tile);
@@ -258,14 +258,166 @@ __global__ void k_flash_delta_f32(FlashArgs a) {
   if (lane == 0) a.delta[row] = s;
 }
 
+// ------------------------------------------------------------------------------------------ backward on the bf16 matrix pipes
+// A value cut into three bf16 parts and six products of 32 cycles per 16 steps of a contraction, as in the fp32 products of
+// gemm_f32.hip, where sixteen halves of v_mfma_f32_32x32x2_f32 take 512.  Every accumulator that is a matrix instruction's takes
+// at most 24 of them (one 64-feature score, or one tile of 32 rows) and is then added, rounded to nearest, to an fp32 one.
+// The tile of 32 streamed rows is cut once for the four waves and laid out in LDS both ways, three planes each:
+//   rows     [row][feature]                  an operand is 8 features of a row
+//   columns  [feature][row'], row' = 16 j + 8 h + 4 i + r of row 16 j + 8 i + 4 h + r: an operand is the 8 rows whose scores the
+//            lanes of half h hold in accumulator elements 8 j .. 8 j + 7, so that those go straight into the other operand
+// 16-byte pieces are permuted within a row so that 16 lanes that read the same piece of 16 rows meet 64 different banks.
+// A result that is not finite (an operand that is infinite, NaN or rounds to infinity in bf16) has the block computed again with the
+// fp32 instruction, whose result stands.
+// (Of a number below 2^-100 the last part, below 2^-110 the second one too, loses bits to bf16's subnormals.)
+// 192 heads x 1024 x 64: dK and dV 945 -> 486 us, dQ 520 -> 316; 512 x 256 x 32: 112 -> 84 and 81 -> 60; 4 x 70 x 64: 29 -> 24 and
+// 26 -> 20.  Relative error against 64 bits at 4 x 512 x 64: dQ 4.6e-7 -> 3.7e-7, dK 6.4e-7 -> 3.8e-7, dV 6.0e-7 -> 3.3e-7.  What bounds
+// it now is vector issue: tanh, exp and the cut of scores, K and V for every 32 x 32 tile beside 3072 cycles of matrix instructions.
+struct Split2 { uint32_t h, m, l; };       // two values side by side
+__device__ __forceinline__ Split2 split2(float x0, float x1) {
+  Split2 s;
+  s.h = pack_bf16x2(x0, x1);
+  x0 -= __uint_as_float(s.h << 16);
+  x1 -= __uint_as_float(s.h & 0xffff0000u);
+  s.m = pack_bf16x2(x0, x1);
+  x0 -= __uint_as_float(s.m << 16);
+  x1 -= __uint_as_float(s.m & 0xffff0000u);
+  s.l = pack_bf16x2(x0, x1);
+  return s;
+}
+// 8 consecutive values of a contraction in the three parts
+__device__ __forceinline__ void split8(const float (&x)[8], bf16x8 (&f)[3]) {
+  uint32_t w[3][4];
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    const Split2 s = split2(x[2 * e], x[2 * e + 1]);
+    w[0][e] = s.h; w[1][e] = s.m; w[2][e] = s.l;
+  }
+#pragma unroll
+  for (int p = 0; p < 3; p++) f[p] = __builtin_bit_cast(bf16x8, make_uint4(w[p][0], w[p][1], w[p][2], w[p][3]));
+}
+// acc += the six products, the smallest first; element (row of a, column of b)
+__device__ __forceinline__ void mfma6(const bf16x8 (&a)[3], const bf16x8 (&b)[3], f32x16 &acc) {
+  constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+  for (int p = 0; p < 6; p++) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[PA[p]], b[PB[p]], acc, 0, 0, 0);
+}
+template <int D>
+struct SplitTile {                          // D = 32 or 64
+  static constexpr int F = D / 32, PLANE = 64 * D, BYTES = 3 * PLANE;      // either layout
+  // A thread's patch of the tile: rows 4 (t / 32) .. + 3, features F (t % 32) ..
+  static __device__ __forceinline__ void load(float (&x)[4][F], const float *__restrict__ base, int64_t st, int row0, int rows, int hd) {
+    const int g = threadIdx.x >> 5, f = F * (threadIdx.x & 31);
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int row = row0 + 4 * g + r;
+      const bool in = row < rows && f < hd;
+      const float *p = base + (int64_t)row * st + f;
+      if (F == 2) {
+        const float2 v = in ? *reinterpret_cast<const float2 *>(p) : make_float2(0.f, 0.f);
+        x[r][0] = v.x; x[r][F - 1] = v.y;
+      } else {
+        x[r][0] = in ? p[0] : 0.f;
+      }
+    }
+  }
+  static __device__ __forceinline__ int row_ofs(int row, int chunk) { return row * 2 * D + ((chunk ^ ((row * D >> 7) & (D / 8 - 1))) << 4); }
+  static __device__ __forceinline__ int col_ofs(int d, int chunk) { return d * 64 + ((chunk ^ ((d >> 2) & 3)) << 4); }
+  static __device__ __forceinline__ uint32_t lows(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x05040100u); }
+  static __device__ __forceinline__ uint32_t highs(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
+  // into the layouts that are asked for
+  template <bool ROWS, bool COLS>
+  static __device__ __forceinline__ void put(const float (&x)[4][F], float mul, char *rows, char *cols) {
+    const int g = threadIdx.x >> 5, f = F * (threadIdx.x & 31);
+    Split2 s[F][2];                         // rows (0, 1) and (2, 3) of a feature
+#pragma unroll
+    for (int d = 0; d < F; d++)
+#pragma unroll
+      for (int i = 0; i < 2; i++) s[d][i] = split2(x[2 * i][d] * mul, x[2 * i + 1][d] * mul);
+#pragma unroll
+    for (int p = 0; p < 3; p++) {
+      auto part = [&](int d, int i) { return p == 0 ? s[d][i].h : p == 1 ? s[d][i].m : s[d][i].l; };
+      if (COLS) {
+        const int chunk = 2 * (g >> 2) + (g & 1), half = 8 * ((g >> 1) & 1);
+#pragma unroll
+        for (int d = 0; d < F; d++) *reinterpret_cast<uint2 *>(cols + p * PLANE + col_ofs(f + d, chunk) + half) = make_uint2(part(d, 0), part(d, 1));
+      }
+      if (ROWS) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          char *q = rows + p * PLANE + row_ofs(4 * g + r, f >> 3) + (f & 7) * 2;
+          const uint32_t a = part(0, r >> 1), b = part(F - 1, r >> 1);
+          if (F == 2) *reinterpret_cast<uint32_t *>(q) = r & 1 ? highs(a, b) : lows(a, b);
+          else *reinterpret_cast<uint16_t *>(q) = (uint16_t)(r & 1 ? a >> 16 : a);
+        }
+      }
+    }
+  }
+  // 8 features 16 step + 8 half of row lane % 32; 8 rows (elements 8 j .. + 7 of the half) of feature d
+  static __device__ __forceinline__ void get_row(const char *rows, int row, int chunk, bf16x8 (&f)[3]) {
+#pragma unroll
+    for (int p = 0; p < 3; p++) f[p] = *reinterpret_cast<const bf16x8 *>(rows + p * PLANE + row_ofs(row, chunk));
+  }
+  static __device__ __forceinline__ void get_col(const char *cols, int d, int chunk, bf16x8 (&f)[3]) {
+#pragma unroll
+    for (int p = 0; p < 3; p++) f[p] = *reinterpret_cast<const bf16x8 *>(cols + p * PLANE + col_ofs(d, chunk));
+  }
+  // the wave's own row, features 16 step + 8 half .. + 7
+  static __device__ __forceinline__ void whole(const float *row, bool live, float mul, int hd, int lk, float (&x)[D / 16][8]) {
+#pragma unroll
+    for (int i = 0; i < D / 16; i++) {
+      const int d = 16 * i + 8 * lk;
+      float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
+      if (live && d < hd) { a = *reinterpret_cast<const float4 *>(row + d); b = *reinterpret_cast<const float4 *>(row + d + 4); }
+      x[i][0] = a.x * mul; x[i][1] = a.y * mul; x[i][2] = a.z * mul; x[i][3] = a.w * mul;
+      x[i][4] = b.x * mul; x[i][5] = b.y * mul; x[i][6] = b.z * mul; x[i][7] = b.w * mul;
+    }
+  }
+  static __device__ __forceinline__ void own(const float *row, bool live, float mul, int hd, int lk, bf16x8 (&f)[D / 16][3]) {
+    float x[D / 16][8];
+    whole(row, live, mul, hd, lk, x);
+#pragma unroll
+    for (int i = 0; i < D / 16; i++) split8(x[i], f[i]);
+  }
+  // acc[d][.] += columns (features) x the scores in x
+  static __device__ __forceinline__ void contract_rows(const char *cols, const f32x16 &x, int lr, int lk, f32x16 (&acc)[F]) {
+    bf16x8 b[2][3];
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      const float v[8] = {x[8 * j], x[8 * j + 1], x[8 * j + 2], x[8 * j + 3], x[8 * j + 4], x[8 * j + 5], x[8 * j + 6], x[8 * j + 7]};
+      split8(v, b[j]);
+    }
+#pragma unroll
+    for (int d = 0; d < F; d++) {
+      f32x16 t;
+#pragma unroll
+      for (int e = 0; e < 16; e++) t[e] = 0.f;
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        bf16x8 a[3];
+        get_col(cols, 32 * d + lr, 2 * j + lk, a);
+        mfma6(a, b[j], t);
+      }
+#pragma unroll
+      for (int e = 0; e < 16; e++) acc[d][e] += t[e];
+    }
+  }
+};
+template <int N>
+__device__ __forceinline__ bool all_finite(const f32x16 (&acc)[N]) {
+  float z = 0.f;
+#pragma unroll
+  for (int d = 0; d < N; d++)
+#pragma unroll
+    for (int e = 0; e < 16; e++) z = __builtin_fmaf(acc[d][e], 0.f, z);      // 0 unless one is infinite or NaN
+  return z == 0.f;
+}
+
 // ------------------------------------------------------------------------------------------ dQ
 template <int D>
-__global__ __launch_bounds__(256) void k_flash_dq_f32(FlashArgs a) {
+__device__ void flash_dq_exact(const FlashArgs &a, int bh, int xblk, float *smem) {
   constexpr int P = D + 1, DB = D / 32;
-  __shared__ float Ks[BC * P], Vs[BC * P];
-  int bh, xblk;
-  flash_block(bh, xblk, flash_head_group(a.T, D, 4));
-  xblk = gridDim.x - 1 - xblk;                                     // longest (latest) query blocks are scheduled first
+  float *Ks = smem, *Vs = Ks + BC * P;
   int b = bh / a.H, h = bh % a.H;
   int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 31, lk = lane >> 5;
   int q0 = xblk * (WAVES * 32) + wave * 32, qi = q0 + lr;
@@ -333,13 +485,92 @@ __global__ __launch_bounds__(256) void k_flash_dq_f32(FlashArgs a) {
   }
 }
 
-// ------------------------------------------------------------------------------------------ dK, dV
+// Four waves of 32 queries.  Head sizes over 64 keep the fp32 instruction: their operands do not fit the registers in three parts.
 template <int D>
-__global__ __launch_bounds__(256) void k_flash_dkv_f32(FlashArgs a) {
-  constexpr int P = D + 1, DB = D / 32;
-  __shared__ float Qs[BC * P], dOs[BC * P], Ls[BC], Ds[BC];
+__global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_dq_f32(FlashArgs a) {
+  constexpr int EXACT = 2 * BC * (D + 1) * 4;
   int bh, xblk;
   flash_block(bh, xblk, flash_head_group(a.T, D, 4));
+  xblk = gridDim.x - 1 - xblk;                                     // longest (latest) query blocks are scheduled first
+  if constexpr (D > 64) {
+    __shared__ float smem[EXACT / 4];
+    flash_dq_exact<D>(a, bh, xblk, smem);
+  } else {
+    using S = SplitTile<D>;
+    __shared__ __attribute__((aligned(16))) char smem[3 * S::BYTES > EXACT ? 3 * S::BYTES : EXACT];
+    char *Kr = smem, *Kc = smem + S::BYTES, *Vr = smem + 2 * S::BYTES;
+    const int b = bh / a.H, h = bh % a.H;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 31, lk = lane >> 5;
+    const int q0 = xblk * (WAVES * 32) + wave * 32, qi = q0 + lr;
+    const float *K = (const float *)a.k + b * a.k_sb + h * a.k_sh;
+    const float *V = (const float *)a.v + b * a.v_sb + h * a.v_sh;
+    const float inv_cap = a.cap > 0.f ? 1.0f / a.cap : 0.f;
+    const bool live = qi < a.T;
+    bf16x8 q[D / 16][3], go[D / 16][3];
+    S::own((const float *)a.q + b * a.q_sb + h * a.q_sh + (int64_t)qi * a.q_st, live, a.scale, a.hd, lk, q);
+    S::own((const float *)a.d_o + b * a.o_sb + h * a.o_sh + (int64_t)qi * a.o_st, live, 1.0f, a.hd, lk, go);
+    const int64_t srow = ((int64_t)b * a.H + h) * a.T + qi;
+    const float lse = live ? a.lse[srow] : 0.f, delta = live ? a.delta[srow] : 0.f;
+    f32x16 dq[S::F];
+#pragma unroll
+    for (int d = 0; d < S::F; d++)
+#pragma unroll
+      for (int e = 0; e < 16; e++) dq[d][e] = 0.f;
+    const int end = min(a.T, (xblk + 1) * (WAVES * 32));
+    float kx[4][S::F], vx[4][S::F];
+    S::load(kx, K, a.k_st, 0, a.T, a.hd);
+    S::load(vx, V, a.v_st, 0, a.T, a.hd);
+    for (int kv0 = 0; kv0 < end; kv0 += BC) {
+      __syncthreads();
+      S::template put<true, true>(kx, 1.0f, Kr, Kc);
+      S::template put<true, false>(vx, 1.0f, Vr, nullptr);
+      S::load(kx, K, a.k_st, kv0 + BC, a.T, a.hd);                 // the next tile, while this one is multiplied; rows past the end read as zero
+      S::load(vx, V, a.v_st, kv0 + BC, a.T, a.hd);
+      __syncthreads();
+      if (kv0 > q0 + 31) continue;                                 // whole tile is in this wave's future (uniform per wave)
+      f32x16 s, dp;
+#pragma unroll
+      for (int e = 0; e < 16; e++) s[e] = dp[e] = 0.f;
+#pragma unroll
+      for (int i = 0; i < D / 16; i++) {
+        bf16x8 f[3];
+        S::get_row(Kr, lr, 2 * i + lk, f);
+        mfma6(f, q[i], s);
+        S::get_row(Vr, lr, 2 * i + lk, f);
+        mfma6(f, go[i], dp);
+      }
+#pragma unroll
+      for (int e = 0; e < 16; e++) {
+        const int kv = kv0 + 8 * (e >> 2) + 4 * lk + (e & 3);
+        const float sc = softcap_fwd(s[e], a.cap, inv_cap);
+        const float p = (kv > qi || kv >= a.T || !live) ? 0.f : expf(sc - lse);
+        float ds = p * (dp[e] - delta);
+        if (a.cap > 0.f) { const float t = sc * inv_cap; ds *= (1.0f - t * t); }
+        s[e] = ds * a.scale;
+      }
+      S::contract_rows(Kc, s, lr, lk, dq);
+    }
+    if (__syncthreads_or(!all_finite<S::F>(dq))) {
+      flash_dq_exact<D>(a, bh, xblk, (float *)smem);
+      return;
+    }
+    if (live) {
+      float *dQ = (float *)a.dq + b * a.q_sb + h * a.q_sh + (int64_t)qi * a.q_st;
+#pragma unroll
+      for (int d = 0; d < S::F; d++)
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+          if (32 * d + 8 * j + 4 * lk < a.hd)
+            *reinterpret_cast<float4 *>(dQ + 32 * d + 8 * j + 4 * lk) = make_float4(dq[d][4 * j], dq[d][4 * j + 1], dq[d][4 * j + 2], dq[d][4 * j + 3]);
+    }
+  }
+}
+
+// ------------------------------------------------------------------------------------------ dK, dV
+template <int D>
+__device__ void flash_dkv_exact(const FlashArgs &a, int bh, int xblk, float *smem) {
+  constexpr int P = D + 1, DB = D / 32;
+  float *Qs = smem, *dOs = Qs + BC * P, *Ls = dOs + BC * P, *Ds = Ls + BC;
   int b = bh / a.H, h = bh % a.H;
   int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 31, lk = lane >> 5;
   int kv_blk0 = xblk * (WAVES * 32), kv0 = kv_blk0 + wave * 32, kvi = kv0 + lr;
@@ -412,6 +643,103 @@ __global__ __launch_bounds__(256) void k_flash_dkv_f32(FlashArgs a) {
         *reinterpret_cast<float4 *>(dK + 32 * d + 8 * j + 4 * lk) = make_float4(dk[d][4 * j], dk[d][4 * j + 1], dk[d][4 * j + 2], dk[d][4 * j + 3]);
         *reinterpret_cast<float4 *>(dV + 32 * d + 8 * j + 4 * lk) = make_float4(dv[d][4 * j], dv[d][4 * j + 1], dv[d][4 * j + 2], dv[d][4 * j + 3]);
       }
+  }
+}
+
+template <int D>
+__global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_dkv_f32(FlashArgs a) {
+  constexpr int EXACT = (2 * BC * (D + 1) + 2 * BC) * 4;
+  int bh, xblk;
+  flash_block(bh, xblk, flash_head_group(a.T, D, 4));
+  if constexpr (D > 64) {
+    __shared__ float smem[EXACT / 4];
+    flash_dkv_exact<D>(a, bh, xblk, smem);
+  } else {
+    using S = SplitTile<D>;
+    constexpr int LDS = 4 * S::BYTES + 2 * BC * 4;
+    __shared__ __attribute__((aligned(16))) char smem[LDS > EXACT ? LDS : EXACT];
+    char *Qr = smem, *Qc = smem + S::BYTES, *Gr = smem + 2 * S::BYTES, *Gc = smem + 3 * S::BYTES;
+    float *Ls = (float *)(smem + 4 * S::BYTES), *Ds = Ls + BC;
+    const int b = bh / a.H, h = bh % a.H;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 31, lk = lane >> 5;
+    const int kv_blk0 = xblk * (WAVES * 32), kv0 = kv_blk0 + wave * 32, kvi = kv0 + lr;
+    const float *Q = (const float *)a.q + b * a.q_sb + h * a.q_sh;
+    const float *dO = (const float *)a.d_o + b * a.o_sb + h * a.o_sh;
+    const float inv_cap = a.cap > 0.f ? 1.0f / a.cap : 0.f;
+    const bool live = kvi < a.T;
+    // K's and V's rows stay whole and are cut where they are used: in three parts, they, the accumulators and the next tile are more
+    // registers than a wave of two per SIMD has (the empty assembler statements keep the cuts from being moved out of the loop).
+    float k[D / 16][8], v[D / 16][8];
+    S::whole((const float *)a.k + b * a.k_sb + h * a.k_sh + (int64_t)kvi * a.k_st, live, 1.0f, a.hd, lk, k);
+    S::whole((const float *)a.v + b * a.v_sb + h * a.v_sh + (int64_t)kvi * a.v_st, live, 1.0f, a.hd, lk, v);
+    f32x16 dk[S::F], dv[S::F];
+#pragma unroll
+    for (int d = 0; d < S::F; d++)
+#pragma unroll
+      for (int e = 0; e < 16; e++) { dk[d][e] = 0.f; dv[d][e] = 0.f; }
+    const int64_t srow0 = ((int64_t)b * a.H + h) * a.T;
+    float qx[4][S::F], gx[4][S::F], stat = 0.f;
+    auto load = [&](int q0) {
+      S::load(qx, Q, a.q_st, q0, a.T, a.hd);
+      S::load(gx, dO, a.o_st, q0, a.T, a.hd);
+      const int qi = q0 + (threadIdx.x & 31);
+      if (threadIdx.x < 64) stat = qi < a.T ? (threadIdx.x < 32 ? a.lse : a.delta)[srow0 + qi] : 0.f;
+    };
+    load(kv_blk0);
+    for (int q0 = kv_blk0; q0 < a.T; q0 += BC) {                   // causal: queries at or after this block's first key
+      __syncthreads();
+      S::template put<true, true>(qx, a.scale, Qr, Qc);
+      S::template put<true, true>(gx, 1.0f, Gr, Gc);
+      if (threadIdx.x < 64) Ls[threadIdx.x] = stat;                // the second 32 are Ds
+      load(q0 + BC);                                               // the next tile, while this one is multiplied; rows past the end read as zero
+      __syncthreads();
+      if (q0 + 31 < kv0) continue;                                 // every query of the tile precedes this wave's keys
+      f32x16 s, dp;
+#pragma unroll
+      for (int e = 0; e < 16; e++) s[e] = dp[e] = 0.f;
+#pragma unroll
+      for (int i = 0; i < D / 16; i++) {                           // rows = queries, columns = this wave's keys
+        bf16x8 f[3];
+        S::get_row(Qr, lr, 2 * i + lk, f);
+        bf16x8 u[3], w[3];
+#pragma unroll
+        for (int e = 0; e < 8; e++) asm volatile("" : "+v"(k[i][e]), "+v"(v[i][e]));
+        split8(k[i], u);
+        split8(v[i], w);
+        mfma6(f, u, s);
+        S::get_row(Gr, lr, 2 * i + lk, f);
+        mfma6(f, w, dp);
+      }
+      f32x16 pm;
+#pragma unroll
+      for (int e = 0; e < 16; e++) {
+        const int qr = 8 * (e >> 2) + 4 * lk + (e & 3), qi = q0 + qr;
+        const float sc = softcap_fwd(s[e], a.cap, inv_cap);
+        const float p = (kvi > qi || qi >= a.T || !live) ? 0.f : expf(sc - Ls[qr]);
+        float ds = p * (dp[e] - Ds[qr]);
+        if (a.cap > 0.f) { const float t = sc * inv_cap; ds *= (1.0f - t * t); }
+        pm[e] = p;
+        s[e] = ds;                                                 // Qc already carries `scale`, so dK = dS^T (scale*Q)
+      }
+      S::contract_rows(Gc, pm, lr, lk, dv);
+      S::contract_rows(Qc, s, lr, lk, dk);
+    }
+    if (__syncthreads_or(!all_finite<S::F>(dk) || !all_finite<S::F>(dv))) {
+      flash_dkv_exact<D>(a, bh, xblk, (float *)smem);
+      return;
+    }
+    if (live) {
+      float *dK = (float *)a.dk + b * a.k_sb + h * a.k_sh + (int64_t)kvi * a.k_st;
+      float *dV = (float *)a.dv + b * a.v_sb + h * a.v_sh + (int64_t)kvi * a.v_st;
+#pragma unroll
+      for (int d = 0; d < S::F; d++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          if (32 * d + 8 * j + 4 * lk >= a.hd) continue;
+          *reinterpret_cast<float4 *>(dK + 32 * d + 8 * j + 4 * lk) = make_float4(dk[d][4 * j], dk[d][4 * j + 1], dk[d][4 * j + 2], dk[d][4 * j + 3]);
+          *reinterpret_cast<float4 *>(dV + 32 * d + 8 * j + 4 * lk) = make_float4(dv[d][4 * j], dv[d][4 * j + 1], dv[d][4 * j + 2], dv[d][4 * j + 3]);
+        }
+    }
   }
 }
 

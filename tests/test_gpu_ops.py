@@ -1694,6 +1694,64 @@ def test_flash_attention_f32_forward_with_keys_shared_by_waves(B, BH, T, D, cap)
         assert_close(np.asarray(r["lse"].data).reshape(BH, T)[h], (m + np.log(e.sum(1, keepdims=True)))[:, 0], rel=rel, what="LSE")
 
 
+def _attention_grads_64(q, k, v, do, scale, cap):
+    """dQ, dK, dV of one head in 64 bits, by the kernels' own formulas (an infinite score has a capped value and no slope)."""
+    q, k, v, do = (x.astype(np.float64) for x in (q, k, v, do))
+    with np.errstate(invalid="ignore"):
+        s = (q * scale) @ k.T
+        t = np.tanh(s / cap) if cap > 0 else np.zeros_like(s)
+        s = np.where(np.tril(np.ones_like(s, dtype=bool)), cap * t if cap > 0 else s, -np.inf)
+        p = np.exp(s - s.max(1, keepdims=True))
+        p /= p.sum(1, keepdims=True)
+        ds = p * (do @ v.T - (do * (p @ v)).sum(1, keepdims=True)) * (1 - t * t) * scale
+        return ds @ k, ds.T @ q, p.T @ do
+
+
+@pytest.mark.parametrize("BH,T,D,cap", [(1, 1, 64, 30.0), (2, 32, 32, 30.0), (3, 33, 64, 0.0), (2, 127, 40, 30.0), (2, 129, 24, 30.0), (9, 160, 64, 30.0), (1, 1057, 64, 30.0)])
+def test_flash_attention_f32_backward_in_bf16_parts(B, BH, T, D, cap):
+    """Edges of the 32-row tiles and 128-row blocks.  Three parts hold an fp32 value; what six products leave out, 3 x 2^-26 of a product,
+    is under the rounding of its sum: 2^-24 sqrt(T) of the terms' sizes at random, 64 times that with the cancellation in dP - delta."""
+    q, k, v, do = (rs.randn(BH, T, D).astype(np.float32) for _ in range(4))
+    Q, K, V, scale = dev(B, q), dev(B, k), dev(B, v), 1 / math.sqrt(D)
+    r = B.flashAttention(Q, K, V, T, scale, cap)
+    g = B.flashAttentionBackward(Q, K, V, r["output"], dev(B, do), r["lse"], T, scale, cap)
+    rel = 64 * 2.0 ** -24 * math.sqrt(max(T, D))
+    for h in {0, BH - 1}:
+        for name, want in zip(("dQ", "dK", "dV"), _attention_grads_64(q[h], k[h], v[h], do[h], scale, cap)):
+            assert_close(np.asarray(g[name].data).reshape(BH, T, D)[h], want, rel=rel, what=name, scale=float(np.abs(do).max() * np.abs(v).max()) if T < 4 else 0.0)
+
+
+def test_flash_attention_f32_backward_of_values_a_bf16_part_cannot_hold(B):
+    """An infinite query feature saturates its row's scores: its gradients are zero where nothing multiplies the infinity itself.  A value
+    that only rounds to infinity in bf16 gives what fp32 gives.  (The small feature is 1e-30: of a number x below 2^-100 = 8e-31 the last
+    part, 2^-16 x .. 2^-24 x, begins to reach bf16's subnormals under 2^-126, and at 1e-36 the second, 2^-8 x, is one.)"""
+    T, D, cap, scale = 200, 64, 30.0, 0.125
+    q, k, v, do = (rs.randn(1, T, D).astype(np.float32) for _ in range(4))
+
+    def run(q, v, do):
+        Q, K, V = dev(B, q), dev(B, k), dev(B, v)
+        r = B.flashAttention(Q, K, V, T, scale, cap)
+        g = B.flashAttentionBackward(Q, K, V, r["output"], dev(B, do), r["lse"], T, scale, cap)
+        return [np.asarray(g[n].data).reshape(T, D) for n in ("dQ", "dK", "dV")], _attention_grads_64(q[0], k[0], v[0], do[0], scale, cap)
+
+    infinite = q.copy()
+    infinite[0, 40, 3] = np.inf
+    (dq, dk, dv), (wq, wk, wv) = run(infinite, v, do)
+    others = np.arange(D) != 3
+    assert_close(dq, wq, what="dQ")
+    assert_close(dk[:, others], wk[:, others], what="dK")
+    assert np.isnan(dk[:41, 3]).all()
+    assert_close(dv, wv, what="dV")
+
+    large, small = v.copy(), do.copy()
+    large[0, 150, 5] = 3.4e38
+    small[0, :, 5] *= 1e-30
+    got, want = run(q, large, small)
+    for name, a, b in zip(("dQ", "dK", "dV"), got, want):
+        assert_close(a, b, what=name)
+    assert_close(got[2][:, 5] * 1e30, want[2][:, 5] * 1e30, what="dV of the small feature")
+
+
 @pytest.mark.parametrize("T", [256, 1024, 2048])
 @pytest.mark.parametrize("cap", [0.0, 30.0])
 def test_flash_attention_microbench_shapes(B, bwd_variant, T, cap):
