@@ -4,7 +4,7 @@
 //   s = scale * q.k;  s = cap * tanh(s / cap) when cap > 0;  keys after the query are masked;
 //   P = softmax(s);  O = P V;  LSE = max + log(sum exp).
 //
-// fp32 path: v_mfma_f32_32x32x2_f32 (backward up to head size 64: bf16 matrix instructions on three parts, below).  One wave owns 32 query rows (forward, dQ) or 32 key rows (dK/dV)
+// fp32 path: v_mfma_f32_32x32x2_f32 (head sizes up to 64, but for few queries forward: bf16 matrix instructions on three parts, below).  One wave owns 32 query rows (forward, dQ) or 32 key rows (dK/dV)
 // and the products are arranged so that the owned index is the accumulator COLUMN (= lane % 32):
 //   forward / dQ : S^T[kv, q] = K Q^T, so a lane holds 16 kv entries of one query row and the running
 //                  max / sum / rescale are per-lane scalars (one cross-half shuffle per tile);
@@ -37,228 +37,7 @@ __device__ __forceinline__ void load_tile_f32(float *s, const float *__restrict_
   }
 }
 
-// ------------------------------------------------------------------------------------------ forward
-template <int D>
-__global__ __launch_bounds__(256) void k_flash_fwd_f32(FlashArgs a) {
-  constexpr int P = D + 1, DB = D / 32;
-  __shared__ float Ks[BC * P], Vs[BC * P];
-  int bh, xblk;
-  flash_block(bh, xblk, flash_head_group(a.T, D, 4));
-  xblk = gridDim.x - 1 - xblk;                                     // longest (latest) query blocks are scheduled first
-  int b = bh / a.H, h = bh % a.H;
-  int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 31, lk = lane >> 5;
-  int q0 = xblk * (WAVES * 32) + wave * 32, qi = q0 + lr;
-  const float *Q = (const float *)a.q + b * a.q_sb + h * a.q_sh;
-  const float *K = (const float *)a.k + b * a.k_sb + h * a.k_sh;
-  const float *V = (const float *)a.v + b * a.v_sb + h * a.v_sh;
-  float inv_cap = a.cap > 0.f ? 1.0f / a.cap : 0.f;
-
-  float qreg[D / 2];                                  // Q[qi][2i + lk] * scale
-#pragma unroll
-  for (int i = 0; i < D / 2; i++) qreg[i] = qi < a.T && 2 * i + lk < a.hd ? Q[(int64_t)qi * a.q_st + 2 * i + lk] * a.scale : 0.f;
-
-  f32x16 o[DB];
-#pragma unroll
-  for (int d = 0; d < DB; d++)
-#pragma unroll
-    for (int e = 0; e < 16; e++) o[d][e] = 0.f;
-  float m = -INFINITY, l = 0.f;
-
-  int q_block_end = min(a.T, (xblk + 1) * (WAVES * 32));   // causal: keys < q_block_end
-  for (int kv0 = 0; kv0 < q_block_end; kv0 += BC) {
-    __syncthreads();
-    load_tile_f32<D>(Ks, K, a.k_st, kv0, a.T, 1.0f, a.hd);
-    load_tile_f32<D>(Vs, V, a.v_st, kv0, a.T, 1.0f, a.hd);
-    __syncthreads();
-    if (kv0 > q0 + 31) continue;                      // whole tile is in this wave's future (uniform per wave)
-    f32x16 s;
-#pragma unroll
-    for (int e = 0; e < 16; e++) s[e] = 0.f;
-#pragma unroll
-    for (int i = 0; i < D / 2; i++) s = __builtin_amdgcn_mfma_f32_32x32x2f32(Ks[lr * P + 2 * i + lk], qreg[i], s, 0, 0, 0);
-    float tmax = -INFINITY;
-#pragma unroll
-    for (int e = 0; e < 16; e++) {
-      int kv = kv0 + 8 * (e >> 2) + 4 * lk + (e & 3);
-      float x = softcap_fwd(s[e], a.cap, inv_cap);
-      x = (kv > qi || kv >= a.T) ? -INFINITY : x;
-      s[e] = x;
-      tmax = fmaxf(tmax, x);
-    }
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-    float m_new = fmaxf(m, tmax);
-    float m_use = m_new == -INFINITY ? 0.f : m_new;   // rows with nothing visible yet stay at zero weight
-    float alpha = expf(m - m_use);
-    float psum = 0.f;
-#pragma unroll
-    for (int e = 0; e < 16; e++) { float p = expf(s[e] - m_use); s[e] = p; psum += p; }
-    psum += __shfl_xor(psum, 32, 64);
-    l = l * alpha + psum;
-    m = m_new;
-#pragma unroll
-    for (int d = 0; d < DB; d++)
-#pragma unroll
-      for (int e = 0; e < 16; e++) o[d][e] *= alpha;
-#pragma unroll
-    for (int d = 0; d < DB; d++)
-#pragma unroll
-      for (int e = 0; e < 16; e++) {                  // MFMA (j = e/4, r = e%4): this half supplies kv row 8j + 4lk + r
-        int kvr = 8 * (e >> 2) + 4 * lk + (e & 3);
-        o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(Vs[kvr * P + 32 * d + lr], s[e], o[d], 0, 0, 0);
-      }
-  }
-  if (qi < a.T) {
-    float inv_l = l > 0.f ? 1.0f / l : 0.f;
-    float *O = (float *)a.o + b * a.o_sb + h * a.o_sh + (int64_t)qi * a.o_st;
-#pragma unroll
-    for (int d = 0; d < DB; d++)
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        float4 w = make_float4(o[d][4 * j] * inv_l, o[d][4 * j + 1] * inv_l, o[d][4 * j + 2] * inv_l, o[d][4 * j + 3] * inv_l);
-        if (32 * d + 8 * j + 4 * lk < a.hd) *reinterpret_cast<float4 *>(O + 32 * d + 8 * j + 4 * lk) = w;
-      }
-    if (lk == 0) a.lse[((int64_t)b * a.H + h) * a.T + qi] = m + logf(l);
-  }
-}
-
-// The same for few blocks of 128 queries: a block owns 32 query rows and its W waves share the keys, wave w taking the tiles
-// w, w + W, ... with a running max / sum / output of its own; the W of them are joined in LDS at the end, in the order of the waves.
-// K and V go from memory straight into the operand registers: the contraction over features may take them in any order as long as
-// both operands do, so half lane/32 owns the features (D/2)*half .. and reads 16 bytes of its key's row at a time; a V operand is 32
-// features of one key side by side.  No LDS and no barrier before the join.
-// What bounded the kernel above there is its serial chain: a tile is 4096 cycles of matrix instructions at D = 64 after two barriers
-// and an unhidden load, T / 32 tiles one after the other on a few CUs.
-template <int D, int W>
-__global__ __launch_bounds__(64 * W) void k_flash_fwd_f32_keys(FlashArgs a) {
-  constexpr int DB = D / 32, H4 = D / 8;
-  __shared__ float4 part[W * 4 * 64];
-  __shared__ float Ms[W * 32], Lsum[W * 32];
-  int bh, xblk;
-  flash_block(bh, xblk, flash_head_group(a.T, D, 4));
-  xblk = gridDim.x - 1 - xblk;                                     // longest (latest) query blocks are scheduled first
-  const int b = bh / a.H, h = bh % a.H;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 31, lk = lane >> 5;
-  const int q0 = xblk * 32, qi = q0 + lr;
-  const float *Q = (const float *)a.q + b * a.q_sb + h * a.q_sh;
-  const float *K = (const float *)a.k + b * a.k_sb + h * a.k_sh;
-  const float *V = (const float *)a.v + b * a.v_sb + h * a.v_sh;
-  const float inv_cap = a.cap > 0.f ? 1.0f / a.cap : 0.f;
-  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-  // 4 H4 features of a row, those of this half
-  auto row = [&](const float *p, float mul, float4 (&r)[H4]) {
-#pragma unroll
-    for (int i = 0; i < H4; i++) {
-      const int d = lk * (D / 2) + 4 * i;
-      r[i] = d < a.hd ? *reinterpret_cast<const float4 *>(p + d) : zero;
-      r[i].x *= mul; r[i].y *= mul; r[i].z *= mul; r[i].w *= mul;
-    }
-  };
-  float4 q[H4], k[H4];
-  row(Q + (int64_t)min(qi, a.T - 1) * a.q_st, a.scale, q);         // rows past the end repeat the last one: not stored, masked as keys
-
-  f32x16 o[DB];
-#pragma unroll
-  for (int d = 0; d < DB; d++)
-#pragma unroll
-    for (int e = 0; e < 16; e++) o[d][e] = 0.f;
-  float m = -INFINITY, l = 0.f;
-  for (int kv0 = wave * 32; kv0 <= q0; kv0 += W * 32) {
-    row(K + (int64_t)min(kv0 + lr, a.T - 1) * a.k_st, 1.0f, k);
-    float v[DB][16];
-#pragma unroll
-    for (int d = 0; d < DB; d++)
-#pragma unroll
-      for (int e = 0; e < 16; e++) {
-        const int kv = min(kv0 + 8 * (e >> 2) + 4 * lk + (e & 3), a.T - 1);
-        v[d][e] = 32 * d + lr < a.hd ? V[(int64_t)kv * a.v_st + 32 * d + lr] : 0.f;
-      }
-    f32x16 s;
-#pragma unroll
-    for (int e = 0; e < 16; e++) s[e] = 0.f;
-#pragma unroll
-    for (int i = 0; i < H4; i++) {
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(k[i].x, q[i].x, s, 0, 0, 0);
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(k[i].y, q[i].y, s, 0, 0, 0);
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(k[i].z, q[i].z, s, 0, 0, 0);
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(k[i].w, q[i].w, s, 0, 0, 0);
-    }
-    float tmax = -INFINITY;
-#pragma unroll
-    for (int e = 0; e < 16; e++) {
-      const int kv = kv0 + 8 * (e >> 2) + 4 * lk + (e & 3);
-      float x = softcap_fwd(s[e], a.cap, inv_cap);
-      x = (kv > qi || kv >= a.T) ? -INFINITY : x;
-      s[e] = x;
-      tmax = fmaxf(tmax, x);
-    }
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-    const float m_new = fmaxf(m, tmax), m_use = m_new == -INFINITY ? 0.f : m_new;
-    const float alpha = expf(m - m_use);
-    float psum = 0.f;
-#pragma unroll
-    for (int e = 0; e < 16; e++) { const float p = expf(s[e] - m_use); s[e] = p; psum += p; }
-    psum += __shfl_xor(psum, 32, 64);
-    l = l * alpha + psum;
-    m = m_new;
-#pragma unroll
-    for (int d = 0; d < DB; d++)
-#pragma unroll
-      for (int e = 0; e < 16; e++) o[d][e] *= alpha;
-#pragma unroll
-    for (int d = 0; d < DB; d++)
-#pragma unroll
-      for (int e = 0; e < 16; e++) o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[d][e], s[e], o[d], 0, 0, 0);
-  }
-
-  if (lk == 0) { Ms[wave * 32 + lr] = m; Lsum[wave * 32 + lr] = l; }
-  __syncthreads();
-  float top = -INFINITY;
-#pragma unroll
-  for (int w = 0; w < W; w++) top = fmaxf(top, Ms[w * 32 + lr]);
-  const float use = top == -INFINITY ? 0.f : top;
-  float total = 0.f;
-#pragma unroll
-  for (int w = 0; w < W; w++) total += Lsum[w * 32 + lr] * expf(Ms[w * 32 + lr] - use);
-  const float factor = expf(m - use) * (total > 0.f ? 1.0f / total : 0.f);
-  if (wave == 0 && lk == 0 && qi < a.T) a.lse[((int64_t)b * a.H + h) * a.T + qi] = top + logf(total);
-  // 8 threads to a row: piece ch of its 32 features is the accumulator quarter ch / 2 of half ch % 2
-  const int r = threadIdx.x >> 3, ch = threadIdx.x & 7;
-#pragma unroll
-  for (int d = 0; d < DB; d++) {
-    if (d) __syncthreads();
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-      part[(wave * 4 + j) * 64 + lane] = make_float4(o[d][4 * j] * factor, o[d][4 * j + 1] * factor, o[d][4 * j + 2] * factor, o[d][4 * j + 3] * factor);
-    __syncthreads();
-    if (threadIdx.x < 256 && q0 + r < a.T && 32 * d + 4 * ch < a.hd) {
-      float4 sum = part[(ch >> 1) * 64 + 32 * (ch & 1) + r];
-#pragma unroll
-      for (int w = 1; w < W; w++) {
-        const float4 x = part[(w * 4 + (ch >> 1)) * 64 + 32 * (ch & 1) + r];
-        sum.x += x.x; sum.y += x.y; sum.z += x.z; sum.w += x.w;
-      }
-      *reinterpret_cast<float4 *>((float *)a.o + b * a.o_sb + h * a.o_sh + (int64_t)(q0 + r) * a.o_st + 32 * d + 4 * ch) = sum;
-    }
-  }
-}
-
-// delta[b,h,t] = sum_d dO[t,d] * O[t,d]
-template <int D>
-__global__ void k_flash_delta_f32(FlashArgs a) {
-  int64_t row = blockIdx.x * (int64_t)(blockDim.x >> 6) + (threadIdx.x >> 6);
-  int64_t total = (int64_t)a.B * a.H * a.T;
-  if (row >= total) return;
-  int lane = threadIdx.x & 63;
-  int t = (int)(row % a.T), h = (int)((row / a.T) % a.H), b = (int)(row / ((int64_t)a.T * a.H));
-  const float *O = (const float *)a.o + b * a.o_sb + h * a.o_sh + (int64_t)t * a.o_st;
-  const float *dO = (const float *)a.d_o + b * a.o_sb + h * a.o_sh + (int64_t)t * a.o_st;
-  float s = 0.f;
-  for (int d = lane; d < a.hd; d += 64) s += O[d] * dO[d];
-  s = wave_sum(s);
-  if (lane == 0) a.delta[row] = s;
-}
-
-// ------------------------------------------------------------------------------------------ backward on the bf16 matrix pipes
+// ------------------------------------------------------------------------------------------ products on the bf16 matrix pipes
 // A value cut into three bf16 parts and six products of 32 cycles per 16 steps of a contraction, as in the fp32 products of
 // gemm_f32.hip, where sixteen halves of v_mfma_f32_32x32x2_f32 take 512.  Every accumulator that is a matrix instruction's takes
 // at most 24 of them (one 64-feature score, or one tile of 32 rows) and is then added, rounded to nearest, to an fp32 one.
@@ -413,6 +192,318 @@ __device__ __forceinline__ bool all_finite(const f32x16 (&acc)[N]) {
   return z == 0.f;
 }
 
+// ------------------------------------------------------------------------------------------ forward
+template <int D>
+__device__ void flash_fwd_exact(const FlashArgs &a, int bh, int xblk, float *smem) {
+  constexpr int P = D + 1, DB = D / 32;
+  float *Ks = smem, *Vs = Ks + BC * P;
+  int b = bh / a.H, h = bh % a.H;
+  int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 31, lk = lane >> 5;
+  int q0 = xblk * (WAVES * 32) + wave * 32, qi = q0 + lr;
+  const float *Q = (const float *)a.q + b * a.q_sb + h * a.q_sh;
+  const float *K = (const float *)a.k + b * a.k_sb + h * a.k_sh;
+  const float *V = (const float *)a.v + b * a.v_sb + h * a.v_sh;
+  float inv_cap = a.cap > 0.f ? 1.0f / a.cap : 0.f;
+
+  float qreg[D / 2];                                  // Q[qi][2i + lk] * scale
+#pragma unroll
+  for (int i = 0; i < D / 2; i++) qreg[i] = qi < a.T && 2 * i + lk < a.hd ? Q[(int64_t)qi * a.q_st + 2 * i + lk] * a.scale : 0.f;
+
+  f32x16 o[DB];
+#pragma unroll
+  for (int d = 0; d < DB; d++)
+#pragma unroll
+    for (int e = 0; e < 16; e++) o[d][e] = 0.f;
+  float m = -INFINITY, l = 0.f;
+
+  int q_block_end = min(a.T, (xblk + 1) * (WAVES * 32));   // causal: keys < q_block_end
+  for (int kv0 = 0; kv0 < q_block_end; kv0 += BC) {
+    __syncthreads();
+    load_tile_f32<D>(Ks, K, a.k_st, kv0, a.T, 1.0f, a.hd);
+    load_tile_f32<D>(Vs, V, a.v_st, kv0, a.T, 1.0f, a.hd);
+    __syncthreads();
+    if (kv0 > q0 + 31) continue;                      // whole tile is in this wave's future (uniform per wave)
+    f32x16 s;
+#pragma unroll
+    for (int e = 0; e < 16; e++) s[e] = 0.f;
+#pragma unroll
+    for (int i = 0; i < D / 2; i++) s = __builtin_amdgcn_mfma_f32_32x32x2f32(Ks[lr * P + 2 * i + lk], qreg[i], s, 0, 0, 0);
+    float tmax = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+      int kv = kv0 + 8 * (e >> 2) + 4 * lk + (e & 3);
+      float x = softcap_fwd(s[e], a.cap, inv_cap);
+      x = (kv > qi || kv >= a.T) ? -INFINITY : x;
+      s[e] = x;
+      tmax = fmaxf(tmax, x);
+    }
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+    float m_new = fmaxf(m, tmax);
+    float m_use = m_new == -INFINITY ? 0.f : m_new;   // rows with nothing visible yet stay at zero weight
+    float alpha = expf(m - m_use);
+    float psum = 0.f;
+#pragma unroll
+    for (int e = 0; e < 16; e++) { float p = expf(s[e] - m_use); s[e] = p; psum += p; }
+    psum += __shfl_xor(psum, 32, 64);
+    l = l * alpha + psum;
+    m = m_new;
+#pragma unroll
+    for (int d = 0; d < DB; d++)
+#pragma unroll
+      for (int e = 0; e < 16; e++) o[d][e] *= alpha;
+#pragma unroll
+    for (int d = 0; d < DB; d++)
+#pragma unroll
+      for (int e = 0; e < 16; e++) {                  // MFMA (j = e/4, r = e%4): this half supplies kv row 8j + 4lk + r
+        int kvr = 8 * (e >> 2) + 4 * lk + (e & 3);
+        o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(Vs[kvr * P + 32 * d + lr], s[e], o[d], 0, 0, 0);
+      }
+  }
+  if (qi < a.T) {
+    float inv_l = l > 0.f ? 1.0f / l : 0.f;
+    float *O = (float *)a.o + b * a.o_sb + h * a.o_sh + (int64_t)qi * a.o_st;
+#pragma unroll
+    for (int d = 0; d < DB; d++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        float4 w = make_float4(o[d][4 * j] * inv_l, o[d][4 * j + 1] * inv_l, o[d][4 * j + 2] * inv_l, o[d][4 * j + 3] * inv_l);
+        if (32 * d + 8 * j + 4 * lk < a.hd) *reinterpret_cast<float4 *>(O + 32 * d + 8 * j + 4 * lk) = w;
+      }
+    if (lk == 0) a.lse[((int64_t)b * a.H + h) * a.T + qi] = m + logf(l);
+  }
+}
+
+// Four waves of 32 queries.  192 heads x 1024 x 64: 383 us with the fp32 instruction, now 294; 48 heads 199 -> 128; 512 x 256 x 32 61 -> 48;
+// relative error against 64 bits at 4 x 512 x 64 2.0e-7 (fp32 instruction, keys among waves: 2.4e-7).  Vector issue bounds it, as in backward.
+// Head sizes over 64 keep the fp32 instruction: their operands do not fit the registers in three parts.
+template <int D>
+__global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_fwd_f32(FlashArgs a) {
+  constexpr int EXACT = 2 * BC * (D + 1) * 4;
+  int bh, xblk;
+  flash_block(bh, xblk, flash_head_group(a.T, D, 4));
+  xblk = gridDim.x - 1 - xblk;                                     // longest (latest) query blocks are scheduled first
+  if constexpr (D > 64) {
+    __shared__ float smem[EXACT / 4];
+    flash_fwd_exact<D>(a, bh, xblk, smem);
+  } else {
+    using S = SplitTile<D>;
+    __shared__ __attribute__((aligned(16))) char smem[2 * S::BYTES > EXACT ? 2 * S::BYTES : EXACT];
+    char *Kr = smem, *Vc = smem + S::BYTES;
+    const int b = bh / a.H, h = bh % a.H;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 31, lk = lane >> 5;
+    const int q0 = xblk * (WAVES * 32) + wave * 32, qi = q0 + lr;
+    const float *K = (const float *)a.k + b * a.k_sb + h * a.k_sh;
+    const float *V = (const float *)a.v + b * a.v_sb + h * a.v_sh;
+    const float inv_cap = a.cap > 0.f ? 1.0f / a.cap : 0.f;
+    bf16x8 q[D / 16][3];
+    S::own((const float *)a.q + b * a.q_sb + h * a.q_sh + (int64_t)qi * a.q_st, qi < a.T, a.scale, a.hd, lk, q);
+    f32x16 o[S::F];
+#pragma unroll
+    for (int d = 0; d < S::F; d++)
+#pragma unroll
+      for (int e = 0; e < 16; e++) o[d][e] = 0.f;
+    float m = -INFINITY, l = 0.f;
+    const int end = min(a.T, (xblk + 1) * (WAVES * 32));           // causal: keys < end
+    float kx[4][S::F], vx[4][S::F];
+    S::load(kx, K, a.k_st, 0, a.T, a.hd);
+    S::load(vx, V, a.v_st, 0, a.T, a.hd);
+    bool fine = true;
+    for (int kv0 = 0; kv0 < end; kv0 += BC) {
+      __syncthreads();
+      S::template put<true, false>(kx, 1.0f, Kr, nullptr);
+      S::template put<false, true>(vx, 1.0f, nullptr, Vc);
+      S::load(kx, K, a.k_st, kv0 + BC, a.T, a.hd);                 // the next tile, while this one is multiplied; rows past the end read as zero
+      S::load(vx, V, a.v_st, kv0 + BC, a.T, a.hd);
+      __syncthreads();
+      if (kv0 > q0 + 31) continue;                                 // whole tile is in this wave's future (uniform per wave)
+      f32x16 s[1];
+#pragma unroll
+      for (int e = 0; e < 16; e++) s[0][e] = 0.f;
+#pragma unroll
+      for (int i = 0; i < D / 16; i++) {
+        bf16x8 f[3];
+        S::get_row(Kr, lr, 2 * i + lk, f);
+        mfma6(f, q[i], s[0]);
+      }
+      fine = fine && all_finite<1>(s);                             // a maximum passes NaN by
+      float tmax = -INFINITY;
+#pragma unroll
+      for (int e = 0; e < 16; e++) {
+        const int kv = kv0 + 8 * (e >> 2) + 4 * lk + (e & 3);
+        float x = softcap_fwd(s[0][e], a.cap, inv_cap);
+        x = (kv > qi || kv >= a.T) ? -INFINITY : x;
+        s[0][e] = x;
+        tmax = fmaxf(tmax, x);
+      }
+      tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+      const float m_new = fmaxf(m, tmax), m_use = m_new == -INFINITY ? 0.f : m_new;
+      const float alpha = expf(m - m_use);
+      float psum = 0.f;
+#pragma unroll
+      for (int e = 0; e < 16; e++) { const float p = expf(s[0][e] - m_use); s[0][e] = p; psum += p; }
+      psum += __shfl_xor(psum, 32, 64);
+      l = l * alpha + psum;
+      m = m_new;
+#pragma unroll
+      for (int d = 0; d < S::F; d++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) o[d][e] *= alpha;
+      S::contract_rows(Vc, s[0], lr, lk, o);
+    }
+    if (__syncthreads_or(!fine || !all_finite<S::F>(o))) {
+      flash_fwd_exact<D>(a, bh, xblk, (float *)smem);
+      return;
+    }
+    if (qi < a.T) {
+      const float inv_l = l > 0.f ? 1.0f / l : 0.f;
+      float *O = (float *)a.o + b * a.o_sb + h * a.o_sh + (int64_t)qi * a.o_st;
+#pragma unroll
+      for (int d = 0; d < S::F; d++)
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+          if (32 * d + 8 * j + 4 * lk < a.hd)
+            *reinterpret_cast<float4 *>(O + 32 * d + 8 * j + 4 * lk) = make_float4(o[d][4 * j] * inv_l, o[d][4 * j + 1] * inv_l, o[d][4 * j + 2] * inv_l, o[d][4 * j + 3] * inv_l);
+      if (lk == 0) a.lse[((int64_t)b * a.H + h) * a.T + qi] = m + logf(l);
+    }
+  }
+}
+
+// The same for few blocks of 128 queries: a block owns 32 query rows and its W waves share the keys, wave w taking the tiles
+// w, w + W, ... with a running max / sum / output of its own; the W of them are joined in LDS at the end, in the order of the waves.
+// K and V go from memory straight into the operand registers: the contraction over features may take them in any order as long as
+// both operands do, so half lane/32 owns the features (D/2)*half .. and reads 16 bytes of its key's row at a time; a V operand is 32
+// features of one key side by side.  No LDS and no barrier before the join.
+// What bounds the kernel above there is its serial chain, T / 32 tiles one after the other on a few CUs.
+template <int D, int W>
+__global__ __launch_bounds__(64 * W) void k_flash_fwd_f32_keys(FlashArgs a) {
+  constexpr int DB = D / 32, H4 = D / 8;
+  __shared__ float4 part[W * 4 * 64];
+  __shared__ float Ms[W * 32], Lsum[W * 32];
+  int bh, xblk;
+  flash_block(bh, xblk, flash_head_group(a.T, D, 4));
+  xblk = gridDim.x - 1 - xblk;                                     // longest (latest) query blocks are scheduled first
+  const int b = bh / a.H, h = bh % a.H;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 31, lk = lane >> 5;
+  const int q0 = xblk * 32, qi = q0 + lr;
+  const float *Q = (const float *)a.q + b * a.q_sb + h * a.q_sh;
+  const float *K = (const float *)a.k + b * a.k_sb + h * a.k_sh;
+  const float *V = (const float *)a.v + b * a.v_sb + h * a.v_sh;
+  const float inv_cap = a.cap > 0.f ? 1.0f / a.cap : 0.f;
+  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+  // 4 H4 features of a row, those of this half
+  auto row = [&](const float *p, float mul, float4 (&r)[H4]) {
+#pragma unroll
+    for (int i = 0; i < H4; i++) {
+      const int d = lk * (D / 2) + 4 * i;
+      r[i] = d < a.hd ? *reinterpret_cast<const float4 *>(p + d) : zero;
+      r[i].x *= mul; r[i].y *= mul; r[i].z *= mul; r[i].w *= mul;
+    }
+  };
+  float4 q[H4], k[H4];
+  row(Q + (int64_t)min(qi, a.T - 1) * a.q_st, a.scale, q);         // rows past the end repeat the last one: not stored, masked as keys
+
+  f32x16 o[DB];
+#pragma unroll
+  for (int d = 0; d < DB; d++)
+#pragma unroll
+    for (int e = 0; e < 16; e++) o[d][e] = 0.f;
+  float m = -INFINITY, l = 0.f;
+  for (int kv0 = wave * 32; kv0 <= q0; kv0 += W * 32) {
+    row(K + (int64_t)min(kv0 + lr, a.T - 1) * a.k_st, 1.0f, k);
+    float v[DB][16];
+#pragma unroll
+    for (int d = 0; d < DB; d++)
+#pragma unroll
+      for (int e = 0; e < 16; e++) {
+        const int kv = min(kv0 + 8 * (e >> 2) + 4 * lk + (e & 3), a.T - 1);
+        v[d][e] = 32 * d + lr < a.hd ? V[(int64_t)kv * a.v_st + 32 * d + lr] : 0.f;
+      }
+    f32x16 s;
+#pragma unroll
+    for (int e = 0; e < 16; e++) s[e] = 0.f;
+#pragma unroll
+    for (int i = 0; i < H4; i++) {
+      s = __builtin_amdgcn_mfma_f32_32x32x2f32(k[i].x, q[i].x, s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_32x32x2f32(k[i].y, q[i].y, s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_32x32x2f32(k[i].z, q[i].z, s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_32x32x2f32(k[i].w, q[i].w, s, 0, 0, 0);
+    }
+    float tmax = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+      const int kv = kv0 + 8 * (e >> 2) + 4 * lk + (e & 3);
+      float x = softcap_fwd(s[e], a.cap, inv_cap);
+      x = (kv > qi || kv >= a.T) ? -INFINITY : x;
+      s[e] = x;
+      tmax = fmaxf(tmax, x);
+    }
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+    const float m_new = fmaxf(m, tmax), m_use = m_new == -INFINITY ? 0.f : m_new;
+    const float alpha = expf(m - m_use);
+    float psum = 0.f;
+#pragma unroll
+    for (int e = 0; e < 16; e++) { const float p = expf(s[e] - m_use); s[e] = p; psum += p; }
+    psum += __shfl_xor(psum, 32, 64);
+    l = l * alpha + psum;
+    m = m_new;
+#pragma unroll
+    for (int d = 0; d < DB; d++)
+#pragma unroll
+      for (int e = 0; e < 16; e++) o[d][e] *= alpha;
+#pragma unroll
+    for (int d = 0; d < DB; d++)
+#pragma unroll
+      for (int e = 0; e < 16; e++) o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[d][e], s[e], o[d], 0, 0, 0);
+  }
+
+  if (lk == 0) { Ms[wave * 32 + lr] = m; Lsum[wave * 32 + lr] = l; }
+  __syncthreads();
+  float top = -INFINITY;
+#pragma unroll
+  for (int w = 0; w < W; w++) top = fmaxf(top, Ms[w * 32 + lr]);
+  const float use = top == -INFINITY ? 0.f : top;
+  float total = 0.f;
+#pragma unroll
+  for (int w = 0; w < W; w++) total += Lsum[w * 32 + lr] * expf(Ms[w * 32 + lr] - use);
+  const float factor = expf(m - use) * (total > 0.f ? 1.0f / total : 0.f);
+  if (wave == 0 && lk == 0 && qi < a.T) a.lse[((int64_t)b * a.H + h) * a.T + qi] = top + logf(total);
+  // 8 threads to a row: piece ch of its 32 features is the accumulator quarter ch / 2 of half ch % 2
+  const int r = threadIdx.x >> 3, ch = threadIdx.x & 7;
+#pragma unroll
+  for (int d = 0; d < DB; d++) {
+    if (d) __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      part[(wave * 4 + j) * 64 + lane] = make_float4(o[d][4 * j] * factor, o[d][4 * j + 1] * factor, o[d][4 * j + 2] * factor, o[d][4 * j + 3] * factor);
+    __syncthreads();
+    if (threadIdx.x < 256 && q0 + r < a.T && 32 * d + 4 * ch < a.hd) {
+      float4 sum = part[(ch >> 1) * 64 + 32 * (ch & 1) + r];
+#pragma unroll
+      for (int w = 1; w < W; w++) {
+        const float4 x = part[(w * 4 + (ch >> 1)) * 64 + 32 * (ch & 1) + r];
+        sum.x += x.x; sum.y += x.y; sum.z += x.z; sum.w += x.w;
+      }
+      *reinterpret_cast<float4 *>((float *)a.o + b * a.o_sb + h * a.o_sh + (int64_t)(q0 + r) * a.o_st + 32 * d + 4 * ch) = sum;
+    }
+  }
+}
+
+// delta[b,h,t] = sum_d dO[t,d] * O[t,d]
+template <int D>
+__global__ void k_flash_delta_f32(FlashArgs a) {
+  int64_t row = blockIdx.x * (int64_t)(blockDim.x >> 6) + (threadIdx.x >> 6);
+  int64_t total = (int64_t)a.B * a.H * a.T;
+  if (row >= total) return;
+  int lane = threadIdx.x & 63;
+  int t = (int)(row % a.T), h = (int)((row / a.T) % a.H), b = (int)(row / ((int64_t)a.T * a.H));
+  const float *O = (const float *)a.o + b * a.o_sb + h * a.o_sh + (int64_t)t * a.o_st;
+  const float *dO = (const float *)a.d_o + b * a.o_sb + h * a.o_sh + (int64_t)t * a.o_st;
+  float s = 0.f;
+  for (int d = lane; d < a.hd; d += 64) s += O[d] * dO[d];
+  s = wave_sum(s);
+  if (lane == 0) a.delta[row] = s;
+}
+
 // ------------------------------------------------------------------------------------------ dQ
 template <int D>
 __device__ void flash_dq_exact(const FlashArgs &a, int bh, int xblk, float *smem) {
@@ -485,7 +576,6 @@ __device__ void flash_dq_exact(const FlashArgs &a, int bh, int xblk, float *smem
   }
 }
 
-// Four waves of 32 queries.  Head sizes over 64 keep the fp32 instruction: their operands do not fit the registers in three parts.
 template <int D>
 __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_dq_f32(FlashArgs a) {
   constexpr int EXACT = 2 * BC * (D + 1) * 4;
@@ -776,14 +866,15 @@ int32_t check(const AhFlash *f, bool bwd, FlashArgs &a) {
 template <int D>
 int32_t run_fwd(const FlashArgs &a) {
   if constexpr (D <= 64) {
-    // Blocks of 128 queries until there is one for every CU; before that the keys go to 8 waves where that gives each at least one
+    // Blocks of 128 queries from one for every second CU on; before that the keys go to 8 waves where that gives each at least one
     // tile, or where all workgroups run at once.  us, 128-query blocks / keys among waves, soft cap on:
-    //   D = 64, 12 heads: T = 64 16 / 16, T = 256 46 / 23, T = 500 88 / 36, T = 1024 172 / 95; T = 1024 24 heads 176 / 122, 32 heads 178 / 157;
-    //   160 heads x T = 100 26 / 42;  D = 32, 8 heads: T = 32 7.9 / 10, T = 128 17 / 11, T = 256 32 / 14
+    //   D = 64, 12 heads: T = 256 33 / 23, T = 500 60 / 36, T = 777 91 / 67, T = 1024 115 / 95; T = 1024 24 heads 119 / 122, 32 heads 121 / 157;
+    //   16 heads x 2048 234 / 254; 64 heads x 512 x 48 63 / 88; 160 heads x T = 100 20 / 42;  12 heads x T = 64 12 / 16
+    //   D = 32: 8 heads x T = 32 7 / 10, x T = 128 16 / 12, x T = 256 28 / 14
     // Larger heads keep the one kernel: there a call over many heads and calls over each alone give the same bits.
     constexpr int W = 8;
     const int64_t heads = (int64_t)a.B * a.H, blocks = cdiv(a.T, 32) * heads;
-    if (a.T > 64 && cdiv(a.T, WAVES * 32) * heads <= num_cus() && (a.T >= W * 32 || blocks <= num_cus())) {
+    if (a.T > 64 && 2 * cdiv(a.T, WAVES * 32) * heads <= num_cus() && (a.T >= W * 32 || blocks <= num_cus())) {
       ah::launch_kernel((k_flash_fwd_f32_keys<D, W>), dim3((unsigned)cdiv(a.T, 32), (unsigned)heads), dim3(64 * W), 0, a);
       AH_LAUNCH_CHECK();
       return AH_OK;
