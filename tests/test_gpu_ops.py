@@ -1677,7 +1677,7 @@ def test_flash_attention_heads_are_independent_of_how_blocks_are_dealt_out(B, st
 
 
 @pytest.mark.parametrize("BH,T,D,cap", [(1, 31, 32, 30.0), (3, 33, 64, 0.0), (12, 256, 64, 30.0), (2, 257, 64, 30.0), (2, 545, 64, 0.0), (1, 300, 40, 30.0),
-                                        (2, 161, 128, 30.0), (256, 128, 32, 30.0), (257, 128, 32, 30.0), (129, 130, 64, 30.0), (2, 2050, 32, 0.0)])
+                                        (2, 161, 128, 30.0), (64, 128, 32, 30.0), (65, 128, 32, 30.0), (64, 256, 64, 30.0), (65, 256, 64, 30.0), (129, 130, 64, 30.0), (2, 2050, 32, 0.0)])
 def test_flash_attention_f32_forward_with_keys_shared_by_waves(B, BH, T, D, cap):
     """Where one key tile, W of them and one more end, and both sides of the grid size from which blocks of 128 queries are taken.
     A sum of T fp32 products rounds by at most T 2^-24 of its terms' sizes, 2^-24 sqrt(T) at random: 16 times that, and 1e-5 at most."""
