@@ -169,10 +169,11 @@ class HipBackend:
             check(self.lib.ah_download(out.ctypes.data_as(C.c_void_p), t._buf.ptr + t._off, out.nbytes))
         return out
 
-    def _own(self, t: TensorData):
-        """Before an in-place write: a clone's block becomes `t`'s own (a tensor not on the device yet has no clone)."""
+    def _own(self, t: TensorData, copy: bool = True):
+        """Before an in-place write: a clone's block becomes `t`'s own (a tensor not on the device yet has no clone); copy=False:
+        the write fills all of it."""
         if t._buf is not None and t._dev_valid:
-            t._buf.own()
+            t._buf.own(copy)
 
     def _dirty(self, t: TensorData):
         """An in-place device op changed `t`: the cached host copy is stale (backend.ts:706-729)."""

@@ -727,13 +727,14 @@ class FastHipBackend(HipBackend):
         self._own(a)
         super().addInplace(a, b)
 
-    def _own(self, t: TensorData):
-        """Before an in-place write: give `t` a buffer nobody else shares."""
+    def _own(self, t: TensorData, copy: bool = True):
+        """Before an in-place write: give `t` a buffer nobody else shares (copy=False: the write fills all of it)."""
         self._launch_flash()                                    # (a pending attention reads its operands as they are now)
         if t._buf is not None and t._buf.refs > 1 and t._dev_valid:
             n = t.size * ffi.DTYPE_BYTES[t.store]
             buf = _Buf(self.lib, n)
-            check(self.lib.ah_copy(buf.ptr, self._ptr(t), n))
+            if copy:
+                check(self.lib.ah_copy(buf.ptr, self._ptr(t), n))
             t._buf.release()
             t._buf, t._off = buf, 0
 

@@ -224,6 +224,7 @@ class DataLoader:
                 fresh = B_._new(t.shape, "i32")
                 t._buf, t._off, t._dev_valid, t._backend = fresh._buf, 0, True, B_
                 fresh._buf = None
+            B_._own(t, copy=False)                              # a clone of an earlier batch keeps the block it shares
         st = TensorData((Bt,), "f64", np.asarray(starts, dtype=np.int64).view(np.float64))     # 8-byte slots holding the int64 starts
         B = self.B
         check(B.lib.ah_token_windows(B._ptr(self._corpus), N, B._ptr(st), Bt, T, B._ptr(inputs), B._ptr(targets)))
