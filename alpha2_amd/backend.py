@@ -69,6 +69,11 @@ class _Buf:
         if self.refs == 0 and self.ptr:
             self._drop()
 
+    @property
+    def shared(self) -> bool:
+        """Is the block named by more than one tensor, as a view or as a clone?"""
+        return self.refs > 1 or self.owners[0] > 1
+
     def own(self, copy: bool = True):
         """A block of its own, for a writer; copy=False: the writer is about to fill all of it from the old address."""
         if self.owners[0] > 1:

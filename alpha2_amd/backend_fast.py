@@ -662,7 +662,7 @@ class FastHipBackend(HipBackend):
         if self._wgrads and b._buf is not None and id(b._buf) in self._wq_out:
             for w in self._wgrads:
                 if b._buf is w.out_buf and w.into is None and a.store == "f32" and a.size == b.size and a._buf is not None and a._dev_valid \
-                        and a._buf.refs == 1 and id(a._buf) not in self._wq_out and id(a._buf) not in self._wq_into \
+                        and not a._buf.shared and id(a._buf) not in self._wq_out and id(a._buf) not in self._wq_into \
                         and not any(a._buf is x for x in w.holds):      # (`a` may be an operand of the very product: it cannot be written while it is read)
                     w.into = (a._buf, a._off)                    # the grouped launch adds into `a`; `b` itself is never computed
                     a._buf.refs += 1
@@ -705,7 +705,7 @@ class FastHipBackend(HipBackend):
         self._ptr(a), self._ptr(b)                               # launches whatever still has to produce (or add into) them
         if a.store == b.store == "bf16" and a.size == b.size and a._dev_valid and (self._ptr(a) | self._ptr(b)) % 16 == 0:
             pa, pb = self._ptr(a), self._ptr(b)
-            if a._buf.refs > 1:                                  # copy-on-write, as below
+            if a._buf.shared:                                    # copy-on-write, as below
                 buf = _Buf(self.lib, a.size * 2)
                 check(self.lib.ah_add_bf16(pa, pb, buf.ptr, a.size))
                 a._buf.release()
@@ -714,7 +714,7 @@ class FastHipBackend(HipBackend):
                 check(self.lib.ah_add_bf16(pa, pb, pa, a.size))
             self._dirty(a)
             return
-        if a._buf is not None and a._buf.refs > 1 and a._dev_valid and a.store == "f32" and b.store == "f32":
+        if a._buf is not None and a._buf.shared and a._dev_valid and a.store == "f32" and b.store == "f32":
             # copy-on-write: `a` shares its buffer (clone): the sum goes to a buffer of its own in one pass
             pa, pb = self._ptr(a), self._ptr(b)
             buf = _Buf(self.lib, a.size * 4)
@@ -730,7 +730,7 @@ class FastHipBackend(HipBackend):
     def _own(self, t: TensorData, copy: bool = True):
         """Before an in-place write: give `t` a buffer nobody else shares (copy=False: the write fills all of it)."""
         self._launch_flash()                                    # (a pending attention reads its operands as they are now)
-        if t._buf is not None and t._buf.refs > 1 and t._dev_valid:
+        if t._buf is not None and t._buf.shared and t._dev_valid:
             n = t.size * ffi.DTYPE_BYTES[t.store]
             buf = _Buf(self.lib, n)
             if copy:

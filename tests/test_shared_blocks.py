@@ -68,6 +68,10 @@ class HostLibrary:
         self.view(out, n)[:] = self.view(a, n) + self.view(b, n)
         return 0
 
+    def ah_add_bf16(self, a, b, out, n):                        # (bf16 words added as whole numbers: not the kernel's arithmetic)
+        self.view(out, n, np.uint16)[:] = self.view(a, n, np.uint16) + self.view(b, n, np.uint16)
+        return 0
+
     def ah_scale_inplace(self, a, s, n):
         return self.touch(n, a)
 
@@ -100,6 +104,9 @@ class HostLibrary:
         return 0
 
     def ah_step_kick(self):
+        return 0
+
+    def ah_sync(self):
         return 0
 
 
@@ -144,3 +151,48 @@ def test_a_cloned_batch_survives_the_batches_that_follow(lib, kind, packed):
         for cx, cy, wx, wy in kept:
             assert np.array_equal(_device(lib, B, cx), wx) and np.array_equal(_device(lib, B, cy), wy)
     assert len({tuple(wx) for _, _, wx, _ in kept}) == 6
+
+
+def _in_place_calls(B):
+    """name -> (sizes of the operands, the call, which operands it writes)."""
+    one = (12,)
+    return {
+        "addInplace": ((one, one), lambda a, b: B.addInplace(a, b), (0,)),
+        "scaleInplace": ((one,), lambda a: B.scaleInplace(a, 2.0), (0,)),
+        "adamwStep": ((one,) * 4, lambda p, g, m, v: B.adamwStep(p, g, m, v, 1e-3, 0.9, 0.95, 1e-8, 0.0, 0.1, 0.05), (0, 2, 3)),
+        "lionStep": ((one,) * 3, lambda p, g, m: B.lionStep(p, g, m, 1e-3, 0.9, 0.99, 0.0), (0, 2)),
+        "sgdStep": ((one,) * 2, lambda p, g: B.sgdStep(p, g, 0.1), (0,)),
+        "adafactorStep2d": (((3, 4), (3, 4), (3,), (4,)), lambda p, g, r, c: B.adafactorStep2d(p, g, r, c, 1e-3, 0.9, 1e-8, 1.0, 0.0), (0, 2, 3)),
+        "adafactorStepFlat": ((one,) * 3, lambda p, g, v: B.adafactorStepFlat(p, g, v, 1e-3, 0.9, 1e-8, 1.0, 0.0), (0, 2)),
+    }
+
+
+@pytest.mark.parametrize("writer", ["f32", "fast"])
+@pytest.mark.parametrize("name", ["addInplace", "scaleInplace", "adamwStep", "lionStep", "sgdStep", "adafactorStep2d", "adafactorStepFlat"])
+@pytest.mark.parametrize("side", ["original", "clone"])
+def test_in_place_calls_leave_the_other_side_of_a_clone_alone(lib, writer, name, side):
+    """Clones made by the fp32 backend, written through either backend, from either side."""
+    maker, B = _backend("f32"), _backend(writer)
+    shapes, call, written = _in_place_calls(B)[name]
+    originals = [_floats(maker, int(np.prod(s)), i, s) for i, s in enumerate(shapes)]
+    before = [np.array(t.data) for t in originals]
+    clones = [maker.clone(t) for t in originals]
+    operands, others = (originals, clones) if side == "original" else (clones, originals)
+    call(*operands)
+    B.syncGpu()
+    for i, (t, o) in enumerate(zip(operands, others)):
+        assert np.array_equal(_device(lib, maker, o), before[i]), i
+        assert np.array_equal(_device(lib, maker, t), before[i]) == (i not in written), i
+
+
+@pytest.mark.parametrize("side", ["original", "clone"])
+def test_bf16_add_in_place_leaves_the_other_side_of_a_clone_alone(lib, side):
+    maker, B = _backend("f32"), _backend("fast")
+    a, b = B._new((16,), "f32", "bf16"), B._new((16,), "f32", "bf16")
+    lib.view(a._buf.ptr, 16, np.uint16)[:] = np.arange(16) + 16256
+    lib.view(b._buf.ptr, 16, np.uint16)[:] = 1
+    c = maker.clone(a)
+    w, other = (a, c) if side == "original" else (c, a)
+    B.addInplace(w, b)
+    assert np.array_equal(lib.view(other._buf.ptr, 16, np.uint16), np.arange(16) + 16256)
+    assert np.array_equal(lib.view(w._buf.ptr, 16, np.uint16), np.arange(16) + 16257)
