@@ -59,10 +59,10 @@ class _Buf:
         return out.value
 
     def _drop(self):
-        self.owners[0] -= 1
-        if self.owners[0] == 0:
-            self.lib.ah_free(self.ptr)
-        self.ptr = 0
+        ptr, owners, self.ptr = self.ptr, self.owners, 0
+        owners[0] -= 1
+        if owners[0] == 0:
+            self.lib.ah_free(ptr)
 
     def release(self):
         self.refs -= 1
@@ -75,12 +75,16 @@ class _Buf:
         return self.refs > 1 or self.owners[0] > 1
 
     def own(self, copy: bool = True):
-        """A block of its own, for a writer; copy=False: the writer is about to fill all of it from the old address."""
+        """A block of its own, for a writer; copy=False: the writer is about to fill all of it, at the latest now from the old address."""
         if self.owners[0] > 1:
             mine = _Buf._block(self.lib, self.nbytes)
             if copy:
-                check(self.lib.ah_copy(mine, self.ptr, self.nbytes))
-            self.owners[0] -= 1
+                try:
+                    check(self.lib.ah_copy(mine, self.ptr, self.nbytes))
+                except Exception:
+                    self.lib.ah_free(mine)
+                    raise
+            self._drop()                    # (the others may have gone meanwhile - a collected clone's __del__: then the block goes too)
             self.ptr, self.owners = mine, [1]
 
     def __del__(self):          # backstop, like the reference's FinalizationRegistry

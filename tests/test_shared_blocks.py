@@ -196,3 +196,33 @@ def test_bf16_add_in_place_leaves_the_other_side_of_a_clone_alone(lib, side):
     B.addInplace(w, b)
     assert np.array_equal(lib.view(other._buf.ptr, 16, np.uint16), np.arange(16) + 16256)
     assert np.array_equal(lib.view(w._buf.ptr, 16, np.uint16), np.arange(16) + 16257)
+
+
+@pytest.mark.parametrize("moment", ["while the writer's block is made", "before"])
+def test_the_shared_block_is_freed_by_whoever_leaves_it_last(lib, moment):
+    """The other side may be collected inside the writer's own allocation: the block has no owner then once the writer has moved."""
+    B = _backend("f32")
+    a = _floats(B, 12, 1)
+    want = np.array(a.data)
+    held = [B.clone(a)]
+    if moment == "before":
+        held.clear()
+    else:
+        lib.on_alloc = held.clear
+    B.scaleInplace(a, 2.0)
+    assert np.array_equal(_device(lib, B, a), want + 1000) and len(lib.blocks) == 1
+    B.releaseGpuTensor(a)
+    assert not lib.blocks
+
+
+def test_a_refused_copy_leaves_both_sides_as_they_were(lib):
+    B = _backend("f32")
+    a = _floats(B, 12, 1)
+    want, c = np.array(a.data), B.clone(a)
+    lib.refuse_copy = True
+    with pytest.raises(Exception):
+        B.scaleInplace(a, 2.0)
+    assert len(lib.blocks) == 1 and a._buf.ptr == c._buf.ptr
+    lib.refuse_copy = False
+    B.scaleInplace(a, 2.0)
+    assert np.array_equal(_device(lib, B, a), want + 1000) and np.array_equal(_device(lib, B, c), want)
