@@ -75,7 +75,7 @@ class _Buf:
         return self.refs > 1 or self.owners[0] > 1
 
     def own(self, copy: bool = True):
-        """A block of its own, for a writer; copy=False: the writer is about to fill all of it, at the latest now from the old address."""
+        """A block of its own, for a writer; copy=False: the writer is about to fill all of it from the old address."""
         if self.owners[0] > 1:
             mine = _Buf._block(self.lib, self.nbytes)
             if copy:

@@ -20,7 +20,7 @@
   attention kernels, whose time goes to per-score vector instructions, are read against.
 
 Every call goes through the C ABI; timing is by HIP events on the library's stream.  Peaks used for the last column:
-2.5 PFLOP/s (bf16 MFMA), 157.3 TFLOP/s (fp32 MFMA), 8 TB/s (HBM).
+2.5 PFLOP/s (bf16 MFMA), a sixth of it (fp32 products: six bf16 products each), 8 TB/s (HBM).
 """
 from __future__ import annotations
 
@@ -34,7 +34,7 @@ import numpy as np
 
 from . import HipBackend, _ffi as ffi
 
-PEAK_TFLOPS = {"bf16": 2500.0, "f32": 157.3}
+PEAK_TFLOPS = {"bf16": 2500.0, "f32": 2500.0 / 6}
 PEAK_GBS = 8000.0
 
 

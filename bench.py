@@ -46,7 +46,7 @@ WORKLOADS = {        # name -> (model, micro-batch, accumulated micro-steps, tok
                  "350M-shape train step: vocab 50304, d_model 1024, 24 layers, 16 heads, ctx 1024, batch 8 x 4 accumulated micro-steps, "
                  "untied lmHead (406.2M params), AdamW lr 3e-4 betas (0.9,0.95) wd 0.1, grad-clip 1.0"),
 }
-PEAK = {"bf16": 2500.0, "f32": 157.3}          # MI355X dense MFMA, TFLOP/s
+PEAK = {"bf16": 2500.0, "f32": 2500.0 / 6}     # MI355X dense MFMA, TFLOP/s (an fp32 product is six bf16 ones)
 # Counter summaries of this benchmark (rocprofv3 --pmc passes; the files say how they were made and calibrated).  What the
 # JSON line reports from counters -- HBM-side bytes per launch of the dominant kernel, time-weighted MFMA-busy fraction of the
 # step -- is read from the table in the file of the workload, never typed in here.
