@@ -239,9 +239,11 @@ int32_t launch(const GemmArgs &ga, int batch, int out_dtype) {
 // LDS traffic per flop of the 128x128 tile.  It holds one block per CU, so what matters is how evenly the tiles fill
 // whole rounds of CUs: take 256 x 256, 256 x 192 or 256 x 128 tiles, whichever wastes least of its last round, and keep the
 // tiles of this file (two blocks per CU, finer grain) when none fills 70 % and they need no second round.  Returns the tile width, 0 = the
-// 128x128 kernel.  A product with planes only gets tile widths that divide a plane of C, and always gets one.
+// tiles of this file.  A product with planes only gets tile widths that divide a plane of C, and always gets one.
+// Its epilogue addresses 128 rows of C with 31-bit byte offsets, and moves four columns at a time: where C ends inside four (an
+// A B^T product; the other layouts have n % 8 == 0) it would write beside the result.
 int pick_large_tile(const GemmArgs &ga, int batch, bool akm, bool bkm) {
-  if (!(ga.M >= 256 && ga.N >= 128 && ga.ldc < (1 << 22))) return 0;      // (its epilogue addresses 128 rows of C with 31-bit byte offsets)
+  if (!(ga.M >= 256 && ga.N >= 128 && ga.N % 4 == 0 && ga.ldc < (1 << 22))) return 0;
   const int64_t cus = num_cus(), per = (int64_t)batch * ga.nsplit;
   auto fill = [&](int bn) {
     if (ga.c_plane_n > 0 && ga.c_plane_n % bn != 0) return 0.0;

@@ -379,7 +379,8 @@ int32_t ah_gemm_planes(const AhGemm *g, int64_t c_plane_cols, int64_t c_plane_st
  * grid, so small outputs with a long contraction fill the chip without split-K).  Used for the weight gradients
  * dW_i = G_i^T X_i of all layers at the end of backward; the reference computes them one matmul at a time
  * (packages/autograd/src/ops.ts:197-234).  Requirements per problem: bf16 operands, batch 1, k a multiple of 64,
- * 16-byte aligned rows, epilogue NONE or ACCUM; all problems share layout and output type.  The plan copies the
+ * 16-byte aligned rows, epilogue NONE or ACCUM; all problems share layout and output type; where n is no multiple of 4
+ * (layout NT) the columns of C up to the next one are written too, so C is no block of a wider matrix there.  The plan copies the
  * descriptors to the device once; ah_gemm_grouped_run only launches (safe inside graph capture) and takes the
  * epilogue (AH_EPI_NONE, or AH_EPI_ACCUM for f32 outputs) so one plan serves first and later micro-batches.
  * Tiles run one per CU in rounds of 256; when the last round of an f32 plan is at most half full, the plan cuts the

@@ -1256,6 +1256,32 @@ def test_gemm_bf16_tile_by_the_number_of_tiles(B, M, N, K, kernel, layout):
     assert np.all(np.abs(tc.data.reshape(M, N) - want) <= 2.0 ** -8 * np.abs(want) + K * 2.0 ** -24 * size)
 
 
+# a last round that the large tiles fill well, one that they do not (more 128-wide tiles than CUs), a few tiles; columns beside C
+@pytest.mark.parametrize("M,N,ldc", [(16384, 1022, 1024), (11000, 770, 772), (300, 129, 140), (256, 131, 132)])
+@pytest.mark.parametrize("out", ["f32", "bf16", "accumulate", "residual"])
+def test_gemm_bf16_writes_nothing_beside_a_result_that_ends_inside_four_columns(B, M, N, ldc, out):
+    """C is a column block of a wider matrix: what lies beside it stays.  Against the float64 product of the same operands, as above."""
+    import ctypes
+    from alpha2_amd import _ffi as ffi
+    K, g = 64, np.random.default_rng(N)
+    a, b = _bf16_round(g.standard_normal((M, K), dtype=np.float32))[0], _bf16_round(g.standard_normal((N, K), dtype=np.float32))[0]
+    c0 = _bf16_round(g.standard_normal((M, ldc), dtype=np.float32))[0]
+    bf = out == "bf16" or out == "residual"
+    ta, tb, tc, tr = B.castStore(dev(B, a), "bf16"), B.castStore(dev(B, b), "bf16"), dev(B, c0), dev(B, c0)
+    if bf:
+        tc, tr = B.castStore(tc, "bf16"), B.castStore(tr, "bf16")
+    epi = {"accumulate": ffi.EPI_ACCUM, "residual": ffi.EPI_RESIDUAL}.get(out, ffi.EPI_NONE)
+    q = ffi.AhGemm(ffi.GEMM_NT, ffi.BF16, ffi.BF16 if bf else ffi.F32, epi, M, N, K, K, K, ldc, 1, 0, 0, 0, B._ptr(ta), B._ptr(tb), B._ptr(tc), B._ptr(tr) if out == "residual" else 0)
+    ffi.check(B.lib.ah_gemm(ctypes.byref(q)))
+    B._dirty(tc)
+    got = tc.data.reshape(M, ldc)
+    assert np.array_equal(got[:, N:], c0[:, N:]), B.lastGemmKernel()
+    want, size = a.astype(np.float64) @ b.T.astype(np.float64), np.abs(a).astype(np.float64) @ np.abs(b).T.astype(np.float64)
+    if epi != ffi.EPI_NONE:
+        want, size = want + c0[:, :N], size + np.abs(c0[:, :N])
+    assert np.all(np.abs(got[:, :N] - want) <= (2.0 ** -8 if bf else 2.0 ** -23) * np.abs(want) + K * 2.0 ** -24 * size)
+
+
 def test_gemm_bf16_split_k_weight_gradient(B):
     """dW = G^T X with a long token axis and few output tiles takes the split-K path (slices of the token axis into a
     workspace, summed in a fixed order by a second kernel)."""
