@@ -1,15 +1,10 @@
 // fp32 products on the bf16 matrix pipes.
 //
-// Every operand value x is cut, on its way to the matrix pipe, into three bf16 numbers h = bf16(x), m = bf16(x - h),
-// l = bf16(x - h - m), each rounded to nearest: 8 + 8 + 8 bits hold the 24 of an fp32 significand, so h + m + l IS x (down to
-// the last bits of numbers below 2^-110).  A product x y is then accumulated in fp32 as
-//     l h' + h l' + m m' + m h' + h m' + h h'
-// (what is left out, m l' + l m' + l l', is at most 2^-24 |x y| and of either sign), six v_mfma_f32_32x32x16_bf16 of 32 cycles
-// for 16 steps of the contraction where eight v_mfma_f32_32x32x2_f32 take 512: 2.7 times the fp32 rate.  How the sums are kept as
-// close to the 64-bit ones as the fp32 instruction's: S_FLUSH below.
-// An operand that is infinite, NaN or rounds to infinity in bf16 leaves a result that is not finite; a workgroup that finds one
-// computes its tile again with the fp32 instruction (f32_tile), whose result stands.
+// Every operand value is cut, on its way to the matrix pipe, into three bf16 numbers, and a product is six of theirs (split_bf16.h):
+// 2.7 times the rate of the fp32 instruction.  How the sums are kept as close to the 64-bit ones as that instruction's: S_FLUSH below.
+// A workgroup that finds a result that is not finite computes its tile again with the fp32 instruction (f32_tile), whose result stands.
 #include "gemm_common.h"
+#include "split_bf16.h"
 #include <cmath>
 
 using namespace ah;
@@ -138,39 +133,15 @@ __device__ __forceinline__ void f32_tile(const GemmArgs &g, const float *A, cons
 }
 
 // ================================================================ the split
-struct Split2 { uint32_t h, m, l; };       // two values side by side
-__device__ __forceinline__ Split2 split2(float x0, float x1) {
-  Split2 s;
-  s.h = pack_bf16x2(x0, x1);
-  x0 -= __uint_as_float(s.h << 16);
-  x1 -= __uint_as_float(s.h & 0xffff0000u);
-  s.m = pack_bf16x2(x0, x1);
-  x0 -= __uint_as_float(s.m << 16);
-  x1 -= __uint_as_float(s.m & 0xffff0000u);
-  s.l = pack_bf16x2(x0, x1);
-  return s;
-}
 // TM x TN accumulators (C^T orientation) += the six products, the smallest first
 template <int TM, int TN>
-__device__ __forceinline__ void mfma6(const bf16x8 (&a)[3][TM], const bf16x8 (&b)[3][TN], f32x16 (&acc)[TM][TN]) {
-  constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
+__device__ __forceinline__ void mfma6_tiles(const bf16x8 (&a)[3][TM], const bf16x8 (&b)[3][TN], f32x16 (&acc)[TM][TN]) {
 #pragma unroll
   for (int p = 0; p < 6; p++)
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
-      for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[PB[p]][j], a[PA[p]][i], acc[i][j], 0, 0, 0);
-}
-template <int TM, int TN>
-__device__ __forceinline__ bool all_finite(const f32x16 (&acc)[TM][TN]) {
-  float z = 0.f;
-#pragma unroll
-  for (int i = 0; i < TM; i++)
-#pragma unroll
-    for (int j = 0; j < TN; j++)
-#pragma unroll
-      for (int e = 0; e < 16; e++) z = __builtin_fmaf(acc[i][j][e], 0.f, z);      // 0 unless one is infinite or NaN
-  return z == 0.f;
+      for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[SPLIT_B[p]][j], a[SPLIT_A[p]][i], acc[i][j], 0, 0, 0);
 }
 
 // ================================================================ tiles through LDS
@@ -196,7 +167,7 @@ __device__ __forceinline__ void store_split(char *s, const float4 (&v)[ROWS / 64
 #pragma unroll
   for (int i = 0; i < ROWS / 64; i++) {
     const int r = (KCONTIG ? t >> 2 : t & 63) + 64 * i, k4 = KCONTIG ? t & 3 : t >> 6;
-    const Split2 a = split2(v[i].x, v[i].y), b = split2(v[i].z, v[i].w);
+    const Split2 a = split2(v[i].x * SPLIT_UP, v[i].y * SPLIT_UP), b = split2(v[i].z * SPLIT_UP, v[i].w * SPLIT_UP);
     char *p = s + plane_ofs(r, k4);
     *reinterpret_cast<uint2 *>(p) = make_uint2(a.h, b.h);
     *reinterpret_cast<uint2 *>(p + ROWS * 32) = make_uint2(a.m, b.m);
@@ -254,7 +225,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f32_split(GemmArgs g, int vec_c
 #pragma unroll
       for (int j = 0; j < TN; j++)
 #pragma unroll
-        for (int e = 0; e < 16; e++) { sum[i][j][e] += acc[i][j][e]; acc[i][j][e] = 0.f; }
+        for (int e = 0; e < 16; e++) { sum[i][j][e] = __builtin_fmaf(acc[i][j][e], SPLIT_DOWN, sum[i][j][e]); acc[i][j][e] = 0.f; }
   };
 
   float4 ra[BM / 64], rb[BN / 64];
@@ -282,7 +253,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f32_split(GemmArgs g, int vec_c
     for (int t = 0; t < full; t++) {
       if (t > 0 && t % S_FLUSH == 0) flush();
       get(smem + (t & 1) * (ABYTES + BBYTES));
-      mfma6<TM, TN>(fa, fb, acc);
+      mfma6_tiles<TM, TN>(fa, fb, acc);
       put(smem + ((t & 1) ^ 1) * (ABYTES + BBYTES));
       load(min(t + 2, full - 1));
       // one matrix instruction (32 cycles), then the vector instructions of the split that fit beside it
@@ -305,11 +276,16 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f32_split(GemmArgs g, int vec_c
     put(smem);
     __syncthreads();
     get(smem);
-    mfma6<TM, TN>(fa, fb, acc);
+    mfma6_tiles<TM, TN>(fa, fb, acc);
     __syncthreads();
   }
   flush();
-  if (__syncthreads_or(!all_finite<TM, TN>(sum))) {
+  bool fine = true;
+#pragma unroll
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int j = 0; j < TN; j++) fine = fine && all_finite(sum[i][j]);
+  if (__syncthreads_or(!fine)) {
     for (int i = 0; i < BM; i += FM)
       for (int j = 0; j < BN; j += FN) {
         if (m0 + i >= g.M || n0 + j >= g.N) continue;
@@ -367,26 +343,16 @@ __device__ __forceinline__ void contract_pieces(const GemmArgs &g, const float *
 #pragma unroll
         for (int e = 0; e < 8; e++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(b[u][e], a[u][e], acc, 0, 0, 0);
       } else {
-        uint32_t wa[3][4], wb[3][4];
+        bf16x8 fa[3], fb[3];
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-          const Split2 x = split2(a[u][2 * e], a[u][2 * e + 1]), y = split2(b[u][2 * e], b[u][2 * e + 1]);
-          wa[0][e] = x.h; wa[1][e] = x.m; wa[2][e] = x.l;
-          wb[0][e] = y.h; wb[1][e] = y.m; wb[2][e] = y.l;
-        }
-        bf16x8 fa[3][1], fb[3][1];
-#pragma unroll
-        for (int p = 0; p < 3; p++) {
-          fa[p][0] = __builtin_bit_cast(bf16x8, make_uint4(wa[p][0], wa[p][1], wa[p][2], wa[p][3]));
-          fb[p][0] = __builtin_bit_cast(bf16x8, make_uint4(wb[p][0], wb[p][1], wb[p][2], wb[p][3]));
-        }
-        f32x16 one[1][1] = {{acc}};
-        mfma6<1, 1>(fa, fb, one);
-        acc = one[0][0];
+        for (int e = 0; e < 8; e++) { a[u][e] *= SPLIT_UP; b[u][e] *= SPLIT_UP; }
+        split8(a[u], fa);
+        split8(b[u], fb);
+        mfma6(fb, fa, acc);                                     // C^T
       }
     }
 #pragma unroll
-    for (int e = 0; e < 16; e++) sum[e] += acc[e];      // short sums, added rounded to nearest (S_FLUSH)
+    for (int e = 0; e < 16; e++) sum[e] = __builtin_fmaf(acc[e], EXACT ? 1.0f : SPLIT_DOWN, sum[e]);      // short sums, added rounded to nearest (S_FLUSH)
   }
 }
 template <int LAYOUT, int WAVES>

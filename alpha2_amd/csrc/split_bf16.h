@@ -8,8 +8,8 @@
 // and A. Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype for Higher-Precision Computations", ARITH 2019.
 //
 // Both operands are multiplied by 2^24 before the cut and the sums by 2^-48 after it: every fp32 number is a multiple of 2^-149,
-// so every part is a multiple of 2^-125 and none is subnormal, which bf16 would hold in fewer bits (unscaled, a number of 2^-120
-// keeps 16 of its 24 bits and one of 2^-126 ten).  Where a value times 2^24 rounds to infinity (from 2^104 on), or a short sum
+// so every part is a multiple of 2^-125 and none is subnormal, which bf16 holds in fewer bits (unscaled, the parts of a number of
+// 2^-112 are 1e-7 of it off, of 2^-120 2.5e-5 and of 2^-126 1.6e-3).  Where a value times 2^24 rounds to infinity (from 2^104 on), or a short sum
 // times 2^48 does (from 2^80 on), or an operand is infinite or NaN, the sum is not finite: a workgroup that finds one computes its
 // results again with the fp32 instruction, and those stand.
 #pragma once
@@ -55,6 +55,13 @@ __device__ __forceinline__ bool all_finite(const f32x16 &acc) {
 #pragma unroll
   for (int e = 0; e < 16; e++) z = __builtin_fmaf(acc[e], 0.f, z);      // 0 unless one is infinite or NaN
   return z == 0.f;
+}
+template <int N>
+__device__ __forceinline__ bool all_finite(const f32x16 (&acc)[N]) {
+  bool fine = true;
+#pragma unroll
+  for (int d = 0; d < N; d++) fine = fine && all_finite(acc[d]);
+  return fine;
 }
 
 }  // namespace ah

@@ -965,6 +965,23 @@ def test_gemm_f32_with_numbers_the_split_cannot_hold(B, M, N, K):
         assert np.all(np.abs(got[fin] - want[fin]) <= (K + 40) * 2.0 ** -24 * size[fin]), layout      # (K roundings where the fp32 instruction ran)
 
 
+# 32-wide pieces by waves, 64-wide tiles, the same in slices, 128-wide tiles, the same in slices
+@pytest.mark.parametrize("M,N,K", [(127, 260, 1000), (65, 129, 47), (384, 128, 1030), (8200, 640, 33), (640, 768, 4096)])
+@pytest.mark.parametrize("ea,eb", [(-118, 100), (100, -126), (-140, 100), (-60, -60), (-70, -72), (110, -100), (60, 45)])
+def test_gemm_f32_keeps_its_bits_at_the_ends_of_the_range(B, M, N, K, ea, eb):
+    """Numbers about 2^ea times numbers about 2^eb, against the float64 product of the same fp32 numbers: below 2^-110 the parts of
+    an unscaled cut are bf16 subnormals, a number of 2^-140 is an fp32 subnormal itself, 2^110 and sums of 2^105 run the fp32
+    instruction.  Bound: as above, K roundings for that instruction, and a subnormal result is rounded to 2^-149 at each of them."""
+    from alpha2_amd import _ffi as ffi
+    g = np.random.default_rng(K + 200 + ea)
+    a, b = (g.standard_normal((M, K)) * 2.0 ** ea).astype(np.float32), (g.standard_normal((K, N)) * 2.0 ** eb).astype(np.float32)
+    want, size = a.astype(np.float64) @ b.astype(np.float64), np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
+    bound = ((K if max(ea, eb) > 103 or ea + eb > 70 else 6 * -(-K // 16)) + 40) * 2.0 ** -24 * size + (K + 1) * 2.0 ** -149
+    for layout in (ffi.GEMM_NN, ffi.GEMM_NT, ffi.GEMM_TN):
+        got = _gemm_f32(B, layout, a, b)
+        assert np.all(np.abs(got - want) <= bound), (layout, B.lastGemmKernel(), float(np.max(np.abs(got - want) / size)))
+
+
 def test_gemm_f32_batched_and_broadcast(B):
     a, b = rs.randn(2, 3, 40, 16).astype(np.float32), rs.randn(2, 3, 16, 24).astype(np.float32)
     assert_close(B.matmul(dev(B, a), dev(B, b)).data, O.matmul(orc(a), orc(b)).data)
