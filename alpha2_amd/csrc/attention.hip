@@ -14,6 +14,7 @@
 // MFMA number (j, r) of a 32-deep contraction contracts rows {8j + r, 8j + 4 + r}: half lane/32 = h owns
 // row 8j + 4h + r in the accumulator and must supply exactly that row as operand -> no data movement.
 #include "attention_common.h"
+#include "split_bf16.h"
 
 using namespace ah;
 
@@ -38,49 +39,18 @@ __device__ __forceinline__ void load_tile_f32(float *s, const float *__restrict_
 }
 
 // ------------------------------------------------------------------------------------------ products on the bf16 matrix pipes
-// A value cut into three bf16 parts and six products of 32 cycles per 16 steps of a contraction, as in the fp32 products of
-// gemm_f32.hip, where sixteen halves of v_mfma_f32_32x32x2_f32 take 512.  Every accumulator that is a matrix instruction's takes
-// at most 24 of them (one 64-feature score, or one tile of 32 rows) and is then added, rounded to nearest, to an fp32 one.
+// The cut and the six products are those of the fp32 products (split_bf16.h).  Every accumulator that is a matrix instruction's
+// takes at most 24 of them (one 64-feature score, or one tile of 32 rows) and is then added, rounded to nearest, to an fp32 one.
 // The tile of 32 streamed rows is cut once for the four waves and laid out in LDS both ways, three planes each:
 //   rows     [row][feature]                  an operand is 8 features of a row
 //   columns  [feature][row'], row' = 16 j + 8 h + 4 i + r of row 16 j + 8 i + 4 h + r: an operand is the 8 rows whose scores the
 //            lanes of half h hold in accumulator elements 8 j .. 8 j + 7, so that those go straight into the other operand
 // 16-byte pieces are permuted within a row so that 16 lanes that read the same piece of 16 rows meet 64 different banks.
-// A result that is not finite (an operand that is infinite, NaN or rounds to infinity in bf16) has the block computed again with the
-// fp32 instruction, whose result stands.
-// (Of a number below 2^-100 the last part, below 2^-110 the second one too, loses bits to bf16's subnormals.)
+// A result that is not finite has the block computed again with the fp32 instruction, whose result stands; so does a score (an
+// infinite one gives weights that look like any other).
 // 192 heads x 1024 x 64: dK and dV 945 -> 486 us, dQ 520 -> 316; 512 x 256 x 32: 112 -> 84 and 81 -> 60; 4 x 70 x 64: 29 -> 24 and
 // 26 -> 20.  Relative error against 64 bits at 4 x 512 x 64: dQ 4.6e-7 -> 3.7e-7, dK 6.4e-7 -> 3.8e-7, dV 6.0e-7 -> 3.3e-7.  What bounds
 // it now is vector issue: tanh, exp and the cut of scores, K and V for every 32 x 32 tile beside 3072 cycles of matrix instructions.
-struct Split2 { uint32_t h, m, l; };       // two values side by side
-__device__ __forceinline__ Split2 split2(float x0, float x1) {
-  Split2 s;
-  s.h = pack_bf16x2(x0, x1);
-  x0 -= __uint_as_float(s.h << 16);
-  x1 -= __uint_as_float(s.h & 0xffff0000u);
-  s.m = pack_bf16x2(x0, x1);
-  x0 -= __uint_as_float(s.m << 16);
-  x1 -= __uint_as_float(s.m & 0xffff0000u);
-  s.l = pack_bf16x2(x0, x1);
-  return s;
-}
-// 8 consecutive values of a contraction in the three parts
-__device__ __forceinline__ void split8(const float (&x)[8], bf16x8 (&f)[3]) {
-  uint32_t w[3][4];
-#pragma unroll
-  for (int e = 0; e < 4; e++) {
-    const Split2 s = split2(x[2 * e], x[2 * e + 1]);
-    w[0][e] = s.h; w[1][e] = s.m; w[2][e] = s.l;
-  }
-#pragma unroll
-  for (int p = 0; p < 3; p++) f[p] = __builtin_bit_cast(bf16x8, make_uint4(w[p][0], w[p][1], w[p][2], w[p][3]));
-}
-// acc += the six products, the smallest first; element (row of a, column of b)
-__device__ __forceinline__ void mfma6(const bf16x8 (&a)[3], const bf16x8 (&b)[3], f32x16 &acc) {
-  constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
-#pragma unroll
-  for (int p = 0; p < 6; p++) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[PA[p]], b[PB[p]], acc, 0, 0, 0);
-}
 template <int D>
 struct SplitTile {                          // D = 32 or 64
   static constexpr int F = D / 32, PLANE = 64 * D, BYTES = 3 * PLANE;      // either layout
@@ -158,8 +128,8 @@ struct SplitTile {                          // D = 32 or 64
 #pragma unroll
     for (int i = 0; i < D / 16; i++) split8(x[i], f[i]);
   }
-  // acc[d][.] += columns (features) x the scores in x
-  static __device__ __forceinline__ void contract_rows(const char *cols, const f32x16 &x, int lr, int lk, f32x16 (&acc)[F]) {
+  // acc[d][.] = alpha acc[d][.] + columns (features) x the weights in x (times SPLIT_UP)
+  static __device__ __forceinline__ void contract_rows(const char *cols, const f32x16 &x, int lr, int lk, float alpha, f32x16 (&acc)[F]) {
     bf16x8 b[2][3];
 #pragma unroll
     for (int j = 0; j < 2; j++) {
@@ -178,18 +148,13 @@ struct SplitTile {                          // D = 32 or 64
         mfma6(a, b[j], t);
       }
 #pragma unroll
-      for (int e = 0; e < 16; e++) acc[d][e] += t[e];
+      for (int e = 0; e < 16; e++) acc[d][e] = __builtin_fmaf(acc[d][e], alpha, t[e]);
     }
   }
 };
-template <int N>
-__device__ __forceinline__ bool all_finite(const f32x16 (&acc)[N]) {
-  float z = 0.f;
-#pragma unroll
-  for (int d = 0; d < N; d++)
-#pragma unroll
-    for (int e = 0; e < 16; e++) z = __builtin_fmaf(acc[d][e], 0.f, z);      // 0 unless one is infinite or NaN
-  return z == 0.f;
+// quarter j of an accumulator of products, as it is stored
+__device__ __forceinline__ float4 summed(const f32x16 &x, int j) {
+  return make_float4(x[4 * j] * SPLIT_DOWN, x[4 * j + 1] * SPLIT_DOWN, x[4 * j + 2] * SPLIT_DOWN, x[4 * j + 3] * SPLIT_DOWN);
 }
 
 // ------------------------------------------------------------------------------------------ forward
@@ -296,7 +261,7 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_fwd_f32(FlashArgs
     const float *V = (const float *)a.v + b * a.v_sb + h * a.v_sh;
     const float inv_cap = a.cap > 0.f ? 1.0f / a.cap : 0.f;
     bf16x8 q[D / 16][3];
-    S::own((const float *)a.q + b * a.q_sb + h * a.q_sh + (int64_t)qi * a.q_st, qi < a.T, a.scale, a.hd, lk, q);
+    S::own((const float *)a.q + b * a.q_sb + h * a.q_sh + (int64_t)qi * a.q_st, qi < a.T, a.scale * SPLIT_UP, a.hd, lk, q);
     f32x16 o[S::F];
 #pragma unroll
     for (int d = 0; d < S::F; d++)
@@ -310,8 +275,8 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_fwd_f32(FlashArgs
     bool fine = true;
     for (int kv0 = 0; kv0 < end; kv0 += BC) {
       __syncthreads();
-      S::template put<true, false>(kx, 1.0f, Kr, nullptr);
-      S::template put<false, true>(vx, 1.0f, nullptr, Vc);
+      S::template put<true, false>(kx, SPLIT_UP, Kr, nullptr);
+      S::template put<false, true>(vx, SPLIT_UP, nullptr, Vc);
       S::load(kx, K, a.k_st, kv0 + BC, a.T, a.hd);                 // the next tile, while this one is multiplied; rows past the end read as zero
       S::load(vx, V, a.v_st, kv0 + BC, a.T, a.hd);
       __syncthreads();
@@ -330,7 +295,7 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_fwd_f32(FlashArgs
 #pragma unroll
       for (int e = 0; e < 16; e++) {
         const int kv = kv0 + 8 * (e >> 2) + 4 * lk + (e & 3);
-        float x = softcap_fwd(s[0][e], a.cap, inv_cap);
+        float x = softcap_fwd(s[0][e] * SPLIT_DOWN, a.cap, inv_cap);
         x = (kv > qi || kv >= a.T) ? -INFINITY : x;
         s[0][e] = x;
         tmax = fmaxf(tmax, x);
@@ -340,22 +305,18 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_fwd_f32(FlashArgs
       const float alpha = expf(m - m_use);
       float psum = 0.f;
 #pragma unroll
-      for (int e = 0; e < 16; e++) { const float p = expf(s[0][e] - m_use); s[0][e] = p; psum += p; }
+      for (int e = 0; e < 16; e++) { const float p = expf(s[0][e] - m_use); s[0][e] = p * SPLIT_UP; psum += p; }
       psum += __shfl_xor(psum, 32, 64);
       l = l * alpha + psum;
       m = m_new;
-#pragma unroll
-      for (int d = 0; d < S::F; d++)
-#pragma unroll
-        for (int e = 0; e < 16; e++) o[d][e] *= alpha;
-      S::contract_rows(Vc, s[0], lr, lk, o);
+      S::contract_rows(Vc, s[0], lr, lk, alpha, o);
     }
     if (__syncthreads_or(!fine || !all_finite<S::F>(o))) {
       flash_fwd_exact<D>(a, bh, xblk, (float *)smem);
       return;
     }
     if (qi < a.T) {
-      const float inv_l = l > 0.f ? 1.0f / l : 0.f;
+      const float inv_l = (l > 0.f ? 1.0f / l : 0.f) * SPLIT_DOWN;
       float *O = (float *)a.o + b * a.o_sb + h * a.o_sh + (int64_t)qi * a.o_st;
 #pragma unroll
       for (int d = 0; d < S::F; d++)
@@ -597,8 +558,8 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_dq_f32(FlashArgs 
     const float inv_cap = a.cap > 0.f ? 1.0f / a.cap : 0.f;
     const bool live = qi < a.T;
     bf16x8 q[D / 16][3], go[D / 16][3];
-    S::own((const float *)a.q + b * a.q_sb + h * a.q_sh + (int64_t)qi * a.q_st, live, a.scale, a.hd, lk, q);
-    S::own((const float *)a.d_o + b * a.o_sb + h * a.o_sh + (int64_t)qi * a.o_st, live, 1.0f, a.hd, lk, go);
+    S::own((const float *)a.q + b * a.q_sb + h * a.q_sh + (int64_t)qi * a.q_st, live, a.scale * SPLIT_UP, a.hd, lk, q);
+    S::own((const float *)a.d_o + b * a.o_sb + h * a.o_sh + (int64_t)qi * a.o_st, live, SPLIT_UP, a.hd, lk, go);
     const int64_t srow = ((int64_t)b * a.H + h) * a.T + qi;
     const float lse = live ? a.lse[srow] : 0.f, delta = live ? a.delta[srow] : 0.f;
     f32x16 dq[S::F];
@@ -610,10 +571,11 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_dq_f32(FlashArgs 
     float kx[4][S::F], vx[4][S::F];
     S::load(kx, K, a.k_st, 0, a.T, a.hd);
     S::load(vx, V, a.v_st, 0, a.T, a.hd);
+    bool fine = true;
     for (int kv0 = 0; kv0 < end; kv0 += BC) {
       __syncthreads();
-      S::template put<true, true>(kx, 1.0f, Kr, Kc);
-      S::template put<true, false>(vx, 1.0f, Vr, nullptr);
+      S::template put<true, true>(kx, SPLIT_UP, Kr, Kc);
+      S::template put<true, false>(vx, SPLIT_UP, Vr, nullptr);
       S::load(kx, K, a.k_st, kv0 + BC, a.T, a.hd);                 // the next tile, while this one is multiplied; rows past the end read as zero
       S::load(vx, V, a.v_st, kv0 + BC, a.T, a.hd);
       __syncthreads();
@@ -629,18 +591,19 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_dq_f32(FlashArgs 
         S::get_row(Vr, lr, 2 * i + lk, f);
         mfma6(f, go[i], dp);
       }
+      fine = fine && all_finite(s);
 #pragma unroll
       for (int e = 0; e < 16; e++) {
         const int kv = kv0 + 8 * (e >> 2) + 4 * lk + (e & 3);
-        const float sc = softcap_fwd(s[e], a.cap, inv_cap);
+        const float sc = softcap_fwd(s[e] * SPLIT_DOWN, a.cap, inv_cap);
         const float p = (kv > qi || kv >= a.T || !live) ? 0.f : expf(sc - lse);
-        float ds = p * (dp[e] - delta);
+        float ds = p * __builtin_fmaf(dp[e], SPLIT_DOWN, -delta);
         if (a.cap > 0.f) { const float t = sc * inv_cap; ds *= (1.0f - t * t); }
-        s[e] = ds * a.scale;
+        s[e] = ds * (a.scale * SPLIT_UP);
       }
-      S::contract_rows(Kc, s, lr, lk, dq);
+      S::contract_rows(Kc, s, lr, lk, 1.0f, dq);
     }
-    if (__syncthreads_or(!all_finite<S::F>(dq))) {
+    if (__syncthreads_or(!fine || !all_finite<S::F>(dq))) {
       flash_dq_exact<D>(a, bh, xblk, (float *)smem);
       return;
     }
@@ -651,7 +614,7 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_dq_f32(FlashArgs 
 #pragma unroll
         for (int j = 0; j < 4; j++)
           if (32 * d + 8 * j + 4 * lk < a.hd)
-            *reinterpret_cast<float4 *>(dQ + 32 * d + 8 * j + 4 * lk) = make_float4(dq[d][4 * j], dq[d][4 * j + 1], dq[d][4 * j + 2], dq[d][4 * j + 3]);
+            *reinterpret_cast<float4 *>(dQ + 32 * d + 8 * j + 4 * lk) = summed(dq[d], j);
     }
   }
 }
@@ -760,8 +723,8 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_dkv_f32(FlashArgs
     // K's and V's rows stay whole and are cut where they are used: in three parts, they, the accumulators and the next tile are more
     // registers than a wave of two per SIMD has (the empty assembler statements keep the cuts from being moved out of the loop).
     float k[D / 16][8], v[D / 16][8];
-    S::whole((const float *)a.k + b * a.k_sb + h * a.k_sh + (int64_t)kvi * a.k_st, live, 1.0f, a.hd, lk, k);
-    S::whole((const float *)a.v + b * a.v_sb + h * a.v_sh + (int64_t)kvi * a.v_st, live, 1.0f, a.hd, lk, v);
+    S::whole((const float *)a.k + b * a.k_sb + h * a.k_sh + (int64_t)kvi * a.k_st, live, SPLIT_UP, a.hd, lk, k);
+    S::whole((const float *)a.v + b * a.v_sb + h * a.v_sh + (int64_t)kvi * a.v_st, live, SPLIT_UP, a.hd, lk, v);
     f32x16 dk[S::F], dv[S::F];
 #pragma unroll
     for (int d = 0; d < S::F; d++)
@@ -776,10 +739,11 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_dkv_f32(FlashArgs
       if (threadIdx.x < 64) stat = qi < a.T ? (threadIdx.x < 32 ? a.lse : a.delta)[srow0 + qi] : 0.f;
     };
     load(kv_blk0);
+    bool fine = true;
     for (int q0 = kv_blk0; q0 < a.T; q0 += BC) {                   // causal: queries at or after this block's first key
       __syncthreads();
-      S::template put<true, true>(qx, a.scale, Qr, Qc);
-      S::template put<true, true>(gx, 1.0f, Gr, Gc);
+      S::template put<true, true>(qx, a.scale * SPLIT_UP, Qr, Qc);
+      S::template put<true, true>(gx, SPLIT_UP, Gr, Gc);
       if (threadIdx.x < 64) Ls[threadIdx.x] = stat;                // the second 32 are Ds
       load(q0 + BC);                                               // the next tile, while this one is multiplied; rows past the end read as zero
       __syncthreads();
@@ -800,21 +764,22 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_dkv_f32(FlashArgs
         S::get_row(Gr, lr, 2 * i + lk, f);
         mfma6(f, w, dp);
       }
+      fine = fine && all_finite(s);
       f32x16 pm;
 #pragma unroll
       for (int e = 0; e < 16; e++) {
         const int qr = 8 * (e >> 2) + 4 * lk + (e & 3), qi = q0 + qr;
-        const float sc = softcap_fwd(s[e], a.cap, inv_cap);
+        const float sc = softcap_fwd(s[e] * SPLIT_DOWN, a.cap, inv_cap);
         const float p = (kvi > qi || qi >= a.T || !live) ? 0.f : expf(sc - Ls[qr]);
-        float ds = p * (dp[e] - Ds[qr]);
+        float ds = p * __builtin_fmaf(dp[e], SPLIT_DOWN, -Ds[qr]);
         if (a.cap > 0.f) { const float t = sc * inv_cap; ds *= (1.0f - t * t); }
-        pm[e] = p;
-        s[e] = ds;                                                 // Qc already carries `scale`, so dK = dS^T (scale*Q)
+        pm[e] = p * SPLIT_UP;
+        s[e] = ds * SPLIT_UP;                                      // Qc already carries `scale`, so dK = dS^T (scale*Q)
       }
-      S::contract_rows(Gc, pm, lr, lk, dv);
-      S::contract_rows(Qc, s, lr, lk, dk);
+      S::contract_rows(Gc, pm, lr, lk, 1.0f, dv);
+      S::contract_rows(Qc, s, lr, lk, 1.0f, dk);
     }
-    if (__syncthreads_or(!all_finite<S::F>(dk) || !all_finite<S::F>(dv))) {
+    if (__syncthreads_or(!fine || !all_finite<S::F>(dk) || !all_finite<S::F>(dv))) {
       flash_dkv_exact<D>(a, bh, xblk, (float *)smem);
       return;
     }
@@ -826,8 +791,8 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_dkv_f32(FlashArgs
 #pragma unroll
         for (int j = 0; j < 4; j++) {
           if (32 * d + 8 * j + 4 * lk >= a.hd) continue;
-          *reinterpret_cast<float4 *>(dK + 32 * d + 8 * j + 4 * lk) = make_float4(dk[d][4 * j], dk[d][4 * j + 1], dk[d][4 * j + 2], dk[d][4 * j + 3]);
-          *reinterpret_cast<float4 *>(dV + 32 * d + 8 * j + 4 * lk) = make_float4(dv[d][4 * j], dv[d][4 * j + 1], dv[d][4 * j + 2], dv[d][4 * j + 3]);
+          *reinterpret_cast<float4 *>(dK + 32 * d + 8 * j + 4 * lk) = summed(dk[d], j);
+          *reinterpret_cast<float4 *>(dV + 32 * d + 8 * j + 4 * lk) = summed(dv[d], j);
         }
     }
   }

@@ -1795,6 +1795,59 @@ def test_flash_attention_f32_backward_of_values_a_bf16_part_cannot_hold(B):
     assert_close(got[2][:, 5] * 1e30, want[2][:, 5] * 1e30, what="dV of the small feature")
 
 
+@pytest.mark.parametrize("T,D", [(70, 64), (300, 32), (140, 48)])
+@pytest.mark.parametrize("eq,ek,ev,eg", [(-118, 119, 0, 0), (119, -118, 0, 0), (0, 0, -120, 0), (0, 0, 0, -121), (0, 0, -122, 100), (-140, 110, 0, -60), (0, 0, 90, 20)])
+def test_flash_attention_f32_keeps_its_bits_at_the_ends_of_the_range(B, T, D, eq, ek, ev, eg):
+    """q, k, v and the output's gradient about 2^eq, 2^ek, 2^ev and 2^eg: numbers below 2^-110, whose bf16 parts would be subnormal, and
+    sums that run the fp32 instruction.  The results are those of ordinary numbers times powers of two, so the bounds are the ones above;
+    a result about 2^-149 is rounded to that."""
+    BH, scale = 3, 1 / math.sqrt(D)
+    g = np.random.default_rng(T + D)
+    q, k, v, do = ((g.standard_normal((BH, T, D)) * 2.0 ** e).astype(np.float32) for e in (eq, ek, ev, eg))
+    Q, K, V = dev(B, q), dev(B, k), dev(B, v)
+    r = B.flashAttention(Q, K, V, T, scale, 30.0)
+    gr = B.flashAttentionBackward(Q, K, V, r["output"], dev(B, do), r["lse"], T, scale, 30.0)
+    rel = 64 * 2.0 ** -24 * math.sqrt(max(T, D))
+    for h in range(BH):
+        s = 30.0 * np.tanh((q[h].astype(np.float64) @ k[h].astype(np.float64).T) * scale / 30.0)
+        s = np.where(np.tril(np.ones((T, T), bool)), s, -np.inf)
+        e = np.exp(s - s.max(1, keepdims=True))
+        wants = {"output": e @ v[h].astype(np.float64) / e.sum(1, keepdims=True)}
+        wants.update(zip(("dQ", "dK", "dV"), _attention_grads_64(q[h], k[h], v[h], do[h], scale, 30.0)))
+        for name, want in wants.items():
+            got = np.asarray((r if name == "output" else gr)[name].data).reshape(BH, T, D)[h].astype(np.float64)
+            off = np.max(np.abs(got - want))
+            assert off <= rel * np.max(np.abs(want)) + T * 2.0 ** -149, (name, h, off / np.max(np.abs(want)))
+
+
+@pytest.mark.parametrize("large", [False, True])
+def test_flash_attention_f32_small_weights_and_large_scores_without_a_cap(B, large):
+    """Weights of 2^-115 meet the only values that are not zero; a row whose scores are all below -2^80 (the sums of the parts overflow
+    there) still has weights that add up to one."""
+    T, D, scale = 64, 64, 1.0
+    g = np.random.default_rng(1)
+    q, k, v, do = (g.standard_normal((1, T, D)).astype(np.float32) for _ in range(4))
+    q[0, :, :], k[0, :, :] = 0.0, 0.0
+    q[0, :, 0], k[0, :, 0] = 1.0, 0.0
+    k[0, :8, 0] = -80.0 - g.random(8).astype(np.float32)
+    v[0, 8:, :] = 0.0
+    v[0, :8, :] *= np.float32(2.0 ** 60)
+    if large:
+        q[0, 5, 0] = np.float32(2.0 ** 90)                          # scores of -2^96 at every visible key
+    Q, K, V = dev(B, q), dev(B, k), dev(B, v)
+    r = B.flashAttention(Q, K, V, T, scale, 0.0)
+    gr = B.flashAttentionBackward(Q, K, V, r["output"], dev(B, do), r["lse"], T, scale, 0.0)
+    s = q[0].astype(np.float64) @ k[0].astype(np.float64).T
+    s = np.where(np.tril(np.ones((T, T), bool)), s, -np.inf)
+    e = np.exp(s - s.max(1, keepdims=True))
+    want = e @ v[0].astype(np.float64) / e.sum(1, keepdims=True)
+    got = np.asarray(r["output"].data).reshape(T, D).astype(np.float64)
+    rows = np.abs(want).max(1)
+    assert np.all(np.abs(got - want).max(1) <= 64 * 2.0 ** -24 * 8 * rows)
+    dv = np.asarray(gr["dV"].data).reshape(T, D)
+    assert_close(dv, _attention_grads_64(q[0], k[0], v[0], do[0], scale, 0.0)[2], rel=64 * 2.0 ** -24 * 8, what="dV")
+
+
 @pytest.mark.parametrize("T", [256, 1024, 2048])
 @pytest.mark.parametrize("cap", [0.0, 30.0])
 def test_flash_attention_microbench_shapes(B, bwd_variant, T, cap):
