@@ -462,7 +462,8 @@ int32_t launch_choice(const F32Choice &c, const GemmArgs &ga, int batch, int vec
   return launch_split<LAYOUT, 128, 128>(ga, batch, vec_a, vec_b, vec_c, out_bf16);
 }
 
-int32_t run_choice(const F32Choice &c, const GemmArgs &ga, int layout, int batch, int out_dtype, int vec_a, int vec_b, int vec_c) {
+// Where the memory for the slices is refused, the product runs without any.
+int32_t run_choice(const F32Choice &c, const GemmArgs &ga, int layout, int batch, int out_dtype, int vec_a, int vec_b, int vec_c, bool long_rows) {
   const int ob = out_dtype == AH_BF16;
   auto go = [&](const GemmArgs &g, int nb, int vc) -> int32_t {
     switch (layout) {
@@ -480,6 +481,7 @@ int32_t run_choice(const F32Choice &c, const GemmArgs &ga, int layout, int batch
   }
   ah_ptr ws = 0;
   int32_t rc = ah_alloc((uint64_t)slices * ga.M * ga.N * 4, &ws);
+  if (rc == AH_ERR_OOM) return run_choice(choose(ga, layout, batch, false, long_rows), ga, layout, batch, out_dtype, vec_a, vec_b, vec_c, long_rows);
   if (rc) return rc;
   GemmArgs gs = ga;
   gs.ksplit = (int)slice; gs.nsplit = slices;
@@ -499,6 +501,6 @@ namespace ah {
 int32_t gemm_f32(const GemmArgs &ga, int layout, int batch, int out_dtype, int vec_a, int vec_b, int vec_c) {
   const bool may_split = batch == 1 && out_dtype == AH_F32 && (ga.epi == AH_EPI_NONE || ga.epi == AH_EPI_ACCUM) && ga.N % 4 == 0 && vec_c;
   const bool long_rows = (layout != AH_GEMM_TN && ga.lda >= (1 << 22)) || (layout == AH_GEMM_NT && ga.ldb >= (1 << 22));
-  return run_choice(choose(ga, layout, batch, may_split, long_rows), ga, layout, batch, out_dtype, vec_a, vec_b, vec_c);
+  return run_choice(choose(ga, layout, batch, may_split, long_rows), ga, layout, batch, out_dtype, vec_a, vec_b, vec_c, long_rows);
 }
 }  // namespace ah

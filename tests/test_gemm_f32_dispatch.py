@@ -1,0 +1,38 @@
+"""Which kernel an fp32 product takes, without a GPU: the built object linked with a stand-in for the runtime (gemm_f32_dispatch.hip),
+which prints what would be launched."""
+import os
+import subprocess
+from collections import namedtuple
+
+import pytest
+
+from alpha2_amd import _ffi as ffi, build
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+Launched = namedtuple("Launched", "code kernel slices blocks launches")
+
+
+@pytest.fixture(scope="module")
+def dispatch(tmp_path_factory):
+    d = tmp_path_factory.mktemp("dispatch")
+    subprocess.run([build._hipcc(), "--offload-arch=gfx950", "--cuda-host-only", "-std=c++17", "-O1", "-fPIC", "-c",
+                    os.path.join(HERE, "gemm_f32_dispatch.hip"), "-o", str(d / "main.o")], check=True, capture_output=True)
+    subprocess.run(["g++", str(d / "main.o"), build._compile("gemm_f32", False), "-o", str(d / "main")], check=True, capture_output=True)
+
+    def ask(m, n, k, layout, epi=ffi.EPI_NONE, refuse=False, lda=0):
+        line = "%d %d %d %d %d %d %d\n" % (m, n, k, layout, epi, refuse, lda)
+        out = subprocess.run([str(d / "main")], input=line, capture_output=True, text=True, check=True).stdout
+        code, kernel, slices, blocks, launches = out.rstrip("\n").split("|")
+        return Launched(int(code), kernel, int(slices), int(blocks), launches.split())
+    return ask
+
+
+def test_a_product_whose_slices_get_no_memory_runs_without_them(dispatch):
+    """64-wide and 128-wide tiles in slices, all layouts, and accumulating: the same product in one launch, nothing left allocated."""
+    for m, n, k in ((384, 128, 1030), (700, 256, 4750), (640, 768, 4096)):
+        for layout in (ffi.GEMM_NN, ffi.GEMM_NT, ffi.GEMM_TN):
+            for epi in (ffi.EPI_NONE, ffi.EPI_ACCUM):
+                sliced = dispatch(m, n, k, layout, epi)
+                assert sliced.code == 0 and sliced.slices > 1 and sliced.launches[-1] == "join" and sliced.blocks == 0
+                whole = dispatch(m, n, k, layout, epi, refuse=True)
+                assert whole.code == 0 and whole.blocks == 0 and len(whole.launches) == 1 and whole.launches[0].endswith(",%d" % k)
