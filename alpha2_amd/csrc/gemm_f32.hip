@@ -476,7 +476,7 @@ int32_t run_choice(const F32Choice &c, const GemmArgs &ga, int layout, int batch
   const int slices = c.splits > 1 ? (int)cdiv(ga.K, slice) : 1;
   if (slices <= 1) {
     const int32_t rc = go(ga, batch, vec_c);
-    note_gemm_split(c.bm == 32 ? c.waves : 1);                      // partial sums added up in fixed order
+    note_gemm_split(1);
     return rc;
   }
   ah_ptr ws = 0;

@@ -36,3 +36,12 @@ def test_a_product_whose_slices_get_no_memory_runs_without_them(dispatch):
                 assert sliced.code == 0 and sliced.slices > 1 and sliced.launches[-1] == "join" and sliced.blocks == 0
                 whole = dispatch(m, n, k, layout, epi, refuse=True)
                 assert whole.code == 0 and whole.blocks == 0 and len(whole.launches) == 1 and whole.launches[0].endswith(",%d" % k)
+
+
+def test_slices_are_reported_where_a_second_launch_joins_them(dispatch):
+    """The waves of a 32-wide piece add up their sums inside the launch: one slice."""
+    for m, n, k, layout in ((127, 260, 1000, ffi.GEMM_NN), (1, 64, 768, ffi.GEMM_NT), (500, 300, 512, ffi.GEMM_TN), (384, 128, 1030, ffi.GEMM_NN), (4000, 1200, 64, ffi.GEMM_NT)):
+        got = dispatch(m, n, k, layout)
+        assert (got.slices > 1) == (got.launches[-1] == "join"), got
+        if "pieces" in got.kernel:
+            assert got.slices == 1
