@@ -428,18 +428,21 @@ F32Choice choose(const GemmArgs &ga, int layout, int batch, bool may_split, bool
   static constexpr Tile TILES[2] = {{64, 0.26, 0.24}, {128, 1.2, 0.65}};
   static constexpr double FIRST[3] = {0.56, 1.1, 1.4}, GROUP[3] = {0.74, 0.58, 0.63}, RATE[3] = {61e6, 50e6, 100e6};      // NN, NT, TN: operations per us
   const double M = ga.M, N = ga.N, K = ga.K;
+  // a launch has fewer than 2^32 threads: a row of more than 2^30 columns leaves only the widest tiles
+  auto fits = [&](int bm, int threads) { return cdiv(ga.M, bm) * cdiv(ga.N, bm) * threads < (1ll << 32); };
   F32Choice best{32, 16, 1};
   double least = 1e300;
   for (int w = 0; w < 3; w++) {
     const int waves = 4 << w;
+    if (!fits(32, 64 * waves)) continue;
     double t = FIRST[w] + GROUP[w] * (double)cdiv(cdiv(ga.K, 16), waves * (w == 2 ? 2 : 4)) +
                (double)(cdiv(ga.M, 32) * cdiv(ga.N, 32) * batch) * 2048.0 * K / RATE[layout] * (w == 0 ? 1.0 : 1.6);
     if (layout == AH_GEMM_TN && w == 2) t += 3.5;               // spills registers
     if (t < least) { least = t; best = F32Choice{32, waves, 1}; }
   }
-  if (long_rows) return best;                                   // the tile loaders' 32-bit offsets
+  if (long_rows) return best;
   for (const Tile &q : TILES)
-    for (int s = 1; s <= (may_split ? 32 : 1); s *= 2) {
+    for (int s = 1; fits(q.bm, 256) && s <= (may_split ? 32 : 1); s *= 2) {
       if (s > 1 && (K / s < 64 || s * M * N > (1 << 27))) break;
       const double per_cu = (double)(cdiv(ga.M, q.bm) * cdiv(ga.N, q.bm) * batch * s) / num_cus();
       const double b = per_cu < 4 ? ceil(per_cu) : per_cu + 0.5, alone = q.step * (layout == AH_GEMM_TN ? 1.1 : 1.0);
@@ -500,7 +503,9 @@ int32_t run_choice(const F32Choice &c, const GemmArgs &ga, int layout, int batch
 namespace ah {
 int32_t gemm_f32(const GemmArgs &ga, int layout, int batch, int out_dtype, int vec_a, int vec_b, int vec_c) {
   const bool may_split = batch == 1 && out_dtype == AH_F32 && (ga.epi == AH_EPI_NONE || ga.epi == AH_EPI_ACCUM) && ga.N % 4 == 0 && vec_c;
-  const bool long_rows = (layout != AH_GEMM_TN && ga.lda >= (1 << 22)) || (layout == AH_GEMM_NT && ga.ldb >= (1 << 22));
+  // the tile loaders' offsets within a tile are 32 bits: its rows, 128 at most, span less than 4 GiB
+  auto spans = [](int rows, int64_t ld) { return ((rows < 128 ? rows : 128) - 1) * ld + 16 >= (1ll << 30); };
+  const bool long_rows = (layout != AH_GEMM_TN && spans(ga.M, ga.lda)) || (layout == AH_GEMM_NT && spans(ga.N, ga.ldb));
   return run_choice(choose(ga, layout, batch, may_split, long_rows), ga, layout, batch, out_dtype, vec_a, vec_b, vec_c, long_rows);
 }
 }  // namespace ah

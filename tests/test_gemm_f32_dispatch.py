@@ -45,3 +45,19 @@ def test_slices_are_reported_where_a_second_launch_joins_them(dispatch):
         assert (got.slices > 1) == (got.launches[-1] == "join"), got
         if "pieces" in got.kernel:
             assert got.slices == 1
+
+
+def test_a_launch_stays_below_two_to_the_32_threads(dispatch):
+    """Rows of more than 2^30 columns, also where the rows of A lie far apart, and 2^30 rows of one column."""
+    for m, n, k, lda in ((1, 1100000000, 1, 0), (1, 2100000000, 1, 0), (1, 1100000000, 1, 1 << 22), (2, 600000000, 1, 1 << 22), (1 << 30, 1, 1, 0)):
+        for layout in (ffi.GEMM_NN, ffi.GEMM_NT, ffi.GEMM_TN):
+            got = dispatch(m, n, k, layout, lda=lda)
+            assert got.code == 0 and all(int(x.split(",")[0]) < 1 << 32 for x in got.launches if x != "join"), (m, n, lda, layout, got)
+
+
+def test_rows_that_lie_far_apart_keep_the_tiles_out(dispatch):
+    """128 rows of A (or B) a tile spans: less than 4 GiB for its 32-bit offsets."""
+    inside, outside = (1 << 30) // 127 - 16, (1 << 30) // 127 + 16
+    assert "split" in dispatch(8200, 640, 33, ffi.GEMM_NN, lda=inside).kernel
+    assert "pieces" in dispatch(8200, 640, 33, ffi.GEMM_NN, lda=outside).kernel
+    assert "split" in dispatch(8200, 640, 33, ffi.GEMM_TN, lda=outside).kernel
