@@ -84,7 +84,7 @@ __device__ __forceinline__ void finish_tile(const GemmArgs &g, int64_t cbase, in
 }
 
 // The BM x BN tile at (m0, n0) by v_mfma_f32_32x32x2_f32, 2 x 2 waves; smem holds 2 * F_BK * (BM + BN + 2 F_PAD) floats.
-template <bool A_KC, bool B_KC, int BM, int BN>
+template <bool A_KC, bool B_KC, int BM, int BN, bool VEC>
 __device__ __forceinline__ void f32_tile(const GemmArgs &g, const float *A, const float *B, int64_t cbase, int m0, int n0, bool vec_c, int out_bf16, float *smem) {
   constexpr int PA = BM + F_PAD, PB = BN + F_PAD, TM = BM / 64, TN = BN / 64;
   float *As = smem, *Bs = smem + 2 * F_BK * PA;
@@ -102,15 +102,24 @@ __device__ __forceinline__ void f32_tile(const GemmArgs &g, const float *A, cons
     const int r = (kc ? t >> 2 : t & 63) + 64 * i, k = kc ? (t & 3) * 4 : (t >> 6) * 4;
     s[(k + 0) * pitch + r] = v.x; s[(k + 1) * pitch + r] = v.y; s[(k + 2) * pitch + r] = v.z; s[(k + 3) * pitch + r] = v.w;
   };
-  const int nt = (g.K + F_BK - 1) / F_BK;
+  const int full = g.K / F_BK, nt = (g.K + F_BK - 1) / F_BK;
+  auto load = [&](int kt) {
+    if (kt < full) {
+      load_tile<A_KC, BM, VEC, false>(A, g.lda, m0, kt * F_BK, g.M, g.K, ra);
+      load_tile<B_KC, BN, VEC, false>(B, g.ldb, n0, kt * F_BK, g.N, g.K, rb);
+    } else if (kt < nt) {
+      load_tile<A_KC, BM, VEC, true>(A, g.lda, m0, kt * F_BK, g.M, g.K, ra);
+      load_tile<B_KC, BN, VEC, true>(B, g.ldb, n0, kt * F_BK, g.N, g.K, rb);
+    }
+  };
+  load(0);
   for (int kt = 0; kt < nt; kt++) {
-    load_tile<A_KC, BM, false, true>(A, g.lda, m0, kt * F_BK, g.M, g.K, ra);
-    load_tile<B_KC, BN, false, true>(B, g.ldb, n0, kt * F_BK, g.N, g.K, rb);
     float *as = As + (kt & 1) * F_BK * PA, *bs = Bs + (kt & 1) * F_BK * PB;
 #pragma unroll
     for (int i = 0; i < BM / 64; i++) store(as, PA, A_KC, ra[i], i);
 #pragma unroll
     for (int i = 0; i < BN / 64; i++) store(bs, PB, B_KC, rb[i], i);
+    load(kt + 1);                               // on its way while this one is multiplied
     __syncthreads();                            // the other buffer was last read before the previous barrier
 #pragma unroll
     for (int kk = 0; kk < F_BK / 2; kk++) {
@@ -199,8 +208,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f32_split(GemmArgs g, int vec_c
   constexpr bool B_KC = (LAYOUT == AH_GEMM_NT);     // B is [N][K] only for NT
   constexpr int TM = BM / 64, TN = BN / 64;
   constexpr int ABYTES = 3 * BM * 32, BBYTES = 3 * BN * 32;
-  constexpr int FM = BM < 128 ? BM : 128, FN = BN < 128 ? BN : 128;         // the piece of the tile f32_tile takes at a time
-  constexpr int SPLIT_LDS = 2 * (ABYTES + BBYTES), F32_LDS = 2 * F_BK * (FM + FN + 2 * F_PAD) * 4;
+  constexpr int SPLIT_LDS = 2 * (ABYTES + BBYTES), F32_LDS = 2 * F_BK * (BM + BN + 2 * F_PAD) * 4;
   __shared__ __attribute__((aligned(16))) char smem[SPLIT_LDS > F32_LDS ? SPLIT_LDS : F32_LDS];
   const float *A = (const float *)g.a + (int64_t)blockIdx.z * g.sa;
   const float *B = (const float *)g.b + (int64_t)blockIdx.z * g.sb;
@@ -286,12 +294,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f32_split(GemmArgs g, int vec_c
 #pragma unroll
     for (int j = 0; j < TN; j++) fine = fine && all_finite(sum[i][j]);
   if (__syncthreads_or(!fine)) {
-    for (int i = 0; i < BM; i += FM)
-      for (int j = 0; j < BN; j += FN) {
-        if (m0 + i >= g.M || n0 + j >= g.N) continue;
-        f32_tile<A_KC, B_KC, FM, FN>(g, A, B, cbase, m0 + i, n0 + j, vec_c, out_bf16, (float *)smem);
-        __syncthreads();
-      }
+    f32_tile<A_KC, B_KC, BM, BN, VEC>(g, A, B, cbase, m0, n0, vec_c, out_bf16, (float *)smem);
     return;
   }
 #pragma unroll
