@@ -46,10 +46,9 @@ __device__ __forceinline__ void load_tile_f32(float *s, const float *__restrict_
 //   columns  [feature][row'], row' = 16 j + 8 h + 4 i + r of row 16 j + 8 i + 4 h + r: an operand is the 8 rows whose scores the
 //            lanes of half h hold in accumulator elements 8 j .. 8 j + 7, so that those go straight into the other operand
 // 16-byte pieces are permuted within a row so that 16 lanes that read the same piece of 16 rows meet 64 different banks.
-// A result that is not finite has the block computed again with the fp32 instruction, whose result stands; so does a score (an
-// infinite one gives weights that look like any other).
+// A result that is not finite has the block computed again with the fp32 instruction, whose result stands; so does a score.
 // 192 heads x 1024 x 64: dK and dV 945 -> 486 us, dQ 520 -> 316; 512 x 256 x 32: 112 -> 84 and 81 -> 60; 4 x 70 x 64: 29 -> 24 and
-// 26 -> 20.  Relative error against 64 bits at 4 x 512 x 64: dQ 4.6e-7 -> 3.7e-7, dK 6.4e-7 -> 3.8e-7, dV 6.0e-7 -> 3.3e-7.  What bounds
+// 26 -> 20 (before both operands were scaled, which costs 2 % of the backward pass at 192 x 1024 x 64 and 6 % at 12 x 64 x 64).  Relative error against 64 bits at 4 x 512 x 64: dQ 4.6e-7 -> 3.7e-7, dK 6.4e-7 -> 3.8e-7, dV 6.0e-7 -> 3.3e-7.  What bounds
 // it now is vector issue: tanh, exp and the cut of scores, K and V for every 32 x 32 tile beside 3072 cycles of matrix instructions.
 template <int D>
 struct SplitTile {                          // D = 32 or 64
@@ -69,6 +68,12 @@ struct SplitTile {                          // D = 32 or 64
         x[r][0] = in ? p[0] : 0.f;
       }
     }
+  }
+  static __device__ __forceinline__ float largest(const float (&x)[4][F]) {
+    float top = 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; r++) top = F == 2 ? fmaxf(fmaxf(top, fabsf(x[r][0])), fabsf(x[r][F - 1])) : fmaxf(top, fabsf(x[r][0]));
+    return top;
   }
   static __device__ __forceinline__ int row_ofs(int row, int chunk) { return row * 2 * D + ((chunk ^ ((row * D >> 7) & (D / 8 - 1))) << 4); }
   static __device__ __forceinline__ int col_ofs(int d, int chunk) { return d * 64 + ((chunk ^ ((d >> 2) & 3)) << 4); }
@@ -152,6 +157,20 @@ struct SplitTile {                          // D = 32 or 64
     }
   }
 };
+// A raw score (times 2^48) scaled back and capped; factor: what split_cap_factor gives
+__device__ __forceinline__ float split_cap(float s, float cap, float factor) { return softcap_fwd(s * factor, cap, 1.0f); }
+__device__ __forceinline__ float split_cap_factor(float cap) { return (cap > 0.f ? 1.0f / cap : 1.0f) * SPLIT_DOWN; }
+// (a cap whose factor is no normal number is left to the fp32 instruction)
+__device__ __forceinline__ bool split_cap_ok(float cap) { return !(cap > 0x1p70f); }
+// An infinite score has to be found before it is capped or weighed: what is made of it looks like any other.  (NaN shows in that.)  Either
+// at the scores, or where the operands of all of them are below LARGE_OPERAND: 64 products of those, times 2^48, stay below 2^127.
+__device__ __forceinline__ bool scores_finite(const f32x16 &s) {
+  float top = 0.f;
+#pragma unroll
+  for (int e = 0; e < 16; e += 2) top = fmaxf(fmaxf(top, fabsf(s[e])), fabsf(s[e + 1]));
+  return top < INFINITY;
+}
+constexpr float LARGE_OPERAND = 0x1p36f;
 // quarter j of an accumulator of products, as it is stored
 __device__ __forceinline__ float4 summed(const f32x16 &x, int j) {
   return make_float4(x[4 * j] * SPLIT_DOWN, x[4 * j + 1] * SPLIT_DOWN, x[4 * j + 2] * SPLIT_DOWN, x[4 * j + 3] * SPLIT_DOWN);
@@ -259,7 +278,7 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_fwd_f32(FlashArgs
     const int q0 = xblk * (WAVES * 32) + wave * 32, qi = q0 + lr;
     const float *K = (const float *)a.k + b * a.k_sb + h * a.k_sh;
     const float *V = (const float *)a.v + b * a.v_sb + h * a.v_sh;
-    const float inv_cap = a.cap > 0.f ? 1.0f / a.cap : 0.f;
+    const float factor = split_cap_factor(a.cap);
     bf16x8 q[D / 16][3];
     S::own((const float *)a.q + b * a.q_sb + h * a.q_sh + (int64_t)qi * a.q_st, qi < a.T, a.scale * SPLIT_UP, a.hd, lk, q);
     f32x16 o[S::F];
@@ -272,7 +291,7 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_fwd_f32(FlashArgs
     float kx[4][S::F], vx[4][S::F];
     S::load(kx, K, a.k_st, 0, a.T, a.hd);
     S::load(vx, V, a.v_st, 0, a.T, a.hd);
-    bool fine = true;
+    bool fine = split_cap_ok(a.cap);
     for (int kv0 = 0; kv0 < end; kv0 += BC) {
       __syncthreads();
       S::template put<true, false>(kx, SPLIT_UP, Kr, nullptr);
@@ -290,12 +309,12 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_fwd_f32(FlashArgs
         S::get_row(Kr, lr, 2 * i + lk, f);
         mfma6(f, q[i], s[0]);
       }
-      fine = fine && all_finite<1>(s);                             // a maximum passes NaN by
+      fine = fine && all_finite(s[0]);
       float tmax = -INFINITY;
 #pragma unroll
       for (int e = 0; e < 16; e++) {
         const int kv = kv0 + 8 * (e >> 2) + 4 * lk + (e & 3);
-        float x = softcap_fwd(s[0][e] * SPLIT_DOWN, a.cap, inv_cap);
+        float x = split_cap(s[0][e], a.cap, factor);
         x = (kv > qi || kv >= a.T) ? -INFINITY : x;
         s[0][e] = x;
         tmax = fmaxf(tmax, x);
@@ -555,7 +574,7 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_dq_f32(FlashArgs 
     const int q0 = xblk * (WAVES * 32) + wave * 32, qi = q0 + lr;
     const float *K = (const float *)a.k + b * a.k_sb + h * a.k_sh;
     const float *V = (const float *)a.v + b * a.v_sb + h * a.v_sh;
-    const float inv_cap = a.cap > 0.f ? 1.0f / a.cap : 0.f;
+    const float inv_cap = a.cap > 0.f ? 1.0f / a.cap : 0.f, factor = split_cap_factor(a.cap);
     const bool live = qi < a.T;
     bf16x8 q[D / 16][3], go[D / 16][3];
     S::own((const float *)a.q + b * a.q_sb + h * a.q_sh + (int64_t)qi * a.q_st, live, a.scale * SPLIT_UP, a.hd, lk, q);
@@ -571,7 +590,7 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_dq_f32(FlashArgs 
     float kx[4][S::F], vx[4][S::F];
     S::load(kx, K, a.k_st, 0, a.T, a.hd);
     S::load(vx, V, a.v_st, 0, a.T, a.hd);
-    bool fine = true;
+    bool fine = split_cap_ok(a.cap);
     for (int kv0 = 0; kv0 < end; kv0 += BC) {
       __syncthreads();
       S::template put<true, true>(kx, SPLIT_UP, Kr, Kc);
@@ -591,11 +610,11 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_dq_f32(FlashArgs 
         S::get_row(Vr, lr, 2 * i + lk, f);
         mfma6(f, go[i], dp);
       }
-      fine = fine && all_finite(s);
+      fine = fine && scores_finite(s);
 #pragma unroll
       for (int e = 0; e < 16; e++) {
         const int kv = kv0 + 8 * (e >> 2) + 4 * lk + (e & 3);
-        const float sc = softcap_fwd(s[e] * SPLIT_DOWN, a.cap, inv_cap);
+        const float sc = split_cap(s[e], a.cap, factor);
         const float p = (kv > qi || kv >= a.T || !live) ? 0.f : expf(sc - lse);
         float ds = p * __builtin_fmaf(dp[e], SPLIT_DOWN, -delta);
         if (a.cap > 0.f) { const float t = sc * inv_cap; ds *= (1.0f - t * t); }
@@ -718,13 +737,19 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_dkv_f32(FlashArgs
     const int kv_blk0 = xblk * (WAVES * 32), kv0 = kv_blk0 + wave * 32, kvi = kv0 + lr;
     const float *Q = (const float *)a.q + b * a.q_sb + h * a.q_sh;
     const float *dO = (const float *)a.d_o + b * a.o_sb + h * a.o_sh;
-    const float inv_cap = a.cap > 0.f ? 1.0f / a.cap : 0.f;
+    const float inv_cap = a.cap > 0.f ? 1.0f / a.cap : 0.f, factor = split_cap_factor(a.cap);
     const bool live = kvi < a.T;
     // K's and V's rows stay whole and are cut where they are used: in three parts, they, the accumulators and the next tile are more
     // registers than a wave of two per SIMD has (the empty assembler statements keep the cuts from being moved out of the loop).
     float k[D / 16][8], v[D / 16][8];
     S::whole((const float *)a.k + b * a.k_sb + h * a.k_sh + (int64_t)kvi * a.k_st, live, SPLIT_UP, a.hd, lk, k);
     S::whole((const float *)a.v + b * a.v_sb + h * a.v_sh + (int64_t)kvi * a.v_st, live, SPLIT_UP, a.hd, lk, v);
+    float top = 0.f;
+#pragma unroll
+    for (int i = 0; i < D / 16; i++)
+#pragma unroll
+      for (int e = 0; e < 8; e++) top = fmaxf(top, fabsf(k[i][e]));
+    bool fine = split_cap_ok(a.cap) && top < LARGE_OPERAND * SPLIT_UP;
     f32x16 dk[S::F], dv[S::F];
 #pragma unroll
     for (int d = 0; d < S::F; d++)
@@ -739,9 +764,9 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_dkv_f32(FlashArgs
       if (threadIdx.x < 64) stat = qi < a.T ? (threadIdx.x < 32 ? a.lse : a.delta)[srow0 + qi] : 0.f;
     };
     load(kv_blk0);
-    bool fine = true;
     for (int q0 = kv_blk0; q0 < a.T; q0 += BC) {                   // causal: queries at or after this block's first key
       __syncthreads();
+      fine = fine && S::largest(qx) * fabsf(a.scale) < LARGE_OPERAND;
       S::template put<true, true>(qx, a.scale * SPLIT_UP, Qr, Qc);
       S::template put<true, true>(gx, SPLIT_UP, Gr, Gc);
       if (threadIdx.x < 64) Ls[threadIdx.x] = stat;                // the second 32 are Ds
@@ -764,17 +789,16 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_dkv_f32(FlashArgs
         S::get_row(Gr, lr, 2 * i + lk, f);
         mfma6(f, w, dp);
       }
-      fine = fine && all_finite(s);
       f32x16 pm;
 #pragma unroll
       for (int e = 0; e < 16; e++) {
         const int qr = 8 * (e >> 2) + 4 * lk + (e & 3), qi = q0 + qr;
-        const float sc = softcap_fwd(s[e] * SPLIT_DOWN, a.cap, inv_cap);
-        const float p = (kvi > qi || qi >= a.T || !live) ? 0.f : expf(sc - Ls[qr]);
+        const float sc = split_cap(s[e], a.cap, factor);
+        const float p = (kvi > qi || qi >= a.T || !live) ? 0.f : expf(sc - Ls[qr]) * SPLIT_UP;
         float ds = p * __builtin_fmaf(dp[e], SPLIT_DOWN, -Ds[qr]);
         if (a.cap > 0.f) { const float t = sc * inv_cap; ds *= (1.0f - t * t); }
-        pm[e] = p * SPLIT_UP;
-        s[e] = ds * SPLIT_UP;                                      // Qc already carries `scale`, so dK = dS^T (scale*Q)
+        pm[e] = p;
+        s[e] = ds;                                      // Qc already carries `scale`, so dK = dS^T (scale*Q)
       }
       S::contract_rows(Gc, pm, lr, lk, 1.0f, dv);
       S::contract_rows(Qc, s, lr, lk, 1.0f, dk);
