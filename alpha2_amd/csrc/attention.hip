@@ -4,8 +4,8 @@
 //   s = scale * q.k;  s = cap * tanh(s / cap) when cap > 0;  keys after the query are masked;
 //   P = softmax(s);  O = P V;  LSE = max + log(sum exp).
 //
-// fp32 path: v_mfma_f32_32x32x2_f32 (head sizes up to 64, but for few queries forward: bf16 matrix instructions on three parts, below).  One wave owns 32 query rows (forward, dQ) or 32 key rows (dK/dV)
-// and the products are arranged so that the owned index is the accumulator COLUMN (= lane % 32):
+// fp32 path: v_mfma_f32_32x32x2_f32; for head sizes up to 64 bf16 matrix instructions on three parts of every operand (below).
+// One wave owns 32 query rows (forward, dQ) or 32 key rows (dK/dV), and the products are arranged so that the owned index is the accumulator COLUMN (= lane % 32):
 //   forward / dQ : S^T[kv, q] = K Q^T, so a lane holds 16 kv entries of one query row and the running
 //                  max / sum / rescale are per-lane scalars (one cross-half shuffle per tile);
 //                  O^T[d, q] += V^T[d, kv] P^T[kv, q] takes P^T straight from the accumulator registers.
@@ -177,13 +177,14 @@ __device__ __forceinline__ float4 summed(const f32x16 &x, int j) {
 }
 
 // ------------------------------------------------------------------------------------------ forward
+// The 32 queries from q0 on of every wave that asks for them (`redo`, the same for a wave), keys below `end` (the same for the block)
 template <int D>
-__device__ void flash_fwd_exact(const FlashArgs &a, int bh, int xblk, float *smem) {
+__device__ void flash_fwd_exact(const FlashArgs &a, int bh, int q0, int end, bool redo, float *smem) {
   constexpr int P = D + 1, DB = D / 32;
   float *Ks = smem, *Vs = Ks + BC * P;
   int b = bh / a.H, h = bh % a.H;
-  int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 31, lk = lane >> 5;
-  int q0 = xblk * (WAVES * 32) + wave * 32, qi = q0 + lr;
+  int lane = threadIdx.x & 63, lr = lane & 31, lk = lane >> 5;
+  int qi = q0 + lr;
   const float *Q = (const float *)a.q + b * a.q_sb + h * a.q_sh;
   const float *K = (const float *)a.k + b * a.k_sb + h * a.k_sh;
   const float *V = (const float *)a.v + b * a.v_sb + h * a.v_sh;
@@ -200,13 +201,12 @@ __device__ void flash_fwd_exact(const FlashArgs &a, int bh, int xblk, float *sme
     for (int e = 0; e < 16; e++) o[d][e] = 0.f;
   float m = -INFINITY, l = 0.f;
 
-  int q_block_end = min(a.T, (xblk + 1) * (WAVES * 32));   // causal: keys < q_block_end
-  for (int kv0 = 0; kv0 < q_block_end; kv0 += BC) {
+  for (int kv0 = 0; kv0 < end; kv0 += BC) {
     __syncthreads();
     load_tile_f32<D>(Ks, K, a.k_st, kv0, a.T, 1.0f, a.hd);
     load_tile_f32<D>(Vs, V, a.v_st, kv0, a.T, 1.0f, a.hd);
     __syncthreads();
-    if (kv0 > q0 + 31) continue;                      // whole tile is in this wave's future (uniform per wave)
+    if (!redo || kv0 > q0 + 31) continue;             // whole tile is in this wave's future (uniform per wave)
     f32x16 s;
 #pragma unroll
     for (int e = 0; e < 16; e++) s[e] = 0.f;
@@ -243,7 +243,7 @@ __device__ void flash_fwd_exact(const FlashArgs &a, int bh, int xblk, float *sme
         o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(Vs[kvr * P + 32 * d + lr], s[e], o[d], 0, 0, 0);
       }
   }
-  if (qi < a.T) {
+  if (redo && qi < a.T) {
     float inv_l = l > 0.f ? 1.0f / l : 0.f;
     float *O = (float *)a.o + b * a.o_sb + h * a.o_sh + (int64_t)qi * a.o_st;
 #pragma unroll
@@ -257,8 +257,36 @@ __device__ void flash_fwd_exact(const FlashArgs &a, int bh, int xblk, float *sme
   }
 }
 
-// Four waves of 32 queries.  192 heads x 1024 x 64: 383 us with the fp32 instruction, now 294; 48 heads 199 -> 128; 512 x 256 x 32 61 -> 48;
-// relative error against 64 bits at 4 x 512 x 64 2.0e-7 (fp32 instruction, keys among waves: 2.4e-7).  Vector issue bounds it, as in backward.
+// Two kernels compute the forward pass of head sizes up to 64, and a row's result does not depend on which: both do the operations
+// below on the tiles of 32 keys in ascending order, each with the same operands and roundings.
+// Raw scores of the tile at key kv0 (times 2^48, row = key, column = this lane's query qi) -> capped and masked; the column's largest
+__device__ __forceinline__ float tile_scores(f32x16 &s, const FlashArgs &a, float factor, int kv0, int qi, int lk) {
+#pragma clang fp contract(off)
+  float top = -INFINITY;
+#pragma unroll
+  for (int e = 0; e < 16; e++) {
+    const int kv = kv0 + 8 * (e >> 2) + 4 * lk + (e & 3);
+    float x = split_cap(s[e], a.cap, factor);
+    x = (kv > qi || kv >= a.T) ? -INFINITY : x;
+    s[e] = x;
+    top = fmaxf(top, x);
+  }
+  return fmaxf(top, __shfl_xor(top, 32, 64));
+}
+// Scores -> weights against the largest score so far, times 2^24; the column's sum of them, and what sums so far are multiplied by
+__device__ __forceinline__ float tile_weights(f32x16 &s, float before, float top, float &alpha) {
+#pragma clang fp contract(off)
+  const float m = fmaxf(before, top), use = m == -INFINITY ? 0.f : m;
+  alpha = expf(before - use);
+  float sum = 0.f;
+#pragma unroll
+  for (int e = 0; e < 16; e++) { const float p = expf(s[e] - use); s[e] = p * SPLIT_UP; sum += p; }
+  return sum + __shfl_xor(sum, 32, 64);
+}
+__device__ __forceinline__ float output_factor(float l) { return (l > 0.f ? 1.0f / l : 0.f) * SPLIT_DOWN; }
+
+// Four waves of 32 queries.  192 heads x 1024 x 64: 383 us with the fp32 instruction, now 308; 512 x 256 x 32 61 -> 52; relative error
+// against 64 bits at 4 x 512 x 64 2.0e-7 (fp32 instruction: 2.4e-7).  Vector issue bounds it, as in backward.
 // Head sizes over 64 keep the fp32 instruction: their operands do not fit the registers in three parts.
 template <int D>
 __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_fwd_f32(FlashArgs a) {
@@ -266,16 +294,16 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_fwd_f32(FlashArgs
   int bh, xblk;
   flash_block(bh, xblk, flash_head_group(a.T, D, 4));
   xblk = gridDim.x - 1 - xblk;                                     // longest (latest) query blocks are scheduled first
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 31, lk = lane >> 5;
+  const int q0 = xblk * (WAVES * 32) + wave * 32, qi = q0 + lr, end = min(a.T, (xblk + 1) * (WAVES * 32));      // causal: keys < end
   if constexpr (D > 64) {
     __shared__ float smem[EXACT / 4];
-    flash_fwd_exact<D>(a, bh, xblk, smem);
+    flash_fwd_exact<D>(a, bh, q0, end, true, smem);
   } else {
     using S = SplitTile<D>;
     __shared__ __attribute__((aligned(16))) char smem[2 * S::BYTES > EXACT ? 2 * S::BYTES : EXACT];
     char *Kr = smem, *Vc = smem + S::BYTES;
     const int b = bh / a.H, h = bh % a.H;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 31, lk = lane >> 5;
-    const int q0 = xblk * (WAVES * 32) + wave * 32, qi = q0 + lr;
     const float *K = (const float *)a.k + b * a.k_sb + h * a.k_sh;
     const float *V = (const float *)a.v + b * a.v_sb + h * a.v_sh;
     const float factor = split_cap_factor(a.cap);
@@ -287,7 +315,6 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_fwd_f32(FlashArgs
 #pragma unroll
       for (int e = 0; e < 16; e++) o[d][e] = 0.f;
     float m = -INFINITY, l = 0.f;
-    const int end = min(a.T, (xblk + 1) * (WAVES * 32));           // causal: keys < end
     float kx[4][S::F], vx[4][S::F];
     S::load(kx, K, a.k_st, 0, a.T, a.hd);
     S::load(vx, V, a.v_st, 0, a.T, a.hd);
@@ -300,172 +327,172 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_fwd_f32(FlashArgs
       S::load(vx, V, a.v_st, kv0 + BC, a.T, a.hd);
       __syncthreads();
       if (kv0 > q0 + 31) continue;                                 // whole tile is in this wave's future (uniform per wave)
-      f32x16 s[1];
+      f32x16 s;
 #pragma unroll
-      for (int e = 0; e < 16; e++) s[0][e] = 0.f;
+      for (int e = 0; e < 16; e++) s[e] = 0.f;
 #pragma unroll
       for (int i = 0; i < D / 16; i++) {
         bf16x8 f[3];
         S::get_row(Kr, lr, 2 * i + lk, f);
-        mfma6(f, q[i], s[0]);
+        mfma6(f, q[i], s);
       }
-      fine = fine && all_finite(s[0]);
-      float tmax = -INFINITY;
-#pragma unroll
-      for (int e = 0; e < 16; e++) {
-        const int kv = kv0 + 8 * (e >> 2) + 4 * lk + (e & 3);
-        float x = split_cap(s[0][e], a.cap, factor);
-        x = (kv > qi || kv >= a.T) ? -INFINITY : x;
-        s[0][e] = x;
-        tmax = fmaxf(tmax, x);
-      }
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-      const float m_new = fmaxf(m, tmax), m_use = m_new == -INFINITY ? 0.f : m_new;
-      const float alpha = expf(m - m_use);
-      float psum = 0.f;
-#pragma unroll
-      for (int e = 0; e < 16; e++) { const float p = expf(s[0][e] - m_use); s[0][e] = p * SPLIT_UP; psum += p; }
-      psum += __shfl_xor(psum, 32, 64);
-      l = l * alpha + psum;
-      m = m_new;
-      S::contract_rows(Vc, s[0], lr, lk, alpha, o);
+      fine = fine && all_finite(s);
+      const float top = tile_scores(s, a, factor, kv0, qi, lk);
+      float alpha;
+      const float sum = tile_weights(s, m, top, alpha);
+      l = __builtin_fmaf(l, alpha, sum);
+      m = fmaxf(m, top);
+      S::contract_rows(Vc, s, lr, lk, alpha, o);
     }
-    if (__syncthreads_or(!fine || !all_finite<S::F>(o))) {
-      flash_fwd_exact<D>(a, bh, xblk, (float *)smem);
-      return;
-    }
-    if (qi < a.T) {
-      const float inv_l = (l > 0.f ? 1.0f / l : 0.f) * SPLIT_DOWN;
+    fine = __all(fine && all_finite<S::F>(o));
+    if (fine && qi < a.T) {
+      const float f = output_factor(l);
       float *O = (float *)a.o + b * a.o_sb + h * a.o_sh + (int64_t)qi * a.o_st;
 #pragma unroll
       for (int d = 0; d < S::F; d++)
 #pragma unroll
         for (int j = 0; j < 4; j++)
           if (32 * d + 8 * j + 4 * lk < a.hd)
-            *reinterpret_cast<float4 *>(O + 32 * d + 8 * j + 4 * lk) = make_float4(o[d][4 * j] * inv_l, o[d][4 * j + 1] * inv_l, o[d][4 * j + 2] * inv_l, o[d][4 * j + 3] * inv_l);
+            *reinterpret_cast<float4 *>(O + 32 * d + 8 * j + 4 * lk) = make_float4(o[d][4 * j] * f, o[d][4 * j + 1] * f, o[d][4 * j + 2] * f, o[d][4 * j + 3] * f);
       if (lk == 0) a.lse[((int64_t)b * a.H + h) * a.T + qi] = m + logf(l);
     }
+    if (__syncthreads_or(!fine)) flash_fwd_exact<D>(a, bh, q0, end, !fine, (float *)smem);
   }
 }
 
-// The same for few blocks of 128 queries: a block owns 32 query rows and its W waves share the keys, wave w taking the tiles
-// w, w + W, ... with a running max / sum / output of its own; the W of them are joined in LDS at the end, in the order of the waves.
-// K and V go from memory straight into the operand registers: the contraction over features may take them in any order as long as
-// both operands do, so half lane/32 owns the features (D/2)*half .. and reads 16 bytes of its key's row at a time; a V operand is 32
-// features of one key side by side.  No LDS and no barrier before the join.
-// What bounds the kernel above there is its serial chain, T / 32 tiles one after the other on a few CUs.
-template <int D, int W>
-__global__ __launch_bounds__(64 * W) void k_flash_fwd_f32_keys(FlashArgs a) {
-  constexpr int DB = D / 32, H4 = D / 8;
-  __shared__ float4 part[W * 4 * 64];
-  __shared__ float Ms[W * 32], Lsum[W * 32];
+// The same for few blocks of 128 queries, where the chain of T / 32 tiles one after the other on a few CUs bounds the kernel above: a
+// block owns 32 queries, and its 8 waves take 8 tiles at a time.  Each has its tile's scores, K and V straight from memory in the
+// operand registers; the waves tell one another their columns' largest scores, so that each weighs its tile against the largest
+// up to it, as the kernel above does; and the 8 products are added up in LDS in the order of the tiles, a thread holding two
+// features of a query from each 32.  12 heads x 500 x 64: 61 us by the kernel above, 23 here (36 with sums of its own for every wave, by
+// the fp32 instruction, whose last bits then depended on the number of heads); x 1024: 118, 61 (95); x 64: 11.7, 9.8.
+template <int D>
+__global__ __launch_bounds__(512, 2) void k_flash_fwd_f32_keys(FlashArgs a) {
+  using S = SplitTile<D>;
+  constexpr int W = 8, EXACT = 2 * BC * (D + 1) * 4, PART = W * 4096;
+  __shared__ __attribute__((aligned(16))) char smem[PART > EXACT ? PART : EXACT];
+  __shared__ float Top[W * 32], Alpha[W * 32], Sum[W * 32];
   int bh, xblk;
   flash_block(bh, xblk, flash_head_group(a.T, D, 4));
   xblk = gridDim.x - 1 - xblk;                                     // longest (latest) query blocks are scheduled first
   const int b = bh / a.H, h = bh % a.H;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 31, lk = lane >> 5;
-  const int q0 = xblk * 32, qi = q0 + lr;
-  const float *Q = (const float *)a.q + b * a.q_sb + h * a.q_sh;
+  const int q0 = xblk * 32, qi = q0 + lr, tiles = xblk + 1;
+  const int r = threadIdx.x >> 4, c = threadIdx.x & 15;            // the sums: query q0 + r, features 2 c and 2 c + 1 of each 32
   const float *K = (const float *)a.k + b * a.k_sb + h * a.k_sh;
   const float *V = (const float *)a.v + b * a.v_sb + h * a.v_sh;
-  const float inv_cap = a.cap > 0.f ? 1.0f / a.cap : 0.f;
-  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-  // 4 H4 features of a row, those of this half
-  auto row = [&](const float *p, float mul, float4 (&r)[H4]) {
+  const float factor = split_cap_factor(a.cap);
+  bf16x8 q[D / 16][3];
+  S::own((const float *)a.q + b * a.q_sb + h * a.q_sh + (int64_t)qi * a.q_st, qi < a.T, a.scale * SPLIT_UP, a.hd, lk, q);
+  float k[D / 16][8], v[S::F][16];
+  auto load = [&](int i) {                                         // rows past the end read as zero
+    if (i >= tiles) return;
+    S::whole(K + (int64_t)(32 * i + lr) * a.k_st, 32 * i + lr < a.T, 1.0f, a.hd, lk, k);
 #pragma unroll
-    for (int i = 0; i < H4; i++) {
-      const int d = lk * (D / 2) + 4 * i;
-      r[i] = d < a.hd ? *reinterpret_cast<const float4 *>(p + d) : zero;
-      r[i].x *= mul; r[i].y *= mul; r[i].z *= mul; r[i].w *= mul;
-    }
-  };
-  float4 q[H4], k[H4];
-  row(Q + (int64_t)min(qi, a.T - 1) * a.q_st, a.scale, q);         // rows past the end repeat the last one: not stored, masked as keys
-
-  f32x16 o[DB];
-#pragma unroll
-  for (int d = 0; d < DB; d++)
-#pragma unroll
-    for (int e = 0; e < 16; e++) o[d][e] = 0.f;
-  float m = -INFINITY, l = 0.f;
-  for (int kv0 = wave * 32; kv0 <= q0; kv0 += W * 32) {
-    row(K + (int64_t)min(kv0 + lr, a.T - 1) * a.k_st, 1.0f, k);
-    float v[DB][16];
-#pragma unroll
-    for (int d = 0; d < DB; d++)
+    for (int d = 0; d < S::F; d++)
 #pragma unroll
       for (int e = 0; e < 16; e++) {
-        const int kv = min(kv0 + 8 * (e >> 2) + 4 * lk + (e & 3), a.T - 1);
-        v[d][e] = 32 * d + lr < a.hd ? V[(int64_t)kv * a.v_st + 32 * d + lr] : 0.f;
+        const int kv = 32 * i + 8 * (e >> 2) + 4 * lk + (e & 3);
+        v[d][e] = kv < a.T && 32 * d + lr < a.hd ? V[(int64_t)kv * a.v_st + 32 * d + lr] : 0.f;
       }
-    f32x16 s;
+  };
+  float o[S::F][2], m = -INFINITY, l = 0.f;                        // m of query qi, l of query q0 + r
 #pragma unroll
-    for (int e = 0; e < 16; e++) s[e] = 0.f;
+  for (int d = 0; d < S::F; d++) o[d][0] = o[d][1] = 0.f;
+  bool fine = split_cap_ok(a.cap);
+  load(wave);
+  for (int first = 0; first < tiles; first += W) {
+    const int i = first + wave;
+    f32x16 s, t[S::F];
+    float top = -INFINITY;
+    if (i < tiles) {
 #pragma unroll
-    for (int i = 0; i < H4; i++) {
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(k[i].x, q[i].x, s, 0, 0, 0);
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(k[i].y, q[i].y, s, 0, 0, 0);
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(k[i].z, q[i].z, s, 0, 0, 0);
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(k[i].w, q[i].w, s, 0, 0, 0);
+      for (int e = 0; e < 16; e++) s[e] = 0.f;
+#pragma unroll
+      for (int u = 0; u < D / 16; u++) {
+        bf16x8 f[3];
+#pragma unroll
+        for (int e = 0; e < 8; e++) k[u][e] *= SPLIT_UP;
+        split8(k[u], f);
+        mfma6(f, q[u], s);
+      }
+      fine = fine && all_finite(s);
+      top = tile_scores(s, a, factor, 32 * i, qi, lk);
     }
-    float tmax = -INFINITY;
-#pragma unroll
-    for (int e = 0; e < 16; e++) {
-      const int kv = kv0 + 8 * (e >> 2) + 4 * lk + (e & 3);
-      float x = softcap_fwd(s[e], a.cap, inv_cap);
-      x = (kv > qi || kv >= a.T) ? -INFINITY : x;
-      s[e] = x;
-      tmax = fmaxf(tmax, x);
-    }
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-    const float m_new = fmaxf(m, tmax), m_use = m_new == -INFINITY ? 0.f : m_new;
-    const float alpha = expf(m - m_use);
-    float psum = 0.f;
-#pragma unroll
-    for (int e = 0; e < 16; e++) { const float p = expf(s[e] - m_use); s[e] = p; psum += p; }
-    psum += __shfl_xor(psum, 32, 64);
-    l = l * alpha + psum;
-    m = m_new;
-#pragma unroll
-    for (int d = 0; d < DB; d++)
-#pragma unroll
-      for (int e = 0; e < 16; e++) o[d][e] *= alpha;
-#pragma unroll
-    for (int d = 0; d < DB; d++)
-#pragma unroll
-      for (int e = 0; e < 16; e++) o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[d][e], s[e], o[d], 0, 0, 0);
-  }
-
-  if (lk == 0) { Ms[wave * 32 + lr] = m; Lsum[wave * 32 + lr] = l; }
-  __syncthreads();
-  float top = -INFINITY;
-#pragma unroll
-  for (int w = 0; w < W; w++) top = fmaxf(top, Ms[w * 32 + lr]);
-  const float use = top == -INFINITY ? 0.f : top;
-  float total = 0.f;
-#pragma unroll
-  for (int w = 0; w < W; w++) total += Lsum[w * 32 + lr] * expf(Ms[w * 32 + lr] - use);
-  const float factor = expf(m - use) * (total > 0.f ? 1.0f / total : 0.f);
-  if (wave == 0 && lk == 0 && qi < a.T) a.lse[((int64_t)b * a.H + h) * a.T + qi] = top + logf(total);
-  // 8 threads to a row: piece ch of its 32 features is the accumulator quarter ch / 2 of half ch % 2
-  const int r = threadIdx.x >> 3, ch = threadIdx.x & 7;
-#pragma unroll
-  for (int d = 0; d < DB; d++) {
-    if (d) __syncthreads();
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-      part[(wave * 4 + j) * 64 + lane] = make_float4(o[d][4 * j] * factor, o[d][4 * j + 1] * factor, o[d][4 * j + 2] * factor, o[d][4 * j + 3] * factor);
+    if (lk == 0) Top[wave * 32 + lr] = top;
     __syncthreads();
-    if (threadIdx.x < 256 && q0 + r < a.T && 32 * d + 4 * ch < a.hd) {
-      float4 sum = part[(ch >> 1) * 64 + 32 * (ch & 1) + r];
+    float before = m;                                              // the largest score ahead of this wave's tile
 #pragma unroll
-      for (int w = 1; w < W; w++) {
-        const float4 x = part[(w * 4 + (ch >> 1)) * 64 + 32 * (ch & 1) + r];
-        sum.x += x.x; sum.y += x.y; sum.z += x.z; sum.w += x.w;
+    for (int w = 0; w < W; w++) {
+      const float x = Top[w * 32 + lr];
+      m = fmaxf(m, x);
+      if (w < wave) before = fmaxf(before, x);
+    }
+    if (i < tiles) {
+      float alpha;
+      const float sum = tile_weights(s, before, top, alpha);
+      if (lk == 0) { Alpha[wave * 32 + lr] = alpha; Sum[wave * 32 + lr] = sum; }
+      bf16x8 p[2][3];
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        const float x[8] = {s[8 * j], s[8 * j + 1], s[8 * j + 2], s[8 * j + 3], s[8 * j + 4], s[8 * j + 5], s[8 * j + 6], s[8 * j + 7]};
+        split8(x, p[j]);
       }
-      *reinterpret_cast<float4 *>((float *)a.o + b * a.o_sb + h * a.o_sh + (int64_t)(q0 + r) * a.o_st + 32 * d + 4 * ch) = sum;
+#pragma unroll
+      for (int d = 0; d < S::F; d++) {
+#pragma unroll
+        for (int e = 0; e < 16; e++) t[d][e] = 0.f;
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+          float x[8];
+#pragma unroll
+          for (int e = 0; e < 8; e++) x[e] = v[d][8 * j + e] * SPLIT_UP;
+          bf16x8 f[3];
+          split8(x, f);
+          mfma6(f, p[j], t[d]);
+        }
+      }
+    }
+    load(i + W);
+    // features 4 g .. 4 g + 3 of a query are 16 bytes, in a row of 32 queries turned by 4 g: neither side meets a bank twice
+#pragma unroll
+    for (int d = 0; d < S::F; d++) {
+      if (d) __syncthreads();
+      if (i < tiles) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          const int g = 2 * j + lk;
+          *reinterpret_cast<float4 *>(smem + ((wave * 8 + g) * 32 + ((lr + 4 * g) & 31)) * 16) = make_float4(t[d][4 * j], t[d][4 * j + 1], t[d][4 * j + 2], t[d][4 * j + 3]);
+        }
+      }
+      __syncthreads();
+      const int g = c >> 1;
+      for (int w = 0; w < min(W, tiles - first); w++) {
+        const float alpha = Alpha[w * 32 + r];
+        const float2 x = *reinterpret_cast<const float2 *>(smem + ((w * 8 + g) * 32 + ((r + 4 * g) & 31)) * 16 + 8 * (c & 1));
+        if (d == 0) l = __builtin_fmaf(l, alpha, Sum[w * 32 + r]);
+        o[d][0] = __builtin_fmaf(o[d][0], alpha, x.x);
+        o[d][1] = __builtin_fmaf(o[d][1], alpha, x.y);
+      }
     }
   }
+  float z = 0.f;
+#pragma unroll
+  for (int d = 0; d < S::F; d++) z = __builtin_fmaf(o[d][0], 0.f, __builtin_fmaf(o[d][1], 0.f, z));      // 0 unless one is infinite or NaN
+  if (__syncthreads_or(!fine || !(z == 0.f))) {
+    flash_fwd_exact<D>(a, bh, q0, min(a.T, q0 + 32), wave == 0, (float *)smem);
+    return;
+  }
+  if (q0 + r < a.T) {
+    const float f = output_factor(l);
+    float *O = (float *)a.o + b * a.o_sb + h * a.o_sh + (int64_t)(q0 + r) * a.o_st;
+#pragma unroll
+    for (int d = 0; d < S::F; d++)
+      if (32 * d + 2 * c < a.hd) *reinterpret_cast<float2 *>(O + 32 * d + 2 * c) = make_float2(o[d][0] * f, o[d][1] * f);
+  }
+  if (c == 0) Sum[r] = l;
+  __syncthreads();
+  if (threadIdx.x < 32 && qi < a.T) a.lse[((int64_t)b * a.H + h) * a.T + qi] = m + logf(Sum[lr]);
 }
 
 // delta[b,h,t] = sum_d dO[t,d] * O[t,d]
@@ -855,16 +882,16 @@ int32_t check(const AhFlash *f, bool bwd, FlashArgs &a) {
 template <int D>
 int32_t run_fwd(const FlashArgs &a) {
   if constexpr (D <= 64) {
-    // Blocks of 128 queries from one for every second CU on; before that the keys go to 8 waves where that gives each at least one
-    // tile, or where all workgroups run at once.  us, 128-query blocks / keys among waves, soft cap on:
-    //   D = 64, 12 heads: T = 256 33 / 23, T = 500 60 / 36, T = 777 91 / 67, T = 1024 115 / 95; T = 1024 24 heads 119 / 122, 32 heads 121 / 157;
-    //   16 heads x 2048 234 / 254; 64 heads x 512 x 48 63 / 88; 160 heads x T = 100 20 / 42;  12 heads x T = 64 12 / 16
-    //   D = 32: 8 heads x T = 32 7 / 10, x T = 128 16 / 12, x T = 256 28 / 14
-    // Larger heads keep the one kernel: there a call over many heads and calls over each alone give the same bits.
-    constexpr int W = 8;
-    const int64_t heads = (int64_t)a.B * a.H, blocks = cdiv(a.T, 32) * heads;
-    if (a.T > 64 && 2 * cdiv(a.T, WAVES * 32) * heads <= num_cus() && (a.T >= W * 32 || blocks <= num_cus())) {
-      ah::launch_kernel((k_flash_fwd_f32_keys<D, W>), dim3((unsigned)cdiv(a.T, 32), (unsigned)heads), dim3(64 * W), 0, a);
+    // What the two take, as measured: a block of 128 queries 3.7 us for each tile of its chain, whatever else is on its CU (up to two), a CU
+    // 10 us for every 8 tiles of 32 queries that share their keys (`eights` of them per head).  us, blocks of 128 / keys among waves:
+    //   D = 64, 12 heads: T = 64 11.7 / 9.8, 256 33 / 14.6, 500 61 / 23, 1024 118 / 61, 2048 232 / 158; T = 1024 24 heads 121 / 81, 32 heads 124 / 103,
+    //   192 heads 305 / 571; T = 256 64 heads 35 / 25, 96 heads 36 / 37; 64 heads x 512 x 48 65 / 60; 160 heads x T = 100 20 / 28
+    //   D = 32: 8 heads x T = 40 9.8 / 7.3, x T = 256 29 / 10; 64 x 128 16 / 8.8; 152 x 250 31 / 41; 2 x 2050 210 / 49
+    // A row has the same bits from both, so a head's result does not depend on how many others are in the call.
+    const int64_t tiles = cdiv(a.T, 32), whole = tiles / 8, eights = 4 * whole * (whole + 1) + tiles % 8 * (whole + 1);
+    const int64_t heads = (int64_t)a.B * a.H;
+    if (26 * eights * heads <= 10 * num_cus() * tiles) {
+      ah::launch_kernel(k_flash_fwd_f32_keys<D>, dim3((unsigned)tiles, (unsigned)heads), dim3(512), 0, a);
       AH_LAUNCH_CHECK();
       return AH_OK;
     }

@@ -1737,6 +1737,25 @@ def test_flash_attention_f32_forward_with_keys_shared_by_waves(B, BH, T, D, cap)
         assert_close(np.asarray(r["lse"].data).reshape(BH, T)[h], (m + np.log(e.sum(1, keepdims=True)))[:, 0], rel=rel, what="LSE")
 
 
+# one tile short of eight, eight, one more, a last tile that is not whole, several rounds of eight; head sizes the tiles fill and do not
+@pytest.mark.parametrize("BH,T,D,cap", [(300, 65, 64, 30.0), (140, 224, 32, 30.0), (140, 256, 64, 0.0), (70, 257, 48, 30.0), (44, 300, 64, 30.0),
+                                        (130, 250, 24, 30.0), (20, 1100, 64, 30.0), (17, 2050, 32, 0.0)])
+@pytest.mark.parametrize("special", [False, True])
+def test_flash_attention_f32_of_a_head_does_not_depend_on_the_number_of_heads(B, BH, T, D, cap, special):
+    """Many heads take blocks of 128 queries, one head shares its keys among waves: the same bits.  Special: with an infinite value, an
+    infinite key, a key of 1e25 (its sums run the fp32 instruction) and a NaN, the rows of 32 queries that meet none of them too."""
+    q, k, v = (rs.randn(BH, T, D).astype(np.float32) for _ in range(3))
+    if special:
+        v[:, T - 3, 1], k[0, T // 2, 2], k[1, T // 3, 0], q[2, T // 4, 3] = np.inf, np.inf, 1e25, np.nan
+    whole = B.flashAttention(dev(B, q), dev(B, k), dev(B, v), T, 1 / math.sqrt(D), cap)
+    O, L = np.asarray(whole["output"].data).reshape(BH, T, D), np.asarray(whole["lse"].data).reshape(BH, T)
+    for h in (0, 1, 2, BH // 2, BH - 1):
+        one = B.flashAttention(dev(B, q[h:h + 1]), dev(B, k[h:h + 1]), dev(B, v[h:h + 1]), T, 1 / math.sqrt(D), cap)
+        assert np.array_equal(np.asarray(one["output"].data).reshape(T, D), O[h], equal_nan=True), h
+        assert np.array_equal(np.asarray(one["lse"].data).reshape(T), L[h], equal_nan=True), h
+        assert special or np.isfinite(O[h]).all()
+
+
 def _attention_grads_64(q, k, v, do, scale, cap):
     """dQ, dK, dV of one head in 64 bits, by the kernels' own formulas (an infinite score has a capped value and no slope)."""
     q, k, v, do = (x.astype(np.float64) for x in (q, k, v, do))
