@@ -324,7 +324,7 @@ __device__ __forceinline__ void load_piece(const float *__restrict__ base, int64
 }
 template <bool A_KC, bool B_KC, int WAVES, bool EXACT>
 __device__ __forceinline__ void contract_pieces(const GemmArgs &g, const float *A, const float *B, int m0, int n0, bool vec_a, bool vec_b, f32x16 &sum) {
-  constexpr int U = WAVES > 8 ? 2 : 4;               // 16 waves: 128 registers each
+  constexpr int U = 4;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 31, lk = lane >> 5;
   const int ra = min(m0 + lr, g.M - 1), rb = min(n0 + lr, g.N - 1), nc = (g.K + 15) >> 4;
 #pragma unroll
@@ -420,7 +420,7 @@ struct F32Choice { int bm, waves, splits; };
 
 // The choice is the least of what the candidates are expected to take, in microseconds beyond a launch, from figures measured over 71 shapes
 // (1 x 4096 x 1024 to 16384 x 50304 x 768, in the three layouts; the choice is 3 % slower than the fastest candidate on average, 32 % at worst):
-//   32 x 32     FIRST, the first round trip; then GROUP per 4 (16 waves: 2) pieces of a wave, and the rate that all of them together reach
+//   32 x 32     FIRST, the first round trip; then GROUP per 4 pieces of a wave, and the rate that all of them together reach
 //   LDS tiles   a tile takes `step` per 16 of the contraction alone on its CU, and `full` of the CU's time where others fill its gaps
 //   slices      another launch, and the workspace written and read
 // Against 128 x 128 tiles of v_mfma_f32_32x32x2_f32 (in slices where there were fewer than 256 tiles and K >= 2048), in us:
@@ -429,18 +429,17 @@ struct F32Choice { int bm, waves, splits; };
 F32Choice choose(const GemmArgs &ga, int layout, int batch, bool may_split, bool long_rows) {
   struct Tile { int bm; double step, full; };
   static constexpr Tile TILES[2] = {{64, 0.26, 0.24}, {128, 1.2, 0.65}};
-  static constexpr double FIRST[3] = {0.56, 1.1, 1.4}, GROUP[3] = {0.74, 0.58, 0.63}, RATE[3] = {61e6, 50e6, 100e6};      // NN, NT, TN: operations per us
+  static constexpr double FIRST[2] = {0.56, 1.1}, GROUP[2] = {0.74, 0.58}, RATE[3] = {61e6, 50e6, 100e6};      // NN, NT, TN: operations per us
   const double M = ga.M, N = ga.N, K = ga.K;
   // a launch has fewer than 2^32 threads: a row of more than 2^30 columns leaves only the widest tiles
   auto fits = [&](int bm, int threads) { return cdiv(ga.M, bm) * cdiv(ga.N, bm) * threads < (1ll << 32); };
-  F32Choice best{32, 16, 1};
+  F32Choice best{32, 8, 1};
   double least = 1e300;
-  for (int w = 0; w < 3; w++) {
+  for (int w = 0; w < 2; w++) {
     const int waves = 4 << w;
     if (!fits(32, 64 * waves)) continue;
-    double t = FIRST[w] + GROUP[w] * (double)cdiv(cdiv(ga.K, 16), waves * (w == 2 ? 2 : 4)) +
+    double t = FIRST[w] + GROUP[w] * (double)cdiv(cdiv(ga.K, 16), waves * 4) +
                (double)(cdiv(ga.M, 32) * cdiv(ga.N, 32) * batch) * 2048.0 * K / RATE[layout] * (w == 0 ? 1.0 : 1.6);
-    if (layout == AH_GEMM_TN && w == 2) t += 3.5;               // spills registers
     if (t < least) { least = t; best = F32Choice{32, waves, 1}; }
   }
   if (long_rows) return best;
@@ -458,11 +457,8 @@ F32Choice choose(const GemmArgs &ga, int layout, int batch, bool may_split, bool
 template <int LAYOUT>
 int32_t launch_choice(const F32Choice &c, const GemmArgs &ga, int batch, int vec_a, int vec_b, int vec_c, int out_bf16) {
   if (c.bm == 32) {
-    switch (c.waves) {
-      case 4: return launch_pieces<LAYOUT, 4>(ga, batch, vec_a, vec_b, vec_c, out_bf16);
-      case 8: return launch_pieces<LAYOUT, 8>(ga, batch, vec_a, vec_b, vec_c, out_bf16);
-      default: return launch_pieces<LAYOUT, 16>(ga, batch, vec_a, vec_b, vec_c, out_bf16);
-    }
+    return c.waves == 4 ? launch_pieces<LAYOUT, 4>(ga, batch, vec_a, vec_b, vec_c, out_bf16)
+                        : launch_pieces<LAYOUT, 8>(ga, batch, vec_a, vec_b, vec_c, out_bf16);
   }
   if (c.bm == 64) return launch_split<LAYOUT, 64, 64>(ga, batch, vec_a, vec_b, vec_c, out_bf16);
   return launch_split<LAYOUT, 128, 128>(ga, batch, vec_a, vec_b, vec_c, out_bf16);
