@@ -924,11 +924,16 @@ def _gemm_f32(B, layout, a, b, c0=None, pad=(0, 0, 0)):
     return out[:, :N]
 
 
-# sizes one off the tiles (32, 64, 128, 256), contractions one off the 16 of a step, with and without slices, and each kernel of the dispatch
-@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (33, 31, 17), (64, 64, 16), (65, 129, 15), (127, 260, 1000), (384, 128, 1030), (700, 256, 4750), (1100, 520, 33),
-                                   (2100, 1300, 130), (4097, 640, 64), (8200, 3100, 50)])
+# sizes one off the tiles (32, 64, 128), contractions one off the 16 of a step, with and without slices, and each kernel of the dispatch:
+# what runs in the layouts NN, NT and TN (without padding: rows of C that are not 16-byte aligned take no slices; slices are whole steps of
+# 16, so 1030 in 16 is 13 of 80)
+S64, S64_8, S64_13, S64_16, S128, S128_16 = ("split", 64, 1), ("split", 64, 8), ("split", 64, 13), ("split", 64, 16), ("split", 128, 1), ("split", 128, 16)
+P4, P8 = ("pieces", 4, 1), ("pieces", 8, 1)
+@pytest.mark.parametrize("M,N,K,runs", [(1, 1, 1, (S64,) * 3), (33, 31, 17, (S64,) * 3), (64, 64, 16, (S64,) * 3), (65, 129, 15, (S64,) * 3), (127, 260, 1000, (P8, S64_8, P8)),
+                                        (384, 128, 1030, (S64_13,) * 3), (700, 256, 4750, (S64_16,) * 3), (1100, 520, 33, (S64,) * 3), (2100, 1300, 130, (S64,) * 3),
+                                        (4097, 640, 64, (S64,) * 3), (8200, 3100, 50, (S128,) * 3), (500, 300, 512, (P4, ("split", 64, 4), P4)), (640, 768, 4096, (S128_16,) * 3)])
 @pytest.mark.parametrize("pad", [(0, 0, 0), (1, 3, 2), (4, 8, 4)])
-def test_gemm_f32_edges_of_tiles_slices_and_strides(B, M, N, K, pad):
+def test_gemm_f32_edges_of_tiles_slices_and_strides(B, M, N, K, runs, pad):
     """Every layout against a float64 product.  Bound: the six partial products of a step of 16 are rounded into the sum one after
     the other (0.375 K roundings, at most one more per slice, wave or partial product), and what the split leaves out is 2^-24 of a term."""
     from alpha2_amd import _ffi as ffi
@@ -938,12 +943,15 @@ def test_gemm_f32_edges_of_tiles_slices_and_strides(B, M, N, K, pad):
     bound = (6 * -(-K // 16) + 40) * 2.0 ** -24 * size
     for layout in (ffi.GEMM_NN, ffi.GEMM_NT, ffi.GEMM_TN):
         assert np.all(np.abs(_gemm_f32(B, layout, a, b, pad=pad) - want) <= bound), (layout, B.lastGemmKernel())
+        if pad == (0, 0, 0):
+            kind, width, slices = runs[layout]
+            assert B.lastGemmKernel() == ("k_gemm_f32_%s<%d, %s>" % (kind, layout, "%d, %d" % (width, width) if kind == "split" else width), slices)
     c0 = g.standard_normal((M, N), dtype=np.float32)
     got = _gemm_f32(B, ffi.GEMM_TN, a, b, c0, pad)
     assert np.all(np.abs(got - (want + c0)) <= bound + 2.0 ** -23 * np.abs(want + c0)), B.lastGemmKernel()
 
 
-@pytest.mark.parametrize("M,N,K", [(40, 40, 40), (500, 300, 512), (300, 2000, 36), (4000, 1200, 64)])
+@pytest.mark.parametrize("M,N,K", [(40, 40, 40), (500, 300, 512), (300, 2000, 36), (4000, 1200, 64), (8200, 648, 40), (640, 768, 4096)])
 def test_gemm_f32_with_numbers_the_split_cannot_hold(B, M, N, K):
     """Infinities, NaNs and numbers above the largest bf16 (3.39e38): the result is the fp32 product's, entry by entry, also in the
     tiles' other rows; numbers down to 1e-30 lose nothing."""
@@ -1203,7 +1211,7 @@ def test_gemm_over_an_empty_contraction(B, m, n):
 
 
 @pytest.mark.parametrize("in_bf16,out_bf16", [(False, False), (True, False), (True, True)])
-@pytest.mark.parametrize("M,N,K", [(128, 128, 64), (256, 384, 96), (300, 200, 72), (1024, 768, 256)])
+@pytest.mark.parametrize("M,N,K", [(128, 128, 64), (256, 384, 96), (300, 200, 72), (1024, 768, 256), (8200, 648, 40)])
 def test_gemm_layouts_epilogues_dtypes(B, in_bf16, out_bf16, M, N, K):
     from alpha2_amd import _ffi as ffi
     idt, odt = (ffi.BF16 if in_bf16 else ffi.F32), (ffi.BF16 if out_bf16 else ffi.F32)
