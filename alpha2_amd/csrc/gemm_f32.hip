@@ -154,9 +154,10 @@ __device__ __forceinline__ void mfma6_tiles(const bf16x8 (&a)[3][TM], const bf16
 }
 
 // ================================================================ tiles through LDS
-// 2 x 2 waves of 64 x 64 (or 32 x 32): 24 matrix instructions per step and wave, 768 cycles, against some 150 vector instructions for the
+// 2 x 2 waves of 64 x 64 (or 32 x 32): 24 matrix instructions per step and wave, 768 cycles, against some 170 vector instructions for the
 // split, which go into the gaps between them (sched_group_barrier: 16384 x 768 x 2304 NN 547 -> 330 us with it and the loads a step
-// earlier).  What bounds it now is what one SIMD issues: the matrix pipes are busy 45 % of the time at 2 waves per SIMD.
+// earlier; 4, 6, 7 or 8 vector instructions to a gap instead of 5 are the same within 3 %).  What bounds it now is what one SIMD issues:
+// at 2 waves per SIMD the matrix pipes are busy 40 to 54 % of the time and the vector units as long.
 // LDS: three planes of [row][16 k] bf16 per operand, 32 bytes a row, two buffers.  The 16-byte half of a row that holds k 0..7 is
 // the first one in rows whose bit 3 is clear and the second one in the others: the fragment reads and the 8-byte writes of either
 // operand order then spread over all banks.
@@ -425,7 +426,9 @@ struct F32Choice { int bm, waves, splits; };
 //   slices      another launch, and the workspace written and read
 // Against 128 x 128 tiles of v_mfma_f32_32x32x2_f32 (in slices where there were fewer than 256 tiles and K >= 2048), in us:
 //   16384 x 3072 x 768 NT 720 -> 430 (128 x 128), 768 x 768 x 16384 TN 329 -> 157 (128 x 128 in 32 slices), 490 x 768 x 768 NT 77 -> 16
-//   (64 x 64 in 4 slices), 48 x 768 x 256 NT 26 -> 7 and 512 x 128 x 1024 TN 97 -> 9 (32 x 32)
+//   (64 x 64 in 4 slices), 48 x 768 x 256 NT 26 -> 7 and 512 x 128 x 1024 TN 97 -> 9 (32 x 32); with the operands scaled 1 to 5 % more,
+//   16384 x 3072 x 768 NT 549 -> 557 and 490 x 768 x 768 16.7 -> 17.5 back to back on standard normal operands.  Operands that are not
+//   finite take the fp32 instruction as well: 16384 x 3072 x 768 of NaNs 1070 (720 by that instruction's own kernel).
 F32Choice choose(const GemmArgs &ga, int layout, int batch, bool may_split, bool long_rows) {
   struct Tile { int bm; double step, full; };
   static constexpr Tile TILES[2] = {{64, 0.26, 0.24}, {128, 1.2, 0.65}};

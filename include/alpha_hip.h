@@ -336,7 +336,7 @@ int32_t ah_cross_entropy_fwd_bwd(ah_ptr logits, int32_t dtype, ah_ptr targets_i3
  *        AH_GEMM_NN: A[M,K] * B[K,N]      (matmul;            dX = G * W)
  *        AH_GEMM_NT: A[M,K] * B[N,K]^T    (matmulTransposed;  Y = X * W^T)
  *        AH_GEMM_TN: A[K,M]^T * B[K,N]    (matmulTransposedA; dW = G^T * X)
- *      f32 operands -> fp32 MFMA (parity mode); bf16 operands -> bf16 MFMA with fp32 accumulation.
+ *      f32 operands -> six bf16 MFMA products that hold all 24 bits (parity mode); bf16 operands -> bf16 MFMA; fp32 accumulation.
  *      lda/ldb/ldc are row strides in elements.  batch > 1 repeats with the given element strides
  *      (0 = operand shared across the batch).
  *      Epilogues: AH_EPI_NONE; AH_EPI_ACCUM  C += acc (gradient accumulation);
@@ -430,7 +430,7 @@ int32_t ah_probe_issue(int32_t kind, int32_t waves_per_simd, int32_t iters, doub
  *      LSE is [B, H, T] f32.  head_dim: a multiple of 8 from 8 to 128 (the kernels are built for 32, 64 and 128; another size
  *      runs the next larger one with the missing features read as zeros and never stored). ---- */
 typedef struct {
-  int32_t dtype;             /* AH_F32 (fp32 MFMA) or AH_BF16 */
+  int32_t dtype;             /* AH_F32 (parity mode) or AH_BF16 */
   int32_t batch, heads, seq, head_dim;
   int64_t q_sb, q_sh, q_st;
   int64_t k_sb, k_sh, k_st;
