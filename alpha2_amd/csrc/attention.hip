@@ -48,7 +48,7 @@ __device__ __forceinline__ void load_tile_f32(float *s, const float *__restrict_
 // 16-byte pieces are permuted within a row so that 16 lanes that read the same piece of 16 rows meet 64 different banks.
 // A result that is not finite has the block computed again with the fp32 instruction, whose result stands; so does a score.
 // 192 heads x 1024 x 64: dK and dV 945 -> 486 us, dQ 520 -> 316; 512 x 256 x 32: 112 -> 84 and 81 -> 60; 4 x 70 x 64: 29 -> 24 and
-// 26 -> 20 (before both operands were scaled, which costs 2 % of the backward pass at 192 x 1024 x 64 and 6 % at 12 x 64 x 64).  Relative error against 64 bits at 4 x 512 x 64: dQ 4.6e-7 -> 3.7e-7, dK 6.4e-7 -> 3.8e-7, dV 6.0e-7 -> 3.3e-7.  What bounds
+// 26 -> 20 (before both operands were scaled, which costs 1 % of the backward pass at 192 x 1024 x 64 and 3 to 6 % of smaller ones).  Relative error against 64 bits at 4 x 512 x 64: dQ 4.6e-7 -> 3.7e-7, dK 6.4e-7 -> 3.8e-7, dV 6.0e-7 -> 3.3e-7.  What bounds
 // it now is vector issue: tanh, exp and the cut of scores, K and V for every 32 x 32 tile beside 3072 cycles of matrix instructions.
 template <int D>
 struct SplitTile {                          // D = 32 or 64
@@ -69,6 +69,12 @@ struct SplitTile {                          // D = 32 or 64
       }
     }
   }
+  static __device__ __forceinline__ void scale(float (&x)[4][F], float mul) {
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+#pragma unroll
+      for (int d = 0; d < F; d++) x[r][d] = here(x[r][d]) * mul;
+  }
   static __device__ __forceinline__ float largest(const float (&x)[4][F]) {
     float top = 0.f;
 #pragma unroll
@@ -81,13 +87,13 @@ struct SplitTile {                          // D = 32 or 64
   static __device__ __forceinline__ uint32_t highs(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
   // into the layouts that are asked for
   template <bool ROWS, bool COLS>
-  static __device__ __forceinline__ void put(const float (&x)[4][F], float mul, char *rows, char *cols) {
+  static __device__ __forceinline__ void put(const float (&x)[4][F], char *rows, char *cols) {
     const int g = threadIdx.x >> 5, f = F * (threadIdx.x & 31);
     Split2 s[F][2];                         // rows (0, 1) and (2, 3) of a feature
 #pragma unroll
     for (int d = 0; d < F; d++)
 #pragma unroll
-      for (int i = 0; i < 2; i++) s[d][i] = split2(x[2 * i][d] * mul, x[2 * i + 1][d] * mul);
+      for (int i = 0; i < 2; i++) s[d][i] = split2(x[2 * i][d], x[2 * i + 1][d]);
 #pragma unroll
     for (int p = 0; p < 3; p++) {
       auto part = [&](int d, int i) { return p == 0 ? s[d][i].h : p == 1 ? s[d][i].m : s[d][i].l; };
@@ -116,20 +122,26 @@ struct SplitTile {                          // D = 32 or 64
 #pragma unroll
     for (int p = 0; p < 3; p++) f[p] = *reinterpret_cast<const bf16x8 *>(cols + p * PLANE + col_ofs(d, chunk));
   }
-  // the wave's own row, features 16 step + 8 half .. + 7
-  static __device__ __forceinline__ void whole(const float *row, bool live, float mul, int hd, int lk, float (&x)[D / 16][8]) {
+  // a row of a wave's own, features 16 step + 8 half .. + 7; then times mul, and cut.  (All loads of a kernel's start come before the
+  // first of these two: each waits for what it takes.)
+  static __device__ __forceinline__ void row(const float *p, bool live, int hd, int lk, float (&x)[D / 16][8]) {
 #pragma unroll
     for (int i = 0; i < D / 16; i++) {
       const int d = 16 * i + 8 * lk;
       float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
-      if (live && d < hd) { a = *reinterpret_cast<const float4 *>(row + d); b = *reinterpret_cast<const float4 *>(row + d + 4); }
-      x[i][0] = a.x * mul; x[i][1] = a.y * mul; x[i][2] = a.z * mul; x[i][3] = a.w * mul;
-      x[i][4] = b.x * mul; x[i][5] = b.y * mul; x[i][6] = b.z * mul; x[i][7] = b.w * mul;
+      if (live && d < hd) { a = *reinterpret_cast<const float4 *>(p + d); b = *reinterpret_cast<const float4 *>(p + d + 4); }
+      x[i][0] = a.x; x[i][1] = a.y; x[i][2] = a.z; x[i][3] = a.w;
+      x[i][4] = b.x; x[i][5] = b.y; x[i][6] = b.z; x[i][7] = b.w;
     }
   }
-  static __device__ __forceinline__ void own(const float *row, bool live, float mul, int hd, int lk, bf16x8 (&f)[D / 16][3]) {
-    float x[D / 16][8];
-    whole(row, live, mul, hd, lk, x);
+  static __device__ __forceinline__ void scale(float (&x)[D / 16][8], float mul) {
+#pragma unroll
+    for (int i = 0; i < D / 16; i++)
+#pragma unroll
+      for (int e = 0; e < 8; e++) x[i][e] = here(x[i][e]) * mul;
+  }
+  static __device__ __forceinline__ void cut(float (&x)[D / 16][8], float mul, bf16x8 (&f)[D / 16][3]) {
+    scale(x, mul);
 #pragma unroll
     for (int i = 0; i < D / 16; i++) split8(x[i], f[i]);
   }
@@ -307,8 +319,8 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_fwd_f32(FlashArgs
     const float *K = (const float *)a.k + b * a.k_sb + h * a.k_sh;
     const float *V = (const float *)a.v + b * a.v_sb + h * a.v_sh;
     const float factor = split_cap_factor(a.cap);
-    bf16x8 q[D / 16][3];
-    S::own((const float *)a.q + b * a.q_sb + h * a.q_sh + (int64_t)qi * a.q_st, qi < a.T, a.scale * SPLIT_UP, a.hd, lk, q);
+    float qx[D / 16][8];
+    S::row((const float *)a.q + b * a.q_sb + h * a.q_sh + (int64_t)qi * a.q_st, qi < a.T, a.hd, lk, qx);
     f32x16 o[S::F];
 #pragma unroll
     for (int d = 0; d < S::F; d++)
@@ -318,11 +330,15 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_fwd_f32(FlashArgs
     float kx[4][S::F], vx[4][S::F];
     S::load(kx, K, a.k_st, 0, a.T, a.hd);
     S::load(vx, V, a.v_st, 0, a.T, a.hd);
+    bf16x8 q[D / 16][3];
+    S::cut(qx, a.scale * SPLIT_UP, q);
     bool fine = split_cap_ok(a.cap);
     for (int kv0 = 0; kv0 < end; kv0 += BC) {
+      S::scale(kx, SPLIT_UP);
+      S::scale(vx, SPLIT_UP);
       __syncthreads();
-      S::template put<true, false>(kx, SPLIT_UP, Kr, nullptr);
-      S::template put<false, true>(vx, SPLIT_UP, nullptr, Vc);
+      S::template put<true, false>(kx, Kr, nullptr);
+      S::template put<false, true>(vx, nullptr, Vc);
       S::load(kx, K, a.k_st, kv0 + BC, a.T, a.hd);                 // the next tile, while this one is multiplied; rows past the end read as zero
       S::load(vx, V, a.v_st, kv0 + BC, a.T, a.hd);
       __syncthreads();
@@ -382,12 +398,11 @@ __global__ __launch_bounds__(512, 2) void k_flash_fwd_f32_keys(FlashArgs a) {
   const float *K = (const float *)a.k + b * a.k_sb + h * a.k_sh;
   const float *V = (const float *)a.v + b * a.v_sb + h * a.v_sh;
   const float factor = split_cap_factor(a.cap);
-  bf16x8 q[D / 16][3];
-  S::own((const float *)a.q + b * a.q_sb + h * a.q_sh + (int64_t)qi * a.q_st, qi < a.T, a.scale * SPLIT_UP, a.hd, lk, q);
-  float k[D / 16][8], v[S::F][16];
+  float qx[D / 16][8], k[D / 16][8], v[S::F][16];
+  S::row((const float *)a.q + b * a.q_sb + h * a.q_sh + (int64_t)qi * a.q_st, qi < a.T, a.hd, lk, qx);
   auto load = [&](int i) {                                         // rows past the end read as zero
     if (i >= tiles) return;
-    S::whole(K + (int64_t)(32 * i + lr) * a.k_st, 32 * i + lr < a.T, 1.0f, a.hd, lk, k);
+    S::row(K + (int64_t)(32 * i + lr) * a.k_st, 32 * i + lr < a.T, a.hd, lk, k);
 #pragma unroll
     for (int d = 0; d < S::F; d++)
 #pragma unroll
@@ -401,6 +416,8 @@ __global__ __launch_bounds__(512, 2) void k_flash_fwd_f32_keys(FlashArgs a) {
   for (int d = 0; d < S::F; d++) o[d][0] = o[d][1] = 0.f;
   bool fine = split_cap_ok(a.cap);
   load(wave);
+  bf16x8 q[D / 16][3];
+  S::cut(qx, a.scale * SPLIT_UP, q);
   for (int first = 0; first < tiles; first += W) {
     const int i = first + wave;
     f32x16 s, t[S::F];
@@ -412,7 +429,7 @@ __global__ __launch_bounds__(512, 2) void k_flash_fwd_f32_keys(FlashArgs a) {
       for (int u = 0; u < D / 16; u++) {
         bf16x8 f[3];
 #pragma unroll
-        for (int e = 0; e < 8; e++) k[u][e] *= SPLIT_UP;
+        for (int e = 0; e < 8; e++) k[u][e] = here(k[u][e]) * SPLIT_UP;
         split8(k[u], f);
         mfma6(f, q[u], s);
       }
@@ -446,7 +463,7 @@ __global__ __launch_bounds__(512, 2) void k_flash_fwd_f32_keys(FlashArgs a) {
         for (int j = 0; j < 2; j++) {
           float x[8];
 #pragma unroll
-          for (int e = 0; e < 8; e++) x[e] = v[d][8 * j + e] * SPLIT_UP;
+          for (int e = 0; e < 8; e++) x[e] = here(v[d][8 * j + e]) * SPLIT_UP;
           bf16x8 f[3];
           split8(x, f);
           mfma6(f, p[j], t[d]);
@@ -603,9 +620,9 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_dq_f32(FlashArgs 
     const float *V = (const float *)a.v + b * a.v_sb + h * a.v_sh;
     const float inv_cap = a.cap > 0.f ? 1.0f / a.cap : 0.f, factor = split_cap_factor(a.cap);
     const bool live = qi < a.T;
-    bf16x8 q[D / 16][3], go[D / 16][3];
-    S::own((const float *)a.q + b * a.q_sb + h * a.q_sh + (int64_t)qi * a.q_st, live, a.scale * SPLIT_UP, a.hd, lk, q);
-    S::own((const float *)a.d_o + b * a.o_sb + h * a.o_sh + (int64_t)qi * a.o_st, live, SPLIT_UP, a.hd, lk, go);
+    float qx[D / 16][8], gx[D / 16][8];
+    S::row((const float *)a.q + b * a.q_sb + h * a.q_sh + (int64_t)qi * a.q_st, live, a.hd, lk, qx);
+    S::row((const float *)a.d_o + b * a.o_sb + h * a.o_sh + (int64_t)qi * a.o_st, live, a.hd, lk, gx);
     const int64_t srow = ((int64_t)b * a.H + h) * a.T + qi;
     const float lse = live ? a.lse[srow] : 0.f, delta = live ? a.delta[srow] : 0.f;
     f32x16 dq[S::F];
@@ -617,11 +634,16 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_dq_f32(FlashArgs 
     float kx[4][S::F], vx[4][S::F];
     S::load(kx, K, a.k_st, 0, a.T, a.hd);
     S::load(vx, V, a.v_st, 0, a.T, a.hd);
+    bf16x8 q[D / 16][3], go[D / 16][3];
+    S::cut(qx, a.scale * SPLIT_UP, q);
+    S::cut(gx, SPLIT_UP, go);
     bool fine = split_cap_ok(a.cap);
     for (int kv0 = 0; kv0 < end; kv0 += BC) {
+      S::scale(kx, SPLIT_UP);
+      S::scale(vx, SPLIT_UP);
       __syncthreads();
-      S::template put<true, true>(kx, SPLIT_UP, Kr, Kc);
-      S::template put<true, false>(vx, SPLIT_UP, Vr, nullptr);
+      S::template put<true, true>(kx, Kr, Kc);
+      S::template put<true, false>(vx, Vr, nullptr);
       S::load(kx, K, a.k_st, kv0 + BC, a.T, a.hd);                 // the next tile, while this one is multiplied; rows past the end read as zero
       S::load(vx, V, a.v_st, kv0 + BC, a.T, a.hd);
       __syncthreads();
@@ -769,14 +791,8 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_dkv_f32(FlashArgs
     // K's and V's rows stay whole and are cut where they are used: in three parts, they, the accumulators and the next tile are more
     // registers than a wave of two per SIMD has (the empty assembler statements keep the cuts from being moved out of the loop).
     float k[D / 16][8], v[D / 16][8];
-    S::whole((const float *)a.k + b * a.k_sb + h * a.k_sh + (int64_t)kvi * a.k_st, live, SPLIT_UP, a.hd, lk, k);
-    S::whole((const float *)a.v + b * a.v_sb + h * a.v_sh + (int64_t)kvi * a.v_st, live, SPLIT_UP, a.hd, lk, v);
-    float top = 0.f;
-#pragma unroll
-    for (int i = 0; i < D / 16; i++)
-#pragma unroll
-      for (int e = 0; e < 8; e++) top = fmaxf(top, fabsf(k[i][e]));
-    bool fine = split_cap_ok(a.cap) && top < LARGE_OPERAND * SPLIT_UP;
+    S::row((const float *)a.k + b * a.k_sb + h * a.k_sh + (int64_t)kvi * a.k_st, live, a.hd, lk, k);
+    S::row((const float *)a.v + b * a.v_sb + h * a.v_sh + (int64_t)kvi * a.v_st, live, a.hd, lk, v);
     f32x16 dk[S::F], dv[S::F];
 #pragma unroll
     for (int d = 0; d < S::F; d++)
@@ -791,11 +807,21 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_dkv_f32(FlashArgs
       if (threadIdx.x < 64) stat = qi < a.T ? (threadIdx.x < 32 ? a.lse : a.delta)[srow0 + qi] : 0.f;
     };
     load(kv_blk0);
+    S::scale(k, SPLIT_UP);
+    S::scale(v, SPLIT_UP);
+    float top = 0.f;
+#pragma unroll
+    for (int i = 0; i < D / 16; i++)
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) top = fmaxf(fmaxf(top, fabsf(k[i][e])), fabsf(k[i][e + 1]));
+    bool fine = split_cap_ok(a.cap) && top < LARGE_OPERAND * SPLIT_UP;
     for (int q0 = kv_blk0; q0 < a.T; q0 += BC) {                   // causal: queries at or after this block's first key
+      S::scale(qx, a.scale * SPLIT_UP);
+      S::scale(gx, SPLIT_UP);
+      fine = fine && S::largest(qx) < LARGE_OPERAND * SPLIT_UP;
       __syncthreads();
-      fine = fine && S::largest(qx) * fabsf(a.scale) < LARGE_OPERAND;
-      S::template put<true, true>(qx, a.scale * SPLIT_UP, Qr, Qc);
-      S::template put<true, true>(gx, SPLIT_UP, Gr, Gc);
+      S::template put<true, true>(qx, Qr, Qc);
+      S::template put<true, true>(gx, Gr, Gc);
       if (threadIdx.x < 64) Ls[threadIdx.x] = stat;                // the second 32 are Ds
       load(q0 + BC);                                               // the next tile, while this one is multiplied; rows past the end read as zero
       __syncthreads();
@@ -883,14 +909,15 @@ template <int D>
 int32_t run_fwd(const FlashArgs &a) {
   if constexpr (D <= 64) {
     // What the two take, as measured: a block of 128 queries 3.7 us for each tile of its chain, whatever else is on its CU (up to two), a CU
-    // 10 us for every 8 tiles of 32 queries that share their keys (`eights` of them per head).  us, blocks of 128 / keys among waves:
+    // 10 us for every 8 tiles of 32 queries that share their keys (`eights` of them per head); a single tile has nobody to share with
+    // (5 heads x 29 x 64 6.6 / 8.4).  us, blocks of 128 / keys among waves:
     //   D = 64, 12 heads: T = 64 11.7 / 9.8, 256 33 / 14.6, 500 61 / 23, 1024 118 / 61, 2048 232 / 158; T = 1024 24 heads 121 / 81, 32 heads 124 / 103,
     //   192 heads 305 / 571; T = 256 64 heads 35 / 25, 96 heads 36 / 37; 64 heads x 512 x 48 65 / 60; 160 heads x T = 100 20 / 28
     //   D = 32: 8 heads x T = 40 9.8 / 7.3, x T = 256 29 / 10; 64 x 128 16 / 8.8; 152 x 250 31 / 41; 2 x 2050 210 / 49
     // A row has the same bits from both, so a head's result does not depend on how many others are in the call.
     const int64_t tiles = cdiv(a.T, 32), whole = tiles / 8, eights = 4 * whole * (whole + 1) + tiles % 8 * (whole + 1);
     const int64_t heads = (int64_t)a.B * a.H;
-    if (26 * eights * heads <= 10 * num_cus() * tiles) {
+    if (tiles > 1 && 26 * eights * heads <= 10 * num_cus() * tiles) {
       ah::launch_kernel(k_flash_fwd_f32_keys<D>, dim3((unsigned)tiles, (unsigned)heads), dim3(512), 0, a);
       AH_LAUNCH_CHECK();
       return AH_OK;

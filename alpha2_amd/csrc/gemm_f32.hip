@@ -171,13 +171,14 @@ constexpr int S_BK = 16;
 constexpr int S_FLUSH = 4;
 __device__ __forceinline__ int plane_ofs(int row, int k4) { return row * 32 + ((((k4 >> 1) ^ (row >> 3)) & 1) << 4) + (k4 & 1) * 8; }
 
-template <bool KCONTIG, int ROWS>
+template <bool KCONTIG, int ROWS, bool TAIL>
 __device__ __forceinline__ void store_split(char *s, const float4 (&v)[ROWS / 64]) {
   const int t = threadIdx.x;
 #pragma unroll
   for (int i = 0; i < ROWS / 64; i++) {
     const int r = (KCONTIG ? t >> 2 : t & 63) + 64 * i, k4 = KCONTIG ? t & 3 : t >> 6;
-    const Split2 a = split2(v[i].x * SPLIT_UP, v[i].y * SPLIT_UP), b = split2(v[i].z * SPLIT_UP, v[i].w * SPLIT_UP);
+    const float4 x = TAIL ? make_float4(here(v[i].x), here(v[i].y), here(v[i].z), here(v[i].w)) : v[i];
+    const Split2 a = split2(x.x * SPLIT_UP, x.y * SPLIT_UP), b = split2(x.z * SPLIT_UP, x.w * SPLIT_UP);
     char *p = s + plane_ofs(r, k4);
     *reinterpret_cast<uint2 *>(p) = make_uint2(a.h, b.h);
     *reinterpret_cast<uint2 *>(p + ROWS * 32) = make_uint2(a.m, b.m);
@@ -244,8 +245,8 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f32_split(GemmArgs g, int vec_c
     load_tile<B_KC, BN, VEC, false>(B, g.ldb, n0, t * S_BK, g.N, g.K, rb);
   };
   auto put = [&](char *buf) {
-    store_split<A_KC, BM>(buf, ra);
-    store_split<B_KC, BN>(buf + ABYTES, rb);
+    store_split<A_KC, BM, false>(buf, ra);
+    store_split<B_KC, BN, false>(buf + ABYTES, rb);
   };
   bf16x8 fa[3][TM], fb[3][TN];
   auto get = [&](const char *buf) {
@@ -282,7 +283,8 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f32_split(GemmArgs g, int vec_c
     if (full % S_FLUSH == 0) flush();
     load_tile<A_KC, BM, VEC, true>(A, g.lda, m0, full * S_BK, g.M, g.K, ra);
     load_tile<B_KC, BN, VEC, true>(B, g.ldb, n0, full * S_BK, g.N, g.K, rb);
-    put(smem);
+    store_split<A_KC, BM, true>(smem, ra);
+    store_split<B_KC, BN, true>(smem + ABYTES, rb);
     __syncthreads();
     get(smem);
     mfma6_tiles<TM, TN>(fa, fb, acc);
@@ -349,7 +351,7 @@ __device__ __forceinline__ void contract_pieces(const GemmArgs &g, const float *
       } else {
         bf16x8 fa[3], fb[3];
 #pragma unroll
-        for (int e = 0; e < 8; e++) { a[u][e] *= SPLIT_UP; b[u][e] *= SPLIT_UP; }
+        for (int e = 0; e < 8; e++) { a[u][e] = here(a[u][e]) * SPLIT_UP; b[u][e] = here(b[u][e]) * SPLIT_UP; }
         split8(a[u], fa);
         split8(b[u], fb);
         mfma6(fb, fa, acc);                                     // C^T
@@ -426,8 +428,8 @@ struct F32Choice { int bm, waves, splits; };
 //   slices      another launch, and the workspace written and read
 // Against 128 x 128 tiles of v_mfma_f32_32x32x2_f32 (in slices where there were fewer than 256 tiles and K >= 2048), in us:
 //   16384 x 3072 x 768 NT 720 -> 430 (128 x 128), 768 x 768 x 16384 TN 329 -> 157 (128 x 128 in 32 slices), 490 x 768 x 768 NT 77 -> 16
-//   (64 x 64 in 4 slices), 48 x 768 x 256 NT 26 -> 7 and 512 x 128 x 1024 TN 97 -> 9 (32 x 32); with the operands scaled 1 to 5 % more,
-//   16384 x 3072 x 768 NT 549 -> 557 and 490 x 768 x 768 16.7 -> 17.5 back to back on standard normal operands.  Operands that are not
+//   (64 x 64 in 4 slices), 48 x 768 x 256 NT 26 -> 7 and 512 x 128 x 1024 TN 97 -> 9 (32 x 32); with the operands scaled 1 % more over
+//   132 random shapes (15 % at worst), 16384 x 3072 x 768 NT 549 -> 557 and 490 x 768 x 768 16.7 -> 17.5 back to back on standard normal operands.  Operands that are not
 //   finite take the fp32 instruction as well: 16384 x 3072 x 768 of NaNs 1070 (720 by that instruction's own kernel).
 F32Choice choose(const GemmArgs &ga, int layout, int batch, bool may_split, bool long_rows) {
   struct Tile { int bm; double step, full; };

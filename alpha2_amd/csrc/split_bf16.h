@@ -19,6 +19,12 @@ namespace ah {
 
 constexpr float SPLIT_UP = 0x1p24f, SPLIT_DOWN = 0x1p-48f;
 
+// A value that was loaded under a condition (zero past the end of a row), where it is used: the compiler would multiply it in the branch
+// that loads it otherwise, and wait for it there.
+__device__ __forceinline__ float here(float x) {
+  asm("" : "+v"(x));
+  return x;
+}
 struct Split2 { uint32_t h, m, l; };       // the parts of two values side by side
 // x0, x1: values that are already multiplied by SPLIT_UP
 __device__ __forceinline__ Split2 split2(float x0, float x1) {
