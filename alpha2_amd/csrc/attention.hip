@@ -48,8 +48,9 @@ __device__ __forceinline__ void load_tile_f32(float *s, const float *__restrict_
 // 16-byte pieces are permuted within a row so that 16 lanes that read the same piece of 16 rows meet 64 different banks.
 // A result that is not finite has the block computed again with the fp32 instruction, whose result stands; so does a score.
 // 192 heads x 1024 x 64: dK and dV 945 -> 486 us, dQ 520 -> 316; 512 x 256 x 32: 112 -> 84 and 81 -> 60; 4 x 70 x 64: 29 -> 24 and
-// 26 -> 20 (before both operands were scaled, which costs 1 % of the backward pass at 192 x 1024 x 64 and 3 to 6 % of smaller ones).  Relative error against 64 bits at 4 x 512 x 64: dQ 4.6e-7 -> 3.7e-7, dK 6.4e-7 -> 3.8e-7, dV 6.0e-7 -> 3.3e-7.  What bounds
-// it now is vector issue: tanh, exp and the cut of scores, K and V for every 32 x 32 tile beside 3072 cycles of matrix instructions.
+// 26 -> 20 (before both operands were scaled, which costs 1 % of the backward pass at 192 x 1024 x 64 and 3 to 6 % of smaller ones).
+// Relative error against 64 bits at 4 x 512 x 64: dQ 4.6e-7 -> 3.7e-7, dK 6.4e-7 -> 3.8e-7, dV 6.0e-7 -> 3.3e-7.  What bounds it now is
+// vector issue: tanh, exp and the cut of scores, K and V for every 32 x 32 tile beside 3072 cycles of matrix instructions.
 template <int D>
 struct SplitTile {                          // D = 32 or 64
   static constexpr int F = D / 32, PLANE = 64 * D, BYTES = 3 * PLANE;      // either layout
@@ -69,6 +70,7 @@ struct SplitTile {                          // D = 32 or 64
       }
     }
   }
+  // (ahead of the barrier in front of put: some of the cut then goes ahead of it too)
   static __device__ __forceinline__ void scale(float (&x)[4][F], float mul) {
 #pragma unroll
     for (int r = 0; r < 4; r++)

@@ -429,8 +429,9 @@ struct F32Choice { int bm, waves, splits; };
 // Against 128 x 128 tiles of v_mfma_f32_32x32x2_f32 (in slices where there were fewer than 256 tiles and K >= 2048), in us:
 //   16384 x 3072 x 768 NT 720 -> 430 (128 x 128), 768 x 768 x 16384 TN 329 -> 157 (128 x 128 in 32 slices), 490 x 768 x 768 NT 77 -> 16
 //   (64 x 64 in 4 slices), 48 x 768 x 256 NT 26 -> 7 and 512 x 128 x 1024 TN 97 -> 9 (32 x 32); with the operands scaled 1 % more over
-//   132 random shapes (15 % at worst), 16384 x 3072 x 768 NT 549 -> 557 and 490 x 768 x 768 16.7 -> 17.5 back to back on standard normal operands.  Operands that are not
-//   finite take the fp32 instruction as well: 16384 x 3072 x 768 of NaNs 1070 (720 by that instruction's own kernel).
+//   132 random shapes (15 % at worst), 16384 x 3072 x 768 NT 549 -> 557 and 490 x 768 x 768 16.7 -> 17.5 back to back on standard
+//   normal operands.  Operands that are not finite take the fp32 instruction as well: 16384 x 3072 x 768 of NaNs 1070 (720 by that
+//   instruction's own kernel).
 F32Choice choose(const GemmArgs &ga, int layout, int batch, bool may_split, bool long_rows) {
   struct Tile { int bm; double step, full; };
   static constexpr Tile TILES[2] = {{64, 0.26, 0.24}, {128, 1.2, 0.65}};
