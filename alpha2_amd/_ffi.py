@@ -18,6 +18,8 @@ GELU_BWD, RELU_BWD, SILU_BWD, CLAMP_BWD, SOFTCAP_BWD = range(5)
 GEMM_NN, GEMM_NT, GEMM_TN = 0, 1, 2
 EPI_NONE, EPI_ACCUM, EPI_GELU, EPI_RESIDUAL, EPI_GELU_BWD, EPI_GELU_GRAD, EPI_MUL_AUX = range(7)
 
+DECODE_GATED = 32
+
 u64, i64, i32, f32 = C.c_uint64, C.c_int64, C.c_int32, C.c_float
 p_i64 = C.POINTER(C.c_int64)
 
@@ -47,6 +49,16 @@ class AhFlash(C.Structure):
                 ("scale", f32), ("soft_cap", f32),
                 ("q", u64), ("k", u64), ("v", u64), ("o", u64), ("lse", u64),
                 ("d_o", u64), ("dq", u64), ("dk", u64), ("dv", u64), ("bwd_variant", i32), ("reserved", i32)]
+
+
+class AhDecodeLayer(C.Structure):
+    _fields_ = [(n, u64) for n in ("ln1_w", "ln1_b", "wqkv", "wo", "ln2_w", "ln2_b", "fc1", "up", "fc2")] + [("coef", u64 * 5)]
+
+
+class AhDecode(C.Structure):
+    _fields_ = [("vocab", i32), ("width", i32), ("heads", i32), ("ffn", i32), ("layers", i32), ("act", i32), ("rows", i32),
+                ("scale", f32), ("cap", f32), ("eps", f32),
+                ("wte", u64), ("wpe", u64), ("lnf_w", u64), ("lnf_b", u64), ("head", u64), ("kv", u64), ("logits", u64)]
 
 
 class AhRng(C.Structure):
@@ -137,6 +149,7 @@ SIGNATURES = {
     "ah_probe_mfma_bf16": [i32, i32, i32, C.POINTER(C.c_double)],
     "ah_probe_issue": [i32, i32, i32, C.POINTER(C.c_double)],
     "ah_flash_fwd": [C.POINTER(AhFlash)], "ah_flash_bwd": [C.POINTER(AhFlash)],
+    "ah_decode": [C.POINTER(AhDecode), C.POINTER(AhDecodeLayer), i32, i32], "ah_decode_head": [C.POINTER(AhDecode), u64],
     "ah_adamw": [u64, u64, u64, u64, u64, C.POINTER(AhAdamW), u64, u64, u64],
     "ah_clip_coef": [u64, f32, f32, u64],
     "ah_side_begin": [], "ah_side_end": [], "ah_side_join": [],

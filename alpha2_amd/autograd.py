@@ -146,6 +146,7 @@ class Ctx:
     backend: object
     dropoutRng: Optional[DropoutRng] = None
     release: Release = None
+    keptQkv: Optional[list] = None      # a list takes each block's q, k, v projection as it is computed
 
 
 def _record(ctx: Ctx, data: TensorData, inputs, backward, cleanup=None) -> Variable:

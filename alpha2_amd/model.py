@@ -142,6 +142,8 @@ def transformerBlock(ctx: Ctx, x: Variable, layer: dict, cfg: ModelConfig, Bt: i
     Bk = ctx.backend
     ln1 = ag.layerNorm(ctx, x, layer["ln1"]["weight"], layer["ln1"]["bias"], 1e-5)
     qkv = ag.matmulTransposed(ctx, ag.reshape(ctx, ln1, [Bt * T, Cc]), layer["attn"]["wqkv"])
+    if ctx.keptQkv is not None:
+        ctx.keptQkv.append(qkv)
     cap = cfg.softCap if cfg.softCap is not None else 30.0
     scl = 1 / math.sqrt(D)
     if cfg.attention == "heads" and cfg.dropout == 0 and ag._has(Bk, "attentionQkv") and flashHeadSize(D):
@@ -209,11 +211,10 @@ def transformerBlock(ctx: Ctx, x: Variable, layer: dict, cfg: ModelConfig, Bt: i
     return ag.residualDropoutAdd(ctx, x, ag.reshape(ctx, mlpH, [Bt, T, Cc]), cfg.dropout, training)
 
 
-def gptForward(cfg: ModelConfig, params: dict, backend, tape: Tape, tokens: TensorData, targets: Optional[TensorData] = None,
-               training: bool = False, activationCheckpointing: bool = False, mixedPrecision: bool = False,
-               dropoutRng=None, release=None):
-    """gpt.ts:344-427.  Returns {"logits": Variable, "loss": Variable | None}."""
-    ctx = Ctx(tape, backend, dropoutRng, release)
+def gptBlocks(ctx: Ctx, cfg: ModelConfig, params: dict, tokens: TensorData, training: bool = False, activationCheckpointing: bool = False,
+              mixedPrecision: bool = False) -> Variable:
+    """gpt.ts:344-412: the embeddings and the blocks, what the last LayerNorm and the head read."""
+    backend, dropoutRng = ctx.backend, ctx.dropoutRng
     Bt, T = tokens.shape
     tok = ag.embedding(ctx, params["wte"], tokens)
     key = (id(backend), Bt, T)
@@ -245,6 +246,16 @@ def gptForward(cfg: ModelConfig, params: dict, backend, tape: Tape, tokens: Tens
             if mixedPrecision and training:
                 x = ag.castToF32(ctx, x)
             x = transformerBlock(ctx, x, layer, cfg, Bt, T, mask, training)
+    return x
+
+
+def gptForward(cfg: ModelConfig, params: dict, backend, tape: Tape, tokens: TensorData, targets: Optional[TensorData] = None,
+               training: bool = False, activationCheckpointing: bool = False, mixedPrecision: bool = False,
+               dropoutRng=None, release=None):
+    """gpt.ts:344-427.  Returns {"logits": Variable, "loss": Variable | None}."""
+    ctx = Ctx(tape, backend, dropoutRng, release)
+    Bt, T = tokens.shape
+    x = gptBlocks(ctx, cfg, params, tokens, training, activationCheckpointing, mixedPrecision)
     x = ag.layerNorm(ctx, x, params["lnF"]["weight"], params["lnF"]["bias"], 1e-5)
     flat = ag.reshape(ctx, x, [Bt * T, cfg.nEmbd])
     logits = ag.reshape(ctx, ag.matmulTransposed(ctx, flat, params["lmHead"]), [Bt, T, cfg.vocabSize])

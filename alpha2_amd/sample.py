@@ -1,6 +1,7 @@
-"""Text generation from a trained model (packages/train/src/sample.ts:23-201): one forward per new token over the last
-blockSize tokens, then greedy / top-k / nucleus / full-softmax selection on the host with the reference's arithmetic (f32
-storage, double accumulation, stable descending sorts) and its use of the seeded rng (one draw per sampled token)."""
+"""Text generation from a trained model (packages/train/src/sample.ts:23-201): for each new token the logits behind the last
+blockSize tokens (by a forward pass over them, or from kept keys and values where the model allows it: decode.py), then greedy /
+top-k / nucleus / full-softmax selection on the host with the reference's arithmetic (f32 storage, double accumulation, stable
+descending sorts) and its use of the seeded rng (one draw per sampled token)."""
 from __future__ import annotations
 
 import math
@@ -11,6 +12,7 @@ import numpy as np
 
 from .autograd import Tape
 from .backend import TensorData
+from .decode import KeptContext
 from .model import ModelConfig, gptForward
 
 
@@ -35,7 +37,7 @@ def selectToken(lastLogits: np.ndarray, rng, temperature: float, topk: int, topP
     if temperature <= 0:                                                    # sample.ts:85-99: first maximum wins
         return int(np.argmax(lastLogits))
     if 0 < topk < V:                                                        # sample.ts:102-109: ties with the k-th value stay
-        threshold = lastLogits[_stable_desc(lastLogits)[topk - 1]]
+        threshold = -np.partition(-lastLogits, topk - 1)[topk - 1]
         lastLogits[lastLogits < threshold] = -np.inf
     if 0 < topP < 1:                                                        # sample.ts:112-163
         maxVal = float(np.max(lastLogits))
@@ -77,6 +79,22 @@ def selectToken(lastLogits: np.ndarray, rng, temperature: float, topk: int, topP
     return int(hit[0]) if hit.size else 0
 
 
+def _lastRow(config: ModelConfig, params: dict, backend, context: np.ndarray, releaseTensor: Optional[Callable]) -> np.ndarray:
+    """The logits behind the last token of `context`, from a forward pass over all of it (sample.ts:48-80)."""
+    V = config.vocabSize
+    inputData = TensorData((1, context.size), "i32", context.copy())
+    tape = Tape()
+    logits = gptForward(config, params, backend, tape, inputData)["logits"]
+    row = backend.slice(logits.data, [0, context.size - 1, 0], [1, context.size, V]) if hasattr(backend, "slice") else None
+    last = np.asarray(row.data if row is not None else logits.data.data.reshape(-1)[(context.size - 1) * V:], dtype=np.float32).reshape(-1).copy()
+    if row is not None and releaseTensor is not None:
+        releaseTensor(row)
+    tape.clear(releaseTensor)
+    if releaseTensor is not None:
+        releaseTensor(inputData)
+    return last
+
+
 def sampleTokens(config: ModelConfig, params: dict, backend, rng, promptTokens: Sequence[int], sampleConfig: SampleConfig,
                  releaseTensor: Optional[Callable] = None, flushGpu: Optional[Callable] = None) -> np.ndarray:
     """The token loop of sample() (sample.ts:36-198) without the tokenizer: returns prompt + generated ids."""
@@ -90,30 +108,25 @@ def sampleTokens(config: ModelConfig, params: dict, backend, rng, promptTokens: 
     if prompt.size > maxLen:                                                # say so instead of truncating silently
         raise ValueError(f"prompt of {prompt.size} tokens exceeds blockSize {config.blockSize}")
     currentLen = int(prompt.size)
-    V = config.vocabSize
-    i = 0
-    while i < steps and currentLen < config.blockSize:
-        ctxStart = max(0, currentLen - config.blockSize)
-        ctx = tokens[ctxStart:currentLen].copy()
-        inputData = TensorData((1, ctx.size), "i32", ctx)
-        tape = Tape()
-        logits = gptForward(config, params, backend, tape, inputData)["logits"]
-        row = backend.slice(logits.data, [0, ctx.size - 1, 0], [1, ctx.size, V]) if hasattr(backend, "slice") else None
-        last = np.asarray(row.data if row is not None else logits.data.data.reshape(-1)[(ctx.size - 1) * V:], dtype=np.float32).reshape(-1).copy()
-        if row is not None and releaseTensor is not None:
-            releaseTensor(row)
-        if temperature > 0:
-            last = (last.astype(np.float64) / temperature).astype(np.float32)
-        tape.clear(releaseTensor)
-        if releaseTensor is not None:
-            releaseTensor(inputData)
-        if flushGpu is not None and (i & 7) == 7:
-            flushGpu()
-        nxt = selectToken(last, rng, temperature, topk, topP)
-        if currentLen < maxLen:
-            tokens[currentLen] = nxt
-            currentLen += 1
-        i += 1
+    kept = KeptContext.of(config, params, backend, maxLen) if 0 < currentLen < maxLen else None
+    try:
+        i = 0
+        while i < steps and currentLen < config.blockSize:
+            last = _lastRow(config, params, backend, tokens[:currentLen], releaseTensor) if kept is None else kept.lastRow(tokens[:currentLen], releaseTensor)
+            if temperature > 0:
+                last = (last.astype(np.float64) / temperature).astype(np.float32)
+            if flushGpu is not None and (i & 7) == 7:
+                flushGpu()
+                if kept is not None:
+                    kept.describe()
+            nxt = selectToken(last, rng, temperature, topk, topP)
+            if currentLen < maxLen:
+                tokens[currentLen] = nxt
+                currentLen += 1
+            i += 1
+    finally:
+        if kept is not None:
+            kept.close()
     return tokens[:currentLen]
 
 

@@ -447,6 +447,28 @@ typedef struct {
 int32_t ah_flash_fwd(const AhFlash *f);
 int32_t ah_flash_bwd(const AhFlash *f);
 
+/* ---- one token of a model of this library, from kept keys and values.  sample() (packages/train/src/sample.ts:36-198) runs the
+ *      forward pass (packages/model/src/gpt.ts:220-427, evaluation: no dropout) over the whole context for every new token;
+ *      under causal attention over heads the rows before the new one are what they were, and reach it through their keys and
+ *      values only.  All tensors f32, 16-byte aligned, matrices [out, in]; width <= 4096 in heads of 8, 16, .. 128 features. ---- */
+#define AH_DECODE_GATED 32   /* AhDecode.act: silu(fc1 x) * (up x); otherwise a mask of bases as in ah_channel_act */
+typedef struct {
+  ah_ptr ln1_w, ln1_b, wqkv, wo, ln2_w, ln2_b, fc1, up, fc2;      /* up: gated only */
+  ah_ptr coef[5];            /* f32[ffn] per basis of the mask, 0: the constant 1 */
+} AhDecodeLayer;
+typedef struct {
+  int32_t vocab, width, heads, ffn, layers, act;
+  int32_t rows;              /* of the cache */
+  float   scale, cap, eps;   /* scores: scale, then cap * tanh(s / cap) if cap > 0; eps of the LayerNorms */
+  ah_ptr  wte, wpe, lnf_w, lnf_b, head;
+  ah_ptr  kv;                /* [layers][rows][3 * width]: q, k, v of every position so far, as the product with wqkv leaves them */
+  ah_ptr  logits;            /* out, f32[vocab] */
+} AhDecode;
+/* `token` at position `pos`: rows 0 .. pos - 1 of kv are read, row pos is written (in every layer), then the logits. */
+int32_t ah_decode(const AhDecode *d, const AhDecodeLayer *layers, int32_t token, int32_t pos);
+/* The logits of one row that has been through all layers: the last LayerNorm and the head. */
+int32_t ah_decode_head(const AhDecode *d, ah_ptr row);
+
 /* ---- optimizer.  Backend.adamwStep (interfaces.ts:149-150; CPU loop optimizers.ts:76-92). ---- */
 typedef struct {
   float lr, beta1, beta2, eps, weight_decay, bc1, bc2, grad_scale;

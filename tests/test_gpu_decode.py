@@ -1,0 +1,151 @@
+"""Kept keys and values (ah_decode) against the same model in 64 bits, beside the pass over the whole context."""
+import math
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def B():
+    from alpha2_amd import HipBackend
+    return HipBackend(0)
+
+
+def _model(B, vocab, ctx, layers, width, heads, **more):
+    from alpha2_amd.model import ModelConfig, initGPT
+    from alpha2_amd.rng import SeededRng
+    cfg = ModelConfig(vocabSize=vocab, blockSize=ctx, nLayer=layers, nEmbd=width, nHead=heads, **more)
+    params = initGPT(cfg, B, SeededRng(3))
+    rs = np.random.RandomState(5)
+    for l in params["layers"]:                  # gains, biases and coefficients that are not all the same
+        for v in (l["ln1"]["weight"], l["ln1"]["bias"], l["ln2"]["weight"], l["ln2"]["bias"],
+                  *(l["mlp"][n] for n in l["mlp"] if n.startswith(("act_", "kan_")))):
+            v.data.data = v.data.data + 0.2 * rs.standard_normal(v.data.data.size).astype(np.float32)
+        l["attn"]["wqkv"].data.data *= 75.0 / math.sqrt(width)      # q and k of 1.5, scores of a few units whatever the width: the softmax is not flat
+    return cfg, params
+
+
+def _logits64(cfg, params, tokens):
+    """All rows' logits in 64 bits."""
+    f = lambda v: v.data.data.reshape(v.data.shape).astype(np.float64)
+    sigmoid = lambda x: 1 / (1 + np.exp(-x))
+    silu = lambda x: x * sigmoid(x)
+    gelu = lambda x: x * sigmoid(2 * math.sqrt(2 / math.pi) * (x + 0.044715 * x ** 3))
+
+    def norm(x, p):
+        c = x - x.mean(1, keepdims=True)
+        return c / np.sqrt((c * c).mean(1, keepdims=True) + 1e-5) * f(p["weight"]) + f(p["bias"])
+    T, H, C = len(tokens), cfg.nHead, cfg.nEmbd
+    cap, act = 30.0 if cfg.softCap is None else cfg.softCap, cfg.ffnActivation
+    x = f(params["wte"])[tokens] + f(params["wpe"])[:T]
+    for l in params["layers"]:
+        q, k, v = ((norm(x, l["ln1"]) @ f(l["attn"]["wqkv"]).T)[:, i * C:(i + 1) * C].reshape(T, H, C // H).transpose(1, 0, 2) for i in range(3))
+        s = q @ k.transpose(0, 2, 1) / math.sqrt(C // H)
+        if cap > 0:
+            s = cap * np.tanh(s / cap)
+        s = np.where(np.tril(np.ones((T, T), bool)), s, -np.inf)
+        p = np.exp(s - s.max(2, keepdims=True))
+        x = x + (p / p.sum(2, keepdims=True) @ v).transpose(1, 0, 2).reshape(T, C) @ f(l["attn"]["wo"]).T
+        y, m = norm(x, l["ln2"]), l["mlp"]
+        if act == "swiglu":
+            x = x + (silu(y @ f(m["fc_gate"]).T) * (y @ f(m["fc_up"]).T)) @ f(m["fc_proj"]).T
+            continue
+        h = y @ f(m["fc1"]).T
+        if act == "universal":
+            h = silu(h) * f(m["act_gate"]) + h * f(m["act_skip"])
+        elif act == "kan_spline":
+            h = silu(h) * f(m["kan_c0"]) + np.maximum(h, 0) * f(m["kan_c1"]) + gelu(h) * f(m["kan_c2"]) + h * f(m["kan_c3"]) + h * h * f(m["kan_c4"])
+        else:
+            h = {"gelu": gelu, "silu": silu, "relu": lambda x: np.maximum(x, 0)}[act](h)
+        x = x + h @ f(m["fc2"]).T
+    return norm(x, params["lnF"]) @ f(params["lmHead"]).T
+
+
+def _compare(kept, cfg, params, B, tokens, lengths, restart):
+    """Both sum the same terms in fp32; the kept row sums its in shorter runs, so over the rows it is no further from 64 bits (root mean
+    square of the rows' relative errors) than the pass over the whole context is, but for the scatter of a few dozen rows of which one
+    ill-conditioned one weighs most: 1.5 times.  Where the sums are so short that both are single roundings away, the bound is those:
+    eight after one another in a block (the norm's three, product, two on a score, exponential, weighted sum) and as many around the
+    blocks, 2^-24 each."""
+    from alpha2_amd.sample import _lastRow
+    exact = _logits64(cfg, params, tokens)
+    ours, theirs = [], []
+    for n in lengths:
+        if restart:
+            kept.known = 0
+            kept.lastRow(tokens[:n - 1], B.releaseGpuTensor)
+        off = lambda row: np.linalg.norm(row.astype(np.float64) - exact[n - 1]) / np.linalg.norm(exact[n - 1])
+        ours.append(off(kept.lastRow(tokens[:n], B.releaseGpuTensor)))
+        theirs.append(off(_lastRow(cfg, params, B, tokens[:n], B.releaseGpuTensor)))
+    ours, theirs = (math.sqrt(np.mean(np.square(e))) for e in (ours, theirs))
+    print("off 64 bits: kept %.2e, whole context %.2e" % (ours, theirs))
+    assert ours <= max(1.5 * theirs, 8 * (cfg.nLayer + 1) * 2.0 ** -24), (ours, theirs)
+
+
+# widths on both sides of a lane's float4 counts (256, 512, 1024, 2048), head sizes of every group width and between two, rows of
+# the head that fill no wave, every activation, with and without the cap
+CASES = [
+    (7, 80, 1, 8, 1, dict()),
+    (97, 80, 2, 64, 4, dict(softCap=0.0)),
+    (256, 80, 2, 256, 8, dict(ffnActivation="swiglu")),
+    (2049, 40, 1, 264, 11, dict(ffnActivation="silu")),
+    (300, 40, 1, 480, 6, dict(ffnActivation="universal")),
+    (301, 40, 2, 768, 12, dict(ffnActivation="kan_spline")),
+    (64, 24, 1, 1024, 8, dict(ffnActivation="relu")),
+    (66, 24, 1, 1040, 13, dict(ffnDim=100)),
+    (66, 24, 1, 2056, 257, dict(ffnDim=4100, ffnActivation="swiglu")),
+]
+
+
+@pytest.mark.parametrize("vocab,ctx,layers,width,heads,more", CASES)
+def test_logits_behind_a_growing_context(B, vocab, ctx, layers, width, heads, more):
+    from alpha2_amd.decode import KeptContext
+    cfg, params = _model(B, vocab, ctx, layers, width, heads, **more)
+    tokens = np.random.RandomState(1).randint(0, vocab, ctx).astype(np.int32)
+    for prompt in (1, ctx // 2):
+        kept = KeptContext.of(cfg, params, B, ctx)
+        assert kept is not None
+        _compare(kept, cfg, params, B, tokens, range(prompt, ctx + 1), False)
+        kept.close()
+
+
+@pytest.mark.parametrize("head_size", [16, 32, 64, 128])
+def test_slices_of_a_long_context(B, head_size):
+    """One key more than so many slices hold, and one less: 64 keys to a slice up to 1024, then 16 longer ones."""
+    from alpha2_amd.decode import KeptContext
+    cfg, params = _model(B, 50, 1200, 1, 2 * head_size, 2)
+    tokens = np.random.RandomState(2).randint(0, 50, 1200).astype(np.int32)
+    kept = KeptContext.of(cfg, params, B, 1200)
+    _compare(kept, cfg, params, B, tokens, (62, 63, 64, 65, 127, 128, 129, 577, 1023, 1024, 1025, 1026, 1199, 1200), True)
+    kept.close()
+
+
+def test_what_the_kernels_do_not_take_runs_the_whole_context(B):
+    from alpha2_amd import FastHipBackend
+    from alpha2_amd.decode import KeptContext
+    for more in (dict(attention="reference-flash"), dict(dropout=0.1), dict(ffnDim=6), dict(attention="unfused")):
+        cfg, params = _model(B, 30, 16, 1, 32, 2, **more)
+        assert KeptContext.of(cfg, params, B, 16) is None, more
+    cfg, params = _model(B, 30, 16, 1, 40, 2)               # head size 20
+    assert KeptContext.of(cfg, params, B, 16) is None
+    cfg, params = _model(B, 30, 16, 1, 32, 2)
+    assert KeptContext.of(cfg, params, FastHipBackend(0), 16) is None
+    kept = KeptContext.of(cfg, params, B, 16)
+    live = B.gpuMemStats()["liveAllocs"]
+    kept.close()
+    assert B.gpuMemStats()["liveAllocs"] == live - 2
+
+
+def test_not_finite_parameters_reach_the_logits(B):
+    from alpha2_amd.decode import KeptContext
+    from alpha2_amd.sample import _lastRow
+    cfg, params = _model(B, 30, 16, 1, 32, 2)
+    params["wpe"].data.data[5 * 32] = np.nan                # position 5: seen from there on
+    tokens = np.arange(8, dtype=np.int32)
+    kept = KeptContext.of(cfg, params, B, 16)
+    for n in range(1, 9):
+        got, want = kept.lastRow(tokens[:n], B.releaseGpuTensor), _lastRow(cfg, params, B, tokens[:n], B.releaseGpuTensor)
+        assert np.array_equal(np.isnan(got), np.isnan(want)), n
+    kept.close()
