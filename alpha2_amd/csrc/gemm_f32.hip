@@ -6,6 +6,7 @@
 #include "gemm_common.h"
 #include "split_bf16.h"
 #include <cmath>
+#include <type_traits>
 
 using namespace ah;
 
@@ -15,31 +16,37 @@ namespace {
 // LDS tiles are k-major: As[k][m], Bs[k][n]; a lane of the 32x32x2 MFMA reads As[2*kk + lane/32][m0 + lane%32].
 constexpr int F_BK = 16, F_PAD = 4;
 
-// Load a [ROWS x F_BK] tile of an operand into registers (ROWS / 64 float4 per thread: 4 consecutive k of one row).
-//   KCONTIG = true : memory is [row][k] (k contiguous), thread -> (row = t/4 + 64*i, k = 4*(t%4)..+3)
-//   KCONTIG = false: memory is [k][row] (row contiguous), thread -> (row = t%64 + 64*i, k = 4*(t/64)..+3)
+// A [rows x F_BK] tile of an operand in registers: a float4 per thread for every 64 rows, 4 consecutive k of one row.  The row and the
+// quarter of the 16 k of a thread's i-th:
+//   KCONTIG = true : memory is [row][k] (k contiguous), 4 threads side by side along a row
+//   KCONTIG = false: memory is [k][row] (row contiguous), a wave along 64 rows
+template <bool KCONTIG>
+__device__ __forceinline__ int part_row(int i) { return (KCONTIG ? threadIdx.x >> 2 : threadIdx.x & 63) + 64 * i; }
+template <bool KCONTIG>
+__device__ __forceinline__ int part_k4() { return KCONTIG ? threadIdx.x & 3 : threadIdx.x >> 6; }
 // TAIL: k from K on reads as zero.  VEC: the rows of a k-contiguous operand are 16-byte aligned.
 // The tile's corner is a scalar address and the thread's part of it 32 bits (the rows of a tile span less than 4 GiB).
-template <bool KCONTIG, int ROWS, bool VEC, bool TAIL>
-__device__ __forceinline__ void load_tile(const float *__restrict__ base, int64_t ld, int row0, int k0, int rows, int K, float4 (&v)[ROWS / 64]) {
-  const int t = threadIdx.x, kw = __builtin_amdgcn_readfirstlane(t >> 6) * 4, last = rows - 1 - row0;
+template <bool KCONTIG, bool VEC, bool TAIL>
+__device__ __forceinline__ float4 load_part(const float *__restrict__ base, int64_t ld, int row0, int k0, int rows, int K, int i) {
+  const int t = threadIdx.x, kw = KCONTIG ? 0 : __builtin_amdgcn_readfirstlane(part_k4<KCONTIG>()) * 4, last = rows - 1 - row0;
   const float *corner = KCONTIG ? base + (int64_t)row0 * ld + k0 : base + (int64_t)(k0 + kw) * ld + row0;
-#pragma unroll
-  for (int i = 0; i < ROWS / 64; i++) {
-    const int r = min((KCONTIG ? t >> 2 : t & 63) + 64 * i, last);      // rows past the end repeat the last one: their results are not stored
-    if (KCONTIG) {
-      const int k = k0 + (t & 3) * 4;
-      const float *p = reinterpret_cast<const float *>(reinterpret_cast<const char *>(corner) + ((uint32_t)r * (uint32_t)ld + (t & 3) * 4) * 4u);
-      if (TAIL) v[i] = make_float4(k < K ? p[0] : 0.f, k + 1 < K ? p[1] : 0.f, k + 2 < K ? p[2] : 0.f, k + 3 < K ? p[3] : 0.f);
-      else if (VEC) v[i] = *reinterpret_cast<const float4 *>(p);
-      else v[i] = make_float4(p[0], p[1], p[2], p[3]);
-    } else {
-      const int k = k0 + kw;
-      const float *p0 = corner, *p1 = p0 + ld, *p2 = p1 + ld, *p3 = p2 + ld;
-      if (TAIL) v[i] = make_float4(k < K ? p0[r] : 0.f, k + 1 < K ? p1[r] : 0.f, k + 2 < K ? p2[r] : 0.f, k + 3 < K ? p3[r] : 0.f);
-      else v[i] = make_float4(p0[(uint32_t)r], p1[(uint32_t)r], p2[(uint32_t)r], p3[(uint32_t)r]);
-    }
+  const int r = min(part_row<KCONTIG>(i), last);      // rows past the end repeat the last one: their results are not stored
+  if (KCONTIG) {
+    const int k = k0 + (t & 3) * 4;
+    const float *p = reinterpret_cast<const float *>(reinterpret_cast<const char *>(corner) + ((uint32_t)r * (uint32_t)ld + (t & 3) * 4) * 4u);
+    if (TAIL) return make_float4(k < K ? p[0] : 0.f, k + 1 < K ? p[1] : 0.f, k + 2 < K ? p[2] : 0.f, k + 3 < K ? p[3] : 0.f);
+    if (VEC) return *reinterpret_cast<const float4 *>(p);
+    return make_float4(p[0], p[1], p[2], p[3]);
   }
+  const int k = k0 + kw;
+  const float *p0 = corner, *p1 = p0 + ld, *p2 = p1 + ld, *p3 = p2 + ld;
+  if (TAIL) return make_float4(k < K ? p0[r] : 0.f, k + 1 < K ? p1[r] : 0.f, k + 2 < K ? p2[r] : 0.f, k + 3 < K ? p3[r] : 0.f);
+  return make_float4(p0[(uint32_t)r], p1[(uint32_t)r], p2[(uint32_t)r], p3[(uint32_t)r]);
+}
+template <bool KCONTIG, int N, bool VEC, bool TAIL>
+__device__ __forceinline__ void load_tile(const float *__restrict__ base, int64_t ld, int row0, int k0, int rows, int K, float4 (&v)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; i++) v[i] = load_part<KCONTIG, VEC, TAIL>(base, ld, row0, k0, rows, K, i);
 }
 
 // Four results side by side: what the epilogue makes of them, 16-byte accesses where vec.  PLAIN: f32 results as they are;
@@ -86,9 +93,9 @@ __device__ __forceinline__ void finish_tile(const GemmArgs &g, int64_t cbase, in
 // The BM x BN tile at (m0, n0) by v_mfma_f32_32x32x2_f32, 2 x 2 waves; smem holds 2 * F_BK * (BM + BN + 2 F_PAD) floats.
 template <bool A_KC, bool B_KC, int BM, int BN, bool VEC>
 __device__ __forceinline__ void f32_tile(const GemmArgs &g, const float *A, const float *B, int64_t cbase, int m0, int n0, bool vec_c, int out_bf16, float *smem) {
-  constexpr int PA = BM + F_PAD, PB = BN + F_PAD, TM = BM / 64, TN = BN / 64;
+  constexpr int PA = BM + F_PAD, PB = BN + F_PAD, TM = BM / 64, TN = BN / 64, NA = BM / 64, NB = BN / 64;
   float *As = smem, *Bs = smem + 2 * F_BK * PA;
-  const int t = threadIdx.x, wave = t >> 6, lane = t & 63, lr = lane & 31, lk = lane >> 5;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 31, lk = lane >> 5;
   const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2);
   f32x16 acc[TM][TN];
 #pragma unroll
@@ -97,28 +104,28 @@ __device__ __forceinline__ void f32_tile(const GemmArgs &g, const float *A, cons
     for (int j = 0; j < TN; j++)
 #pragma unroll
       for (int e = 0; e < 16; e++) acc[i][j][e] = 0.f;
-  float4 ra[BM / 64], rb[BN / 64];
-  auto store = [&](float *s, int pitch, bool kc, const float4 &v, int i) {
-    const int r = (kc ? t >> 2 : t & 63) + 64 * i, k = kc ? (t & 3) * 4 : (t >> 6) * 4;
+  float4 ra[NA], rb[NB];
+  auto store = [&](float *s, int pitch, int r, int k4, const float4 &v) {
+    const int k = 4 * k4;
     s[(k + 0) * pitch + r] = v.x; s[(k + 1) * pitch + r] = v.y; s[(k + 2) * pitch + r] = v.z; s[(k + 3) * pitch + r] = v.w;
   };
   const int full = g.K / F_BK, nt = (g.K + F_BK - 1) / F_BK;
   auto load = [&](int kt) {
     if (kt < full) {
-      load_tile<A_KC, BM, VEC, false>(A, g.lda, m0, kt * F_BK, g.M, g.K, ra);
-      load_tile<B_KC, BN, VEC, false>(B, g.ldb, n0, kt * F_BK, g.N, g.K, rb);
+      load_tile<A_KC, NA, VEC, false>(A, g.lda, m0, kt * F_BK, g.M, g.K, ra);
+      load_tile<B_KC, NB, VEC, false>(B, g.ldb, n0, kt * F_BK, g.N, g.K, rb);
     } else if (kt < nt) {
-      load_tile<A_KC, BM, VEC, true>(A, g.lda, m0, kt * F_BK, g.M, g.K, ra);
-      load_tile<B_KC, BN, VEC, true>(B, g.ldb, n0, kt * F_BK, g.N, g.K, rb);
+      load_tile<A_KC, NA, VEC, true>(A, g.lda, m0, kt * F_BK, g.M, g.K, ra);
+      load_tile<B_KC, NB, VEC, true>(B, g.ldb, n0, kt * F_BK, g.N, g.K, rb);
     }
   };
   load(0);
   for (int kt = 0; kt < nt; kt++) {
     float *as = As + (kt & 1) * F_BK * PA, *bs = Bs + (kt & 1) * F_BK * PB;
 #pragma unroll
-    for (int i = 0; i < BM / 64; i++) store(as, PA, A_KC, ra[i], i);
+    for (int i = 0; i < NA; i++) store(as, PA, part_row<A_KC>(i), part_k4<A_KC>(), ra[i]);
 #pragma unroll
-    for (int i = 0; i < BN / 64; i++) store(bs, PB, B_KC, rb[i], i);
+    for (int i = 0; i < NB; i++) store(bs, PB, part_row<B_KC>(i), part_k4<B_KC>(), rb[i]);
     load(kt + 1);                               // on its way while this one is multiplied
     __syncthreads();                            // the other buffer was last read before the previous barrier
 #pragma unroll
@@ -142,22 +149,26 @@ __device__ __forceinline__ void f32_tile(const GemmArgs &g, const float *A, cons
 }
 
 // ================================================================ the split
-// TM x TN accumulators (C^T orientation) += the six products, the smallest first
-template <int TM, int TN>
+// TM x TN accumulators (C^T orientation) += the six products, the smallest first; FIRST: = the six products
+template <bool FIRST, int TM, int TN>
 __device__ __forceinline__ void mfma6_tiles(const bf16x8 (&a)[3][TM], const bf16x8 (&b)[3][TN], f32x16 (&acc)[TM][TN]) {
+  const f32x16 zero = {0.f};
 #pragma unroll
   for (int p = 0; p < 6; p++)
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
-      for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[SPLIT_B[p]][j], a[SPLIT_A[p]][i], acc[i][j], 0, 0, 0);
+      for (int j = 0; j < TN; j++)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[SPLIT_B[p]][j], a[SPLIT_A[p]][i], FIRST && p == 0 ? zero : acc[i][j], 0, 0, 0);
 }
 
 // ================================================================ tiles through LDS
-// 2 x 2 waves of 64 x 64 (or 32 x 32): 24 matrix instructions per step and wave, 768 cycles, against some 170 vector instructions for the
-// split, which go into the gaps between them (sched_group_barrier: 16384 x 768 x 2304 NN 547 -> 330 us with it and the loads a step
-// earlier; 4, 6, 7 or 8 vector instructions to a gap instead of 5 are the same within 3 %).  What bounds it now is what one SIMD issues:
-// at 2 waves per SIMD the matrix pipes are busy 40 to 54 % of the time and the vector units as long.
+// 2 x 2 waves of 64 x 64 (or 32 x 32): 24 matrix instructions per step and wave, 768 cycles, against 92 vector instructions for the
+// split and the long sums, which go into the gaps between them (sched_group_barrier, four to a gap: with 3 or 6 3 to 12 % slower).
+// What bounds the large tiles: on zeros, where the clock does not fall, 16384 x 3072 x 768 takes 342 us, without the split 275; on
+// standard normal operands the clock falls to 1.9 GHz and it takes 414 (matrix pipes 49 % busy).  One tile on its way instead of two cost
+// 5 % there, the 64 vector instructions more of a split by shifts and subtractions nothing in NT and NN and 5 % in TN.  Tiles of
+// 128 x 64, and 128 x 128 on eight waves, are slower at every size tried (2 to 30 %).
 // LDS: three planes of [row][16 k] bf16 per operand, 32 bytes a row, two buffers.  The 16-byte half of a row that holds k 0..7 is
 // the first one in rows whose bit 3 is clear and the second one in the others: the fragment reads and the 8-byte writes of either
 // operand order then spread over all banks.
@@ -169,21 +180,22 @@ constexpr int S_BK = 16;
 // 512, 4.2e-7.  Flushing every 16 steps is 2 % faster and left the gradients of a 6 x 256 model 1.6 times as far from 64 bits as the
 // fp32 instruction does; every 4 steps leaves them where they were.
 constexpr int S_FLUSH = 4;
+static_assert(S_FLUSH == 4, "the loop of k_gemm_f32_split is written for it");
 __device__ __forceinline__ int plane_ofs(int row, int k4) { return row * 32 + ((((k4 >> 1) ^ (row >> 3)) & 1) << 4) + (k4 & 1) * 8; }
 
 template <bool KCONTIG, int ROWS, bool TAIL>
+__device__ __forceinline__ void store_part(char *s, const float4 &v, int i) {
+  const float4 x = TAIL ? make_float4(here(v.x), here(v.y), here(v.z), here(v.w)) : v;
+  const Split2 a = split2(x.x * SPLIT_UP, x.y * SPLIT_UP), b = split2(x.z * SPLIT_UP, x.w * SPLIT_UP);
+  char *p = s + plane_ofs(part_row<KCONTIG>(i), part_k4<KCONTIG>());
+  *reinterpret_cast<uint2 *>(p) = make_uint2(a.h, b.h);
+  *reinterpret_cast<uint2 *>(p + ROWS * 32) = make_uint2(a.m, b.m);
+  *reinterpret_cast<uint2 *>(p + 2 * ROWS * 32) = make_uint2(a.l, b.l);
+}
+template <bool KCONTIG, int ROWS, bool TAIL>
 __device__ __forceinline__ void store_split(char *s, const float4 (&v)[ROWS / 64]) {
-  const int t = threadIdx.x;
 #pragma unroll
-  for (int i = 0; i < ROWS / 64; i++) {
-    const int r = (KCONTIG ? t >> 2 : t & 63) + 64 * i, k4 = KCONTIG ? t & 3 : t >> 6;
-    const float4 x = TAIL ? make_float4(here(v[i].x), here(v[i].y), here(v[i].z), here(v[i].w)) : v[i];
-    const Split2 a = split2(x.x * SPLIT_UP, x.y * SPLIT_UP), b = split2(x.z * SPLIT_UP, x.w * SPLIT_UP);
-    char *p = s + plane_ofs(r, k4);
-    *reinterpret_cast<uint2 *>(p) = make_uint2(a.h, b.h);
-    *reinterpret_cast<uint2 *>(p + ROWS * 32) = make_uint2(a.m, b.m);
-    *reinterpret_cast<uint2 *>(p + 2 * ROWS * 32) = make_uint2(a.l, b.l);
-  }
+  for (int i = 0; i < ROWS / 64; i++) store_part<KCONTIG, ROWS, TAIL>(s, v[i], i);
 }
 template <int ROWS, int T>
 __device__ __forceinline__ void read_split(const char *s, int row0, int lr, int lk, bf16x8 (&f)[3][T]) {
@@ -208,7 +220,7 @@ template <int LAYOUT, int BM, int BN, bool PLAIN, bool VEC>
 __global__ __launch_bounds__(256, 2) void k_gemm_f32_split(GemmArgs g, int vec_c, int out_bf16) {
   constexpr bool A_KC = (LAYOUT != AH_GEMM_TN);     // A is [M][K] except for TN ([K][M])
   constexpr bool B_KC = (LAYOUT == AH_GEMM_NT);     // B is [N][K] only for NT
-  constexpr int TM = BM / 64, TN = BN / 64;
+  constexpr int TM = BM / 64, TN = BN / 64, NA = BM / 64, NB = BN / 64;
   constexpr int ABYTES = 3 * BM * 32, BBYTES = 3 * BN * 32;
   constexpr int SPLIT_LDS = 2 * (ABYTES + BBYTES), F32_LDS = 2 * F_BK * (BM + BN + 2 * F_PAD) * 4;
   __shared__ __attribute__((aligned(16))) char smem[SPLIT_LDS > F32_LDS ? SPLIT_LDS : F32_LDS];
@@ -235,59 +247,93 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f32_split(GemmArgs g, int vec_c
 #pragma unroll
       for (int j = 0; j < TN; j++)
 #pragma unroll
-        for (int e = 0; e < 16; e++) { sum[i][j][e] = __builtin_fmaf(acc[i][j][e], SPLIT_DOWN, sum[i][j][e]); acc[i][j][e] = 0.f; }
+        for (int e = 0; e < 16; e++) sum[i][j][e] = __builtin_fmaf(acc[i][j][e], SPLIT_DOWN, sum[i][j][e]);
   };
 
-  float4 ra[BM / 64], rb[BN / 64];
+  float4 ra[2][NA], rb[2][NB];                      // two tiles on their way, by the parity of their number
   const int full = g.K / S_BK, rest = g.K - full * S_BK;
-  auto load = [&](int t) {
-    load_tile<A_KC, BM, VEC, false>(A, g.lda, m0, t * S_BK, g.M, g.K, ra);
-    load_tile<B_KC, BN, VEC, false>(B, g.ldb, n0, t * S_BK, g.N, g.K, rb);
-  };
-  auto put = [&](char *buf) {
-    store_split<A_KC, BM, false>(buf, ra);
-    store_split<B_KC, BN, false>(buf + ABYTES, rb);
+  auto load = [&](float4 (&va)[NA], float4 (&vb)[NB], int t) {
+    load_tile<A_KC, NA, VEC, false>(A, g.lda, m0, t * S_BK, g.M, g.K, va);
+    load_tile<B_KC, NB, VEC, false>(B, g.ldb, n0, t * S_BK, g.N, g.K, vb);
   };
   bf16x8 fa[3][TM], fb[3][TN];
   auto get = [&](const char *buf) {
     read_split<BN, TN>(buf + ABYTES, wn, lr, lk, fb);
     read_split<BM, TM>(buf, wm, lr, lk, fa);
   };
-  // Tile t is multiplied while tile t + 1 goes from registers through the split into the other buffer and tile t + 2 is requested.
-  // (Past the last whole tile the last one is loaded again and not used.)
-  if (full > 0) {
-    load(0);
-    put(smem);
-    load(min(1, full - 1));
-    __syncthreads();
-    for (int t = 0; t < full; t++) {
-      if (t > 0 && t % S_FLUSH == 0) flush();
-      get(smem + (t & 1) * (ABYTES + BBYTES));
-      mfma6_tiles<TM, TN>(fa, fb, acc);
-      put(smem + ((t & 1) ^ 1) * (ABYTES + BBYTES));
-      load(min(t + 2, full - 1));
-      // one matrix instruction (32 cycles), then the vector instructions of the split that fit beside it
-      if (TM * TN > 1) {
-        __builtin_amdgcn_sched_group_barrier(0x100, 3 * (TM + TN), 0);        // the fragments
+  // Tile t is multiplied while tile t + 1 goes from registers through the split into the other buffer; tile t + 2 is on its way and
+  // tile t + 3 is requested, each value as soon as the one before it in its registers has been cut.  (Past the last whole tile the last
+  // one is loaded again and not used.)  FIRST: the first step of S_FLUSH, which adds the short sums of the steps before it to the long
+  // ones and starts new ones.
+  auto step = [&](auto first, auto parity, int t) {
+    constexpr bool FIRST = decltype(first)::value;
+    constexpr int ODD = decltype(parity)::value ? 1 : 0;
+    get(smem + ODD * (ABYTES + BBYTES));
+    if (FIRST) flush();
+    mfma6_tiles<FIRST>(fa, fb, acc);
+    char *next = smem + (ODD ^ 1) * (ABYTES + BBYTES);
+    const int k0 = min(t + 3, full - 1) * S_BK;
 #pragma unroll
-        for (int i = 0; i < 6 * TM * TN; i++) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
-          if (i & 1) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
-        }
+    for (int i = 0; i < NA; i++) {
+      store_part<A_KC, BM, false>(next, ra[ODD ^ 1][i], i);
+      ra[ODD ^ 1][i] = load_part<A_KC, VEC, false>(A, g.lda, m0, k0, g.M, g.K, i);
+    }
+#pragma unroll
+    for (int i = 0; i < NB; i++) {
+      store_part<B_KC, BN, false>(next + ABYTES, rb[ODD ^ 1][i], i);
+      rb[ODD ^ 1][i] = load_part<B_KC, VEC, false>(B, g.ldb, n0, k0, g.N, g.K, i);
+    }
+    // The fragments of the first two products, then one matrix instruction (32 cycles) and the vector instructions of the split that fit
+    // beside it, in turn; the middle parts are read once the lowest ones, whose registers they take, have been multiplied.
+    if (TM * TN > 1) {
+      __builtin_amdgcn_sched_group_barrier(0x100, 2 * (TM + TN), 0);
+#pragma unroll
+      for (int i = 0; i < 6 * TM * TN; i++) {
+        if (FIRST && i < TM * TN) __builtin_amdgcn_sched_group_barrier(0x002, 16, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+        if (i == TM * TN - 1) __builtin_amdgcn_sched_group_barrier(0x100, TM + TN, 0);
+        if (i & 1) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+        if (i % 6 == 5) __builtin_amdgcn_sched_group_barrier(0x020, 4, 0);
       }
-      __syncthreads();
+    }
+    __syncthreads();
+  };
+  using yes = std::integral_constant<bool, true>;
+  using no = std::integral_constant<bool, false>;
+  int t = 0;
+  if (full > 0) {
+    load(ra[0], rb[0], 0);
+    load(ra[1], rb[1], min(1, full - 1));
+    store_split<A_KC, BM, false>(smem, ra[0]);
+    store_split<B_KC, BN, false>(smem + ABYTES, rb[0]);
+    load(ra[0], rb[0], min(2, full - 1));
+    __syncthreads();
+    for (; t + S_FLUSH <= full; t += S_FLUSH) {
+      step(yes(), no(), t);
+      step(no(), yes(), t + 1);
+      step(no(), no(), t + 2);
+      step(no(), yes(), t + 3);
+    }
+    if (t < full) {
+      step(yes(), no(), t);
+      if (t + 1 < full) step(no(), yes(), t + 1);
+      if (t + 2 < full) step(no(), no(), t + 2);
     }
   }
   if (rest > 0) {
-    if (full % S_FLUSH == 0) flush();
-    load_tile<A_KC, BM, VEC, true>(A, g.lda, m0, full * S_BK, g.M, g.K, ra);
-    load_tile<B_KC, BN, VEC, true>(B, g.ldb, n0, full * S_BK, g.N, g.K, rb);
-    store_split<A_KC, BM, true>(smem, ra);
-    store_split<B_KC, BN, true>(smem + ABYTES, rb);
+    load_tile<A_KC, NA, VEC, true>(A, g.lda, m0, full * S_BK, g.M, g.K, ra[0]);
+    load_tile<B_KC, NB, VEC, true>(B, g.ldb, n0, full * S_BK, g.N, g.K, rb[0]);
+    store_split<A_KC, BM, true>(smem, ra[0]);
+    store_split<B_KC, BN, true>(smem + ABYTES, rb[0]);
     __syncthreads();
     get(smem);
-    mfma6_tiles<TM, TN>(fa, fb, acc);
+    if (full % S_FLUSH == 0) {
+      flush();
+      mfma6_tiles<true>(fa, fb, acc);
+    } else {
+      mfma6_tiles<false>(fa, fb, acc);
+    }
     __syncthreads();
   }
   flush();
@@ -427,11 +473,9 @@ struct F32Choice { int bm, waves, splits; };
 //   LDS tiles   a tile takes `step` per 16 of the contraction alone on its CU, and `full` of the CU's time where others fill its gaps
 //   slices      another launch, and the workspace written and read
 // Against 128 x 128 tiles of v_mfma_f32_32x32x2_f32 (in slices where there were fewer than 256 tiles and K >= 2048), in us:
-//   16384 x 3072 x 768 NT 720 -> 430 (128 x 128), 768 x 768 x 16384 TN 329 -> 157 (128 x 128 in 32 slices), 490 x 768 x 768 NT 77 -> 16
-//   (64 x 64 in 4 slices), 48 x 768 x 256 NT 26 -> 7 and 512 x 128 x 1024 TN 97 -> 9 (32 x 32); with the operands scaled 1 % more over
-//   132 random shapes (15 % at worst), 16384 x 3072 x 768 NT 549 -> 557 and 490 x 768 x 768 16.7 -> 17.5 back to back on standard
-//   normal operands.  Operands that are not finite take the fp32 instruction as well: 16384 x 3072 x 768 of NaNs 1070 (720 by that
-//   instruction's own kernel).
+//   16384 x 3072 x 768 NT 720 -> 414 (128 x 128), 768 x 768 x 16384 TN 329 -> 137 (128 x 128 in 32 slices), 490 x 768 x 768 NT 77 -> 14
+//   (64 x 64 in 2 slices), 48 x 768 x 256 NT 26 -> 7 and 512 x 128 x 1024 TN 97 -> 9 (32 x 32).  Operands that are not finite take the
+//   fp32 instruction as well: 16384 x 3072 x 768 of NaNs 1070 (720 by that instruction's own kernel).
 F32Choice choose(const GemmArgs &ga, int layout, int batch, bool may_split, bool long_rows) {
   struct Tile { int bm; double step, full; };
   static constexpr Tile TILES[2] = {{64, 0.26, 0.24}, {128, 1.2, 0.65}};

@@ -26,15 +26,30 @@ __device__ __forceinline__ float here(float x) {
   return x;
 }
 struct Split2 { uint32_t h, m, l; };       // the parts of two values side by side
+// x less the low (high) half of h: v_dot2_f32_bf16 with (-1, 0) or (0, -1), in place of an instruction that makes an fp32 number of the
+// half and one that subtracts it: nine instructions for a pair of values in place of 13 (2.0 ns of a SIMD each where a shift takes 1.9 and
+// a subtraction 1.2).  The result is exact for every significand (both ways compared over all of them at eight exponents),
+// and the other half, unless it is infinite or NaN, adds nothing.  The constants are hidden from the compiler, which takes 0xbf80 in the
+// low half alone for the one in both.
+__device__ __forceinline__ uint32_t hidden(uint32_t c) {
+  asm("" : "+s"(c));
+  return c;
+}
+__device__ __forceinline__ float less_low(float x, uint32_t h) {
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, h), __builtin_bit_cast(bf16x2_t, hidden(0x0000bf80u)), x, false);
+}
+__device__ __forceinline__ float less_high(float x, uint32_t h) {
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, h), __builtin_bit_cast(bf16x2_t, hidden(0xbf800000u)), x, false);
+}
 // x0, x1: values that are already multiplied by SPLIT_UP
 __device__ __forceinline__ Split2 split2(float x0, float x1) {
   Split2 s;
   s.h = pack_bf16x2(x0, x1);
-  x0 -= __uint_as_float(s.h << 16);
-  x1 -= __uint_as_float(s.h & 0xffff0000u);
+  x0 = less_low(x0, s.h);
+  x1 = less_high(x1, s.h);
   s.m = pack_bf16x2(x0, x1);
-  x0 -= __uint_as_float(s.m << 16);
-  x1 -= __uint_as_float(s.m & 0xffff0000u);
+  x0 = less_low(x0, s.m);
+  x1 = less_high(x1, s.m);
   s.l = pack_bf16x2(x0, x1);
   return s;
 }
