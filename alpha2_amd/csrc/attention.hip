@@ -15,6 +15,7 @@
 // row 8j + 4h + r in the accumulator and must supply exactly that row as operand -> no data movement.
 #include "attention_common.h"
 #include "split_bf16.h"
+#include <type_traits>
 
 using namespace ah;
 
@@ -48,7 +49,8 @@ __device__ __forceinline__ void load_tile_f32(float *s, const float *__restrict_
 // 16-byte pieces are permuted within a row so that 16 lanes that read the same piece of 16 rows meet 64 different banks.
 // A result that is not finite has the block computed again with the fp32 instruction, whose result stands; so does a score.
 // 192 heads x 1024 x 64: dK and dV 945 -> 486 us, dQ 520 -> 316; 512 x 256 x 32: 112 -> 84 and 81 -> 60; 4 x 70 x 64: 29 -> 24 and
-// 26 -> 20 (before both operands were scaled, which costs 1 % of the backward pass at 192 x 1024 x 64 and 3 to 6 % of smaller ones).
+// 26 -> 20 (before both operands were scaled, which costs 1 % of the backward pass at 192 x 1024 x 64 and 3 to 6 % of smaller ones, and
+// before the scores' functions ran side by side, below).
 // Relative error against 64 bits at 4 x 512 x 64: dQ 4.6e-7 -> 3.7e-7, dK 6.4e-7 -> 3.8e-7, dV 6.0e-7 -> 3.3e-7.  What bounds it now is
 // vector issue: tanh, exp and the cut of scores, K and V for every 32 x 32 tile beside 3072 cycles of matrix instructions.
 template <int D>
@@ -171,8 +173,51 @@ struct SplitTile {                          // D = 32 or 64
     }
   }
 };
-// A raw score (times 2^48) scaled back and capped; factor: what split_cap_factor gives
-__device__ __forceinline__ float split_cap(float s, float cap, float factor) { return softcap_fwd(s * factor, cap, 1.0f); }
+// The functions of a tile's 16 scores in straight-line code, all 16 at once: the library's tanh branches for every score, and so did the cap
+// and the masks, so that the 16 ran one after the other.  Forward / backward (delta, dQ, dK and dV), us, before -> now: 512 heads x 256 x
+// 32 50 / 172 -> 42 / 130, 192 x 1024 x 64 265 / 810 -> 234 / 685 (without a cap 220 / 755 -> 197 / 650), 32 x 128 x 32 8.5 / 42 ->
+// 7.3 / 34, 12 x 500 x 64 22 / 184 -> 20 / 140; errors against 64 bits the same without a cap and up to 20 % less with one.
+// tanh x for |x| < TANH_SMALL as x + x^3 P(x^2), P the fifth-order polynomial of least relative error there (fitted by reweighted least
+// squares): 0.7 last places off at most, 0.3 on average.  Beyond, 1 - 2 / (exp(2 |x|) + 1), which is 1.5 off at most there.
+constexpr float TANH_SMALL = 0.625f, LOG2E = 1.44269502162933349609375f, LOG2E_REST = 1.925963033e-8f;
+__device__ __forceinline__ float tanh_small(float x) {
+  const float z = x * x;
+  float p = -0.005704985465854406f;
+  p = __builtin_fmaf(p, z, 0.02063908614218235f);
+  p = __builtin_fmaf(p, z, -0.05373971536755562f);
+  p = __builtin_fmaf(p, z, 0.13331441581249237f);
+  p = __builtin_fmaf(p, z, -0.3333328068256378f);
+  return __builtin_fmaf(x * z, p, x);
+}
+// 2^UP exp x, x not much above 0 and not below -1e9 (there, as for infinite x, NaN or infinity may come of it): the integer part of
+// x log2 e goes into the exponent, 2 to the rest is the instruction's.  0.96 last places off at most, 0.306 on average (expf: 0.84, 0.300;
+// a single exponential of x log2 e times what that rounds off: 1.25, 0.41).
+template <int UP>
+__device__ __forceinline__ float exp_of(float x) {
+  const float n = __builtin_rintf(x * LOG2E), rest = __builtin_fmaf(x, LOG2E_REST, __builtin_fmaf(x, LOG2E, -n));
+  return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(rest), (int)n + UP);
+}
+__device__ __forceinline__ float tanh_large(float x) {
+  const float e = __builtin_amdgcn_exp2f(fabsf(x) * (2.0f * LOG2E));
+  return copysignf(__builtin_fmaf(-2.0f, __builtin_amdgcn_rcpf(e + 1.0f), 1.0f), x);
+}
+// Raw scores (times 2^48) scaled back by `factor` (split_cap_factor) and, with a cap, put through tanh: a score is cap times that
+__device__ __forceinline__ void scores_tanh(f32x16 &s, float cap, float factor) {
+#pragma clang fp contract(off)
+#pragma unroll
+  for (int e = 0; e < 16; e++) s[e] *= factor;
+  if (!(cap > 0.f)) return;
+  float top = 0.f;
+#pragma unroll
+  for (int e = 0; e < 16; e += 2) top = fmaxf(fmaxf(top, fabsf(s[e])), fabsf(s[e + 1]));
+  if (__all(top < TANH_SMALL)) {                                   // (NaN: either way gives NaN)
+#pragma unroll
+    for (int e = 0; e < 16; e++) s[e] = tanh_small(s[e]);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 16; e++) { const float small = tanh_small(s[e]), large = tanh_large(s[e]); s[e] = fabsf(s[e]) < TANH_SMALL ? small : large; }
+  }
+}
 __device__ __forceinline__ float split_cap_factor(float cap) { return (cap > 0.f ? 1.0f / cap : 1.0f) * SPLIT_DOWN; }
 // (a cap whose factor is no normal number is left to the fp32 instruction)
 __device__ __forceinline__ bool split_cap_ok(float cap) { return !(cap > 0x1p70f); }
@@ -273,34 +318,41 @@ __device__ void flash_fwd_exact(const FlashArgs &a, int bh, int q0, int end, boo
 
 // Two kernels compute the forward pass of head sizes up to 64, and a row's result does not depend on which: both do the operations
 // below on the tiles of 32 keys in ascending order, each with the same operands and roundings.
-// Raw scores of the tile at key kv0 (times 2^48, row = key, column = this lane's query qi) -> capped and masked; the column's largest
+// Raw scores of the tile at key kv0 (times 2^48, row = key, column = this lane's query qi) -> what scores_tanh makes of them, -infinity
+// where masked; the column's largest score, which is cap_mul times that
+__device__ __forceinline__ float cap_mul(const FlashArgs &a) { return a.cap > 0.f ? a.cap : 1.0f; }
 __device__ __forceinline__ float tile_scores(f32x16 &s, const FlashArgs &a, float factor, int kv0, int qi, int lk) {
 #pragma clang fp contract(off)
+  scores_tanh(s, a.cap, factor);
   float top = -INFINITY;
+  if (__all(kv0 + 31 <= qi && kv0 + 32 <= a.T)) {                  // nothing to mask
 #pragma unroll
-  for (int e = 0; e < 16; e++) {
-    const int kv = kv0 + 8 * (e >> 2) + 4 * lk + (e & 3);
-    float x = split_cap(s[e], a.cap, factor);
-    x = (kv > qi || kv >= a.T) ? -INFINITY : x;
-    s[e] = x;
-    top = fmaxf(top, x);
+    for (int e = 0; e < 16; e++) top = fmaxf(top, s[e]);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+      const int kv = kv0 + 8 * (e >> 2) + 4 * lk + (e & 3);
+      s[e] = kv > qi || kv >= a.T ? -INFINITY : s[e];
+      top = fmaxf(top, s[e]);
+    }
   }
-  return fmaxf(top, __shfl_xor(top, 32, 64));
+  return fmaxf(top, __shfl_xor(top, 32, 64)) * cap_mul(a);
 }
 // Scores -> weights against the largest score so far, times 2^24; the column's sum of them, and what sums so far are multiplied by
-__device__ __forceinline__ float tile_weights(f32x16 &s, float before, float top, float &alpha) {
+// (-infinity, a masked score or no score so far, weighs what -200 does: nothing)
+__device__ __forceinline__ float tile_weights(f32x16 &s, float mul, float before, float top, float &alpha) {
 #pragma clang fp contract(off)
   const float m = fmaxf(before, top), use = m == -INFINITY ? 0.f : m;
-  alpha = expf(before - use);
+  alpha = exp_of<0>(fmaxf(before - use, -200.f));
   float sum = 0.f;
 #pragma unroll
-  for (int e = 0; e < 16; e++) { const float p = expf(s[e] - use); s[e] = p * SPLIT_UP; sum += p; }
-  return sum + __shfl_xor(sum, 32, 64);
+  for (int e = 0; e < 16; e++) { s[e] = exp_of<24>(fmaxf(__builtin_fmaf(s[e], mul, -use), -200.f)); sum += s[e]; }
+  return (sum + __shfl_xor(sum, 32, 64)) * 0x1p-24f;
 }
 __device__ __forceinline__ float output_factor(float l) { return (l > 0.f ? 1.0f / l : 0.f) * SPLIT_DOWN; }
 
-// Four waves of 32 queries.  192 heads x 1024 x 64: 383 us with the fp32 instruction, now 308; 512 x 256 x 32 61 -> 52; relative error
-// against 64 bits at 4 x 512 x 64 2.0e-7 (fp32 instruction: 2.4e-7).  Vector issue bounds it, as in backward.
+// Four waves of 32 queries.  192 heads x 1024 x 64: 383 us with the fp32 instruction, now 240; 512 x 256 x 32 61 -> 42; relative error
+// against 64 bits at 4 x 512 x 64 1.9e-7 (fp32 instruction: 2.4e-7).  Vector issue bounds it, as in backward.
 // Head sizes over 64 keep the fp32 instruction: their operands do not fit the registers in three parts.
 template <int D>
 __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_fwd_f32(FlashArgs a) {
@@ -320,7 +372,7 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_fwd_f32(FlashArgs
     const int b = bh / a.H, h = bh % a.H;
     const float *K = (const float *)a.k + b * a.k_sb + h * a.k_sh;
     const float *V = (const float *)a.v + b * a.v_sb + h * a.v_sh;
-    const float factor = split_cap_factor(a.cap);
+    const float factor = split_cap_factor(a.cap), mul = cap_mul(a);
     float qx[D / 16][8];
     S::row((const float *)a.q + b * a.q_sb + h * a.q_sh + (int64_t)qi * a.q_st, qi < a.T, a.hd, lk, qx);
     f32x16 o[S::F];
@@ -357,7 +409,7 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_fwd_f32(FlashArgs
       fine = fine && all_finite(s);
       const float top = tile_scores(s, a, factor, kv0, qi, lk);
       float alpha;
-      const float sum = tile_weights(s, m, top, alpha);
+      const float sum = tile_weights(s, mul, m, top, alpha);
       l = __builtin_fmaf(l, alpha, sum);
       m = fmaxf(m, top);
       S::contract_rows(Vc, s, lr, lk, alpha, o);
@@ -399,7 +451,7 @@ __global__ __launch_bounds__(512, 2) void k_flash_fwd_f32_keys(FlashArgs a) {
   const int r = threadIdx.x >> 4, c = threadIdx.x & 15;            // the sums: query q0 + r, features 2 c and 2 c + 1 of each 32
   const float *K = (const float *)a.k + b * a.k_sb + h * a.k_sh;
   const float *V = (const float *)a.v + b * a.v_sb + h * a.v_sh;
-  const float factor = split_cap_factor(a.cap);
+  const float factor = split_cap_factor(a.cap), mul = cap_mul(a);
   float qx[D / 16][8], k[D / 16][8], v[S::F][16];
   S::row((const float *)a.q + b * a.q_sb + h * a.q_sh + (int64_t)qi * a.q_st, qi < a.T, a.hd, lk, qx);
   auto load = [&](int i) {                                         // rows past the end read as zero
@@ -449,7 +501,7 @@ __global__ __launch_bounds__(512, 2) void k_flash_fwd_f32_keys(FlashArgs a) {
     }
     if (i < tiles) {
       float alpha;
-      const float sum = tile_weights(s, before, top, alpha);
+      const float sum = tile_weights(s, mul, before, top, alpha);
       if (lk == 0) { Alpha[wave * 32 + lr] = alpha; Sum[wave * 32 + lr] = sum; }
       bf16x8 p[2][3];
 #pragma unroll
@@ -514,20 +566,23 @@ __global__ __launch_bounds__(512, 2) void k_flash_fwd_f32_keys(FlashArgs a) {
   if (threadIdx.x < 32 && qi < a.T) a.lse[((int64_t)b * a.H + h) * a.T + qi] = m + logf(Sum[lr]);
 }
 
-// delta[b,h,t] = sum_d dO[t,d] * O[t,d]
+// delta[b,h,t] = sum_d dO[t,d] * O[t,d]: D / 4 lanes to a row of D features, 16 bytes each (a wave to a row, 4 bytes each, half of its
+// lanes without any at head size 32, took 31 us for 512 heads x 256 x 32 and 44 us for 192 x 1024 x 64)
 template <int D>
-__global__ void k_flash_delta_f32(FlashArgs a) {
-  int64_t row = blockIdx.x * (int64_t)(blockDim.x >> 6) + (threadIdx.x >> 6);
-  int64_t total = (int64_t)a.B * a.H * a.T;
-  if (row >= total) return;
-  int lane = threadIdx.x & 63;
-  int t = (int)(row % a.T), h = (int)((row / a.T) % a.H), b = (int)(row / ((int64_t)a.T * a.H));
-  const float *O = (const float *)a.o + b * a.o_sb + h * a.o_sh + (int64_t)t * a.o_st;
-  const float *dO = (const float *)a.d_o + b * a.o_sb + h * a.o_sh + (int64_t)t * a.o_st;
+__global__ __launch_bounds__(256) void k_flash_delta_f32(FlashArgs a) {
+  constexpr int L = D / 4;
+  const int64_t row = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) / L, total = (int64_t)a.B * a.H * a.T;
+  const int d = 4 * (threadIdx.x % L);
   float s = 0.f;
-  for (int d = lane; d < a.hd; d += 64) s += O[d] * dO[d];
-  s = wave_sum(s);
-  if (lane == 0) a.delta[row] = s;
+  if (row < total && d < a.hd) {
+    const int t = (int)(row % a.T), h = (int)((row / a.T) % a.H), b = (int)(row / ((int64_t)a.T * a.H));
+    const int64_t at = b * a.o_sb + h * a.o_sh + (int64_t)t * a.o_st + d;
+    const float4 o = *reinterpret_cast<const float4 *>((const float *)a.o + at), g = *reinterpret_cast<const float4 *>((const float *)a.d_o + at);
+    s = __builtin_fmaf(o.x, g.x, o.y * g.y) + __builtin_fmaf(o.z, g.z, o.w * g.w);
+  }
+#pragma unroll
+  for (int i = 1; i < L; i <<= 1) s += __shfl_xor(s, i, 64);
+  if (row < total && d == 0) a.delta[row] = s;
 }
 
 // ------------------------------------------------------------------------------------------ dQ
@@ -620,7 +675,8 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_dq_f32(FlashArgs 
     const int q0 = xblk * (WAVES * 32) + wave * 32, qi = q0 + lr;
     const float *K = (const float *)a.k + b * a.k_sb + h * a.k_sh;
     const float *V = (const float *)a.v + b * a.v_sb + h * a.v_sh;
-    const float inv_cap = a.cap > 0.f ? 1.0f / a.cap : 0.f, factor = split_cap_factor(a.cap);
+    // a score is mul times what scores_tanh leaves, t, and its derivative 1 - slope t^2
+    const float factor = split_cap_factor(a.cap), mul = cap_mul(a), slope = a.cap > 0.f ? 1.0f : 0.f;
     const bool live = qi < a.T;
     float qx[D / 16][8], gx[D / 16][8];
     S::row((const float *)a.q + b * a.q_sb + h * a.q_sh + (int64_t)qi * a.q_st, live, a.hd, lk, qx);
@@ -662,15 +718,20 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_dq_f32(FlashArgs 
         mfma6(f, go[i], dp);
       }
       fine = fine && scores_finite(s);
+      scores_tanh(s, a.cap, factor);
+      auto weigh = [&](auto masks) {
 #pragma unroll
-      for (int e = 0; e < 16; e++) {
-        const int kv = kv0 + 8 * (e >> 2) + 4 * lk + (e & 3);
-        const float sc = split_cap(s[e], a.cap, factor);
-        const float p = (kv > qi || kv >= a.T || !live) ? 0.f : expf(sc - lse);
-        float ds = p * __builtin_fmaf(dp[e], SPLIT_DOWN, -delta);
-        if (a.cap > 0.f) { const float t = sc * inv_cap; ds *= (1.0f - t * t); }
-        s[e] = ds * (a.scale * SPLIT_UP);
-      }
+        for (int e = 0; e < 16; e++) {
+          const int kv = kv0 + 8 * (e >> 2) + 4 * lk + (e & 3);
+          const float t = s[e];
+          float p = exp_of<0>(__builtin_fmaf(t, mul, -lse));
+          if (decltype(masks)::value) p = kv > qi || kv >= a.T || !live ? 0.f : p;
+          const float ds = p * __builtin_fmaf(dp[e], SPLIT_DOWN, -delta) * __builtin_fmaf(-(t * slope), t, 1.0f);
+          s[e] = ds * (a.scale * SPLIT_UP);
+        }
+      };
+      if (__all(live && kv0 + 31 <= qi && kv0 + 32 <= a.T)) weigh(std::false_type());
+      else weigh(std::true_type());
       S::contract_rows(Kc, s, lr, lk, 1.0f, dq);
     }
     if (__syncthreads_or(!fine || !all_finite<S::F>(dq))) {
@@ -788,7 +849,7 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_dkv_f32(FlashArgs
     const int kv_blk0 = xblk * (WAVES * 32), kv0 = kv_blk0 + wave * 32, kvi = kv0 + lr;
     const float *Q = (const float *)a.q + b * a.q_sb + h * a.q_sh;
     const float *dO = (const float *)a.d_o + b * a.o_sb + h * a.o_sh;
-    const float inv_cap = a.cap > 0.f ? 1.0f / a.cap : 0.f, factor = split_cap_factor(a.cap);
+    const float factor = split_cap_factor(a.cap), mul = cap_mul(a), slope = a.cap > 0.f ? 1.0f : 0.f;      // as in dQ
     const bool live = kvi < a.T;
     // K's and V's rows stay whole and are cut where they are used: in three parts, they, the accumulators and the next tile are more
     // registers than a wave of two per SIMD has (the empty assembler statements keep the cuts from being moved out of the loop).
@@ -845,16 +906,21 @@ __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_dkv_f32(FlashArgs
         mfma6(f, w, dp);
       }
       f32x16 pm;
+      scores_tanh(s, a.cap, factor);
+      auto weigh = [&](auto masks) {
 #pragma unroll
-      for (int e = 0; e < 16; e++) {
-        const int qr = 8 * (e >> 2) + 4 * lk + (e & 3), qi = q0 + qr;
-        const float sc = split_cap(s[e], a.cap, factor);
-        const float p = (kvi > qi || qi >= a.T || !live) ? 0.f : expf(sc - Ls[qr]) * SPLIT_UP;
-        float ds = p * __builtin_fmaf(dp[e], SPLIT_DOWN, -Ds[qr]);
-        if (a.cap > 0.f) { const float t = sc * inv_cap; ds *= (1.0f - t * t); }
-        pm[e] = p;
-        s[e] = ds;                                      // Qc already carries `scale`, so dK = dS^T (scale*Q)
-      }
+        for (int e = 0; e < 16; e++) {
+          const int qr = 8 * (e >> 2) + 4 * lk + (e & 3), qi = q0 + qr;
+          const float t = s[e];
+          float p = exp_of<24>(__builtin_fmaf(t, mul, -Ls[qr]));
+          if (decltype(masks)::value) p = kvi > qi || qi >= a.T || !live ? 0.f : p;
+          pm[e] = p;
+          // Qc already carries `scale`, so dK = dS^T (scale*Q)
+          s[e] = p * __builtin_fmaf(dp[e], SPLIT_DOWN, -Ds[qr]) * __builtin_fmaf(-(t * slope), t, 1.0f);
+        }
+      };
+      if (__all(live && kvi <= q0 && q0 + 32 <= a.T)) weigh(std::false_type());
+      else weigh(std::true_type());
       S::contract_rows(Gc, pm, lr, lk, 1.0f, dv);
       S::contract_rows(Qc, s, lr, lk, 1.0f, dk);
     }
@@ -937,7 +1003,7 @@ int32_t run_bwd(FlashArgs &a) {
   int32_t rc = ah_alloc((uint64_t)rows * 4, &delta);
   if (rc) return rc;
   a.delta = dp<float>(delta);
-  ah::launch_kernel(k_flash_delta_f32<D>, dim3((unsigned)cdiv(rows, 4)), dim3(256), 0, a);
+  ah::launch_kernel(k_flash_delta_f32<D>, dim3((unsigned)cdiv(rows * (D / 4), 256)), dim3(256), 0, a);
   AH_LAUNCH_CHECK();
   dim3 grid((unsigned)cdiv(a.T, WAVES * 32), (unsigned)(a.B * a.H));
   ah::launch_kernel(k_flash_dq_f32<D>, grid, dim3(256), 0, a);
