@@ -938,6 +938,40 @@ class HipBackend:
         for t in (params, m, v):
             self._dirty(t)
 
+    def adamwSteps(self, items, lr, beta1, beta2, eps, bc1, bc2, gradScale=1.0):
+        """adamwStep for every (params, grads, m, v, weightDecay) of an optimizer pass, in as few launches as their table takes: the
+        first eight at once, since the device idles here (the norm was just read back), then 48 at a time."""
+        if type(self).adamwStep is not HipBackend.adamwStep or "adamwStep" in self.__dict__:      # somebody's own update of one tensor
+            for p, g, m, v, wd in items:
+                self.adamwStep(p, g, m, v, lr, beta1, beta2, eps, wd, bc1, bc2, gradScale)
+            return
+        h, dev = self._adam_hyper(lr, beta1, beta2, eps, 0.0, bc1, bc2, gradScale)
+        queue, written, most = [], set(), 8
+
+        def launch():
+            if queue:
+                check(self.lib.ah_adamw_list((ffi.AhAdamWItem * len(queue))(*queue), len(queue), C.byref(h), dev, 0))
+            queue.clear()
+            written.clear()
+        try:
+            for p, g, m, v, wd in items:
+                self._f32(p, g, m, v)
+                n = p.size
+                if not (n == g.size == m.size == v.size):
+                    raise ValueError("adamwStep: params, grads, m, v must have the same size")
+                for t in (p, m, v):
+                    self._own(t)
+                ptrs = self._ptr(p), self._ptr(g), self._ptr(m), self._ptr(v)
+                if len(queue) >= most or not written.isdisjoint(ptrs):      # (a tensor listed twice is updated twice, in order)
+                    most = 48 if len(queue) >= most else most
+                    launch()
+                written.update((ptrs[0], ptrs[2], ptrs[3]))
+                queue.append(ffi.AhAdamWItem(*ptrs, 0, n, wd, 0))
+                for t in (p, m, v):
+                    self._dirty(t)
+        finally:
+            launch()
+
     def _adam_hyper(self, lr, beta1, beta2, eps, weightDecay, bc1, bc2, gradScale):
         """The optimizer's scalars are the same for every tensor of a step except the weight decay (optimizers.ts:54-94): they
         are written to a small device struct once per step, which the kernel reads, and the by-value argument carries only

@@ -508,14 +508,11 @@ class FusedTrainer:
         self._norm_done = False
         # clip coefficient, non-finite guard and the bias corrections, all on the device (trainer.ts:1248-1262,1495-1522,1650-1656)
         check(lib.ah_step_guard(self.sumsq, self.loss, 1.0 / self.accum, tc.gradClip, tc.beta1, tc.beta2, self.guard, self.hyper, self.clip))
-        h = ffi.AhAdamW(tc.lr, tc.beta1, tc.beta2, tc.eps, tc.weightDecay, 1.0, 1.0, 1.0 / self.accum)
-        if split > 0:
-            check(lib.ah_adamw(self.P, self.G, self.M, self.Vm, split, C.byref(h), self.hyper, self.clip, self.Pb))
-        h.weight_decay = 0.0
-        n2 = self.nparam - split
-        if n2 > 0:
-            check(lib.ah_adamw(self.P + split * 4, self.G + split * 4, self.M + split * 4, self.Vm + split * 4, n2, C.byref(h), self.hyper,
-                               self.clip, self.Pb + split * 2))
+        h = ffi.AhAdamW(tc.lr, tc.beta1, tc.beta2, tc.eps, 0.0, 1.0, 1.0, 1.0 / self.accum)
+        parts = [(at, n, wd) for at, n, wd in ((0, split, tc.weightDecay), (split, self.nparam - split, 0.0)) if n > 0]
+        items = (ffi.AhAdamWItem * len(parts))(*[ffi.AhAdamWItem(self.P + at * 4, self.G + at * 4, self.M + at * 4, self.Vm + at * 4, self.Pb + at * 2, n, wd, 0)
+                                                for at, n, wd in parts])
+        check(lib.ah_adamw_list(items, len(parts), C.byref(h), self.hyper, self.clip))
 
     def _whole_step(self):
         for m in range(self.accum):               # gradients of the micro-steps are summed in place; scaled once in the optimizer

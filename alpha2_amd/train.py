@@ -74,24 +74,20 @@ class AdamW:
         self._beta2Pow *= self.beta2
         return 1 - self._beta1Pow, 1 - self._beta2Pow
 
-    def stepParamEntries(self, entries, gradScale: float = 1.0):
+    def _update(self, tensors, gradScale: float):
         bc1, bc2 = self._next_bias_corrections()
-        for name, var in entries:
-            if var.grad is None:
-                continue
-            m, v = self._moments(name, var.data)
-            wd = 0.0 if name in self.noDecayNames else self.weightDecay
-            self.backend.adamwStep(var.data, var.grad, m, v, self.lr, self.beta1, self.beta2, self.eps, wd, bc1, bc2, gradScale)
+        items = ((p, g, *self._moments(name, p), 0.0 if name in self.noDecayNames else self.weightDecay) for name, p, g in tensors)
+        if hasattr(self.backend, "adamwSteps"):             # a backend that takes a whole pass
+            self.backend.adamwSteps(items, self.lr, self.beta1, self.beta2, self.eps, bc1, bc2, gradScale)
+            return
+        for p, g, m, v, wd in items:
+            self.backend.adamwStep(p, g, m, v, self.lr, self.beta1, self.beta2, self.eps, wd, bc1, bc2, gradScale)
+
+    def stepParamEntries(self, entries, gradScale: float = 1.0):
+        self._update([(name, var.data, var.grad) for name, var in entries if var.grad is not None], gradScale)
 
     def step(self, params: Dict[str, TensorData], grads: Dict[str, TensorData], gradScale: float = 1.0):
-        bc1, bc2 = self._next_bias_corrections()
-        for name, p in params.items():
-            g = grads.get(name)
-            if g is None:
-                continue
-            m, v = self._moments(name, p)
-            wd = 0.0 if name in self.noDecayNames else self.weightDecay
-            self.backend.adamwStep(p, g, m, v, self.lr, self.beta1, self.beta2, self.eps, wd, bc1, bc2, gradScale)
+        self._update([(name, p, grads[name]) for name, p in params.items() if grads.get(name) is not None], gradScale)
 
     def stateDict(self) -> dict:
         """Reads the moments back from the device (the reference copies stale host arrays after any GPU adamwStep,

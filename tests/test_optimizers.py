@@ -212,3 +212,34 @@ def test_optimizer_registry_and_state_round_trip(B):
         a.stepParamEntries(ent, 0.45)
         b.step({"w": ent_b[0][1].data}, {"w": ent_b[0][1].grad}, 0.45)
         assert np.array_equal(ent[0][1].data.data, ent_b[0][1].data.data)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("count", [1, 8, 9, 56, 57])
+def test_a_pass_of_adamw_in_tables_is_the_tensors_one_by_one(count):
+    """Table ends (8, then 48 tensors), sizes that are no multiple of a vector or a chunk, a tensor listed twice, an error on the way:
+    bit for bit what adamwStep does in the same order."""
+    from alpha2_amd import HipBackend
+    from alpha2_amd.backend import TensorData
+    B = HipBackend(0)
+    rs = np.random.RandomState(count)
+    sizes = [int(n) for n in rs.choice([1, 3, 4, 257, 1024, 1025, 5000], size=count)]
+    host = [[rs.standard_normal(n).astype(np.float32) for _ in range(3)] + [rs.rand(n).astype(np.float32)] for n in sizes]
+    hyper = (1e-2, 0.9, 0.95, 1e-8)
+
+    def tensors():
+        t = [tuple(TensorData((x.size,), "f32", x.copy()) for x in row) + (0.1 * (i % 3),) for i, row in enumerate(host)]
+        return t + t[:1] + t[-1:]
+    one, many = tensors(), tensors()
+    for p, g, m, v, wd in one:
+        B.adamwStep(p, g, m, v, *hyper, wd, 0.1, 0.05, 0.5)
+    B.adamwSteps(many, *hyper, 0.1, 0.05, 0.5)
+    for a, b in zip(one, many):
+        assert all(np.array_equal(x.data, y.data) for x, y in zip(a[:4], b[:4]))
+    bad = tensors()
+    bad.insert(1, (bad[0][0], TensorData((sizes[0] + 1,), "f32", np.zeros(sizes[0] + 1, np.float32)), bad[0][2], bad[0][3], 0.0))
+    with pytest.raises(ValueError):
+        B.adamwSteps(bad, *hyper, 0.1, 0.05, 0.5)
+    p, g, m, v, wd = tensors()[0]
+    B.adamwStep(p, g, m, v, *hyper, wd, 0.1, 0.05, 0.5)
+    assert np.array_equal(bad[0][0].data, p.data)                       # the tensors before the bad one were updated
