@@ -51,6 +51,10 @@ class AhFlash(C.Structure):
                 ("d_o", u64), ("dq", u64), ("dk", u64), ("dv", u64), ("bwd_variant", i32), ("reserved", i32)]
 
 
+class AhCopy(C.Structure):
+    _fields_ = [("dst", u64), ("src", u64), ("bytes", u64), ("value", u64)]
+
+
 class AhDecodeLayer(C.Structure):
     _fields_ = [(n, u64) for n in ("ln1_w", "ln1_b", "wqkv", "wo", "ln2_w", "ln2_b", "fc1", "up", "fc2")] + [("coef", u64 * 5)]
 
@@ -93,7 +97,7 @@ SIGNATURES = {
     "ah_init": [i32], "ah_shutdown": [], "ah_device_info": [C.POINTER(AhDeviceInfo)], "ah_sync": [],
     "ah_alloc": [u64, C.POINTER(u64)], "ah_free": [u64], "ah_upload": [u64, C.c_void_p, u64],
     "ah_download": [C.c_void_p, u64, u64], "ah_download_begin": [u64, u64, C.POINTER(u64)], "ah_download_end": [u64, C.c_void_p, u64],
-    "ah_copy": [u64, u64, u64], "ah_fill_f32": [u64, f32, u64],
+    "ah_copy": [u64, u64, u64], "ah_copy_list": [C.POINTER(AhCopy), i32], "ah_fill_f32": [u64, f32, u64],
     "ah_fill_i32": [u64, i32, u64], "ah_stats": [C.POINTER(AhStats)], "ah_reset_op_count": [], "ah_trim_pool": [],
     "ah_graph_begin": [], "ah_graph_end": [C.POINTER(u64)], "ah_graph_launch": [u64], "ah_graph_destroy": [u64],
     "ah_event_create": [C.POINTER(u64)], "ah_event_record": [u64], "ah_event_elapsed_ms": [u64, u64, C.POINTER(f32)],

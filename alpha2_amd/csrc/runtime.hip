@@ -167,6 +167,24 @@ __global__ void k_step_copy(char *__restrict__ dst, const char *__restrict__ src
     for (uint64_t i = tid; i < bytes; i += stride) dst[i] = src[i];
   }
 }
+// blockIdx.y: which of the copies
+constexpr int COPY_LIST = 24;
+struct CopyList { AhCopy item[COPY_LIST]; };
+__global__ __launch_bounds__(256) void k_copy_list(CopyList l) {
+  const AhCopy &c = l.item[blockIdx.y];
+  char *dst = reinterpret_cast<char *>(c.dst);
+  const char *src = reinterpret_cast<const char *>(c.src);
+  const uint64_t tid = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x, stride = (uint64_t)gridDim.x * blockDim.x;
+  if (c.src == 0) {
+    if (tid < c.bytes) dst[tid] = (char)(c.value >> (8 * tid));
+  } else if (((c.dst | c.src | c.bytes) & 15u) == 0) {
+    for (uint64_t i = tid; i < c.bytes >> 4; i += stride) reinterpret_cast<uint4 *>(dst)[i] = reinterpret_cast<const uint4 *>(src)[i];
+  } else if (((c.dst | c.src | c.bytes) & 3u) == 0) {
+    for (uint64_t i = tid; i < c.bytes >> 2; i += stride) reinterpret_cast<uint32_t *>(dst)[i] = reinterpret_cast<const uint32_t *>(src)[i];
+  } else {
+    for (uint64_t i = tid; i < c.bytes; i += stride) dst[i] = src[i];
+  }
+}
 void step_copy(void *dst, const void *src, uint64_t bytes) {
   uint64_t blocks = (bytes / 16 + 255) / 256;
   if (blocks < 1) blocks = 1;
@@ -636,6 +654,31 @@ int32_t ah_copy(ah_ptr dst, ah_ptr src, uint64_t bytes) {
   }
   AH_HIP(hipMemcpyAsync(dp<void>(dst), dp<void>(src), bytes, hipMemcpyDeviceToDevice, g.stream));
   g.ops++;
+  return AH_OK;
+}
+
+int32_t ah_copy_list(const AhCopy *items, int32_t count) {
+  AH_REQUIRE_READY();
+  AH_ARG(count >= 0 && (count == 0 || items != nullptr), "ah_copy_list: bad list");
+  for (int i = 0; i < count; i++) {
+    const AhCopy &c = items[i];
+    AH_ARG(c.bytes == 0 || (c.dst != 0 && (c.src != 0 || c.bytes <= sizeof(c.value))), "ah_copy_list: item %d: null pointer", i);
+  }
+  for (int i = 0; i < count;) {
+    CopyList l;
+    memset(&l, 0, sizeof(l));                      // (a step plan compares the whole argument)
+    int n = 0;
+    uint64_t most = 0;
+    for (; i < count && n < COPY_LIST; i++) {
+      if (items[i].bytes == 0) continue;
+      l.item[n++] = items[i];
+      if (items[i].bytes > most) most = items[i].bytes;
+    }
+    if (n == 0) break;
+    const uint64_t blocks = (most / 16 + 255) / 256;
+    ah::launch_kernel(k_copy_list, dim3((unsigned)(blocks < 1 ? 1 : blocks > 1024 ? 1024 : blocks), (unsigned)n), dim3(256), 0, l);
+    AH_LAUNCH_CHECK();
+  }
   return AH_OK;
 }
 

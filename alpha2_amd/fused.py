@@ -24,6 +24,7 @@ from __future__ import annotations
 
 import ctypes as C
 import math
+import struct
 from dataclasses import dataclass
 from typing import Dict, List, Optional, Tuple
 
@@ -40,11 +41,6 @@ F32, BF16 = ffi.F32, ffi.BF16
 
 def _align(n: int, a: int = 64) -> int:
     return (n + a - 1) // a * a
-
-
-def _i32(x: int) -> int:
-    x &= 0xFFFFFFFF
-    return x - (1 << 32) if x >> 31 else x
 
 
 @dataclass
@@ -556,21 +552,20 @@ class FusedTrainer:
                     self._bufs.remove(b)
         self._batches = []
 
-    def _use_batch(self, i, micro: int = 0):
-        """Copy stored batch i into the resident slot of micro-step `micro` (a sequence fills slots 0, 1, ...)."""
-        if isinstance(i, (list, tuple)):
-            if len(i) != self.micro_steps:
-                raise ValueError(f"need {self.micro_steps} batch indices, one per micro-step")
-            for m, bi in enumerate(i):
-                self._use_batch(bi, m)
-            return
-        ti, tt, ix = self._batches[i]
-        at = (micro % self.per_pass) * self.BTm * 4
-        check(self.lib.ah_copy(self.toks[micro // self.per_pass] + at, ti, self.BTm * 4))
-        check(self.lib.ah_copy(self.tgts[micro // self.per_pass] + at, tt, self.BTm * 4))
-        if ix:
-            check(self.lib.ah_copy(self.tok_index[micro], ix, self._index_bytes))
+    def _use_batch(self, i) -> list:
+        """Copies of stored batch i into the resident slot (a sequence: of each micro-step's into slots 0, 1, ...)."""
+        indices = i if isinstance(i, (list, tuple)) else (i,)
+        if len(indices) != self.micro_steps and isinstance(i, (list, tuple)):
+            raise ValueError(f"need {self.micro_steps} batch indices, one per micro-step")
+        copies, n = [], self.BTm * 4
+        for micro, bi in enumerate(indices):
+            ti, tt, ix = self._batches[bi]
+            at = (micro % self.per_pass) * n
+            copies += [ffi.AhCopy(self.toks[micro // self.per_pass] + at, ti, n, 0), ffi.AhCopy(self.tgts[micro // self.per_pass] + at, tt, n, 0)]
+            if ix:
+                copies.append(ffi.AhCopy(self.tok_index[micro], ix, self._index_bytes, 0))
         self._have_batch = True
+        return copies
 
     def _write_guard_state(self, b1p: float = 1.0, b2p: float = 1.0, skipped: float = 0.0):
         st = (C.c_double * 3)(b1p, b2p, skipped)
@@ -579,26 +574,27 @@ class FusedTrainer:
         h = ffi.AhAdamW(tc.lr, tc.beta1, tc.beta2, tc.eps, tc.weightDecay, 1 - b1p, 1 - b2p, 1.0 / self.accum)
         check(self.lib.ah_upload(self.hyper, C.byref(h), C.sizeof(h)))
 
-    def _write_hyper(self) -> float:
+    def _hyper_items(self) -> list:
         """The learning rate of this step: the first field of the device AhAdamW.  Its bias corrections are kept by
         ah_step_guard on the device, which advances them on applied steps only."""
-        lr = lrAt(self.tc, self.stepIdx)
-        v = C.c_float(lr)
-        check(self.lib.ah_upload(self.hyper, C.byref(v), 4))
+        items = [ffi.AhCopy(self.hyper, 0, 4, struct.unpack("<I", struct.pack("<f", lrAt(self.tc, self.stepIdx)))[0])]
         if self.drop > 0:                          # the masks of this step's micro-steps (trainer.ts:1169,1202), as int32 like `seed | 0`
-            seeds = (C.c_int32 * self.micro_steps)(*[_i32(self.tc.seed + self.stepIdx * 1000 + m) for m in range(self.micro_steps)])
-            check(self.lib.ah_upload(self.seed_dev, seeds, 4 * self.micro_steps))
-        return lr
+            items += [ffi.AhCopy(self.seed_dev + 4 * m, 0, 4, (self.tc.seed + self.stepIdx * 1000 + m) & 0xFFFFFFFF) for m in range(self.micro_steps)]
+        return items
+
+    def _write_hyper(self):
+        self._copy(self._hyper_items())
+
+    def _copy(self, items: list):
+        check(self.lib.ah_copy_list((ffi.AhCopy * len(items))(*items), len(items)))
 
     def step(self, batch_index=None) -> int:
         """Enqueue one optimizer step (no host synchronisation); returns the step index whose loss / grad-norm can be
         read later with history().  `batch_index`: a stored batch, or with gradient accumulation a sequence of `accum`
         stored batches (micro-steps run in that order); None keeps the resident ones."""
-        if batch_index is not None:
-            self._use_batch(batch_index)
-        elif not self._have_batch:
+        if batch_index is None and not self._have_batch:
             raise RuntimeError("no batch set")
-        self._write_hyper()
+        self._copy((self._use_batch(batch_index) if batch_index is not None else []) + self._hyper_items())
         if self.use_graph:
             if self._graph is None:
                 self.prepare()
@@ -616,8 +612,7 @@ class FusedTrainer:
         else:
             self._whole_step()
         i = self.stepIdx % self.loss_hist_cap
-        check(self.lib.ah_copy(self.loss_hist + i * 4, self.loss, 4))
-        check(self.lib.ah_copy(self.norm_hist + i * 16, self.clip, 16))
+        self._copy([ffi.AhCopy(self.loss_hist + i * 4, self.loss, 4, 0), ffi.AhCopy(self.norm_hist + i * 16, self.clip, 16, 0)])
         self.stepIdx += 1
         return self.stepIdx - 1
 

@@ -74,6 +74,10 @@ int32_t ah_download(void *host, ah_ptr src, uint64_t bytes);          /* blocks 
 int32_t ah_download_begin(ah_ptr src, uint64_t bytes, uint64_t *out_ticket);
 int32_t ah_download_end(uint64_t ticket, void *host, uint64_t bytes);
 int32_t ah_copy(ah_ptr dst, ah_ptr src, uint64_t bytes);              /* device to device */
+/* Several of them in one launch, for the few small copies around a step (a launch costs some 3 us, a copy of 512 bytes by itself 6):
+ * src == 0: the first `bytes` (at most 8) of `value` are written.  No destination may overlap another item's source or destination. */
+typedef struct { ah_ptr dst, src; uint64_t bytes, value; } AhCopy;
+int32_t ah_copy_list(const AhCopy *items, int32_t count);
 int32_t ah_fill_f32(ah_ptr dst, float value, uint64_t n);
 int32_t ah_fill_i32(ah_ptr dst, int32_t value, uint64_t n);
 

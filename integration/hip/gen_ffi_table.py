@@ -14,7 +14,7 @@ from alpha2_amd import _ffi as ffi  # noqa: E402
 
 SCALARS = {C.c_int32: "i32", C.c_uint64: "u64", C.c_int64: "i64", C.c_float: "f32", C.c_double: "f64"}
 RETURNS = {"ah_last_error": "cstring", "ah_step_note": "cstring", "ah_layernorm_bwd_partials_bytes": "i64", "ah_embedding_index_bytes": "i64"}
-STRUCTS = ("AhGemm", "AhFlash", "AhAdamW", "AhAdamWItem", "AhStats", "AhDeviceInfo", "AhColsumJob", "AhLion", "AhAdafactor", "AhRng", "AhDecode", "AhDecodeLayer")
+STRUCTS = ("AhGemm", "AhFlash", "AhAdamW", "AhAdamWItem", "AhStats", "AhDeviceInfo", "AhColsumJob", "AhLion", "AhAdafactor", "AhRng", "AhCopy", "AhDecode", "AhDecodeLayer")
 
 
 def ts_type(t) -> str:

@@ -34,6 +34,7 @@ export const lib = dlopen(process.env.ALPHA_HIP_LIB ?? "libalpha_hip.so", {
   ah_check_finite:                 { args: [u64, u64, u64], returns: i32 },
   ah_clip_coef:                    { args: [u64, f32, f32, u64], returns: i32 },
   ah_copy:                         { args: [u64, u64, u64], returns: i32 },
+  ah_copy_list:                    { args: [ptr, i32], returns: i32 },
   ah_cross_entropy:                { args: [u64, i32, u64, u64, u64, i64, i64], returns: i32 },
   ah_cross_entropy_bwd:            { args: [u64, i32, u64, u64, u64, f32, u64, i64, i64], returns: i32 },
   ah_cross_entropy_fwd_bwd:        { args: [u64, i32, u64, u64, u64, u64, f32, u64, i64, i64], returns: i32 },
@@ -141,6 +142,7 @@ export const LAYOUT = {
   AhLion: { size: 40, lr: 0, beta1: 8, beta2: 16, weight_decay: 24, grad_scale: 32 },
   AhAdafactor: { size: 48, lr: 0, beta2: 8, eps: 16, clip_threshold: 24, weight_decay: 32, grad_scale: 40 },
   AhRng: { size: 24, s0: 0, s1: 4, has_spare: 8, _pad: 12, spare: 16 },
+  AhCopy: { size: 32, dst: 0, src: 8, bytes: 16, value: 24 },
   AhDecode: { size: 96, vocab: 0, width: 4, heads: 8, ffn: 12, layers: 16, act: 20, rows: 24, scale: 28, cap: 32, eps: 36, wte: 40, wpe: 48, lnf_w: 56, lnf_b: 64, head: 72, kv: 80, logits: 88 },
   AhDecodeLayer: { size: 112, ln1_w: 0, ln1_b: 8, wqkv: 16, wo: 24, ln2_w: 32, ln2_b: 40, fc1: 48, up: 56, fc2: 64, coef: 72 },
   // GENERATED LAYOUTS END
