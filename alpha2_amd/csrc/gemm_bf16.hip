@@ -273,10 +273,14 @@ int32_t run(const GemmArgs &ga, int batch, int out_dtype) {
   // (us, 128 x 128 / 64 x 128 / 64 x 64): 128 x 384 x 128 5.6 / 4.1 / 3.4, 777 x 768 x 768 11.5 / 7.7 / 6.0, 777 x 768 x 3072 31.3 / 20.7 /
   // 19.8, 2048 x 1024 x 4096 (256 tiles of 64 x 128, 512 of 64 x 64) 44.2 / 32.6 / 35.0; beyond one tile to a CU: 777 x 3072 x 768
   // 13.5 / 14.2 / 13.3, 10240 x 384 x 1536 21.9 / 22.5 / 26.3.  The sums are the same, bit for bit.
+  // The 128 x 128 tile has eight waves of 64 x 32, two to a SIMD, one of which multiplies while the other waits at the barrier or for LDS: on
+  // four of 64 x 64 (the figures above) 10240 x 384 x 1536 takes 22.3 us, now 19.3, 10240 x 384 x 384 10.1 -> 9.1, 4096 x 640 x 2560
+  // 27.6 -> 22.4, 777 x 3072 x 768 13.1 -> 12.0, 10240 x 384 x 4096 46.4 -> 40.0.  (Two or four k-tiles on their way in registers
+  // instead of one change nothing but for few tiles of K >= 3072; eight waves on the 64 x 128 tile: 3 % faster to 1 % slower.)
   const int64_t per = (int64_t)batch * ga.nsplit * cdiv(ga.M, 64);
   if (per * cdiv(ga.N, 64) <= num_cus()) return launch<64, 64, 2, 2, AKM, BKM>(ga, batch, out_dtype);
   if (per * cdiv(ga.N, 128) <= num_cus()) return launch<64, 128, 2, 2, AKM, BKM>(ga, batch, out_dtype);
-  return launch<128, 128, 2, 2, AKM, BKM>(ga, batch, out_dtype);
+  return launch<128, 128, 2, 4, AKM, BKM>(ga, batch, out_dtype);
 }
 
 }  // namespace
