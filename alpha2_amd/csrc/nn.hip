@@ -917,8 +917,12 @@ int32_t ah_layernorm(ah_ptr x, ah_ptr w, ah_ptr b, ah_ptr out, int64_t rows, int
 // more: a block beyond that runs alone in a second round.  Resident blocks per CU by registers, the least over the stream and
 // gradient types of a row length: 4 up to 512 elements, 3 up to 768, 2 beyond (16384 x 768: 21.3 us with two blocks per CU of
 // eight rows a wave, 19.5 with three of five or six, 24.4 with four; 8192 x 1024: 22.0 -> 16.1 us).
+// Fewer rows than that leave the choice of how many a wave walks.  Up to 2048 it is one: a row after another is its latency again
+// (bf16, us with four rows a wave / one: 128 x 128 6.3 / 3.9, 1024 x 384 8.9 / 4.8, 2048 x 512 9.2 / 5.6; fp32 with its column sums
+// 8.7 / 6.3, 10.8 / 7.5, 11.2 / 9.9).  Beyond, four: with two, 10240 x 384 in bf16 takes 10.2 instead of 11.5, but the column sums of twice
+// the partials cost as much where they follow at once (fp32 16.7 / 16.3, 4096 x 1024 16.4 / 15.7).
 static int ln_bwd_blocks(int64_t rows, int64_t dim) {
-  int64_t nblk = cdiv(rows, WPB * 4);             // >= 4 rows per wave amortise the partial write
+  int64_t nblk = cdiv(rows, WPB * (rows <= 2048 ? 1 : 4));
   int64_t cap = (int64_t)num_cus() * (dim <= 512 ? 4 : dim <= 768 ? 3 : 2);
   if (nblk > cap) nblk = cap;
   return nblk < 1 ? 1 : (int)nblk;
