@@ -18,6 +18,7 @@ Release = Optional[Callable[[TensorData], None]]
 
 
 class Variable:
+    __slots__ = ("id", "data", "grad", "requiresGrad", "__dict__", "__weakref__")
     _next_id = 0
 
     def __init__(self, data: TensorData, requiresGrad: bool = False):
@@ -64,9 +65,9 @@ class Tape:
                 if entry.cleanup:
                     entry.cleanup(releaseTensor)
                 continue
-            needs = None
-            if any(not v.requiresGrad for v in entry.inputs):
-                needs = [v.requiresGrad for v in entry.inputs]
+            needs = [v.requiresGrad for v in entry.inputs]
+            if all(needs):
+                needs = None
             grads = entry.backward(out_grad, backend, releaseTensor, needs)
             uses = {}
             for inp, g in zip(entry.inputs, grads):

@@ -25,10 +25,7 @@ _NP = {"f32": np.float32, "i32": np.int32, "f16": np.uint16, "bf16": np.uint16, 
 
 
 def shapeSize(shape) -> int:
-    s = 1
-    for d in shape:
-        s *= int(d)
-    return s
+    return int(math.prod(shape))
 
 
 def shapeStrides(shape) -> List[int]:
@@ -54,8 +51,10 @@ class _Buf:
 
     @staticmethod
     def _block(lib, nbytes: int) -> int:
-        out = C.c_uint64(0)
-        check(lib.ah_alloc(max(1, nbytes), C.byref(out)))
+        out = C.c_uint64()
+        rc = lib.ah_alloc(nbytes or 1, C.byref(out))
+        if rc:
+            check(rc)
         return out.value
 
     def _drop(self):
@@ -99,20 +98,27 @@ class TensorData:
     """shape + dtype + data (packages/core/src/interfaces.ts:31-35).  `data` is a flat numpy array; for a
     device-resident tensor it is fetched on demand."""
 
+    # slots, and a dictionary only for the few that are given more: a step makes hundreds, and what the collector counts of them decides
+    # how often it looks at everything
+    __slots__ = ("shape", "dtype", "store", "_host", "_buf", "_off", "_host_valid", "_dev_valid", "_backend", "__dict__", "__weakref__")
+
     def __init__(self, shape, dtype: str = "f32", data: Optional[np.ndarray] = None):
-        self.shape: Tuple[int, ...] = tuple(int(s) for s in shape)
-        self.dtype = dtype
-        self._host: Optional[np.ndarray] = None if data is None else np.ascontiguousarray(data, dtype=_NP[dtype]).reshape(-1)
+        self.shape: Tuple[int, ...] = tuple(map(int, shape))
+        self.dtype = self.store = dtype         # store: device storage type ("bf16" for fast-mode activations)
         self._buf: Optional[_Buf] = None
-        self._off = 0               # byte offset into _buf
-        self._host_valid = data is not None
+        self._off = 0                           # byte offset into _buf
         self._dev_valid = False
         self._backend: Optional["HipBackend"] = None
-        self.store = dtype          # device storage type ("bf16" for fast-mode activations)
+        if data is None:
+            self._host: Optional[np.ndarray] = None
+            self._host_valid = False
+        else:
+            self._host = np.ascontiguousarray(data, dtype=_NP[dtype]).reshape(-1)
+            self._host_valid = True
 
     @property
     def size(self) -> int:
-        return shapeSize(self.shape)
+        return math.prod(self.shape)
 
     @property
     def data(self) -> np.ndarray:
@@ -131,6 +137,7 @@ class TensorData:
 
 class HipBackend:
     name = "hip"
+    _timed: Optional[list] = None              # startTiming(): a record per product
 
     def __init__(self, device: int = 0):
         self.lib = ffi.load()
@@ -146,13 +153,17 @@ class HipBackend:
     # ------------------------------------------------------------------ residency helpers
     def _new(self, shape, dtype="f32", store: Optional[str] = None) -> TensorData:
         t = TensorData(shape, dtype)
-        t.store = store or dtype
-        t._buf = _Buf(self.lib, shapeSize(shape) * ffi.DTYPE_BYTES[t.store])
+        if store:
+            t.store = store
+        t._buf = _Buf(self.lib, math.prod(t.shape) * ffi.DTYPE_BYTES[t.store])
         t._dev_valid, t._backend = True, self
         return t
 
     def _ptr(self, t: TensorData) -> int:
         """Device address of `t`, uploading a host-created tensor on first use."""
+        b = t._buf
+        if b is not None and t._dev_valid:
+            return b.ptr + t._off
         if t._buf is None or not t._dev_valid:
             if not t._host_valid:
                 raise RuntimeError("use of a released tensor")
@@ -200,10 +211,12 @@ class HipBackend:
 
     def releaseGpuTensor(self, t: TensorData):
         """packages/train/src/trainer.ts:1003-1006.  Stream-ordered: safe to call right after enqueueing uses."""
-        if t is None or t._buf is None:
+        if t is None:
             return
-        t._buf.release()
-        t._buf, t._dev_valid = None, False
+        b = t._buf
+        if b is not None:
+            b.release()
+            t._buf, t._dev_valid = None, False
 
     def flush(self):
         """The trainer's end-of-step call (trainer.ts:1776-1784).  Work is already on the stream in call order, so there
@@ -362,9 +375,12 @@ class HipBackend:
               out_dtype=ffi.F32, epilogue=ffi.EPI_NONE, aux=0, planes=None):
         """planes = (c_plane_cols, c_plane_stride, a_plane_k, a_plane_stride): the product goes through ah_gemm_planes."""
         g = ffi.AhGemm(layout, in_dtype, out_dtype, epilogue, m, n, k, lda, ldb, ldc, batch, sa, sb, sc, a_ptr, b_ptr, c_ptr, aux)
+        if planes is None and self._timed is None:
+            check(self.lib.ah_gemm(C.byref(g)))
+            return
         run = (lambda: check(self.lib.ah_gemm(C.byref(g)))) if planes is None else (lambda: check(self.lib.ah_gemm_planes(C.byref(g), *planes, 0)))
         self.planeProducts += planes is not None
-        timed = getattr(self, "_timed", None)
+        timed = self._timed
         if timed is None:
             run()
             return
@@ -405,6 +421,8 @@ class HipBackend:
     def _batched(self, a: TensorData, b: TensorData, a_mat, b_mat):
         """Resolve broadcast batch dims (cpu_ref.ts:184-243).  Returns (batch_shape, batch, stride_a, stride_b)
         when the batch collapses to one uniform stride per operand, else None."""
+        if len(a.shape) == 2 and len(b.shape) == 2:
+            return [], 1, 0, 0
         aB, bB = list(a.shape[:-2]), list(b.shape[:-2])
         nb = max(len(aB), len(bB))
         pa, pb = [1] * (nb - len(aB)) + aB, [1] * (nb - len(bB)) + bB
@@ -804,7 +822,8 @@ class HipBackend:
         """The tape clones every first gradient and most are never written again (tape.ts:116-127): a clone of a whole buffer shares
         its block until one side is written in place.  The copies were 10.9 ms of the 118 ms fp32 step of the 12 x 768 model."""
         self._ptr(a)
-        if a.size and a._off == 0 and a.size * ffi.DTYPE_BYTES[a.store] == a._buf.nbytes:
+        n = a.size * ffi.DTYPE_BYTES[a.store]
+        if n and a._off == 0 and n == a._buf.nbytes:
             out = TensorData(a.shape, a.dtype)
             out.store, out._buf = a.store, _Buf(self.lib, a._buf.nbytes, like=a._buf)
             out._dev_valid, out._backend = True, self
