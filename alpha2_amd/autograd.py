@@ -314,7 +314,13 @@ def matmulTransposed(ctx, a, b):
 def matmulTransposedGelu(ctx, a, b):
     ad, bd = a.data, b.data
     B0 = ctx.backend
-    mm, tB = _mt_forward(B0, ad, bd)
+    both = B0.matmulTransposedGeluSaved(ad, bd) if _has(B0, "matmulTransposedGeluSaved") else None
+    if both is not None:
+        out, mm = both
+        tB = None
+    else:
+        mm, tB = _mt_forward(B0, ad, bd)
+        out = B0.gelu(mm)
     live = [mm, tB]
 
     def cleanup(rel):
@@ -327,7 +333,7 @@ def matmulTransposedGelu(ctx, a, b):
         grads = _mt_backward(B, dmm, ad, bd, rel, needs)
         _rel(rel, dmm)
         return grads
-    return _record(ctx, B0.gelu(mm), [a, b], bw, cleanup)
+    return _record(ctx, out, [a, b], bw, cleanup)
 
 
 # ---- reductions (ops.ts:238-255) ----------------------------------------------------------------------------
