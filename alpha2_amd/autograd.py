@@ -469,6 +469,22 @@ def residualDropoutAdd(ctx, residual, projected, p, training):
                    lambda g, B, rel, n: [_reduce_broadcast(B, g, rs, rel), B.mul(g, mask)], cleanup)
 
 
+def residualProduct(ctx, residual, a, b, p, training):
+    """residual + dropout(A B^T), the end of either half of a block (gpt.ts:281,332)."""
+    B0 = ctx.backend
+    if (not training or p == 0) and _has(B0, "matmulTransposedAdd"):
+        ad, bd = a.data, b.data
+        out = B0.matmulTransposedAdd(ad, bd, residual.data)
+        if out is not None:
+            def bw(g, B, rel, needs):
+                flat = B.reshape(g, [ad.shape[0], bd.shape[0]])
+                ga, gb = _mt_backward(B, flat, ad, bd, rel, None if needs is None else needs[1:])
+                _rel(rel, flat)
+                return [g, ga, gb]
+            return _record(ctx, out, [residual, a, b], bw)
+    return residualDropoutAdd(ctx, residual, reshape(ctx, matmulTransposed(ctx, a, b), list(residual.data.shape)), p, training)
+
+
 def softmax(ctx, a, axis=None):
     out = ctx.backend.softmax(a.data, axis)
     last = axis is None or axis == -1 or axis == len(a.data.shape) - 1

@@ -483,6 +483,19 @@ class HipBackend:
         self._gemm(ffi.GEMM_NT, self._ptr(a), self._ptr(b), out._buf.ptr, M, N, K, K, K, N, epilogue=ffi.EPI_GELU, aux=pre._buf.ptr)
         return out, pre
 
+    def matmulTransposedAdd(self, a: TensorData, b: TensorData, residual: TensorData) -> Optional[TensorData]:
+        """residual + A B^T for two matrices, shaped as the residual, from the product's kernel (or from the one that joins its slices);
+        None where the shapes are no such case."""
+        if len(a.shape) != 2 or len(b.shape) != 2 or not 0 < a.shape[1] == b.shape[1] or residual.shape[-1:] != b.shape[:1]:
+            return None
+        (M, K), N = a.shape, b.shape[0]
+        if M == 0 or N == 0 or residual.size != M * N:
+            return None
+        self._f32(a, b, residual)
+        out = self._new(residual.shape)
+        self._gemm(ffi.GEMM_NT, self._ptr(a), self._ptr(b), out._buf.ptr, M, N, K, K, K, N, epilogue=ffi.EPI_RESIDUAL, aux=self._ptr(residual))
+        return out
+
     def matmulTransposedA(self, a: TensorData, b: TensorData) -> TensorData:
         """A[..,M,K]^T @ B[..,M,N] -> [..,K,N] (interfaces.ts:112; packages/tests/src/gpu-perf.test.ts:211-233)."""
         self._f32(a, b)

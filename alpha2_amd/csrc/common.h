@@ -13,6 +13,7 @@ namespace ah {
 // ---- host-side context (defined in runtime.hip) -------------------------------------------------
 hipStream_t stream();
 bool        ready();
+bool        on_side();              // between ah_side_begin and ah_side_end, where nothing may be allocated
 int32_t     fail(int32_t code, const char *fmt, ...);
 int32_t     hip_fail(hipError_t e, const char *what);
 void        count_op();

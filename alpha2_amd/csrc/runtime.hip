@@ -119,6 +119,7 @@ size_t round_size(size_t b) {
 
 namespace ah {
 hipStream_t stream() { return g.cur; }
+bool on_side() { return g.cur != g.stream; }
 bool ready() { return g.inited; }
 int num_cus() { return g.prop.multiProcessorCount; }
 int current_device() { return g.device; }

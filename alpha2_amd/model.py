@@ -173,8 +173,7 @@ def transformerBlock(ctx: Ctx, x: Variable, layer: dict, cfg: ModelConfig, Bt: i
             ctx.tape.record(masked, [scores], lambda g, B, rel, n: [B.maskedFill(g, mask, 0)])
             att = ag.dropout(ctx, ag.softmax(ctx, masked, -1), cfg.dropout, training)
             concat = ag.reshape(ctx, ag.transpose(ctx, ag.matmul(ctx, att, vH), 1, 2), [Bt * T, Cc])
-    proj = ag.reshape(ctx, ag.matmulTransposed(ctx, concat, layer["attn"]["wo"]), [Bt, T, Cc])
-    x = ag.residualDropoutAdd(ctx, x, proj, cfg.dropout, training)
+    x = ag.residualProduct(ctx, x, concat, layer["attn"]["wo"], cfg.dropout, training)
 
     ln2 = ag.layerNorm(ctx, x, layer["ln2"]["weight"], layer["ln2"]["bias"], 1e-5)
     flat = ag.reshape(ctx, ln2, [Bt * T, Cc])
@@ -183,32 +182,32 @@ def transformerBlock(ctx: Ctx, x: Variable, layer: dict, cfg: ModelConfig, Bt: i
     mt = ag.matmulTransposed
     if act == "composed" and cfg.activationGraph:
         h = mt(ctx, flat, m["fc1"])
-        mlpH = mt(ctx, _eval_activation_graph(ctx, h, cfg.activationGraph), m["fc2"])
+        hidden = _eval_activation_graph(ctx, h, cfg.activationGraph)
     elif act == "swiglu":
-        mlpH = mt(ctx, ag.siluMul(ctx, mt(ctx, flat, m["fc_gate"]), mt(ctx, flat, m["fc_up"])), m["fc_proj"])
+        hidden = ag.siluMul(ctx, mt(ctx, flat, m["fc_gate"]), mt(ctx, flat, m["fc_up"]))
     elif act == "universal" and ag._has(Bk, "channelAct"):
         h = mt(ctx, flat, m["fc1"])
-        mlpH = mt(ctx, ag.channelAct(ctx, h, {"silu": m["act_gate"], "identity": m["act_skip"]}), m["fc2"])
+        hidden = ag.channelAct(ctx, h, {"silu": m["act_gate"], "identity": m["act_skip"]})
     elif act == "kan_spline" and ag._has(Bk, "channelAct"):
         h = mt(ctx, flat, m["fc1"])
         coefs = {"silu": m["kan_c0"], "relu": m["kan_c1"], "gelu": m["kan_c2"], "identity": m["kan_c3"], "square": m["kan_c4"]}
-        mlpH = mt(ctx, ag.channelAct(ctx, h, coefs), m["fc2"])
+        hidden = ag.channelAct(ctx, h, coefs)
     elif act == "universal":
         h = mt(ctx, flat, m["fc1"])
-        mlpH = mt(ctx, ag.add(ctx, ag.mul(ctx, ag.silu(ctx, h), m["act_gate"]), ag.mul(ctx, h, m["act_skip"])), m["fc2"])
+        hidden = ag.add(ctx, ag.mul(ctx, ag.silu(ctx, h), m["act_gate"]), ag.mul(ctx, h, m["act_skip"]))
     elif act == "kan_spline":
         h = mt(ctx, flat, m["fc1"])
         hs, hr = ag.mul(ctx, ag.silu(ctx, h), m["kan_c0"]), ag.mul(ctx, ag.relu(ctx, h), m["kan_c1"])
         hg, hi = ag.mul(ctx, ag.gelu(ctx, h), m["kan_c2"]), ag.mul(ctx, h, m["kan_c3"])
         hq = ag.mul(ctx, ag.mul(ctx, h, h), m["kan_c4"])
-        mlpH = mt(ctx, ag.add(ctx, ag.add(ctx, ag.add(ctx, ag.add(ctx, hs, hr), hg), hi), hq), m["fc2"])
+        hidden = ag.add(ctx, ag.add(ctx, ag.add(ctx, ag.add(ctx, hs, hr), hg), hi), hq)
     elif act == "silu":
-        mlpH = mt(ctx, ag.silu(ctx, mt(ctx, flat, m["fc1"])), m["fc2"])
+        hidden = ag.silu(ctx, mt(ctx, flat, m["fc1"]))
     elif act == "relu":
-        mlpH = mt(ctx, ag.relu(ctx, mt(ctx, flat, m["fc1"])), m["fc2"])
+        hidden = ag.relu(ctx, mt(ctx, flat, m["fc1"]))
     else:
-        mlpH = mt(ctx, ag.matmulTransposedGelu(ctx, flat, m["fc1"]), m["fc2"])
-    return ag.residualDropoutAdd(ctx, x, ag.reshape(ctx, mlpH, [Bt, T, Cc]), cfg.dropout, training)
+        hidden = ag.matmulTransposedGelu(ctx, flat, m["fc1"])
+    return ag.residualProduct(ctx, x, hidden, m["fc_proj" if act == "swiglu" else "fc2"], cfg.dropout, training)
 
 
 def gptBlocks(ctx: Ctx, cfg: ModelConfig, params: dict, tokens: TensorData, training: bool = False, activationCheckpointing: bool = False,
