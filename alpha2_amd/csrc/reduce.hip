@@ -55,6 +55,25 @@ __global__ void k_sum_strided(const float *__restrict__ a, float *__restrict__ o
   out[line] = mean ? (float)((double)sf / (double)dim) : sf;
 }
 
+// The sums of a strided walk, AHEAD loads in flight and added in the order of the walk: one load waited for after the other was what bound
+// short lists (16 trips of a block through memory for a chunk of 2^14).  24 tensors of 65536 to 262144 7.5 -> 6.4 us, 7.1 M elements of one
+// 7.6 -> 6.4, 56.6 M in 24 tensors 38.5 -> 37.7 (memory); the same bits.
+constexpr int AHEAD = 8;
+template <class V, class F>
+__device__ __forceinline__ double walk_sum(const V *__restrict__ a, uint64_t i, uint64_t end, uint64_t step, F term) {
+  double s = 0;
+  for (; i < end && (AHEAD - 1) * step < end - i; i += AHEAD * step) {
+    V v[AHEAD];
+#pragma unroll
+    for (int k = 0; k < AHEAD; k++) v[k] = a[i + k * step];
+#pragma unroll
+    for (int k = 0; k < AHEAD; k++) s += term(v[k]);
+  }
+  for (; i < end; i += step) s += term(a[i]);
+  return s;
+}
+__device__ __forceinline__ double squares(const float4 &v) { return (double)v.x * v.x + (double)v.y * v.y + (double)v.z * v.z + (double)v.w * v.w; }
+
 // stage 1 of a full reduction: partial[b] = sum over a grid-stride slice; SQ squares first
 template <int SQ>
 __global__ void k_partial_sum(const float *__restrict__ a, uint64_t n, double *__restrict__ partial) {
@@ -63,11 +82,8 @@ __global__ void k_partial_sum(const float *__restrict__ a, uint64_t n, double *_
   double s = 0;
   if ((((uintptr_t)a) & 15u) == 0) {
     uint64_t n4 = n >> 2;
-    for (uint64_t i = tid; i < n4; i += stride) {
-      float4 v = reinterpret_cast<const float4 *>(a)[i];
-      if (SQ) s += (double)v.x * v.x + (double)v.y * v.y + (double)v.z * v.z + (double)v.w * v.w;
-      else s += ((double)v.x + (double)v.y) + ((double)v.z + (double)v.w);
-    }
+    s = walk_sum(reinterpret_cast<const float4 *>(a), tid, n4, stride,
+                 [](const float4 &v) { return SQ ? squares(v) : ((double)v.x + (double)v.y) + ((double)v.z + (double)v.w); });
     for (uint64_t i = (n4 << 2) + tid; i < n; i += stride) { double v = a[i]; s += SQ ? v * v : v; }
   } else {
     for (uint64_t i = tid; i < n; i += stride) { double v = a[i]; s += SQ ? v * v : v; }
@@ -101,10 +117,7 @@ __global__ void k_sum_sq_list(SumList L, double *__restrict__ partial) {
   double s = 0;
   if ((((uintptr_t)a) & 15u) == 0) {                 // chunk starts are multiples of SL_CHUNK elements: as aligned as the tensor
     const uint64_t q0 = c0 >> 2, q1 = c1 >> 2;
-    for (uint64_t i = q0 + threadIdx.x; i < q1; i += blockDim.x) {
-      float4 v = reinterpret_cast<const float4 *>(a)[i];
-      s += (double)v.x * v.x + (double)v.y * v.y + (double)v.z * v.z + (double)v.w * v.w;
-    }
+    s = walk_sum(reinterpret_cast<const float4 *>(a), q0 + threadIdx.x, q1, blockDim.x, squares);
     for (uint64_t i = (q1 << 2) + threadIdx.x; i < c1; i += blockDim.x) { double v = a[i]; s += v * v; }
   } else {
     for (uint64_t i = c0 + threadIdx.x; i < c1; i += blockDim.x) { double v = a[i]; s += v * v; }
@@ -115,9 +128,7 @@ __global__ void k_sum_sq_list(SumList L, double *__restrict__ partial) {
 // stage 2: fixed-order sum of the partials by one block
 __global__ void k_final_sum(const double *__restrict__ partial, int nparts, float *__restrict__ out, double div) {
   __shared__ double sh[TPB / 64];
-  double s = 0;
-  for (int i = threadIdx.x; i < nparts; i += blockDim.x) s += partial[i];
-  s = block_sum_d(s, sh);
+  const double s = block_sum_d(walk_sum(partial, threadIdx.x, (uint64_t)nparts, blockDim.x, [](double v) { return v; }), sh);
   if (threadIdx.x == 0) out[0] = (float)(s / div);
 }
 
