@@ -485,6 +485,38 @@ def residualProduct(ctx, residual, a, b, p, training):
     return residualDropoutAdd(ctx, residual, reshape(ctx, matmulTransposed(ctx, a, b), list(residual.data.shape)), p, training)
 
 
+def geluMlp(ctx, residual, x, w1, w2, p, training):
+    """residual + dropout(gelu(x W1^T) W2^T) (gpt.ts:326-332); where the backend joins gelu and its backward to the products, as one entry."""
+    B0 = ctx.backend
+    rd, xd, d1, d2 = residual.data, x.data, w1.data, w2.data
+    both = None
+    if (not training or p == 0) and _has(B0, "matmulGeluBackward") and rd.shape[-1:] + d1.shape[:1] == d2.shape and rd.size == xd.shape[0] * d2.shape[0]:
+        both = B0.matmulTransposedGeluSaved(xd, d1)
+    if both is None:
+        return residualProduct(ctx, residual, matmulTransposedGelu(ctx, x, w1), w2, p, training)
+    live = list(both)
+    out = B0.matmulTransposedAdd(both[0], d2, rd)
+
+    def cleanup(rel):
+        _rel(rel, live[0], live[1])
+        live[0] = live[1] = None
+
+    def bw(g, B, rel, needs):
+        act, pre = live
+        flat = B.reshape(g, [xd.shape[0], d2.shape[0]])
+        dpre = B.matmulGeluBackward(flat, d2, pre)
+        if dpre is None:
+            dact = B.matmul(flat, d2)
+            dpre = B.geluBackward(pre, dact)
+            _rel(rel, dact)
+        g2 = B.matmulTransposedA(flat, act) if needs is None or needs[3] else None
+        cleanup(rel)
+        gx, g1 = _mt_backward(B, dpre, xd, d1, rel, None if needs is None else needs[1:3])
+        _rel(rel, flat, dpre)
+        return [g, gx, g1, g2]
+    return _record(ctx, out, [residual, x, w1, w2], bw, cleanup)
+
+
 def softmax(ctx, a, axis=None):
     out = ctx.backend.softmax(a.data, axis)
     last = axis is None or axis == -1 or axis == len(a.data.shape) - 1

@@ -483,6 +483,18 @@ class HipBackend:
         self._gemm(ffi.GEMM_NT, self._ptr(a), self._ptr(b), out._buf.ptr, M, N, K, K, K, N, epilogue=ffi.EPI_GELU, aux=pre._buf.ptr)
         return out, pre
 
+    def matmulGeluBackward(self, a: TensorData, b: TensorData, pre: TensorData) -> Optional[TensorData]:
+        """geluBackward(pre, A B) from the product's kernel with the arithmetic of the two; or None, for those, as for matmulTransposedGeluSaved."""
+        if len(a.shape) != 2 or len(b.shape) != 2 or not 0 < a.shape[1] == b.shape[0] <= b.shape[1] or a.shape[0] == 0:
+            return None
+        (M, K), N = a.shape, b.shape[1]
+        if pre.shape != (M, N):
+            return None
+        self._f32(a, b, pre)
+        out = self._new((M, N))
+        self._gemm(ffi.GEMM_NN, self._ptr(a), self._ptr(b), out._buf.ptr, M, N, K, K, N, N, epilogue=ffi.EPI_GELU_BWD, aux=self._ptr(pre))
+        return out
+
     def matmulTransposedAdd(self, a: TensorData, b: TensorData, residual: TensorData) -> Optional[TensorData]:
         """residual + A B^T for two matrices, shaped as the residual, from the product's kernel (or from the one that joins its slices);
         None where the shapes are no such case."""

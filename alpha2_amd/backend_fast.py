@@ -123,7 +123,7 @@ class _LazyTranspose:
 
 class FastHipBackend(HipBackend):
     name = "hip"
-    matmulTransposedGeluSaved = matmulTransposedAdd = None      # gelu and a residual join a product that is held back, whoever asks for the two
+    matmulTransposedGeluSaved = matmulGeluBackward = matmulTransposedAdd = None      # gelu, its backward and a residual join a product that is held back, whoever asks for the two
 
     def __init__(self, device: int = 0, group_weight_grads: bool = True, stream_bf16: bool = True, gelu_saves_derivative: bool = True):
         super().__init__(device)

@@ -129,5 +129,11 @@ __device__ __forceinline__ float gelu_grad_f(float x) {
   gelu_both_f(x, v, d);
   return d;
 }
+// gelu' is 1 / 0 beyond +-40 to the last bit; evaluated there, x^3 does not overflow f32 as it would from 7e12 on (the reference
+// computes in f64, ops.ts:401-419).  NaN and the infinities go through as they are (the reference's formula gives NaN for both: 0 x inf).
+__device__ __forceinline__ float gelu_grad_any_f(float x) {
+  const float ax = fabsf(x);
+  return gelu_grad_f(ax > 40.f && ax <= 3.402823466e38f ? copysignf(40.f, x) : x);
+}
 
 }  // namespace ah

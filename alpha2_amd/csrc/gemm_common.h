@@ -60,7 +60,7 @@ __device__ __forceinline__ void epilogue4(const GemmArgs &g, int64_t cbase, int 
       else { uint2 o = *reinterpret_cast<const uint2 *>((const uint16_t *)g.aux + idx);
              x[0] = bf16_bits_to_f32(o.x & 0xffff); x[1] = bf16_bits_to_f32(o.x >> 16); x[2] = bf16_bits_to_f32(o.y & 0xffff); x[3] = bf16_bits_to_f32(o.y >> 16); }
 #pragma unroll
-      for (int i = 0; i < 4; i++) v[i] *= gelu_grad_f(x[i]);
+      for (int i = 0; i < 4; i++) v[i] *= sizeof(OUT) == 4 ? gelu_grad_any_f(x[i]) : gelu_grad_f(x[i]);
     } else if (EPI == AH_EPI_MUL_AUX) {
       float x[4];
       if (sizeof(OUT) == 4) { float4 o = *reinterpret_cast<const float4 *>((const float *)g.aux + idx); x[0] = o.x; x[1] = o.y; x[2] = o.z; x[3] = o.w; }
@@ -90,7 +90,7 @@ __device__ __forceinline__ void epilogue4(const GemmArgs &g, int64_t cbase, int 
       float a = v[i];
       if (EPI == AH_EPI_ACCUM) a += Io<OUT>::ld(c, idx + i);
       else if (EPI == AH_EPI_RESIDUAL) a += Io<OUT>::ld((const OUT *)g.aux, idx + i);
-      else if (EPI == AH_EPI_GELU_BWD) a *= gelu_grad_f(Io<OUT>::ld((const OUT *)g.aux, idx + i));
+      else if (EPI == AH_EPI_GELU_BWD) { const float x = Io<OUT>::ld((const OUT *)g.aux, idx + i); a *= sizeof(OUT) == 4 ? gelu_grad_any_f(x) : gelu_grad_f(x); }
       else if (EPI == AH_EPI_GELU) { Io<OUT>::st((OUT *)g.aux_out, idx + i, a); a = gelu_f(a); }
       else if (EPI == AH_EPI_MUL_AUX) a *= Io<OUT>::ld((const OUT *)g.aux, idx + i);
       else if (EPI == AH_EPI_GELU_GRAD) { float d; gelu_both_f(a, a, d); Io<OUT>::st((OUT *)g.aux_out, idx + i, d); }

@@ -206,7 +206,7 @@ def transformerBlock(ctx: Ctx, x: Variable, layer: dict, cfg: ModelConfig, Bt: i
     elif act == "relu":
         hidden = ag.relu(ctx, mt(ctx, flat, m["fc1"]))
     else:
-        hidden = ag.matmulTransposedGelu(ctx, flat, m["fc1"])
+        return ag.geluMlp(ctx, x, flat, m["fc1"], m["fc2"], cfg.dropout, training)
     return ag.residualProduct(ctx, x, hidden, m["fc_proj" if act == "swiglu" else "fc2"], cfg.dropout, training)
 
 

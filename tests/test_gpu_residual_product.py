@@ -1,5 +1,5 @@
 """residual + A B^T from one call: against the two calls it stands for (same sums in the same order, so the same bits), with its gradients,
-and in one piece on the side stream."""
+the MLP that ends in one, and in one piece on the side stream."""
 import ctypes
 
 import numpy as np
@@ -83,3 +83,20 @@ def test_one_piece_on_the_side_stream(B):
     ffi.check(B.lib.ah_side_join())
     assert pieces() == 1
     _check(out, a, b, r)
+
+
+@pytest.mark.parametrize("rows,width,hidden", [(34, 48, 192), (2, 4, 4), (130, 256, 1024), (66, 96, 40)])      # the last: no wider than the input
+@pytest.mark.parametrize("scale", [1.0, 1e13])                     # 1e13: pre-activations whose cube is past f32
+def test_gelu_mlp_has_the_bits_of_its_parts(B, rows, width, hidden, scale):
+    def run(op):
+        rng = np.random.default_rng(rows)
+        draw = lambda k, *s: Variable(B.fromArray((k * rng.standard_normal(s)).astype(np.float32).ravel(), list(s)), True)
+        v = draw(1.0, 2, rows // 2, width), draw(scale, rows, width), draw(1.0, hidden, width), draw(1.0, width, hidden)
+        ctx = Ctx(Tape(), B)
+        y = op(ctx, *v)
+        ctx.tape.backward(ag.sum(ctx, ag.scale(ctx, y, 0.5)), B, B.releaseGpuTensor)
+        return [np.array(t.grad.data) for t in v]
+    one = run(lambda c, r, x, a, b: ag.geluMlp(c, r, x, a, b, 0.0, True))
+    two = run(lambda c, r, x, a, b: ag.add(c, r, ag.reshape(c, ag.matmulTransposed(c, ag.gelu(c, ag.matmulTransposed(c, x, a)), b), r.data.shape)))
+    for g, w in zip(one, two):
+        assert np.isfinite(w).all() and np.array_equal(g, w)
