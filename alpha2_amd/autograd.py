@@ -490,7 +490,7 @@ def geluMlp(ctx, residual, x, w1, w2, p, training):
     B0 = ctx.backend
     rd, xd, d1, d2 = residual.data, x.data, w1.data, w2.data
     both = None
-    if (not training or p == 0) and _has(B0, "matmulGeluBackward") and rd.shape[-1:] + d1.shape[:1] == d2.shape and rd.size == xd.shape[0] * d2.shape[0]:
+    if (not training or p == 0) and _has(B0, "matmulGeluBackward") and rd.shape[-1:] + d1.shape[:1] == d2.shape and 0 < rd.size == xd.shape[0] * d2.shape[0]:
         both = B0.matmulTransposedGeluSaved(xd, d1)
     if both is None:
         return residualProduct(ctx, residual, matmulTransposedGelu(ctx, x, w1), w2, p, training)
