@@ -995,34 +995,39 @@ class HipBackend:
             self._dirty(t)
 
     def adamwSteps(self, items, lr, beta1, beta2, eps, bc1, bc2, gradScale=1.0):
-        """adamwStep for every (params, grads, m, v, weightDecay) of an optimizer pass, in as few launches as their table takes: the
-        first eight at once, since the device idles here (the norm was just read back), then 48 at a time."""
-        if type(self).adamwStep is not HipBackend.adamwStep or "adamwStep" in self.__dict__:      # somebody's own update of one tensor
+        """adamwStep for every (params, grads, m, v, weightDecay) of an optimizer pass, in their order.  A list (or tuple) takes as few launches
+        as their table does: the first eight tensors at once, since the device idles here (the norm was just read back), then 48 at a
+        time.  Anything else is taken one by one: making an item may read what the items before it update, and its gradient may have no
+        other owner."""
+        own = type(self).adamwStep is not HipBackend.adamwStep or "adamwStep" in self.__dict__      # somebody's own update of one tensor
+        if own or not isinstance(items, (list, tuple)):
             for p, g, m, v, wd in items:
                 self.adamwStep(p, g, m, v, lr, beta1, beta2, eps, wd, bc1, bc2, gradScale)
             return
         h, dev = self._adam_hyper(lr, beta1, beta2, eps, 0.0, bc1, bc2, gradScale)
-        queue, written, most = [], set(), 8
+        queue, used, most = [], set(), 8        # used: buffers that a queued update reads or writes
 
         def launch():
             if queue:
                 check(self.lib.ah_adamw_list((ffi.AhAdamWItem * len(queue))(*queue), len(queue), C.byref(h), dev, 0))
             queue.clear()
-            written.clear()
+            used.clear()
         try:
             for p, g, m, v, wd in items:
                 self._f32(p, g, m, v)
                 n = p.size
                 if not (n == g.size == m.size == v.size):
                     raise ValueError("adamwStep: params, grads, m, v must have the same size")
-                for t in (p, m, v):
-                    self._own(t)
-                ptrs = self._ptr(p), self._ptr(g), self._ptr(m), self._ptr(v)
-                if len(queue) >= most or not written.isdisjoint(ptrs):      # (a tensor listed twice is updated twice, in order)
+                # The tensors of a launch run side by side, so an update that meets a queued one (a tensor listed twice, a gradient that
+                # is a parameter elsewhere, views of one buffer) waits for it - and so does what comes before it: an upload into the
+                # buffer, or a block of its own for a tensor that shares one with a clone.
+                if len(queue) >= most or any(id(t._buf) in used for t in (p, g, m, v)):
                     most = 48 if len(queue) >= most else most
                     launch()
-                written.update((ptrs[0], ptrs[2], ptrs[3]))
-                queue.append(ffi.AhAdamWItem(*ptrs, 0, n, wd, 0))
+                for t in (p, m, v):
+                    self._own(t)
+                queue.append(ffi.AhAdamWItem(self._ptr(p), self._ptr(g), self._ptr(m), self._ptr(v), 0, n, wd, 0))
+                used.update((id(p._buf), id(g._buf), id(m._buf), id(v._buf)))
                 for t in (p, m, v):
                     self._dirty(t)
         finally:

@@ -76,7 +76,7 @@ class AdamW:
 
     def _update(self, tensors, gradScale: float):
         bc1, bc2 = self._next_bias_corrections()
-        items = ((p, g, *self._moments(name, p), 0.0 if name in self.noDecayNames else self.weightDecay) for name, p, g in tensors)
+        items = [(p, g, *self._moments(name, p), 0.0 if name in self.noDecayNames else self.weightDecay) for name, p, g in tensors]
         if hasattr(self.backend, "adamwSteps"):             # a backend that takes a whole pass
             self.backend.adamwSteps(items, self.lr, self.beta1, self.beta2, self.eps, bc1, bc2, gradScale)
             return
