@@ -103,6 +103,8 @@ class KeptContext:
     def lastRow(self, context: np.ndarray, releaseTensor: Optional[Callable]) -> np.ndarray:
         """Logits behind the last token of `context`: the context of the call before and one token, or, the first time, any."""
         lib, n = self.backend.lib, int(context.size)
+        if not 0 < n <= min(self.longest, self.rows):           # past that, rows of the next layer would be overwritten
+            raise ValueError(f"a context of {n} tokens, where 1 to {min(self.longest, self.rows)} were asked for")
         if self.known == n - 1 and self.known > 0:
             check(lib.ah_decode(C.byref(self.model), self.layers, int(context[-1]), n - 1))
         else:
