@@ -24,7 +24,8 @@ _ACTIVATIONS = {"gelu": {2: None}, "silu": {0: None}, "relu": {1: None}, "univer
 
 
 class KeptContext:
-    """Use `of`, then `lastRow` with a context that is one token longer each time, then `close`."""
+    """Use `of`, then `lastRow` with a context that is one token longer each time, then `close`; `refresh` after code that may have moved
+    a parameter.  The parameters' values must stay: the kept keys and values are not computed again."""
 
     @staticmethod
     def of(cfg: ModelConfig, params: dict, backend, longest: int) -> Optional["KeptContext"]:
@@ -38,9 +39,8 @@ class KeptContext:
             return None
         kept = KeptContext(cfg, params, backend, act, longest)
         try:
-            for t, shape in kept._tensors():
-                if t.dtype != "f32" or t.store != "f32" or t.shape != shape or backend._ptr(t) & 15:
-                    return None
+            if not kept._fits():
+                return None
             # as many rows as the next power of two has: contexts of similar length ask the pool for blocks of one size
             kept.rows = min(cfg.blockSize, 1 << max(6, (longest - 1).bit_length()))
             kept.kv = backend._new((cfg.nLayer, kept.rows, 3 * width))
@@ -79,8 +79,21 @@ class KeptContext:
                 if name is not None:
                     yield m[name].data, (1, F)
 
+    def _fits(self) -> bool:
+        return all(t.dtype == "f32" and t.store == "f32" and t.shape == shape and not self.backend._ptr(t) & 15 for t, shape in self._tensors())
+
+    def refresh(self) -> bool:
+        """After code of the caller's, which may have moved a parameter: False where one is no longer what the kernels take."""
+        try:
+            if not self._fits():
+                return False
+        except (ffi.AlphaHipError, KeyError, AttributeError):
+            return False
+        self.describe()
+        return True
+
     def describe(self):
-        """Where the parameters lie now (the caller's own code may have moved one since: call it again after any)."""
+        """Where the parameters lie now."""
         cfg, p, ptr = self.cfg, self.params, self.backend._ptr
         bases = _ACTIVATIONS[self.act]
         gated = self.act == "swiglu"

@@ -97,7 +97,8 @@ def _lastRow(config: ModelConfig, params: dict, backend, context: np.ndarray, re
 
 def sampleTokens(config: ModelConfig, params: dict, backend, rng, promptTokens: Sequence[int], sampleConfig: SampleConfig,
                  releaseTensor: Optional[Callable] = None, flushGpu: Optional[Callable] = None) -> np.ndarray:
-    """The token loop of sample() (sample.ts:36-198) without the tokenizer: returns prompt + generated ids."""
+    """The token loop of sample() (sample.ts:36-198) without the tokenizer: returns prompt + generated ids.  The parameters keep their values
+    meanwhile; releaseTensor and flushGpu may move them."""
     steps, temperature, topk = sampleConfig.steps, sampleConfig.temperature, sampleConfig.topk
     topp = sampleConfig.topp
     topP = min(1.0, max(0.0, topp)) if (topp is not None and math.isfinite(topp)) else 1.0
@@ -115,10 +116,12 @@ def sampleTokens(config: ModelConfig, params: dict, backend, rng, promptTokens: 
             last = _lastRow(config, params, backend, tokens[:currentLen], releaseTensor) if kept is None else kept.lastRow(tokens[:currentLen], releaseTensor)
             if temperature > 0:
                 last = (last.astype(np.float64) / temperature).astype(np.float32)
-            if flushGpu is not None and (i & 7) == 7:
+            flush = flushGpu is not None and (i & 7) == 7
+            if flush:
                 flushGpu()
-                if kept is not None:
-                    kept.describe()
+            if kept is not None and (flush or (i == 0 and releaseTensor is not None)) and not kept.refresh():       # (both are the caller's code)
+                kept.close()
+                kept = None
             nxt = selectToken(last, rng, temperature, topk, topP)
             if currentLen < maxLen:
                 tokens[currentLen] = nxt

@@ -101,3 +101,41 @@ def test_a_context_past_what_was_asked_for_is_refused(monkeypatch, ctx, wpe, lon
         kept.lastRow(tokens[:most + 1], None)
     assert kept.known == most
     kept.close()
+
+
+def _sample(monkeypatch, replace, when):
+    """16 tokens behind a prompt of 5 while the caller's own code replaces the head's tensor, on the way out of the pass over the prompt or in
+    flushGpu; returns what the device saw of the single tokens and the contexts that were run whole."""
+    from alpha2_amd import sample
+    from alpha2_amd.backend import TensorData
+    B, cfg, params = _model(monkeypatch, 64)
+    done, whole = [], []
+
+    def move(now):
+        if now == when and not done:
+            done.append(1)
+            old = params["lmHead"].data
+            params["lmHead"].data = replace(TensorData, old)
+            B.releaseGpuTensor(old)
+    release = lambda t: (B.releaseGpuTensor(t), move("release"))
+    monkeypatch.setattr(sample, "_lastRow", lambda c, p, b, context, r: whole.append(context.size) or np.ones(20, np.float32))
+    monkeypatch.setattr(B, "_download", lambda t: np.ones(20, np.float32))
+    sample.sampleTokens(cfg, params, B, None, np.arange(5), sample.SampleConfig(steps=16, temperature=0), release, lambda: move("flush"))
+    assert done
+    return B, params, B.lib.tokens, whole
+
+
+@pytest.mark.parametrize("when", ["release", "flush"])
+def test_a_parameter_that_moves_is_followed(monkeypatch, when):
+    B, params, tokens, whole = _sample(monkeypatch, lambda T, old: T(old.shape, "f32", old.data), when)
+    assert [pos for _, pos, _ in tokens] == list(range(5, 20)) and not whole
+    assert tokens[-1][2] == B._ptr(params["lmHead"].data)
+
+
+@pytest.mark.parametrize("when", ["release", "flush"])
+def test_a_parameter_of_another_shape_ends_the_kept_context(monkeypatch, when):
+    """The pass over the whole context then says what it thinks of it, as it does for every other backend."""
+    B, params, tokens, whole = _sample(monkeypatch, lambda T, old: T((10, 16), "f32", old.data[:160]), when)
+    last = 5 if when == "release" else 12
+    assert [pos for _, pos, _ in tokens] == list(range(5, last)) and whole == list(range(last + 1, 21))
+    assert not any(n == 2 * 64 * 3 * 16 * 4 for n, _ in B.lib.blocks.values())          # the cache went back
