@@ -458,6 +458,14 @@ __global__ __launch_bounds__(256) void k_join_residual(const float *__restrict__
   }
 }
 
+int32_t join_residual(const float *ws, const GemmArgs &ga, int slices) {
+  const int64_t n4 = (int64_t)ga.M * ga.N / 4;
+  ah::launch_kernel(k_join_residual, dim3((unsigned)(cdiv(n4, 256) < 4096 ? cdiv(n4, 256) : 4096)), dim3(256), 0, ws, (const float *)ga.aux, (float *)ga.c, slices,
+                    n4, ga.N / 4, ga.ldc);
+  AH_LAUNCH_CHECK();
+  return AH_OK;
+}
+
 // ================================================================ dispatch
 template <int LAYOUT, int BM, int BN>
 int32_t launch_split(const GemmArgs &ga, int batch, int vec_a, int vec_b, int vec_c, int out_bf16) {
@@ -558,14 +566,9 @@ int32_t run_choice(const F32Choice &c, const GemmArgs &ga, int layout, int batch
   gs.sb = layout == AH_GEMM_NT ? slice : slice * ga.ldb;
   gs.c = dp<void>(ws); gs.ldc = ga.N; gs.sc = (int64_t)ga.M * ga.N; gs.epi = AH_EPI_NONE;
   rc = go(gs, slices, 1);
-  if (rc == AH_OK && ga.epi == AH_EPI_RESIDUAL) {
-    const int64_t n4 = (int64_t)ga.M * ga.N / 4;
-    ah::launch_kernel(k_join_residual, dim3((unsigned)(cdiv(n4, 256) < 4096 ? cdiv(n4, 256) : 4096)), dim3(256), 0, dp<const float>(ws), (const float *)ga.aux,
-                      (float *)ga.c, slices, n4, ga.N / 4, ga.ldc);
-    AH_LAUNCH_CHECK();
-  } else if (rc == AH_OK) {
-    rc = ah::splitk_reduce(dp<const float>(ws), (float *)ga.c, slices, ga.M, ga.N, ga.ldc, ga.epi == AH_EPI_ACCUM);
-  }
+  if (rc == AH_OK)
+    rc = ga.epi == AH_EPI_RESIDUAL ? join_residual(dp<const float>(ws), ga, slices)
+                                   : ah::splitk_reduce(dp<const float>(ws), (float *)ga.c, slices, ga.M, ga.N, ga.ldc, ga.epi == AH_EPI_ACCUM);
   note_gemm_split(slices);
   const int32_t rf = ah_free(ws);      // stream-ordered: reusable only by later work
   return rc ? rc : rf;

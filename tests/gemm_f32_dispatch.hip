@@ -1,6 +1,8 @@
 // The host side of the fp32 products without a GPU: links with the built gemm_f32 object in place of the runtime, and prints for every
-// line "M N K layout epilogue refuse lda" on the standard input (refuse: device memory is refused) what gemm_f32 would launch:
+// line "M N K layout epilogue refuse lda" on the standard input (refuse: 1 device memory is refused, 2 the second launch fails) what
+// gemm_f32 would launch:
 //   return code | last kernel noted | slices noted | blocks outstanding | launch ...    with launch = grid x * threads, K of a slice
+// or "join" for the launch that adds up the slices
 // Built for the host only (hipcc --cuda-host-only); no HIP runtime is linked.
 #include "../alpha2_amd/csrc/gemm_common.h"
 #include <cstdarg>
@@ -8,10 +10,12 @@
 #include <string>
 
 static std::string g_kernel, g_launches;
-static int g_split = 0, g_live = 0, g_refuse = 0;
+static int g_split = 0, g_live = 0, g_refuse = 0, g_count = 0;
 
 namespace ah {
-void launch_raw(const void *, dim3 grid, dim3 block, unsigned, void **args, const uint32_t *, int) {
+void launch_raw(const void *, dim3 grid, dim3 block, unsigned, void **args, const uint32_t *sizes, int) {
+  g_count++;
+  if (sizes[0] != sizeof(GemmArgs)) { g_launches += " join"; return; }
   const GemmArgs &g = *(const GemmArgs *)args[0];
   char s[96];
   snprintf(s, sizeof s, " %llu,%d", (unsigned long long)grid.x * block.x, g.nsplit > 1 ? g.ksplit : g.K);
@@ -33,13 +37,13 @@ int32_t hip_fail(hipError_t, const char *) { return AH_ERR_HIP; }
 }  // namespace ah
 extern "C" {
 int32_t ah_alloc(uint64_t, ah_ptr *out) {
-  if (g_refuse) return AH_ERR_OOM;
+  if (g_refuse == 1) return AH_ERR_OOM;
   g_live++;
   *out = 1 << 20;
   return AH_OK;
 }
 int32_t ah_free(ah_ptr) { g_live--; return AH_OK; }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() { return g_refuse == 2 && g_count > 1 ? hipErrorLaunchFailure : hipSuccess; }
 hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t) { return hipSuccess; }
 void **__hipRegisterFatBinary(const void *) { static void *handle; return &handle; }
 void __hipUnregisterFatBinary(void **) {}
@@ -59,7 +63,7 @@ int main() {
     g.ldc = n;
     g.epi = epi; g.ksplit = (int)k; g.nsplit = 1;
     g_kernel = g_launches = "";
-    g_split = -1; g_live = 0; g_refuse = refuse;
+    g_split = -1; g_live = 0; g_refuse = refuse; g_count = 0;
     const int rc = ah::gemm_f32(g, layout, 1, AH_F32, 1, 1, 1);
     printf("%d|%s|%d|%d|%s\n", rc, g_kernel.c_str(), g_split, g_live, g_launches.c_str());
   }

@@ -38,6 +38,15 @@ def test_a_product_whose_slices_get_no_memory_runs_without_them(dispatch):
                 assert whole.code == 0 and whole.blocks == 0 and len(whole.launches) == 1 and whole.launches[0].endswith(",%d" % k)
 
 
+def test_a_join_that_fails_to_launch_gives_the_slices_back(dispatch):
+    """The residual's join is launched by the product itself."""
+    for layout in (ffi.GEMM_NN, ffi.GEMM_NT, ffi.GEMM_TN):
+        ok = dispatch(384, 128, 1030, layout, ffi.EPI_RESIDUAL)
+        assert ok.code == 0 and ok.slices > 1 and ok.launches[-1] == "join" and ok.blocks == 0
+        failed = dispatch(384, 128, 1030, layout, ffi.EPI_RESIDUAL, refuse=2)
+        assert failed.code != 0 and len(failed.launches) == 2 and failed.blocks == 0
+
+
 def test_slices_are_reported_where_a_second_launch_joins_them(dispatch):
     """The waves of a 32-wide piece add up their sums inside the launch: one slice."""
     for m, n, k, layout in ((127, 260, 1000, ffi.GEMM_NN), (1, 64, 768, ffi.GEMM_NT), (500, 300, 512, ffi.GEMM_TN), (384, 128, 1030, ffi.GEMM_NN), (4000, 1200, 64, ffi.GEMM_NT)):
