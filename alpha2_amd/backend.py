@@ -472,10 +472,10 @@ class HipBackend:
         return out
 
     def matmulTransposedGeluSaved(self, a: TensorData, b: TensorData):
-        """(gelu(A B^T), A B^T), both from the product's kernel, with the arithmetic of matmulTransposed and gelu (16384 x 1024 x 256: 81
-        us in two passes, 67 in one; x 3072 x 768 500 and 454); or None, for those two: operands that are no matrices of the model's
-        kind, and more to contract than there are columns, where the product may be better off in slices, which have no epilogue."""
-        if len(a.shape) != 2 or len(b.shape) != 2 or not 0 < a.shape[1] == b.shape[1] <= b.shape[0] or a.shape[0] == 0:
+        """(gelu(A B^T), A B^T), both from the product's kernel or from the one that joins its slices, with the arithmetic of matmulTransposed
+        and gelu (16384 x 1024 x 256: 81 us in two passes, 67 in one; x 3072 x 768 500 and 454); or None, for those two: operands that
+        are no matrices of the model's kind."""
+        if len(a.shape) != 2 or len(b.shape) != 2 or not 0 < a.shape[1] == b.shape[1] or a.shape[0] == 0 or b.shape[0] == 0:
             return None
         self._f32(a, b)
         (M, K), N = a.shape, b.shape[0]
@@ -485,7 +485,7 @@ class HipBackend:
 
     def matmulGeluBackward(self, a: TensorData, b: TensorData, pre: TensorData) -> Optional[TensorData]:
         """geluBackward(pre, A B) from the product's kernel with the arithmetic of the two; or None, for those, as for matmulTransposedGeluSaved."""
-        if len(a.shape) != 2 or len(b.shape) != 2 or not 0 < a.shape[1] == b.shape[0] <= b.shape[1] or a.shape[0] == 0:
+        if len(a.shape) != 2 or len(b.shape) != 2 or not 0 < a.shape[1] == b.shape[0] or a.shape[0] == 0 or b.shape[1] == 0:
             return None
         (M, K), N = a.shape, b.shape[1]
         if pre.shape != (M, N):

@@ -560,7 +560,7 @@ int32_t ah_gemm(const AhGemm *p) {
   if (q.in_dtype == AH_F32) {
     int vec_a = aligned16(q.a) && (q.lda % 4 == 0) && (q.stride_a % 4 == 0);
     int vec_b = aligned16(q.b) && (q.ldb % 4 == 0) && (q.stride_b % 4 == 0);
-    if (q.epilogue == AH_EPI_RESIDUAL && ah::on_side()) ga.nsplit = 0;       // in one piece: no workspace there
+    if (q.epilogue != AH_EPI_NONE && q.epilogue != AH_EPI_ACCUM && ah::on_side()) ga.nsplit = 0;       // in one piece: no workspace there
     return ah::gemm_f32(ga, q.layout, batch, q.out_dtype, vec_a, vec_b, vec_c);
   }
 

@@ -441,29 +441,38 @@ __global__ __launch_bounds__(64 * WAVES) void k_gemm_f32_pieces(GemmArgs g, int 
   if (threadIdx.x < 256) finish4<false>(g, cbase, tm * 32 + r, tn * 32 + 4 * ch, s, vec_c, out_bf16);
 }
 
-// The slices of a product added up in their order, and the residual: C = sum + aux.  Memory-bound like the plain join (which adds slices only);
-// a product and an addition of their own became one product, 16384 x 256 x 1024 in two slices 73.4 -> 65.3 us, 1024 x 128 x 512 in eight
-// 11.6 -> 9.9, 16384 x 768 x 768 in one piece 135 -> 119.
-__global__ __launch_bounds__(256) void k_join_residual(const float *__restrict__ ws, const float *aux, float *c, int slices, int64_t n4,
-                                                       int row4, int64_t ldc) {
+// The slices of a product added up in their order, and its epilogue: a residual, gelu (both outputs) or gelu's backward.  Memory-bound like the
+// plain join (which adds slices only).  A product and an addition of their own became one product, 16384 x 256 x 1024 in two slices
+// 73.4 -> 65.3 us, 1024 x 128 x 512 in eight 11.6 -> 9.9, 16384 x 768 x 768 in one piece 135 -> 119.
+// gelu as a pass of its own / joined here / in the epilogue of a product that has to stay in one piece for it: 33 x 5120 x 5120 in 16 slices
+// 35.5 / 31.9 / 114.6 us, 64 x 4096 x 4096 in four 29.1 / 26.2 / 50.0, 490 x 8192 x 2048 in two 110 / 106 / 118; its backward at the same
+// shapes 36.8 / 33.5 / 77.6, 32.0 / 30.0 / 46.7, 113 / 107 / 125.
+template <int EPI>
+__global__ __launch_bounds__(256) void k_join_epilogue(const float *__restrict__ ws, GemmArgs g, int slices, int64_t n4) {
+  const int row4 = g.N / 4;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n4; i += (int64_t)gridDim.x * blockDim.x) {
     float4 s = reinterpret_cast<const float4 *>(ws)[i];
     for (int k = 1; k < slices; k++) {
       const float4 v = reinterpret_cast<const float4 *>(ws)[k * n4 + i];
       s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
     }
-    const int64_t at = i / row4 * ldc + i % row4 * 4;
-    const float4 r = *reinterpret_cast<const float4 *>(aux + at);
-    *reinterpret_cast<float4 *>(c + at) = make_float4(s.x + r.x, s.y + r.y, s.z + r.z, s.w + r.w);
+    epilogue4<EPI, float>(g, 0, (int)(i / row4), (int)(i % row4) * 4, s.x, s.y, s.z, s.w, true);
   }
 }
-
-int32_t join_residual(const float *ws, const GemmArgs &ga, int slices) {
+template <int EPI>
+int32_t join_epilogue(const float *ws, const GemmArgs &ga, int slices) {
   const int64_t n4 = (int64_t)ga.M * ga.N / 4;
-  ah::launch_kernel(k_join_residual, dim3((unsigned)(cdiv(n4, 256) < 4096 ? cdiv(n4, 256) : 4096)), dim3(256), 0, ws, (const float *)ga.aux, (float *)ga.c, slices,
-                    n4, ga.N / 4, ga.ldc);
+  ah::launch_kernel(k_join_epilogue<EPI>, dim3((unsigned)(cdiv(n4, 256) < 4096 ? cdiv(n4, 256) : 4096)), dim3(256), 0, ws, ga, slices, n4);
   AH_LAUNCH_CHECK();
   return AH_OK;
+}
+int32_t join(const float *ws, const GemmArgs &ga, int slices) {
+  switch (ga.epi) {
+    case AH_EPI_RESIDUAL: return join_epilogue<AH_EPI_RESIDUAL>(ws, ga, slices);
+    case AH_EPI_GELU: return join_epilogue<AH_EPI_GELU>(ws, ga, slices);
+    case AH_EPI_GELU_BWD: return join_epilogue<AH_EPI_GELU_BWD>(ws, ga, slices);
+    default: return ah::splitk_reduce(ws, (float *)ga.c, slices, ga.M, ga.N, ga.ldc, ga.epi == AH_EPI_ACCUM);
+  }
 }
 
 // ================================================================ dispatch
@@ -566,9 +575,7 @@ int32_t run_choice(const F32Choice &c, const GemmArgs &ga, int layout, int batch
   gs.sb = layout == AH_GEMM_NT ? slice : slice * ga.ldb;
   gs.c = dp<void>(ws); gs.ldc = ga.N; gs.sc = (int64_t)ga.M * ga.N; gs.epi = AH_EPI_NONE;
   rc = go(gs, slices, 1);
-  if (rc == AH_OK)
-    rc = ga.epi == AH_EPI_RESIDUAL ? join_residual(dp<const float>(ws), ga, slices)
-                                   : ah::splitk_reduce(dp<const float>(ws), (float *)ga.c, slices, ga.M, ga.N, ga.ldc, ga.epi == AH_EPI_ACCUM);
+  if (rc == AH_OK) rc = join(dp<const float>(ws), ga, slices);
   note_gemm_split(slices);
   const int32_t rf = ah_free(ws);      // stream-ordered: reusable only by later work
   return rc ? rc : rf;
@@ -577,10 +584,10 @@ int32_t run_choice(const F32Choice &c, const GemmArgs &ga, int layout, int batch
 }  // namespace
 
 namespace ah {
-// ga.nsplit: 0 keeps a product with a residual in one piece, which it otherwise need not be
+// ga.nsplit: 0 keeps a product in one piece
 int32_t gemm_f32(const GemmArgs &ga, int layout, int batch, int out_dtype, int vec_a, int vec_b, int vec_c) {
-  const bool joins = ga.epi == AH_EPI_NONE || ga.epi == AH_EPI_ACCUM || (ga.epi == AH_EPI_RESIDUAL && ga.nsplit > 0);
-  const bool may_split = batch == 1 && out_dtype == AH_F32 && joins && ga.N % 4 == 0 && vec_c;
+  const bool joins = ga.epi == AH_EPI_NONE || ga.epi == AH_EPI_ACCUM || ga.epi == AH_EPI_RESIDUAL || ga.epi == AH_EPI_GELU || ga.epi == AH_EPI_GELU_BWD;
+  const bool may_split = ga.nsplit > 0 && batch == 1 && out_dtype == AH_F32 && joins && ga.N % 4 == 0 && vec_c;
   // the tile loaders' offsets within a tile are 32 bits: its rows, 128 at most, span less than 4 GiB
   auto spans = [](int rows, int64_t ld) { return ((rows < 128 ? rows : 128) - 1) * ld + 16 >= (1ll << 30); };
   const bool long_rows = (layout != AH_GEMM_TN && spans(ga.M, ga.lda)) || (layout == AH_GEMM_NT && spans(ga.N, ga.ldb));

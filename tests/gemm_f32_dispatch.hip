@@ -1,6 +1,6 @@
 // The host side of the fp32 products without a GPU: links with the built gemm_f32 object in place of the runtime, and prints for every
-// line "M N K layout epilogue refuse lda" on the standard input (refuse: 1 device memory is refused, 2 the second launch fails) what
-// gemm_f32 would launch:
+// line "M N K layout epilogue refuse lda" on the standard input (refuse: 1 device memory is refused, 2 the second launch fails, 3 the
+// caller wants one piece) what gemm_f32 would launch:
 //   return code | last kernel noted | slices noted | blocks outstanding | launch ...    with launch = grid x * threads, K of a slice
 // or "join" for the launch that adds up the slices
 // Built for the host only (hipcc --cuda-host-only); no HIP runtime is linked.
@@ -61,7 +61,7 @@ int main() {
     g.lda = lda ? lda : layout == AH_GEMM_TN ? m : k;
     g.ldb = layout == AH_GEMM_NT ? k : n;
     g.ldc = n;
-    g.epi = epi; g.ksplit = (int)k; g.nsplit = 1;
+    g.epi = epi; g.ksplit = (int)k; g.nsplit = refuse == 3 ? 0 : 1;
     g_kernel = g_launches = "";
     g_split = -1; g_live = 0; g_refuse = refuse; g_count = 0;
     const int rc = ah::gemm_f32(g, layout, 1, AH_F32, 1, 1, 1);

@@ -47,6 +47,20 @@ def test_a_join_that_fails_to_launch_gives_the_slices_back(dispatch):
         assert failed.code != 0 and len(failed.launches) == 2 and failed.blocks == 0
 
 
+def test_an_epilogue_does_not_change_the_kernel(dispatch):
+    """Few rows and a long contraction, and shapes that stay in one piece: the slices join with a residual, gelu or its backward; refused
+    memory, and zero for `nsplit` (nothing may be allocated), leave one piece."""
+    for m, n, k in ((33, 5120, 5120), (64, 4096, 4096), (490, 8192, 2048), (256, 6144, 1536), (16384, 1024, 256), (777, 768, 3072), (1, 4096, 1024)):
+        for layout, epis in ((ffi.GEMM_NT, (ffi.EPI_GELU, ffi.EPI_RESIDUAL)), (ffi.GEMM_NN, (ffi.EPI_GELU_BWD,)), (ffi.GEMM_TN, (ffi.EPI_GELU,))):
+            plain = dispatch(m, n, k, layout)
+            for epi in epis:
+                assert dispatch(m, n, k, layout, epi) == plain
+                whole = dispatch(m, n, k, layout, epi, refuse=1)
+                assert whole.code == 0 and whole.blocks == 0 and len(whole.launches) == 1
+                kept = dispatch(m, n, k, layout, epi, refuse=3)
+                assert kept == whole
+
+
 def test_slices_are_reported_where_a_second_launch_joins_them(dispatch):
     """The waves of a 32-wide piece add up their sums inside the launch: one slice."""
     for m, n, k, layout in ((127, 260, 1000, ffi.GEMM_NN), (1, 64, 768, ffi.GEMM_NT), (500, 300, 512, ffi.GEMM_TN), (384, 128, 1030, ffi.GEMM_NN), (4000, 1200, 64, ffi.GEMM_NT)):
