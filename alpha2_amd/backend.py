@@ -25,7 +25,7 @@ _NP = {"f32": np.float32, "i32": np.int32, "f16": np.uint16, "bf16": np.uint16, 
 
 
 def shapeSize(shape) -> int:
-    return int(math.prod(shape))
+    return math.prod(map(int, shape))
 
 
 def shapeStrides(shape) -> List[int]:
