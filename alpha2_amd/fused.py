@@ -24,7 +24,6 @@ from __future__ import annotations
 
 import ctypes as C
 import math
-import struct
 from dataclasses import dataclass
 from typing import Dict, List, Optional, Tuple
 
@@ -577,7 +576,7 @@ class FusedTrainer:
     def _hyper_items(self) -> list:
         """The learning rate of this step: the first field of the device AhAdamW.  Its bias corrections are kept by
         ah_step_guard on the device, which advances them on applied steps only."""
-        items = [ffi.AhCopy(self.hyper, 0, 4, struct.unpack("<I", struct.pack("<f", lrAt(self.tc, self.stepIdx)))[0])]
+        items = [ffi.AhCopy(self.hyper, 0, 4, C.c_uint32.from_buffer(C.c_float(lrAt(self.tc, self.stepIdx))).value)]
         if self.drop > 0:                          # the masks of this step's micro-steps (trainer.ts:1169,1202), as int32 like `seed | 0`
             items += [ffi.AhCopy(self.seed_dev + 4 * m, 0, 4, (self.tc.seed + self.stepIdx * 1000 + m) & 0xFFFFFFFF) for m in range(self.micro_steps)]
         return items
