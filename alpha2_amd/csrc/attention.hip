@@ -24,7 +24,14 @@ namespace {
 constexpr int BC = 32;     // rows of the streamed tile per iteration
 constexpr int WAVES = 4;   // 4 waves x 32 owned rows = 128 rows per block
 
+// (finite for a cap whose inverse is past the range, so that a score of zero stays one)
+__device__ __forceinline__ float inverse_cap(float cap) { return cap > 0.f ? fminf(1.0f / cap, 3.402823466e38f) : 0.f; }
 __device__ __forceinline__ float softcap_fwd(float s, float cap, float inv_cap) { return cap > 0.f ? tanhf(s * inv_cap) * cap : s; }
+__device__ __forceinline__ float softcap_both(float s, float cap, float inv_cap, float &slope) {
+  const float t = cap > 0.f ? tanhf(s * inv_cap) : 0.f;
+  slope = 1.0f - t * t;
+  return cap > 0.f ? t * cap : s;
+}
 
 // cooperative load of a [32 x D] f32 tile (rows row0.., zero beyond `rows` and beyond feature hd) into LDS with pitch D+1
 template <int D>
@@ -218,7 +225,7 @@ __device__ __forceinline__ void scores_tanh(f32x16 &s, float cap, float factor) 
     for (int e = 0; e < 16; e++) { const float small = tanh_small(s[e]), large = tanh_large(s[e]); s[e] = fabsf(s[e]) < TANH_SMALL ? small : large; }
   }
 }
-__device__ __forceinline__ float split_cap_factor(float cap) { return (cap > 0.f ? 1.0f / cap : 1.0f) * SPLIT_DOWN; }
+__device__ __forceinline__ float split_cap_factor(float cap) { return (cap > 0.f ? inverse_cap(cap) : 1.0f) * SPLIT_DOWN; }
 // (a cap whose factor is no normal number is left to the fp32 instruction)
 __device__ __forceinline__ bool split_cap_ok(float cap) { return !(cap > 0x1p70f); }
 // An infinite score has to be found before it is capped or weighed: what is made of it looks like any other.  (NaN shows in that.)  Either
@@ -247,7 +254,7 @@ __device__ void flash_fwd_exact(const FlashArgs &a, int bh, int q0, int end, boo
   const float *Q = (const float *)a.q + b * a.q_sb + h * a.q_sh;
   const float *K = (const float *)a.k + b * a.k_sb + h * a.k_sh;
   const float *V = (const float *)a.v + b * a.v_sb + h * a.v_sh;
-  float inv_cap = a.cap > 0.f ? 1.0f / a.cap : 0.f;
+  const float inv_cap = inverse_cap(a.cap);
 
   float qreg[D / 2];                                  // Q[qi][2i + lk] * scale
 #pragma unroll
@@ -597,7 +604,7 @@ __device__ void flash_dq_exact(const FlashArgs &a, int bh, int xblk, float *smem
   const float *K = (const float *)a.k + b * a.k_sb + h * a.k_sh;
   const float *V = (const float *)a.v + b * a.v_sb + h * a.v_sh;
   const float *dO = (const float *)a.d_o + b * a.o_sb + h * a.o_sh;
-  float inv_cap = a.cap > 0.f ? 1.0f / a.cap : 0.f;
+  const float inv_cap = inverse_cap(a.cap);
   bool live = qi < a.T;
   float qreg[D / 2], doreg[D / 2];
 #pragma unroll
@@ -632,11 +639,9 @@ __device__ void flash_dq_exact(const FlashArgs &a, int bh, int xblk, float *smem
 #pragma unroll
     for (int e = 0; e < 16; e++) {
       int kv = kv0 + 8 * (e >> 2) + 4 * lk + (e & 3);
-      float sc = softcap_fwd(s[e], a.cap, inv_cap);
+      float slope, sc = softcap_both(s[e], a.cap, inv_cap, slope);
       float p = (kv > qi || kv >= a.T || !live) ? 0.f : expf(sc - lse);
-      float ds = p * (dp[e] - delta);
-      if (a.cap > 0.f) { float t = sc * inv_cap; ds *= (1.0f - t * t); }
-      s[e] = ds * a.scale;
+      s[e] = p * (dp[e] - delta) * slope * a.scale;
     }
 #pragma unroll
     for (int d = 0; d < DB; d++)
@@ -762,7 +767,7 @@ __device__ void flash_dkv_exact(const FlashArgs &a, int bh, int xblk, float *sme
   const float *K = (const float *)a.k + b * a.k_sb + h * a.k_sh;
   const float *V = (const float *)a.v + b * a.v_sb + h * a.v_sh;
   const float *dO = (const float *)a.d_o + b * a.o_sb + h * a.o_sh;
-  float inv_cap = a.cap > 0.f ? 1.0f / a.cap : 0.f;
+  const float inv_cap = inverse_cap(a.cap);
   bool live = kvi < a.T;
   float kreg[D / 2], vreg[D / 2];
 #pragma unroll
@@ -800,12 +805,10 @@ __device__ void flash_dkv_exact(const FlashArgs &a, int bh, int xblk, float *sme
 #pragma unroll
     for (int e = 0; e < 16; e++) {
       int qr = 8 * (e >> 2) + 4 * lk + (e & 3), qi = q0 + qr;
-      float sc = softcap_fwd(s[e], a.cap, inv_cap);
+      float slope, sc = softcap_both(s[e], a.cap, inv_cap, slope);
       float p = (kvi > qi || qi >= a.T || !live) ? 0.f : expf(sc - Ls[qr]);
-      float ds = p * (dp[e] - Ds[qr]);
-      if (a.cap > 0.f) { float t = sc * inv_cap; ds *= (1.0f - t * t); }
       pm[e] = p;
-      s[e] = ds;                                      // Qs already carries `scale`, so dK = dS^T (scale*Q)
+      s[e] = p * (dp[e] - Ds[qr]) * slope;                                      // Qs already carries `scale`, so dK = dS^T (scale*Q)
     }
 #pragma unroll
     for (int d = 0; d < DB; d++)

@@ -56,3 +56,28 @@ def test_scores_on_both_sides_of_the_cap(B, heads, T, D, cap, spread):
     for name, got, w, size in zip(("O", "dQ", "dK", "dV"), out, want, sizes):
         off = np.linalg.norm(got.data.reshape(a[0].shape)[:4].astype(np.float64) - w)
         assert off <= (10 + 2 * largest) * 2.0 ** -24 * size, (name, off / size * 2 ** 24)
+
+
+@pytest.mark.parametrize("cap", [1e-39, 2.0 ** -149, 1e-37])
+@pytest.mark.parametrize("heads,T,D", [(2, 40, 32), (300, 130, 64), (2, 33, 128)])
+def test_scores_of_zero_under_the_smallest_caps(B, heads, T, D, cap):
+    """Down to caps whose inverse is past the range: a score of zero stays one, others weigh the same to 2^-24.  Row 3 of the queries is zero,
+    which a derivative passes (tanh' 0 = 1); at the others, scores of a unit or so, it is nothing.  Bound as above."""
+    from alpha2_amd import _ffi as ffi
+    from alpha2_amd.backend import TensorData
+    rs = np.random.default_rng(T + D)
+    a = [rs.standard_normal((heads, T, D), dtype=np.float32) for _ in range(4)]
+    a[0][:, 3] = 0
+    t = [TensorData(x.shape, "f32", x) for x in a]
+    out = [B._new(a[0].shape) for _ in range(4)]
+    lse = B._new((heads, T))
+    st = (heads * T * D, T * D, D)
+    p = [B._ptr(x) for x in t]
+    f = ffi.AhFlash(ffi.F32, 1, heads, T, D, *st, *st, *st, *st, 1.0, cap, p[0], p[1], p[2], out[0]._buf.ptr, lse._buf.ptr, p[3],
+                    out[1]._buf.ptr, out[2]._buf.ptr, out[3]._buf.ptr, 0, 0)
+    ffi.check(B.lib.ah_flash_fwd(C.byref(f)))
+    ffi.check(B.lib.ah_flash_bwd(C.byref(f)))
+    want, sizes, _ = _exact(*(x[:4].astype(np.float64) for x in a), 1.0, float(np.float32(cap)))
+    for name, got, w, size in zip(("O", "dQ", "dK", "dV"), out, want, sizes):
+        off = np.linalg.norm(got.data.reshape(a[0].shape)[:4].astype(np.float64) - w)
+        assert off <= 10 * 2.0 ** -24 * size, (name, off / size * 2 ** 24)
