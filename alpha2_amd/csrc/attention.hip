@@ -182,10 +182,14 @@ struct SplitTile {                          // D = 32 or 64
 };
 // The functions of a tile's 16 scores in straight-line code, all 16 at once: the library's tanh branches for every score, and so did the cap
 // and the masks, so that the 16 ran one after the other.  Forward / backward (delta, dQ, dK and dV), us, before -> now: 512 heads x 256 x
-// 32 50 / 172 -> 42 / 130, 192 x 1024 x 64 265 / 810 -> 234 / 685 (without a cap 220 / 755 -> 197 / 650), 32 x 128 x 32 8.5 / 42 ->
-// 7.3 / 34, 12 x 500 x 64 22 / 184 -> 20 / 140; errors against 64 bits the same without a cap and up to 20 % less with one.
-// tanh x for |x| < TANH_SMALL as x + x^3 P(x^2), P the fifth-order polynomial of least relative error there (fitted by reweighted least
-// squares): 0.7 last places off at most, 0.3 on average.  Beyond, 1 - 2 / (exp(2 |x|) + 1), which is 1.5 off at most there.
+// 32 51 / 168 -> 45 / 128, 192 x 1024 x 64 269 / 816 -> 240 / 697 (without a cap 239 / 763 -> 219 / 665; the scores all at a cap of 0.75
+// 309 / 888 -> 262 / 736), 32 x 128 x 32 8.5 / 42 ->
+// 7.3 / 34, 12 x 500 x 64 22 / 184 -> 20 / 140.  Results against 64 bits (4 x 256 x 32 and 4 x 512 x 64): the same without a cap, up to 46 %
+// closer with one of 5 or 30; under a cap of 0.75 with nearly every score at it, dQ up to 12 % further off and down to 13 % closer.
+// tanh in the form of Cephes' tanhf (Moshier): for |x| < TANH_SMALL x + x^3 P(x^2), P here the fifth-order polynomial of least relative error
+// there (fitted by reweighted least squares, Lawson's method), beyond that 1 - 2 / (exp(2 |x|) + 1).  Last places off at most, over all
+// values from 0.5 to 1: 0.73 and 1.63 (the library's tanhf 0.78 and 1.39; its two-part argument and a corrected exponential bring the
+// second to 1.56 and cost 5 % of the forward pass where scores are large).
 constexpr float TANH_SMALL = 0.625f, LOG2E = 1.44269502162933349609375f, LOG2E_REST = 1.925963033e-8f;
 __device__ __forceinline__ float tanh_small(float x) {
   const float z = x * x;
@@ -197,8 +201,8 @@ __device__ __forceinline__ float tanh_small(float x) {
   return __builtin_fmaf(x * z, p, x);
 }
 // 2^UP exp x, x not much above 0 and not below -1e9 (there, as for infinite x, NaN or infinity may come of it): the integer part of
-// x log2 e goes into the exponent, 2 to the rest is the instruction's.  0.96 last places off at most, 0.306 on average (expf: 0.84, 0.300;
-// a single exponential of x log2 e times what that rounds off: 1.25, 0.41).
+// x log2 e, whose constant is held in two parts (Cody and Waite), goes into the exponent, 2 to the rest is the instruction's.  0.96 last
+// places off at most, 0.306 root mean square (expf: 0.84, 0.300; a single exponential of x log2 e times what that rounds off: 1.25, 0.41).
 template <int UP>
 __device__ __forceinline__ float exp_of(float x) {
   const float n = __builtin_rintf(x * LOG2E), rest = __builtin_fmaf(x, LOG2E_REST, __builtin_fmaf(x, LOG2E, -n));
@@ -358,8 +362,8 @@ __device__ __forceinline__ float tile_weights(f32x16 &s, float mul, float before
 }
 __device__ __forceinline__ float output_factor(float l) { return (l > 0.f ? 1.0f / l : 0.f) * SPLIT_DOWN; }
 
-// Four waves of 32 queries.  192 heads x 1024 x 64: 383 us with the fp32 instruction, now 240; 512 x 256 x 32 61 -> 42; relative error
-// against 64 bits at 4 x 512 x 64 1.9e-7 (fp32 instruction: 2.4e-7).  Vector issue bounds it, as in backward.
+// Four waves of 32 queries.  With the fp32 instruction 192 heads x 1024 x 64 took 383 us and 512 x 256 x 32 61 (now: beside the functions
+// above); relative error against 64 bits at 4 x 512 x 64 1.9e-7 (fp32 instruction: 2.4e-7).  Vector issue bounds it, as in backward.
 // Head sizes over 64 keep the fp32 instruction: their operands do not fit the registers in three parts.
 template <int D>
 __global__ __launch_bounds__(256, D > 64 ? 1 : 2) void k_flash_fwd_f32(FlashArgs a) {

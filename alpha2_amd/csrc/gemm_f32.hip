@@ -165,9 +165,10 @@ __device__ __forceinline__ void mfma6_tiles(const bf16x8 (&a)[3][TM], const bf16
 // ================================================================ tiles through LDS
 // 2 x 2 waves of 64 x 64 (or 32 x 32): 24 matrix instructions per step and wave, 768 cycles, against 92 vector instructions for the
 // split and the long sums, which go into the gaps between them (sched_group_barrier, four to a gap: with 3 or 6 3 to 12 % slower).
-// What bounds the large tiles: on zeros, where the clock does not fall, 16384 x 3072 x 768 takes 342 us, without the split 275; on
-// standard normal operands the clock falls to 1.9 GHz and it takes 414 (matrix pipes 49 % busy).  One tile on its way instead of two cost
-// 5 % there, the 64 vector instructions more of a split by shifts and subtractions nothing in NT and NN and 5 % in TN.  Tiles of
+// What bounds the large tiles: on zeros, where the clock does not fall, 16384 x 3072 x 768 takes 341 us, without the split 275; on
+// standard normal operands the clock falls to 1.9 GHz and it takes 436 from the hundredth call on, 560 over the first ten (matrix pipes
+// 49 % busy).  One tile on its way instead of two cost 5 % there, the 64 vector instructions more of a split by shifts and subtractions
+// nothing in NT and NN and 5 % in TN.  Tiles of
 // 128 x 64, and 128 x 128 on eight waves, are slower at every size tried (2 to 30 %).
 // LDS: three planes of [row][16 k] bf16 per operand, 32 bytes a row, two buffers.  The 16-byte half of a row that holds k 0..7 is
 // the first one in rows whose bit 3 is clear and the second one in the others: the fragment reads and the 8-byte writes of either
@@ -502,14 +503,15 @@ int32_t launch_pieces(const GemmArgs &ga, int batch, int vec_a, int vec_b, int v
 struct F32Choice { int bm, waves, splits; };
 
 // The choice is the least of what the candidates are expected to take, in microseconds beyond a launch, from figures measured over 71 shapes
-// (1 x 4096 x 1024 to 16384 x 50304 x 768, in the three layouts; the choice is 3 % slower than the fastest candidate on average, 32 % at worst):
+// (1 x 4096 x 1024 to 16384 x 50304 x 768, in the three layouts) on the kernels as they were when a pair of values was cut in 13
+// instructions: the tiles have become 2 to 15 % faster since, and the constants are those of then:
 //   32 x 32     FIRST, the first round trip; then GROUP per 4 pieces of a wave, and the rate that all of them together reach
 //   LDS tiles   a tile takes `step` per 16 of the contraction alone on its CU, and `full` of the CU's time where others fill its gaps
 //   slices      another launch, and the workspace written and read
 // Against 128 x 128 tiles of v_mfma_f32_32x32x2_f32 (in slices where there were fewer than 256 tiles and K >= 2048), in us:
-//   16384 x 3072 x 768 NT 720 -> 414 (128 x 128), 768 x 768 x 16384 TN 329 -> 137 (128 x 128 in 32 slices), 490 x 768 x 768 NT 77 -> 14
+//   16384 x 3072 x 768 NT 720 -> 436 (128 x 128), 768 x 768 x 16384 TN 329 -> 139 (128 x 128 in 32 slices), 490 x 768 x 768 NT 77 -> 14
 //   (64 x 64 in 2 slices), 48 x 768 x 256 NT 26 -> 7 and 512 x 128 x 1024 TN 97 -> 9 (32 x 32).  Operands that are not finite take the
-//   fp32 instruction as well: 16384 x 3072 x 768 of NaNs 1070 (720 by that instruction's own kernel).
+//   fp32 instruction as well: 16384 x 3072 x 768 of NaNs 975 (720 by that instruction's own kernel).
 F32Choice choose(const GemmArgs &ga, int layout, int batch, bool may_split, bool long_rows) {
   struct Tile { int bm; double step, full; };
   static constexpr Tile TILES[2] = {{64, 0.26, 0.24}, {128, 1.2, 0.65}};

@@ -28,8 +28,8 @@ __device__ __forceinline__ float here(float x) {
 struct Split2 { uint32_t h, m, l; };       // the parts of two values side by side
 // x less the low (high) half of h: v_dot2_f32_bf16 with (-1, 0) or (0, -1), in place of an instruction that makes an fp32 number of the
 // half and one that subtracts it: nine instructions for a pair of values in place of 13 (2.0 ns of a SIMD each where a shift takes 1.9 and
-// a subtraction 1.2).  The result is exact for every significand (both ways compared over all of them at eight exponents),
-// and the other half, unless it is infinite or NaN, adds nothing.  The constants are hidden from the compiler, which takes 0xbf80 in the
+// a subtraction 1.2).  The result is exact for every significand (times 1, each comes out of a product as it went in: all of them, at
+// eight pairs of exponents of the two halves), and the other half, unless it is infinite or NaN, adds nothing.  The constants are hidden from the compiler, which takes 0xbf80 in the
 // low half alone for the one in both.
 __device__ __forceinline__ uint32_t hidden(uint32_t c) {
   asm("" : "+s"(c));

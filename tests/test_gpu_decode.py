@@ -149,3 +149,48 @@ def test_not_finite_parameters_reach_the_logits(B):
         got, want = kept.lastRow(tokens[:n], B.releaseGpuTensor), _lastRow(cfg, params, B, tokens[:n], B.releaseGpuTensor)
         assert np.array_equal(np.isnan(got), np.isnan(want)), n
     kept.close()
+
+
+@pytest.mark.parametrize("temperature", [0.0, 0.8])
+@pytest.mark.parametrize("act", ["gelu", "swiglu"])
+def test_the_same_tokens_with_and_without_kept_keys(B, monkeypatch, temperature, act):
+    """Over a prompt of 60 and 20 tokens behind it (a second slice from the 65th on), while flushGpu moves every parameter to another block and
+    fills the one it left with NaN.  The largest logits lie further apart than the two ways' roundings put them (1e-4 of the row; see _compare)."""
+    from alpha2_amd import sample
+    from alpha2_amd.decode import KeptContext
+    from alpha2_amd.model import collectParamEntries
+    from alpha2_amd.rng import SeededRng
+    cfg, params = _model(B, 50, 96, 2, 64, 4, ffnActivation=act)
+    prompt = np.random.RandomState(4).randint(0, 50, 60)
+    config = sample.SampleConfig(steps=20, temperature=temperature, topk=10)
+    whole, gaps = [], []
+
+    def look(row, *rest):
+        top = np.sort(row)[::-1]
+        gaps.append((top[0] - top[1]) / np.linalg.norm(row))
+        return select(row, *rest)
+    select = sample.selectToken
+    with monkeypatch.context() as m:
+        m.setattr(KeptContext, "of", staticmethod(lambda *a: None))
+        if temperature == 0:
+            m.setattr(sample, "selectToken", look)
+        want = sample.sampleTokens(cfg, params, B, SeededRng(7), prompt, config, B.releaseGpuTensor, B.flush)
+    assert not gaps or min(gaps) > 1e-4
+    moved = {}
+
+    def move():
+        B.flush()
+        for _, v in collectParamEntries(params):
+            t = v.data
+            t.data = np.array(t.data)
+            old = t._buf.ptr
+            B.releaseGpuTensor(t)
+            for _ in range(1000):                       # (the pool hands out its lowest block first)
+                x = B.full(t.shape, float("nan"))
+                moved[x._buf.ptr] = x
+                if x._buf.ptr == old:
+                    break
+            assert old in moved
+        whole.append(1)
+    got = sample.sampleTokens(cfg, params, B, SeededRng(7), prompt, config, B.releaseGpuTensor, move)
+    assert len(whole) == 2 and got.size == 80 and np.array_equal(got, want)
