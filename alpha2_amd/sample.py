@@ -12,7 +12,7 @@ import numpy as np
 
 from .autograd import Tape
 from .backend import TensorData
-from .decode import KeptContext
+from .decode import KeptContext, mayMove
 from .model import ModelConfig, gptForward
 
 
@@ -116,10 +116,9 @@ def sampleTokens(config: ModelConfig, params: dict, backend, rng, promptTokens: 
             last = _lastRow(config, params, backend, tokens[:currentLen], releaseTensor) if kept is None else kept.lastRow(tokens[:currentLen], releaseTensor)
             if temperature > 0:
                 last = (last.astype(np.float64) / temperature).astype(np.float32)
-            flush = flushGpu is not None and (i & 7) == 7
-            if flush:
+            if flushGpu is not None and (i & 7) == 7:
                 flushGpu()
-            if kept is not None and (flush or (i == 0 and releaseTensor is not None)) and not kept.refresh():       # (both are the caller's code)
+            if kept is not None and (((i & 7) == 7 and mayMove(flushGpu)) or (i == 0 and mayMove(releaseTensor))) and not kept.refresh():
                 kept.close()
                 kept = None
             nxt = selectToken(last, rng, temperature, topk, topP)
