@@ -1021,7 +1021,7 @@ class HipBackend:
                 # The tensors of a launch run side by side, so an update that meets a queued one (a tensor listed twice, a gradient that
                 # is a parameter elsewhere, views of one buffer) waits for it - and so does what comes before it: an upload into the
                 # buffer, or a block of its own for a tensor that shares one with a clone.
-                if len(queue) >= most or any(id(t._buf) in used for t in (p, g, m, v)):
+                if len(queue) >= most or not used.isdisjoint((id(p._buf), id(g._buf), id(m._buf), id(v._buf))):
                     most = 48 if len(queue) >= most else most
                     launch()
                 for t in (p, m, v):
