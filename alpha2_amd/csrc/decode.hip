@@ -11,7 +11,7 @@
 //   k_decode_attention   keys in slices of at least 64, one workgroup to a slice and head
 //   k_decode_rows<JOIN>  joins the slices (softmax weights of the slices' maxima) in LDS + wo + the residual stream
 //   k_decode_long        fc2 + the residual stream: long rows, few of them, so four waves to a row
-// 64 tokens from a 6 x 256 model 54.3 -> 12.2 ms, 24 tokens behind a prompt of 480 from the GPT-2-small shape 59.4 -> 12.4 (each with
+// 64 tokens from a 6 x 256 model 56.0 -> 11.5 ms, 24 tokens behind a prompt of 480 from the GPT-2-small shape 59.9 -> 12.6 (each with
 // the pass over the finished sequence that follows).  A launch takes 2.9 to 5.7 us there and the next one starts about 1 us later.
 #include "common.h"
 #include <cmath>
