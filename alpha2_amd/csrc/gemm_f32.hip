@@ -500,7 +500,8 @@ int32_t launch_pieces(const GemmArgs &ga, int batch, int vec_a, int vec_b, int v
 
 // bm = 32: 32 x 32 tiles straight from memory, `waves` waves each; otherwise tiles of bm x bm through LDS.  splits: the contraction is cut
 // into that many slices, which run as batch entries into a workspace and are then added up in fixed order.
-struct F32Choice { int bm, waves, splits; };
+// us: what the choice is expected to take.
+struct F32Choice { int bm, waves, splits; double us; };
 
 // The choice is the least of what the candidates are expected to take, in microseconds beyond a launch, from figures measured over 71 shapes
 // (1 x 4096 x 1024 to 16384 x 50304 x 768, in the three layouts) on the kernels as they were when a pair of values was cut in 13
@@ -519,14 +520,13 @@ F32Choice choose(const GemmArgs &ga, int layout, int batch, bool may_split, bool
   const double M = ga.M, N = ga.N, K = ga.K;
   // a launch has fewer than 2^32 threads: a row of more than 2^30 columns leaves only the widest tiles
   auto fits = [&](int bm, int threads) { return cdiv(ga.M, bm) * cdiv(ga.N, bm) * threads < (1ll << 32); };
-  F32Choice best{32, 8, 1};
-  double least = 1e300;
+  F32Choice best{32, 8, 1, 1e300};
   for (int w = 0; w < 2; w++) {
     const int waves = 4 << w;
     if (!fits(32, 64 * waves)) continue;
     double t = FIRST[w] + GROUP[w] * (double)cdiv(cdiv(ga.K, 16), waves * 4) +
                (double)(cdiv(ga.M, 32) * cdiv(ga.N, 32) * batch) * 2048.0 * K / RATE[layout] * (w == 0 ? 1.0 : 1.6);
-    if (t < least) { least = t; best = F32Choice{32, waves, 1}; }
+    if (t < best.us) best = F32Choice{32, waves, 1, t};
   }
   if (long_rows) return best;
   for (const Tile &q : TILES)
@@ -535,7 +535,7 @@ F32Choice choose(const GemmArgs &ga, int layout, int batch, bool may_split, bool
       const double per_cu = (double)(cdiv(ga.M, q.bm) * cdiv(ga.N, q.bm) * batch * s) / num_cus();
       const double b = per_cu < 4 ? ceil(per_cu) : per_cu + 0.5, alone = q.step * (layout == AH_GEMM_TN ? 1.1 : 1.0);
       const double t = K / s / 16 * (b * q.full > alone ? b * q.full : alone) + (s > 1 ? 1.8 + (s + 1) * M * N * 4 / 2.8e6 : 0.0);
-      if (t < least) { least = t; best = F32Choice{q.bm, 0, s}; }
+      if (t < best.us) best = F32Choice{q.bm, 0, s, t};
     }
   return best;
 }
@@ -593,6 +593,19 @@ int32_t gemm_f32(const GemmArgs &ga, int layout, int batch, int out_dtype, int v
   // the tile loaders' offsets within a tile are 32 bits: its rows, 128 at most, span less than 4 GiB
   auto spans = [](int rows, int64_t ld) { return ((rows < 128 ? rows : 128) - 1) * ld + 16 >= (1ll << 30); };
   const bool long_rows = (layout != AH_GEMM_TN && spans(ga.M, ga.lda)) || (layout == AH_GEMM_NT && spans(ga.N, ga.ldb));
-  return run_choice(choose(ga, layout, batch, may_split, long_rows), ga, layout, batch, out_dtype, vec_a, vec_b, vec_c, long_rows);
+  F32Choice c = choose(ga, layout, batch, may_split, long_rows);
+  // With gelu or its backward one piece is one launch and slices are two and a workspace, where the plain product's slices are what its join is
+  // compared with.  So slices have to be expected to gain something: 2.5 us on tiles through LDS, 6 on 32 x 32 pieces, whose estimate is
+  // that much too high beside a join.  Measured in graphs, slices / one piece, forward and backward: tiles that gain 0 to 2.1 us by the
+  // estimate 27.7 / 28.4 and 27.5 / 30.7 (274 x 3456 x 864) to 63.6 / 60.5 and 62.0 / 63.0 (912 x 4096 x 1024), and a second launch
+  // is some 4 us of the host, which is what bounds a pass of a small model; from 2.5 us on 15.8 / 20.9 and 17.0 / 23.1 (108 x 3584 x
+  // 896), 42.3 / 45.3 and 44.5 / 50.8 (256 x 6144 x 1536).  Pieces that gain 0 to 4.5 us 9.8 / 10.1 and 10.3 / 8.1 (88 x 2048 x 512),
+  // 13.2 / 12.7 and 14.1 / 10.6 (65 x 2688 x 672), backward 14.1 / 13.3 (64 x 4096 x 1024); from 6 us on 13.5 / 17.4 (its forward pass),
+  // 18.1 / 28.8 and 20.0 / 23.5 (128 x 2048 x 2048).
+  if (c.splits > 1 && (ga.epi == AH_EPI_GELU || ga.epi == AH_EPI_GELU_BWD)) {
+    const F32Choice one = choose(ga, layout, batch, false, long_rows);
+    if (one.us - c.us < (one.bm == 32 ? 6.0 : 2.5)) c = one;
+  }
+  return run_choice(c, ga, layout, batch, out_dtype, vec_a, vec_b, vec_c, long_rows);
 }
 }  // namespace ah
