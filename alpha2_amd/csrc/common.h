@@ -49,6 +49,7 @@ inline void launch_kernel(void (*kernel)(KArgs...), dim3 grid, dim3 block, unsig
 // inside a step plan the work recorded so far is launched first.  Returns AH_OK or an error code.
 int32_t step_boundary(const char *what);
 bool    step_active();
+bool    capturing();                              // between ah_graph_begin and ah_graph_end
 
 #define AH_REQUIRE_READY() do { if (!ah::ready()) return ah::fail(AH_ERR_STATE, "%s: ah_init has not been called", __func__); } while (0)
 #define AH_HIP(expr) do { hipError_t _e = (expr); if (_e != hipSuccess) return ah::hip_fail(_e, #expr); } while (0)

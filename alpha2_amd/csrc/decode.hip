@@ -4,16 +4,18 @@
 // A single row makes every product a matrix times a vector: nothing is used twice, so there is no tile to share and the bound is the
 // weights read once (4 bytes for 2 operations) - where a launch is long enough to feel it.  At the sizes sampled in earnest (256 to
 // 1024 wide) a matrix is 0.3 to 12 MB, a microsecond or two of the chip, and what a token takes is the chain of dependent launches.
-// So the launches are few, five a layer, each does the small work in front of its product itself, and each asks for its weights before
+// So the launches are few, one for the whole token up to 512 wide (k_decode_chain) and otherwise five a layer, each does the small work in front of its product itself, and each asks for its weights before
 // anything it has to wait for:
 //   k_decode_rows<NORM>  LayerNorm (the first one of all adds the two embeddings) + q, k, v into the row of the cache; + fc1 and its
 //                        activation (gate and up together); + the head.  Every wave normalises the row again, in registers.
 //   k_decode_attention   keys in slices of at least 64, one workgroup to a slice and head
 //   k_decode_rows<JOIN>  joins the slices (softmax weights of the slices' maxima) in LDS + wo + the residual stream
 //   k_decode_long        fc2 + the residual stream: long rows, few of them, so four waves to a row
-// 64 tokens from a 6 x 256 model 56.0 -> 11.5 ms, 24 tokens behind a prompt of 480 from the GPT-2-small shape 59.9 -> 12.6 (each with
+// 64 tokens from a 6 x 256 model 56.0 -> 11.5 ms in launches and 9.0 in one launch a token, 24 tokens behind a prompt of 480 from the GPT-2-small shape 59.9 -> 12.6 (each with
 // the pass over the finished sequence that follows).  A launch takes 2.9 to 5.7 us there and the next one starts about 1 us later.
 #include "common.h"
+#include <algorithm>
+#include <atomic>
 #include <cmath>
 
 using namespace ah;
@@ -52,6 +54,9 @@ __device__ __forceinline__ float4 ldq(const float *p, int j) { return reinterpre
 __device__ __forceinline__ float dot4(float4 a, float4 b, float s) {
   return __builtin_fmaf(a.w, b.w, __builtin_fmaf(a.z, b.z, __builtin_fmaf(a.y, b.y, __builtin_fmaf(a.x, b.x, s))));
 }
+
+// what sums about the maximum m count for beside those about `most`; -inf: no key
+__device__ __forceinline__ float slice_weight(float m, float most) { return m == -INFINITY ? 0.f : expf(m - most); }
 
 enum { NORM = 0, JOIN = 1 };
 // A wave computes R neighbouring results (DUAL: R of the gate and R of the up matrix).  NV: float4 per lane of a row, K <= 256 NV.
@@ -235,13 +240,12 @@ __global__ __launch_bounds__(256) void k_decode_attention(DecodeAttention a) {
       }
     }
   }
-  // the groups of a wave, then the waves; -inf is a group without a key
-  auto weight = [](float m, float most) { return m == -INFINITY ? 0.f : expf(m - most); };
+  // the groups of a wave, then the waves
 #pragma unroll
   for (int d = G; d < 64; d <<= 1) {
     const float om = __shfl_xor(m, d, 64), ol = __shfl_xor(l, d, 64);
     const float4 oo = make_float4(__shfl_xor(o.x, d, 64), __shfl_xor(o.y, d, 64), __shfl_xor(o.z, d, 64), __shfl_xor(o.w, d, 64));
-    const float most = fmaxf(m, om), c = weight(m, most), e = weight(om, most);
+    const float most = fmaxf(m, om), c = slice_weight(m, most), e = slice_weight(om, most);
     l = l * c + ol * e;
     o = make_float4(o.x * c + oo.x * e, o.y * c + oo.y * e, o.z * c + oo.z * e, o.w * c + oo.w * e);
     m = most;
@@ -254,7 +258,7 @@ __global__ __launch_bounds__(256) void k_decode_attention(DecodeAttention a) {
   const float most = fmaxf(fmaxf(all_m[0], all_m[1]), fmaxf(all_m[2], all_m[3]));
   float c[4], sum = 0.f;
 #pragma unroll
-  for (int w = 0; w < 4; w++) { c[w] = weight(all_m[w], most); sum = __builtin_fmaf(c[w], all_l[w], sum); }
+  for (int w = 0; w < 4; w++) { c[w] = slice_weight(all_m[w], most); sum = __builtin_fmaf(c[w], all_l[w], sum); }
   for (int d = threadIdx.x; d < a.head_size; d += 256) {
     float v = 0.f;
 #pragma unroll
@@ -262,6 +266,489 @@ __global__ __launch_bounds__(256) void k_decode_attention(DecodeAttention a) {
     a.sums[(int64_t)blockIdx.x * a.width + h * a.head_size + d] = v;
   }
   if (threadIdx.x == 0) a.top[blockIdx.x * gridDim.y + h] = make_float2(most, sum);
+}
+
+// ================================================================ a token in one launch
+// The five launches of a layer cost 3 to 6 us each and 1 us between them, whatever they compute.  k_decode_chain runs all of them, and the head,
+// as phases of one launch of at most a workgroup to a CU: what a phase hands to the next is written as 64-bit words of a value and a tag, and
+// who needs it reads the words until they bear the tag of this layer of this launch.  A word is written and read whole (relaxed atomics of
+// device scope), so the tag says that the value beside it is the new one: no flag, no fence, no barrier over the grid, one trip
+// through memory from a phase to the next.
+//   waves 4 .. 7 wait for the words of the next phase, normalise or join them and leave them in LDS;
+//   waves 0 .. 3 meanwhile have the rows of the next matrices (and the keys and values of this workgroup's slice) on their way into registers:
+//   the two are different waves because a wave's loads come back in order.
+// A buffer is written again a layer later.  Whoever writes it then has read all results of the phase before, which stand on those of all
+// phases since the earlier use, and those were computed after their inputs had been read: nobody reads the old words any more.
+// All workgroups have to be on the chip at once, which the grid's size allows but nothing guarantees while other processes use the GPU.
+// So every wait ends: after SPIN_TICKS, or as soon as another workgroup has given up, a workgroup leaves `chain_gave_up` and ends, and the launch
+// behind it, of one workgroup that depends on no other, computes the token again (and otherwise ends at once).
+// What bounds it is that chain of trips, 1.3 us at least and 2 to 3 as polled, five a layer, and between them the one wave that has the next step
+// (350 instructions in a row are 1 us).  A token, its logits read and chosen from, 64 of them behind a prompt of 17 (with the prompt's pass and the pass
+// over the result): 6 layers x 256 186 -> 142 us, 4 x 128 112 -> 99, 2 x 64 87 -> 73; 24 behind 200: 8 x 384 327 -> 298, 8 x 512 365 -> 316.  The
+// kernel alone: 6 x 256 96 us, 16 a layer, against 23 in launches.  All rows ahead have to be asked for unconditionally: behind branches the
+// compiler waits for the newest of them before the oldest (attention 2.3 -> 1.9 us).
+constexpr int CHAIN_LAYERS = 32, CHAIN_NV = 2, CHAIN_UNITS = 4;      // at most: layers; 1024 wide, ffn 4096; keys a lane holds
+constexpr int64_t SPIN_TICKS = 5000000;                              // of 10 ns
+enum { WORD_QKV = 0, WORD_SUMS = 3072, WORD_TOPS = WORD_SUMS + MAX_SLICES * 1024, WORD_MID = WORD_TOPS + MAX_SLICES * 128 * 2,
+       WORD_HID = WORD_MID + 1024, WORD_STREAM = WORD_HID + 4096, WORDS = WORD_STREAM + 1024 };
+__device__ uint64_t chain_words[WORDS];
+__device__ uint32_t chain_gave_up;              // the first tag of the launch that did
+
+struct DecodeChain {
+  AhDecodeLayer layer[CHAIN_LAYERS];
+  ah_ptr lnf_w, lnf_b;
+  const float *tok, *pos, *head;
+  float *kv, *logits;
+  int vocab, width, heads, head_size, ffn, layers, mask, n, slices, slice, lanes;      // lanes: of a head's features, four each, a power of two
+  int64_t layer_stride;                         // of kv
+  int64_t ticks;                                // a wait's end
+  float scale, cap, eps;
+  uint32_t tag;                                 // layer i's words bear tag + i
+  uint32_t rescue;                              // 0, or the first tag of the launch that this one computes again if it gave up
+};
+static_assert(sizeof(DecodeChain) <= 4096, "kernel arguments");
+
+__device__ __forceinline__ void put(int at, uint32_t tag, float v) {
+  __hip_atomic_store(chain_words + at, (uint64_t)tag << 32 | __float_as_uint(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint64_t peek(int at) { return __hip_atomic_load(chain_words + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+// The words index(i), i < N, once all of them (of all lanes) bear the tag; false: given up
+template <int N, class Index>
+__device__ __forceinline__ bool take(uint32_t tag, uint32_t launch, int64_t ticks, Index index, float (&v)[N]) {
+  int64_t since = 0;
+  for (int tries = 1;; tries++) {
+    uint64_t w[N];
+#pragma unroll
+    for (int i = 0; i < N; i++) w[i] = peek(index(i));
+    uint32_t other = 0;
+#pragma unroll
+    for (int i = 0; i < N; i++) { other |= (uint32_t)(w[i] >> 32) ^ tag; v[i] = __uint_as_float((uint32_t)w[i]); }
+    if (__all(other == 0)) return true;
+    if ((tries & 63) == 0 || ticks < 0) {
+      const int64_t now = wall_clock64();
+      if (since == 0) since = now;
+      if (now - since > ticks || __hip_atomic_load(&chain_gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == launch) {
+        __hip_atomic_store(&chain_gave_up, launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return false;
+      }
+    }
+  }
+}
+
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float lane_moved(float v) {
+  return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), CTRL, ROWS, 0xf, false));
+}
+// the sum over the lanes of a group of g (a power of two up to 64), in each of them: neighbours, pairs, halves and rows of 16, then by exchange
+__device__ __forceinline__ float group_sum(float v, int g) {
+  if (g >= 2) v += lane_moved<0xB1, 0xf>(v);
+  if (g >= 4) v += lane_moved<0x4E, 0xf>(v);
+  if (g >= 8) v += lane_moved<0x141, 0xf>(v);
+  if (g >= 16) v += lane_moved<0x140, 0xf>(v);
+  if (g >= 32) v += __shfl_xor(v, 16, 64);
+  if (g >= 64) v += __shfl_xor(v, 32, 64);
+  return v;
+}
+// the largest of the wave
+__device__ __forceinline__ float wave_most(float v) {
+  v = fmaxf(v, lane_moved<0xB1, 0xf>(v));
+  v = fmaxf(v, lane_moved<0x4E, 0xf>(v));
+  v = fmaxf(v, lane_moved<0x141, 0xf>(v));
+  v = fmaxf(v, lane_moved<0x140, 0xf>(v));
+  v = fmaxf(v, __shfl_xor(v, 16, 64));
+  return fmaxf(v, __shfl_xor(v, 32, 64));
+}
+// over the wave; row sums go to the next row and to the upper half, so the last lane has all
+__device__ __forceinline__ float wave_total(float v) {
+  v = group_sum(v, 16);
+  v += lane_moved<0x142, 0xa>(v);
+  v += lane_moved<0x143, 0xc>(v);
+  return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), 63));
+}
+
+template <int NV, bool DUAL>
+__global__ __launch_bounds__(512, 2) void k_decode_chain(DecodeChain a) {
+  constexpr int PAIRS = DUAL ? (NV + 1) / 2 : 0, RA = DUAL ? 2 * PAIRS : NV, NF = 4 * NV, U = CHAIN_UNITS, E = 4 * NV;
+  __shared__ __attribute__((aligned(16))) float xn[256 * NV], joined[256 * NV], hid[1024 * NV];
+  __shared__ float stream[256 * NV], mid[256 * NV];
+  __shared__ __attribute__((aligned(16))) float fresh[3][128];         // the new row's q, k, v of a head
+  __shared__ __attribute__((aligned(16))) float part_o[4][128];
+  __shared__ float part_m[4], part_l[4], tops[MAX_SLICES * 128 * 2];
+  __shared__ int quit;
+  if (a.rescue && __hip_atomic_load(&chain_gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != a.rescue) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, C = a.width, F = a.ffn, nv = C >> 2, nf = F >> 2;
+  const int G = gridDim.x, W = 4 * G, gw = blockIdx.x * 4 + wave;      // row gw + r W of a matrix is this wave's
+  const int units = a.slices * a.heads;
+  const bool in_c = blockIdx.x * 4 < (unsigned)C, in_qkv = blockIdx.x * 4 < (unsigned)(3 * C), in_f = blockIdx.x * 4 < (unsigned)F;
+  if (threadIdx.x == 0) quit = 0;
+  __syncthreads();
+
+  auto at = [](ah_ptr p) { return reinterpret_cast<const float *>(static_cast<uintptr_t>(p)); };
+  // The two kinds of waves run loops of their own, so that neither's registers are kept through the other's code; both come to the same barriers.
+  if (wave >= 4) {
+    const int ct = threadIdx.x - 256;
+    float gain[E], bias[E];
+    auto load_norm = [&](ah_ptr g, ah_ptr b) {
+#pragma unroll
+      for (int i = 0; i < E; i++) { const int k = lane + 64 * i; gain[i] = k < C ? at(g)[k] : 0.f; bias[i] = k < C ? at(b)[k] : 0.f; }
+    };
+    // x: elements lane + 64 i of the row, which `raw` takes as they are and xn normalised, in two passes over the registers
+    auto norm = [&](const float (&x)[E], float *raw) {
+      float s = 0.f, q = 0.f;
+#pragma unroll
+      for (int i = 0; i < E; i++) s += lane + 64 * i < C ? x[i] : 0.f;
+      const float inv = 1.0f / (float)C, mean = wave_total(s) * inv;
+#pragma unroll
+      for (int i = 0; i < E; i++) { const float c = x[i] - mean; q += lane + 64 * i < C ? c * c : 0.f; }
+      const float rstd = 1.0f / sqrtf(wave_total(q) * inv + a.eps);
+#pragma unroll
+      for (int i = 0; i < E; i++) {
+        const int k = lane + 64 * i;
+        if (k < C) { raw[k] = x[i]; xn[k] = (x[i] - mean) * rstd * gain[i] + bias[i]; }
+      }
+    };
+    auto take_row = [&](int words, uint32_t tag, float (&x)[E]) {
+      if (!take<E>(tag, a.tag, a.ticks, [&](int i) { return words + min(lane + 64 * i, C - 1); }, x)) quit = 1;
+    };
+    int head2[NV];
+#pragma unroll
+    for (int i = 0; i < NV; i++) head2[i] = min(ct + 256 * i, C - 1) / a.head_size * 2;
+    if (wave == 4) load_norm(a.layer[0].ln1_w, a.layer[0].ln1_b);
+#pragma unroll 1
+    for (int l = 0; l < a.layers; l++) {
+      const uint32_t tag = a.tag + l;
+      if (in_qkv) {
+        if (wave == 4) {
+          float x[E];
+          if (!in_f && !in_c) load_norm(a.layer[l].ln1_w, a.layer[l].ln1_b);
+          if (l == 0) {
+#pragma unroll
+            for (int i = 0; i < E; i++) { const int k = lane + 64 * i; x[i] = k < C ? a.tok[k] + a.pos[k] : 0.f; }
+          } else {
+            take_row(WORD_STREAM, tag - 1, x);
+          }
+          norm(x, stream);
+          load_norm(a.layer[l].ln2_w, a.layer[l].ln2_b);
+        }
+        __syncthreads();
+        if (quit) return;
+      }
+      for (int unit = blockIdx.x; unit < units; unit += G) {
+        if (ct < 128) {
+          float x[3];
+          const int from = WORD_QKV + unit % a.heads * a.head_size + min(ct, a.head_size - 1);
+          if (!take<3>(tag, a.tag, a.ticks, [&](int i) { return from + i * C; }, x)) quit = 1;
+#pragma unroll
+          for (int i = 0; i < 3; i++) fresh[i][ct] = x[i];
+        }
+        __syncthreads();
+        if (quit) return;
+        __syncthreads();
+      }
+      if (in_c) {
+        // the slices' maxima and sums go through LDS; then the slices are joined, S at a time
+        constexpr int S = 4;
+        const int ntops = units * 2;
+        float x[NV * S + 1];
+        auto sums = [&](int s0, int e) { return WORD_SUMS + min(s0 + e % S, a.slices - 1) * C + min(ct + 256 * (e / S), C - 1); };
+        if (!take<NV * S + 1>(tag, a.tag, a.ticks, [&](int e) { return e == 0 ? WORD_TOPS + min(ct, ntops - 1) : sums(0, e - 1); }, x)) quit = 1;
+        if (ct < ntops) tops[ct] = x[0];
+        for (int t = ct + 256; t - ct < ntops; t += 256) {
+          float y[1];
+          if (!take<1>(tag, a.tag, a.ticks, [&](int) { return WORD_TOPS + min(t, ntops - 1); }, y)) quit = 1;
+          if (t < ntops) tops[t] = y[0];
+        }
+        __syncthreads();
+        if (quit) return;
+        float most[NV], sum[NV], v[NV];
+#pragma unroll
+        for (int i = 0; i < NV; i++) { most[i] = -INFINITY; sum[i] = v[i] = 0.f; }
+        for (int s0 = 0; s0 < a.slices; s0 += S) {
+          float y[NV * S];
+          if (s0 > 0 && !take<NV * S>(tag, a.tag, a.ticks, [&](int e) { return sums(s0, e); }, y)) { quit = 1; break; }
+#pragma unroll
+          for (int i = 0; i < NV; i++) {
+            const float *top = tops + head2[i];
+            float now = most[i];
+#pragma unroll
+            for (int s = 0; s < S; s++) if (s0 + s < a.slices) now = fmaxf(now, top[(s0 + s) * a.heads * 2]);
+            const float old = slice_weight(most[i], now);
+            sum[i] *= old;
+            v[i] *= old;
+            most[i] = now;
+#pragma unroll
+            for (int s = 0; s < S; s++)
+              if (s0 + s < a.slices) {
+                const float *t = top + (s0 + s) * a.heads * 2, c = slice_weight(t[0], now);
+                sum[i] = __builtin_fmaf(c, t[1], sum[i]);
+                v[i] = __builtin_fmaf(c, s0 == 0 ? x[i * S + s + 1] : y[i * S + s], v[i]);
+              }
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < NV; i++) if (ct + 256 * i < C) joined[ct + 256 * i] = v[i] / sum[i];
+        __syncthreads();
+        if (quit) return;
+      }
+      if (in_f || in_c) {
+        if (wave == 4) {
+          float x[E];
+          if (!in_qkv) load_norm(a.layer[l].ln2_w, a.layer[l].ln2_b);
+          take_row(WORD_MID, tag, x);
+          norm(x, mid);
+          const bool last = l + 1 == a.layers;
+          load_norm(last ? a.lnf_w : a.layer[l + 1].ln1_w, last ? a.lnf_b : a.layer[l + 1].ln1_b);
+        }
+        __syncthreads();
+        if (quit) return;
+      }
+      if (in_c) {
+        float x[E];
+        if (!take<E>(tag, a.tag, a.ticks, [&](int i) { return WORD_HID + min(ct + 256 * i, F - 1); }, x)) quit = 1;
+#pragma unroll
+        for (int i = 0; i < E; i++) if (ct + 256 * i < F) hid[ct + 256 * i] = x[i];
+        __syncthreads();
+        if (quit) return;
+      }
+    }
+    if (wave == 4) {
+      float x[E];
+      if (!in_f && !in_c) load_norm(a.lnf_w, a.lnf_b);
+      take_row(WORD_STREAM, a.tag + a.layers - 1, x);
+      norm(x, stream);
+    }
+    __syncthreads();
+    return;
+  }
+
+  float4 wa[RA][NV], wo[NV], w2[NF], kk[U], vv[U];
+  auto row_of = [&](float4 (&w)[NV], const float *m, int n, int N) {
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+      w[i] = ldq(m + (int64_t)min(n, N - 1) * C, min(lane + 64 * i, nv - 1));
+    }
+  };
+  auto long_row = [&](const float *m, int n) {
+#pragma unroll
+    for (int i = 0; i < NF; i++) {
+      w2[i] = ldq(m + (int64_t)min(n, C - 1) * F, min(lane + 64 * i, nf - 1));
+    }
+  };
+  auto get = [&](const float *s, float4 (&x)[NV]) {
+#pragma unroll
+    for (int i = 0; i < NV; i++) x[i] = ldq(s, min(lane + 64 * i, nv - 1));
+  };
+  auto dot_row = [&](const float4 (&w)[NV], const float4 (&x)[NV]) {
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; i++) s = lane + 64 * i < nv ? dot4(w[i], x[i], s) : s;
+    return wave_total(s);
+  };
+  // this thread's place in a slice of keys: features 4 f .. of every KEYS-th key
+  const int f = threadIdx.x & (a.lanes - 1), keys = 256 / a.lanes, key = threadIdx.x / a.lanes;
+  const bool has_f = 4 * f < a.head_size;
+  const int64_t pitch = 3 * (int64_t)C;
+  auto load_keys = [&](int l, int unit, int j0) {                      // of keys j0 + key + u KEYS of the unit's slice; the newest comes through `fresh`
+    const int h = unit % a.heads, begin = unit / a.heads * a.slice, count = min(a.slice, a.n - begin);
+    const float *p = a.kv + l * a.layer_stride + C + h * a.head_size + 4 * (has_f ? f : 0);
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const float *row = p + (int64_t)max(0, min(begin + min(j0 + u * keys + key, count - 1), a.n - 2)) * pitch;
+      kk[u] = ldq(row, 0);
+      vv[u] = ldq(row + C, 0);
+    }
+  };
+#pragma unroll
+  for (int r = 0; r < RA; r++) row_of(wa[r], at(a.layer[0].wqkv), gw + r * W, 3 * C);
+  load_keys(0, min((int)blockIdx.x, units - 1), 0);
+  row_of(wo, at(a.layer[0].wo), gw, C);
+#pragma unroll 1
+  for (int l = 0; l < a.layers; l++) {
+    const AhDecodeLayer &w = a.layer[l];
+    const uint32_t tag = a.tag + l;
+    // ---- LayerNorm, q, k, v
+    if (in_qkv) {
+      __syncthreads();
+      if (quit) return;
+      float4 x[NV];
+      get(xn, x);
+      float *row = a.kv + l * a.layer_stride + (a.n - 1) * pitch;
+      auto leave = [&](int n, float s) {
+        if (lane == 0) { put(WORD_QKV + n, tag, s); row[n] = s; }
+      };
+#pragma unroll
+      for (int r = 0; r < RA; r++) {
+        const int n = gw + r * W;
+        if (n < 3 * C) leave(n, dot_row(wa[r], x));
+      }
+      for (int n = gw + RA * W; n < 3 * C; n += W) {
+        row_of(wa[0], at(w.wqkv), n, 3 * C);
+        leave(n, dot_row(wa[0], x));
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < RA; r++) row_of(wa[r], at(DUAL && r >= PAIRS ? w.up : w.fc1), gw + (DUAL ? r % (PAIRS ? PAIRS : 1) : r) * W, F);
+    // ---- the newest query against the keys of a slice, for one head
+    for (int unit = blockIdx.x; unit < units; unit += G) {
+      const int h = unit % a.heads, slice = unit / a.heads, begin = slice * a.slice, count = min(a.slice, a.n - begin);
+      __syncthreads();
+      if (quit) return;
+      const float4 none = make_float4(0.f, 0.f, 0.f, 0.f), q = has_f ? ldq(fresh[0], f) : none;
+      float m = -INFINITY, sum = 0.f;
+      float4 o = none;
+      for (int j0 = 0; j0 < count; j0 += U * keys) {
+        if (j0 > 0 || unit != (int)blockIdx.x) load_keys(l, unit, j0);
+        // the group's U scores, one of them to a lane for what tanh and exp take
+        float mine = 0.f;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const int j = j0 + u * keys + key;
+          if (begin + j == a.n - 1) { kk[u] = ldq(fresh[1], has_f ? f : 0); vv[u] = ldq(fresh[2], has_f ? f : 0); }
+          const float s = group_sum(has_f ? dot4(q, kk[u], 0.f) : 0.f, a.lanes);
+          mine = (f & (U - 1)) == u ? s : mine;
+        }
+        mine *= a.scale;
+        if (a.cap > 0.f) mine = a.cap * tanhf(mine / a.cap);
+        if (j0 + (f & (U - 1)) * keys + key >= count) mine = -INFINITY;
+        const float most = fmaxf(m, wave_most(mine)), old = slice_weight(m, most), p = (f & ~(U - 1)) == 0 ? slice_weight(mine, most) : 0.f;
+        sum = __builtin_fmaf(sum, old, wave_total(p));
+        o.x *= old; o.y *= old; o.z *= old; o.w *= old;
+        m = most;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const float pu = __shfl(p, (lane & ~(a.lanes - 1)) + u, 64);
+          o.x = __builtin_fmaf(pu, vv[u].x, o.x); o.y = __builtin_fmaf(pu, vv[u].y, o.y);
+          o.z = __builtin_fmaf(pu, vv[u].z, o.z); o.w = __builtin_fmaf(pu, vv[u].w, o.w);
+        }
+      }
+      for (int d = a.lanes; d < 64; d <<= 1) {
+        o.x += __shfl_xor(o.x, d, 64); o.y += __shfl_xor(o.y, d, 64);
+        o.z += __shfl_xor(o.z, d, 64); o.w += __shfl_xor(o.w, d, 64);
+      }
+      if (lane < a.lanes && has_f) reinterpret_cast<float4 *>(part_o[wave])[lane] = o;
+      if (lane == 0) { part_m[wave] = m; part_l[wave] = sum; }
+      __syncthreads();
+      const float most = fmaxf(fmaxf(part_m[0], part_m[1]), fmaxf(part_m[2], part_m[3]));
+      float c[4];
+      sum = 0.f;
+#pragma unroll
+      for (int v = 0; v < 4; v++) { c[v] = slice_weight(part_m[v], most); sum = __builtin_fmaf(c[v], part_l[v], sum); }
+      if ((int)threadIdx.x < a.head_size) {
+        float v = 0.f;
+#pragma unroll
+        for (int u = 0; u < 4; u++) v = __builtin_fmaf(c[u], part_o[u][threadIdx.x], v);
+        put(WORD_SUMS + slice * C + h * a.head_size + threadIdx.x, tag, v);
+      }
+      if (threadIdx.x == 0) {
+        put(WORD_TOPS + (slice * a.heads + h) * 2, tag, most);
+        put(WORD_TOPS + (slice * a.heads + h) * 2 + 1, tag, sum);
+      }
+    }
+    // ---- the slices joined, wo, the residual stream
+    if (in_c) {
+      __syncthreads();
+      if (quit) return;
+      __syncthreads();
+      if (quit) return;
+      float4 x[NV];
+      get(joined, x);
+      for (int n = gw; n < C; n += W) {
+        if (n != gw) row_of(wo, at(w.wo), n, C);
+        const float s = dot_row(wo, x);
+        if (lane == 0) put(WORD_MID + n, tag, stream[n] + s);
+      }
+    }
+    long_row(at(w.fc2), gw);
+    // ---- LayerNorm, fc1 and its activation
+    if (in_f || in_c) {
+      __syncthreads();
+      if (quit) return;
+    }
+    if (in_f) {
+      float4 x[NV];
+      get(xn, x);
+      if constexpr (DUAL) {
+        auto leave = [&](int n, float s, float t) {
+          if (lane == 0) put(WORD_HID + n, tag, silu(s) * t);
+        };
+#pragma unroll
+        for (int r = 0; r < PAIRS; r++) {
+          const int n = gw + r * W;
+          if (n < F) leave(n, dot_row(wa[r], x), dot_row(wa[PAIRS + r], x));
+        }
+        for (int n = gw + PAIRS * W; n < F; n += W) {
+          row_of(wa[0], at(w.fc1), n, F);
+          row_of(wa[1], at(w.up), n, F);
+          leave(n, dot_row(wa[0], x), dot_row(wa[1], x));
+        }
+      } else {
+        // a lane for each of the wave's rows: the activation is computed once
+        float mine = 0.f;
+#pragma unroll
+        for (int r = 0; r < RA; r++)
+          if (gw + r * W < F) {
+            const float s = dot_row(wa[r], x);
+            mine = lane == r ? s : mine;
+          }
+        DecodeRows c;
+        c.mask = a.mask;
+#pragma unroll
+        for (int k = 0; k < 5; k++) c.coef[k] = at(w.coef[k]);
+        const int n = gw + lane * W;
+        if (lane < RA && n < F) put(WORD_HID + n, tag, activate(c, n, mine));
+        for (int n = gw + RA * W; n < F; n += W) {
+          row_of(wa[0], at(w.fc1), n, F);
+          const float s = dot_row(wa[0], x);
+          if (lane == 0) put(WORD_HID + n, tag, activate(c, n, s));
+        }
+      }
+    }
+    // of the next layer, or the first rows of the head
+    const bool last = l + 1 == a.layers;
+    const float *next = last ? a.head : at(a.layer[l + 1].wqkv);
+    const int N = last ? a.vocab : 3 * C;
+#pragma unroll
+    for (int r = 0; r < RA; r++) row_of(wa[r], next, gw + r * W, N);
+    // ---- fc2, the residual stream
+    if (in_c) {
+      __syncthreads();
+      if (quit) return;
+      for (int n = gw; n < C; n += W) {
+        if (n != gw) long_row(at(w.fc2), n);
+        float s[2] = {0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < NF; i++) {
+          const int j = lane + 64 * i;
+          s[i & 1] = j < nf ? dot4(w2[i], ldq(hid, min(j, nf - 1)), s[i & 1]) : s[i & 1];
+        }
+        const float t = wave_total(s[0] + s[1]);
+        if (lane == 0) put(WORD_STREAM + n, tag, mid[n] + t);
+      }
+    }
+    const int after = last ? l : l + 1;
+    if ((int)blockIdx.x < units) load_keys(after, blockIdx.x, 0);
+    row_of(wo, at(a.layer[after].wo), gw, C);
+  }
+  // ---- the head
+  __syncthreads();
+  if (quit) return;
+  float4 x[NV];
+  get(xn, x);
+  for (int n = gw; n < a.vocab; n += RA * W) {
+    float4 next[RA][NV];
+#pragma unroll
+    for (int r = 0; r < RA; r++) row_of(next[r], a.head, n + (RA + r) * W, a.vocab);
+#pragma unroll
+    for (int r = 0; r < RA; r++) {
+      const float s = dot_row(wa[r], x);
+      if (lane == 0 && n + r * W < a.vocab) a.logits[n + r * W] = s;
+#pragma unroll
+      for (int i = 0; i < NV; i++) wa[r][i] = next[r][i];
+    }
+  }
+}
+__global__ __launch_bounds__(256) void k_chain_clear() {
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < WORDS; i += gridDim.x * 256) chain_words[i] = 0;
 }
 
 // More results to a wave where that leaves the chip its 1000 waves or so: the row is read and normalised once for them.
@@ -313,9 +800,66 @@ DecodeRows rows_of(const AhDecode *d, ah_ptr gain, ah_ptr bias, ah_ptr w, int n)
   return a;
 }
 
+
+// Where the token runs in one launch: up to 512 wide (ffn 2048), and with the layers that fit the kernel's arguments.  Wider, every phase's words
+// are asked for by every workgroup at 3 to 24 KB a time, their trips through memory take 5 to 7 us instead of 2 to 3, and the rows ahead no longer
+// fit the registers: 768 wide in 12 layers 430 us a token against 400 in launches.  Not inside a captured graph or a step plan, whose replays would bring the same tags again, nor on the side stream, where the launches of a layer are refused too.
+int chain_quads(const AhDecode *d) {
+  if (d->layers > CHAIN_LAYERS || ah::step_active() || ah::capturing() || ah::on_side()) return 0;
+  const int64_t nv = cdiv(d->width, 256) > cdiv(d->ffn, 1024) ? cdiv(d->width, 256) : cdiv(d->ffn, 1024);
+  return nv <= CHAIN_NV ? (int)nv : 0;
+}
+thread_local int64_t next_ticks = SPIN_TICKS;
+int32_t launch_chain(const AhDecode *d, const AhDecodeLayer *layers, int32_t token, int32_t pos, int nv) {
+  static std::atomic<uint32_t> tags{1};
+  const int C = d->width, H = d->heads, hs = C / H, n = pos + 1;
+  const uint32_t used = 2 * (uint32_t)d->layers;
+  uint32_t tag = tags.fetch_add(used);
+  if (tag > 0xf0000000u) {                      // once in 4e9 layers: no word may bear a tag that comes again
+    ah::launch_kernel(k_chain_clear, dim3(64), dim3(256), 0);
+    tags.store(1 + used);
+    tag = 1;
+  }
+  DecodeChain a = {};
+  for (int i = 0; i < d->layers; i++) a.layer[i] = layers[i];
+  a.lnf_w = d->lnf_w; a.lnf_b = d->lnf_b;
+  a.tok = dp<const float>(d->wte) + (int64_t)token * C; a.pos = dp<const float>(d->wpe) + (int64_t)pos * C;
+  a.head = dp<const float>(d->head); a.kv = dp<float>(d->kv); a.logits = dp<float>(d->logits);
+  a.vocab = d->vocab; a.width = C; a.heads = H; a.head_size = hs; a.ffn = d->ffn; a.layers = d->layers;
+  const bool gated = (d->act & AH_DECODE_GATED) != 0;
+  a.mask = gated ? 0 : d->act;
+  a.n = n; a.layer_stride = (int64_t)d->rows * 3 * C;
+  for (a.lanes = 8; 4 * a.lanes < hs;) a.lanes *= 2;
+  // a slice: what the lanes hold at a time, at most 128 keys; longer ones where there would be too many
+  const int most = 256 / a.lanes * CHAIN_UNITS, held = most < 128 ? most : 128;
+  a.slices = (int)(cdiv(n, held) < MAX_SLICES ? cdiv(n, held) : MAX_SLICES);
+  a.slice = (int)cdiv(n, a.slices);
+  a.slices = (int)cdiv(n, a.slice);
+  a.scale = d->scale; a.cap = d->cap; a.eps = d->eps;
+  const int rows = std::max(std::max(3 * C, d->ffn), std::max(d->vocab, 4 * a.slices * H));
+  const unsigned grid = (unsigned)std::min<int64_t>(cdiv(rows, 4), ah::num_cus());
+  auto go = [&](auto kfn) {
+    a.tag = tag; a.rescue = 0; a.ticks = next_ticks;
+    ah::launch_kernel(kfn, dim3(grid), dim3(512), 0, a);
+    a.rescue = tag; a.tag = tag + (uint32_t)d->layers; a.ticks = next_ticks = SPIN_TICKS;
+    ah::launch_kernel(kfn, dim3(1), dim3(512), 0, a);
+  };
+  if (gated) { if (nv == 1) go(k_decode_chain<1, true>); else go(k_decode_chain<2, true>); }
+  else { if (nv == 1) go(k_decode_chain<1, false>); else go(k_decode_chain<2, false>); }
+  AH_LAUNCH_CHECK();
+  return AH_OK;
+}
+
 }  // namespace
 
 extern "C" {
+
+// For tests: when the waits of this thread's next token in one launch end (below 0: a word that is not there at once), so that the launch behind it
+// computes the token.
+int32_t ah_decode_next_ticks(int32_t ticks) {
+  next_ticks = ticks;
+  return AH_OK;
+}
 
 int32_t ah_decode_head(const AhDecode *d, ah_ptr row) {
   AH_REQUIRE_READY();
@@ -343,6 +887,7 @@ int32_t ah_decode(const AhDecode *d, const AhDecodeLayer *layers, int32_t token,
     AH_ARG(l.ln1_w && l.ln1_b && l.wqkv && l.wo && l.ln2_w && l.ln2_b && l.fc1 && l.fc2 && (!gated || l.up), "ah_decode: null weight in layer %d", i);
     AH_ARG(aligned16(l.ln1_w | l.ln1_b | l.wqkv | l.wo | l.ln2_w | l.ln2_b | l.fc1 | l.fc2 | l.up), "ah_decode: weights of layer %d must be 16-byte aligned", i);
   }
+  if (const int nv = chain_quads(d)) return launch_chain(d, layers, token, pos, nv);
   const int C = d->width, H = d->heads, n = pos + 1;
   const int slices = (int)(cdiv(n, MIN_SLICE) < MAX_SLICES ? cdiv(n, MIN_SLICE) : MAX_SLICES);
   // the residual stream, the MLP's hidden row, the slices' sums and their maxima; stream-ordered, so it may go back at once

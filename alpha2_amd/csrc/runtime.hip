@@ -326,6 +326,7 @@ void launch_raw(const void *func, dim3 grid, dim3 block, unsigned shmem, void **
 }
 
 bool step_active() { return g.step_mode != STEP_OFF; }
+bool capturing() { return g.capturing; }
 
 int32_t step_boundary(const char *what) {
   if (g.step_mode == STEP_OFF || g.step_mode == STEP_EAGER) return AH_OK;

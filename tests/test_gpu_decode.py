@@ -194,3 +194,44 @@ def test_the_same_tokens_with_and_without_kept_keys(B, monkeypatch, temperature,
         whole.append(1)
     got = sample.sampleTokens(cfg, params, B, SeededRng(7), prompt, config, B.releaseGpuTensor, move)
     assert len(whole) == 2 and got.size == 80 and np.array_equal(got, want)
+
+
+# in one launch: an MLP that has more rows than q, k, v, one that has fewer than the residual stream, a head with more rows than the grid has waves, the
+# widest model it takes (512, with rows of 2048), swiglu in pairs that fill no round, and one layer more than its arguments hold
+CHAIN_CASES = [
+    (5000, 40, 2, 64, 4, dict(ffnDim=2048)),
+    (33, 40, 1, 256, 4, dict(ffnDim=36)),
+    (260, 70, 2, 512, 4, dict()),
+    (260, 40, 1, 512, 64, dict(ffnActivation="swiglu")),
+    (64, 20, 33, 64, 2, dict()),
+]
+
+
+@pytest.mark.parametrize("vocab,ctx,layers,width,heads,more", CHAIN_CASES)
+def test_a_token_in_one_launch(B, vocab, ctx, layers, width, heads, more):
+    from alpha2_amd.decode import KeptContext
+    cfg, params = _model(B, vocab, ctx, layers, width, heads, **more)
+    tokens = np.random.RandomState(3).randint(0, vocab, ctx).astype(np.int32)
+    kept = KeptContext.of(cfg, params, B, ctx)
+    _compare(kept, cfg, params, B, tokens, range(1, ctx + 1), False)
+    kept.close()
+
+
+@pytest.mark.parametrize("width,heads,act", [(64, 2, "gelu"), (256, 8, "swiglu"), (512, 4, "kan_spline")])
+def test_a_launch_that_gave_up_is_computed_again(B, width, heads, act):
+    """Its waits end at the first word that is not there yet; the one workgroup behind it sums the same terms in the same order."""
+    from alpha2_amd.decode import KeptContext
+    cfg, params = _model(B, 70, 80, 2, width, heads, ffnActivation=act)
+    tokens = np.random.RandomState(6).randint(0, 70, 80).astype(np.int32)
+    kept = KeptContext.of(cfg, params, B, 80)
+    rows = []
+    for given_up in (False, True):
+        kept.known = 0
+        kept.lastRow(tokens[:60], B.releaseGpuTensor)
+        for n in range(61, 81):
+            if given_up and n % 3 == 0:
+                B.lib.ah_decode_next_ticks(-1)
+            rows.append(kept.lastRow(tokens[:n], B.releaseGpuTensor).copy())
+    for n, (a, b) in enumerate(zip(rows[:20], rows[20:])):
+        assert np.array_equal(a, b), n + 61
+    kept.close()
