@@ -291,14 +291,14 @@ __device__ void flash_fwd_exact(const FlashArgs &a, int bh, int q0, int end, boo
       s[e] = x;
       tmax = fmaxf(tmax, x);
     }
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+    tmax = max_lane<32>(tmax);
     float m_new = fmaxf(m, tmax);
     float m_use = m_new == -INFINITY ? 0.f : m_new;   // rows with nothing visible yet stay at zero weight
     float alpha = expf(m - m_use);
     float psum = 0.f;
 #pragma unroll
     for (int e = 0; e < 16; e++) { float p = expf(s[e] - m_use); s[e] = p; psum += p; }
-    psum += __shfl_xor(psum, 32, 64);
+    psum = add_lane<32>(psum);
     l = l * alpha + psum;
     m = m_new;
 #pragma unroll
@@ -347,7 +347,7 @@ __device__ __forceinline__ float tile_scores(f32x16 &s, const FlashArgs &a, floa
       top = fmaxf(top, s[e]);
     }
   }
-  return fmaxf(top, __shfl_xor(top, 32, 64)) * cap_mul(a);
+  return max_lane<32>(top) * cap_mul(a);
 }
 // Scores -> weights against the largest score so far, times 2^24; the column's sum of them, and what sums so far are multiplied by
 // (-infinity, a masked score or no score so far, weighs what -200 does: nothing)
@@ -358,7 +358,7 @@ __device__ __forceinline__ float tile_weights(f32x16 &s, float mul, float before
   float sum = 0.f;
 #pragma unroll
   for (int e = 0; e < 16; e++) { s[e] = exp_of<24>(fmaxf(__builtin_fmaf(s[e], mul, -use), -200.f)); sum += s[e]; }
-  return (sum + __shfl_xor(sum, 32, 64)) * 0x1p-24f;
+  return add_lane<32>(sum) * 0x1p-24f;
 }
 __device__ __forceinline__ float output_factor(float l) { return (l > 0.f ? 1.0f / l : 0.f) * SPLIT_DOWN; }
 
@@ -591,8 +591,7 @@ __global__ __launch_bounds__(256) void k_flash_delta_f32(FlashArgs a) {
     const float4 o = *reinterpret_cast<const float4 *>((const float *)a.o + at), g = *reinterpret_cast<const float4 *>((const float *)a.d_o + at);
     s = __builtin_fmaf(o.x, g.x, o.y * g.y) + __builtin_fmaf(o.z, g.z, o.w * g.w);
   }
-#pragma unroll
-  for (int i = 1; i < L; i <<= 1) s += __shfl_xor(s, i, 64);
+  s = near_sum<L>(s);
   if (row < total && d == 0) a.delta[row] = s;
 }
 

@@ -239,14 +239,14 @@ __device__ __forceinline__ void flash_fwd_bf16_body(const FlashArgs &a) {
           }
 #pragma unroll
           for (int e = 0; e < 16; e++) tmax = fmaxf(tmax, s[e]);
-          tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+          tmax = max_lane<32>(tmax);
           float m_new = fmaxf(m, tmax);
           float m_use = m_new == -INFINITY ? 0.f : m_new;
           float alpha = exp2_fast(m - m_use);
           float psum = 0.f;
 #pragma unroll
           for (int e = 0; e < 16; e++) { float p = exp2_fast(s[e] - m_use); s[e] = p; psum += p; }
-          psum += __shfl_xor(psum, 32, 64);
+          psum = add_lane<32>(psum);
           l = l * alpha + psum;
           m = m_new;
 #pragma unroll
@@ -275,7 +275,7 @@ __device__ __forceinline__ void flash_fwd_bf16_body(const FlashArgs &a) {
     }
     __syncthreads();
   }
-  if (CAPPED) { l += __shfl_xor(l, 32, 64); l_rnd = lacc[0]; } else l_rnd = l;
+  if (CAPPED) { l = add_lane<32>(l); l_rnd = lacc[0]; } else l_rnd = l;
   if (qi < a.T) {
     float inv_l = l_rnd > 0.f ? 1.0f / l_rnd : 0.f;
     store_rows<D, PAD>((uint16_t *)a.o + b * a.o_sb + h * a.o_sh + (int64_t)qi * a.o_st, o, inv_l, lane, a.hd);
@@ -343,7 +343,7 @@ __device__ __forceinline__ void flash_dq_bf16_body(const FlashArgs &a) {
     for (int ks = 0; ks < KS; ks++)
 #pragma unroll
       for (int i = 0; i < 8; i++) delta += (float)dof[ks][i] * (float)of[ks][i];
-    delta += __shfl_xor(delta, 32, 64);
+    delta = add_lane<32>(delta);
     if (live && lk == 0) a.delta[srow] = delta;
   }
   float krow = live ? ((CAPPED ? a.cap : 0.f) - a.lse[srow]) * LOG2E : 0.f;
@@ -633,8 +633,7 @@ __global__ __launch_bounds__(512, 1) void k_flash_bwd_fused_bf16(FlashArgs a, fl
       float dsum = 0.f;
 #pragma unroll
       for (int e = 0; e < 8; e++) dsum += (float)vd[e] * (float)vo[e];
-#pragma unroll
-      for (int o = 1; o < CPR; o <<= 1) dsum += __shfl_xor(dsum, o, 64);
+      dsum = near_sum<CPR>(dsum);
       if (c < TCH) {
         *reinterpret_cast<u32x4 *>(&Qs[buf][r * Geo<D>::PITCH + c8 * 8]) = rq[i];
         *reinterpret_cast<u32x4 *>(&dOs[buf][r * Geo<D>::PITCH + c8 * 8]) = rdo[i];

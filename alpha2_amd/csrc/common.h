@@ -87,21 +87,72 @@ template <> struct Io<uint16_t> {   // bf16 storage
   static __device__ __forceinline__ void  st(uint16_t *p, size_t i, float v) { p[i] = f32_to_bf16_bits(v); }
 };
 
-// wave64 butterfly reductions
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+// What lane ^ O holds; every lane of the wave takes part.  Rows of 16 and halves are exchanged by v_permlane16/32_swap, the rest is moved by DPP: a step
+// of a reduction is one or two vector instructions, where __shfl_xor is a trip through LDS (ds_bpermute, 100 cycles and more), and reductions
+// along a row are what a short row kernel waits for (same bits; the step of 2 layers x 128 at 2 x 64 tokens 294 -> 289 us, of 24 x 1024 at
+// 4 x 8 x 1024 96.4 -> 95.7 ms, 24 tokens sampled from 12 x 768 12.3 -> 11.9).
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_moved(uint32_t v) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true); }
+template <int O>
+__device__ __forceinline__ uint32_t lane_xor(uint32_t v) {
+  static_assert(O == 1 || O == 2 || O == 4 || O == 8 || O == 16 || O == 32, "one bit of the lane");
+  if constexpr (O == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);      // the lower halves, the upper halves
+    return threadIdx.x & 32 ? r[0] : r[1];
+  } else if constexpr (O == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);      // the even rows, the odd rows
+    return threadIdx.x & 16 ? r[0] : r[1];
+  } else if constexpr (O == 8) return dpp_moved<0x128>(v);                    // a row turned by eight
+  else if constexpr (O == 4) return dpp_moved<0x1b>(dpp_moved<0x141>(v));     // eight lanes mirrored, then each four of them
+  else if constexpr (O == 2) return dpp_moved<0x4e>(v);
+  else return dpp_moved<0xb1>(v);
+}
+template <int O>
+__device__ __forceinline__ float lane_xor(float v) { return __uint_as_float(lane_xor<O>(__float_as_uint(v))); }
+template <int O>
+__device__ __forceinline__ double lane_xor(double v) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  return __builtin_bit_cast(double, (uint64_t)lane_xor<O>((uint32_t)(u >> 32)) << 32 | lane_xor<O>((uint32_t)u));
+}
+// v and what lane ^ O holds, in an order that both lanes share: for sums and maxima, which do not ask which is whose
+template <int O>
+__device__ __forceinline__ float2 lane_pair(float v) {
+  if constexpr (O == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return make_float2(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  } else if constexpr (O == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return make_float2(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  } else return make_float2(v, lane_xor<O>(v));
+}
+template <int O> __device__ __forceinline__ float add_lane(float v) { const float2 p = lane_pair<O>(v); return p.x + p.y; }
+template <int O> __device__ __forceinline__ float max_lane(float v) { const float2 p = lane_pair<O>(v); return fmaxf(p.x, p.y); }
+
+// over G neighbours (a power of two), the near ones first
+template <int G>
+__device__ __forceinline__ float near_sum(float v) {
+  if constexpr (G > 1) v = add_lane<1>(v);
+  if constexpr (G > 2) v = add_lane<2>(v);
+  if constexpr (G > 4) v = add_lane<4>(v);
+  if constexpr (G > 8) v = add_lane<8>(v);
+  if constexpr (G > 16) v = add_lane<16>(v);
+  if constexpr (G > 32) v = add_lane<32>(v);
   return v;
 }
+// wave64 reductions, the far lanes first.  (In the step of 4 a row of 16 holds its eight sums twice, so turning it by four does.)
+__device__ __forceinline__ float wave_sum(float v) {
+  v = add_lane<8>(add_lane<16>(add_lane<32>(v)));
+  v += __uint_as_float(dpp_moved<0x124>(__float_as_uint(v)));
+  return add_lane<1>(add_lane<2>(v));
+}
 __device__ __forceinline__ double wave_sum_d(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  v += lane_xor<32>(v); v += lane_xor<16>(v); v += lane_xor<8>(v); v += lane_xor<4>(v); v += lane_xor<2>(v); v += lane_xor<1>(v);
   return v;
 }
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
+  v = max_lane<8>(max_lane<16>(max_lane<32>(v)));
+  v = fmaxf(v, __uint_as_float(dpp_moved<0x124>(__float_as_uint(v))));
+  return max_lane<1>(max_lane<2>(v));
 }
 
 // tanh-approximation GELU and its derivative (cpu_ref.ts:422-427; ops.ts:405-417) on the gate

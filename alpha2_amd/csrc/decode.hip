@@ -335,35 +335,12 @@ __device__ __forceinline__ bool take(uint32_t tag, uint32_t launch, int64_t tick
   }
 }
 
-template <int CTRL, int ROWS>
-__device__ __forceinline__ float lane_moved(float v) {
-  return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), CTRL, ROWS, 0xf, false));
-}
-// the sum over the lanes of a group of g (a power of two up to 64), in each of them: neighbours, pairs, halves and rows of 16, then by exchange
+// the sum over the lanes of a group of g (8 to 64), in each of them
 __device__ __forceinline__ float group_sum(float v, int g) {
-  if (g >= 2) v += lane_moved<0xB1, 0xf>(v);
-  if (g >= 4) v += lane_moved<0x4E, 0xf>(v);
-  if (g >= 8) v += lane_moved<0x141, 0xf>(v);
-  if (g >= 16) v += lane_moved<0x140, 0xf>(v);
-  if (g >= 32) v += __shfl_xor(v, 16, 64);
-  if (g >= 64) v += __shfl_xor(v, 32, 64);
-  return v;
-}
-// the largest of the wave
-__device__ __forceinline__ float wave_most(float v) {
-  v = fmaxf(v, lane_moved<0xB1, 0xf>(v));
-  v = fmaxf(v, lane_moved<0x4E, 0xf>(v));
-  v = fmaxf(v, lane_moved<0x141, 0xf>(v));
-  v = fmaxf(v, lane_moved<0x140, 0xf>(v));
-  v = fmaxf(v, __shfl_xor(v, 16, 64));
-  return fmaxf(v, __shfl_xor(v, 32, 64));
-}
-// over the wave; row sums go to the next row and to the upper half, so the last lane has all
-__device__ __forceinline__ float wave_total(float v) {
-  v = group_sum(v, 16);
-  v += lane_moved<0x142, 0xa>(v);
-  v += lane_moved<0x143, 0xc>(v);
-  return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), 63));
+  v = near_sum<8>(v);
+  if (g >= 16) v = add_lane<8>(v);
+  if (g >= 32) v = add_lane<16>(v);
+  return g >= 64 ? add_lane<32>(v) : v;
 }
 
 template <int NV, bool DUAL>
@@ -397,10 +374,10 @@ __global__ __launch_bounds__(512, 2) void k_decode_chain(DecodeChain a) {
       float s = 0.f, q = 0.f;
 #pragma unroll
       for (int i = 0; i < E; i++) s += lane + 64 * i < C ? x[i] : 0.f;
-      const float inv = 1.0f / (float)C, mean = wave_total(s) * inv;
+      const float inv = 1.0f / (float)C, mean = wave_sum(s) * inv;
 #pragma unroll
       for (int i = 0; i < E; i++) { const float c = x[i] - mean; q += lane + 64 * i < C ? c * c : 0.f; }
-      const float rstd = 1.0f / sqrtf(wave_total(q) * inv + a.eps);
+      const float rstd = 1.0f / sqrtf(wave_sum(q) * inv + a.eps);
 #pragma unroll
       for (int i = 0; i < E; i++) {
         const int k = lane + 64 * i;
@@ -542,7 +519,7 @@ __global__ __launch_bounds__(512, 2) void k_decode_chain(DecodeChain a) {
     float s = 0.f;
 #pragma unroll
     for (int i = 0; i < NV; i++) s = lane + 64 * i < nv ? dot4(w[i], x[i], s) : s;
-    return wave_total(s);
+    return wave_sum(s);
   };
   // this thread's place in a slice of keys: features 4 f .. of every KEYS-th key
   const int f = threadIdx.x & (a.lanes - 1), keys = 256 / a.lanes, key = threadIdx.x / a.lanes;
@@ -610,8 +587,8 @@ __global__ __launch_bounds__(512, 2) void k_decode_chain(DecodeChain a) {
         mine *= a.scale;
         if (a.cap > 0.f) mine = a.cap * tanhf(mine / a.cap);
         if (j0 + (f & (U - 1)) * keys + key >= count) mine = -INFINITY;
-        const float most = fmaxf(m, wave_most(mine)), old = slice_weight(m, most), p = (f & ~(U - 1)) == 0 ? slice_weight(mine, most) : 0.f;
-        sum = __builtin_fmaf(sum, old, wave_total(p));
+        const float most = fmaxf(m, wave_max(mine)), old = slice_weight(m, most), p = (f & ~(U - 1)) == 0 ? slice_weight(mine, most) : 0.f;
+        sum = __builtin_fmaf(sum, old, wave_sum(p));
         o.x *= old; o.y *= old; o.z *= old; o.w *= old;
         m = most;
 #pragma unroll
@@ -621,10 +598,10 @@ __global__ __launch_bounds__(512, 2) void k_decode_chain(DecodeChain a) {
           o.z = __builtin_fmaf(pu, vv[u].z, o.z); o.w = __builtin_fmaf(pu, vv[u].w, o.w);
         }
       }
-      for (int d = a.lanes; d < 64; d <<= 1) {
-        o.x += __shfl_xor(o.x, d, 64); o.y += __shfl_xor(o.y, d, 64);
-        o.z += __shfl_xor(o.z, d, 64); o.w += __shfl_xor(o.w, d, 64);
-      }
+      auto far = [&](auto step) { o.x = step(o.x); o.y = step(o.y); o.z = step(o.z); o.w = step(o.w); };
+      if (a.lanes < 16) far([](float v) { return add_lane<8>(v); });
+      if (a.lanes < 32) far([](float v) { return add_lane<16>(v); });
+      if (a.lanes < 64) far([](float v) { return add_lane<32>(v); });
       if (lane < a.lanes && has_f) reinterpret_cast<float4 *>(part_o[wave])[lane] = o;
       if (lane == 0) { part_m[wave] = m; part_l[wave] = sum; }
       __syncthreads();
@@ -721,7 +698,7 @@ __global__ __launch_bounds__(512, 2) void k_decode_chain(DecodeChain a) {
           const int j = lane + 64 * i;
           s[i & 1] = j < nf ? dot4(w2[i], ldq(hid, min(j, nf - 1)), s[i & 1]) : s[i & 1];
         }
-        const float t = wave_total(s[0] + s[1]);
+        const float t = wave_sum(s[0] + s[1]);
         if (lane == 0) put(WORD_STREAM + n, tag, mid[n] + t);
       }
     }

@@ -593,6 +593,11 @@ __device__ __forceinline__ void online_merge(float &m, float &s, float m2, float
   s = s * expf(m - nm) + s2 * expf(m2 - nm);
   m = nm;
 }
+__device__ __forceinline__ void wave_merge(float &m, float &s) {
+  online_merge(m, s, lane_xor<32>(m), lane_xor<32>(s)); online_merge(m, s, lane_xor<16>(m), lane_xor<16>(s));
+  online_merge(m, s, lane_xor<8>(m), lane_xor<8>(s)); online_merge(m, s, lane_xor<4>(m), lane_xor<4>(s));
+  online_merge(m, s, lane_xor<2>(m), lane_xor<2>(s)); online_merge(m, s, lane_xor<1>(m), lane_xor<1>(s));
+}
 // one block per row: single read of the row with an online (max, sum-exp) pair per thread
 template <class T>
 __global__ void k_ce_fwd(const T *__restrict__ logits, const int32_t *__restrict__ targets, float *__restrict__ row_loss,
@@ -622,8 +627,7 @@ __global__ void k_ce_fwd(const T *__restrict__ logits, const int32_t *__restrict
     float v = Io<T>::ld(p, j);
     if (v > m) { s = s * expf(m - v) + 1.0f; m = v; } else { s += expf(v - m); }
   }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) online_merge(m, s, __shfl_xor(m, off, 64), __shfl_xor(s, off, 64));
+  wave_merge(m, s);
   int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
   if (lane == 0) { shm[wv] = m; shs[wv] = s; }
   __syncthreads();
@@ -733,8 +737,7 @@ __global__ __launch_bounds__(CE_TPB) void k_ce_fwd_bwd(const uint16_t *__restric
       for (int i = 0; i < 8; i++) s += exp_minus(v[i], m);
     }
   }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) online_merge(m, s, __shfl_xor(m, off, 64), __shfl_xor(s, off, 64));
+  wave_merge(m, s);
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
   if (lane == 0) { shm[wv] = m; shs[wv] = s; }
   __syncthreads();

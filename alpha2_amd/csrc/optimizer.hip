@@ -172,14 +172,9 @@ __global__ void k_sgd(float *__restrict__ p, const float *__restrict__ g, uint64
   if (i < n) p[i] = (float)((double)p[i] - lr * ((double)g[i] * gs));
 }
 
-__device__ __forceinline__ double wave_sum_f64(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
 // block-wide sum (256 threads) of doubles; the result is valid in thread 0
 __device__ __forceinline__ double block_sum_f64(double v, double *sh) {
-  v = wave_sum_f64(v);
+  v = wave_sum_d(v);
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
   __syncthreads();
   double r = 0;
