@@ -116,6 +116,8 @@ SIGNATURES = {
     "ah_residual_dropout_add": [u64, u64, u64, u64, u64],
     "ah_dropout_mask": [u64, u64, i32, i32, C.c_double],
     "ah_dropout_apply": [u64, i32, u64, u64, i32, u64, u64, i32, C.c_double],
+    "ah_dropout_layernorm": [u64, u64, u64, u64, u64, u64, i64, i64, f32, u64, i64, i32, C.c_double],
+    "ah_layernorm_bwd_dropout": [u64, u64, u64, u64, u64, u64, u64, u64, i64, i64, f32, u64, i64, i32, C.c_double],
     "ah_masked_fill": [u64, u64, u64, u64, u64, f32], "ah_causal_mask": [u64, i64],
     "ah_cast": [u64, i32, u64, i32, u64], "ah_check_finite": [u64, u64, u64],
     "ah_transpose": [u64, u64, i32, p_i64, i32, i32],

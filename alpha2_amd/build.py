@@ -32,7 +32,7 @@ def _compile(name: str, force: bool) -> str:
     src = os.path.join(CSRC, name + ".hip")
     obj = os.path.join(OBJ, name + ".o")
     deps = [src, os.path.join(CSRC, "common.h"), os.path.join(CSRC, "gemm_common.h"), os.path.join(CSRC, "gemm_bf16_dma.inc"),
-            os.path.join(CSRC, "attention_common.h"), os.path.join(CSRC, "split_bf16.h"), os.path.join(HERE, "..", "include", "alpha_hip.h")]
+            os.path.join(CSRC, "attention_common.h"), os.path.join(CSRC, "split_bf16.h"), os.path.join(CSRC, "dropout.h"), os.path.join(HERE, "..", "include", "alpha_hip.h")]
     if not force and os.path.exists(obj) and all(os.path.getmtime(obj) >= os.path.getmtime(d) for d in deps):
         return obj
     cmd = [_hipcc()] + FLAGS + ["-c", src, "-o", obj]

@@ -9,8 +9,9 @@ Differences from the op-by-op path are layout and fusion only; the arithmetic is
     projection and writes merged heads (attention="heads"), or -- attention="reference-flash", the function gpt.ts:247-254
     computes on a backend with flashAttention -- the projection writes q, k, v as three [BT, C] matrices that are read as
     [B H, T, D] slabs, and its backward reads the three gradients where the attention kernel leaves them;
-  * dropout (reference-flash wiring only): the two residualDropoutAdd of a block become one pass each over the projection
-    with the mask made on the fly, and so do the two mask multiplies of their backward; the seed of a step's masks is read
+  * dropout (reference-flash wiring only): the two residualDropoutAdd of a block become one pass each over the projection, with the
+    mask made on the fly and the LayerNorm behind it in the same pass, and the two mask multiplies of their backward come out of the
+    LayerNorms' backward passes (an f32 stream keeps passes of their own); the seed of a step's masks is read
     from device memory, so the captured graph draws new masks at every replay;
   * every activation is bf16, by default the residual stream and the gradient flowing back along it too (stream="f32"
     keeps those two in f32: 3 % slower, losses equal to 1e-4 relative);
@@ -353,6 +354,28 @@ class FusedTrainer:
             check(self.lib.ah_dropout_apply(x + seg * n * 2, BF16, residual + seg * n * rs if residual else 0, out + seg * n * rs, out_dtype, n,
                                             self.seed_dev + 4 * (micro * self.per_pass + seg), counter, self.drop))
 
+    def _dropped_norm(self, residual: int, stream: int, name: str, out: int, micro: int, counter: int):
+        """stream = residual + the projection times its mask, out = the LayerNorm `name` of it: one pass where the stream is bf16."""
+        w, b = self.p(name + ".weight"), self.p(name + ".bias")
+        if self.SD == BF16:
+            check(self.lib.ah_dropout_layernorm(self.proj, residual, stream, w, b, out, self.BT, self.C, 1e-5, self.seed_dev + 4 * micro * self.per_pass,
+                                                self.BTm, counter, self.drop))
+            return
+        self._dropout(self.proj, residual, stream, self.SD, micro, counter)
+        check(self.lib.ah_layernorm(stream, w, b, out, self.BT, self.C, 1e-5, BF16, self.SD))
+
+    def _norm_bwd(self, name: str, x: int, residual_grad: int, dx: int, dx16: int, dropped: int = 0, micro: int = 0, counter: int = 0):
+        """The backward pass of the LayerNorm `name` over x, its gradient in dlnb.  dropped: also dx16 times the mask `counter`, the gradient of the
+        projection before it (in the same pass where the stream is bf16)."""
+        w, part = self.p(name + ".weight"), self._ln_part[name]
+        if dropped and self.SD == BF16:
+            check(self.lib.ah_layernorm_bwd_dropout(x, w, self.dlnb, residual_grad, dx, dx16, dropped, part, self.BT, self.C, 1e-5,
+                                                    self.seed_dev + 4 * micro * self.per_pass, self.BTm, counter, self.drop))
+            return
+        check(self.lib.ah_layernorm_bwd_deferred(x, w, self.dlnb, BF16, residual_grad, dx, dx16, part, self.BT, self.C, 1e-5, self.SD))
+        if dropped:
+            self._dropout(dx16, 0, dropped, BF16, micro, counter)
+
     def _flash(self, l: int, bwd: bool):
         Cc, T, D = self.C, self.T, self.D
         f = ffi.AhFlash()
@@ -395,7 +418,8 @@ class FusedTrainer:
         check(lib.ah_embedding_tok_pos(self.p("wte"), self.p("wpe"), self.tok, self.x[0], BT, self.T, Cc, V, SD))
         for l in range(L):
             pre = f"layer.{l}."
-            check(lib.ah_layernorm(self.x[l], self.p(pre + "ln1.weight"), self.p(pre + "ln1.bias"), self.ln1[l], BT, Cc, 1e-5, BF16, SD))
+            if l == 0 or self.drop == 0:           # (with dropout the pass that writes the stream has normalised it)
+                check(lib.ah_layernorm(self.x[l], self.p(pre + "ln1.weight"), self.p(pre + "ln1.bias"), self.ln1[l], BT, Cc, 1e-5, BF16, SD))
             if self.slabs:
                 self._gemm(NT, self.ln1[l], self.p(pre + "attn.wqkv", True), self.qkv[l], BT, 3 * Cc, Cc, Cc, Cc, Cc, c_planes=(Cc, BT * Cc))
             else:
@@ -403,10 +427,10 @@ class FusedTrainer:
             self._flash(l, False)
             if self.drop > 0:
                 self._gemm(NT, self.att[l], self.p(pre + "attn.wo", True), self.proj, BT, Cc, Cc, Cc, Cc, Cc)
-                self._dropout(self.proj, self.x[l], self.xmid[l], SD, micro, 2 * l)
+                self._dropped_norm(self.x[l], self.xmid[l], pre + "ln2", self.ln2[l], micro, 2 * l)
             else:
                 self._gemm(NT, self.att[l], self.p(pre + "attn.wo", True), self.xmid[l], BT, Cc, Cc, Cc, Cc, Cc, SD, ffi.EPI_RESIDUAL, self.x[l])
-            check(lib.ah_layernorm(self.xmid[l], self.p(pre + "ln2.weight"), self.p(pre + "ln2.bias"), self.ln2[l], BT, Cc, 1e-5, BF16, SD))
+                check(lib.ah_layernorm(self.xmid[l], self.p(pre + "ln2.weight"), self.p(pre + "ln2.bias"), self.ln2[l], BT, Cc, 1e-5, BF16, SD))
             if self.act == "gelu":
                 self._gemm(NT, self.ln2[l], self.p(pre + "mlp.fc1", True), self.hact[l], BT, Fd, Cc, Cc, Cc, Fd, BF16, ffi.EPI_GELU_GRAD, self.hgrad[l])
             else:
@@ -418,10 +442,12 @@ class FusedTrainer:
                     check(lib.ah_channel_act(BF16, self.hpre[l], self._coef_handles(l, self.p), self._act_mask, self.hact[l], BT, Fd))
             if self.drop > 0:
                 self._gemm(NT, self.hact[l], self.p(pre + self.w2, True), self.proj, BT, Cc, Fd, Fd, Fd, Cc)
-                self._dropout(self.proj, self.xmid[l], self.x[l + 1], SD, micro, 2 * l + 1)
+                name, out = (f"layer.{l + 1}.ln1", self.ln1[l + 1]) if l + 1 < L else ("lnF", self.lnf)
+                self._dropped_norm(self.xmid[l], self.x[l + 1], name, out, micro, 2 * l + 1)
             else:
                 self._gemm(NT, self.hact[l], self.p(pre + self.w2, True), self.x[l + 1], BT, Cc, Fd, Fd, Fd, Cc, SD, ffi.EPI_RESIDUAL, self.xmid[l])
-        check(lib.ah_layernorm(self.x[L], self.p("lnF.weight"), self.p("lnF.bias"), self.lnf, BT, Cc, 1e-5, BF16, SD))
+        if L == 0 or self.drop == 0:
+            check(lib.ah_layernorm(self.x[L], self.p("lnF.weight"), self.p("lnF.bias"), self.lnf, BT, Cc, 1e-5, BF16, SD))
         self._gemm(NT, self.lnf, self.p("lmHead", True), self.logits, BT, V, Cc, Cc, Cc, V)
         # loss and dlogits (in place) from one read of the logits
         if self.accum == 1:
@@ -435,15 +461,12 @@ class FusedTrainer:
         self._gemm(NN, self.logits, self.p("lmHead", True), self.dlnb, BT, Cc, V, V, Cc, Cc)
         cur = 0
         f32s = SD == F32                           # f32 stream: gradient in dx[cur] with bf16 copies; bf16 stream: the copies are the stream
-        check(lib.ah_layernorm_bwd_deferred(self.x[L], self.p("lnF.weight"), self.dlnb, BF16, 0, self.dx[cur] if f32s else 0, self.dy_fc2[L - 1],
-                                            self._ln_part["lnF"], BT, Cc, 1e-5, SD))
+        drop = self.drop > 0
+        self._norm_bwd("lnF", self.x[L], 0, self.dx[cur] if f32s else 0, self.dy_fc2[L - 1], self.dproj_fc2[L - 1] if drop else 0, micro, 2 * L - 1)
         for l in reversed(range(L)):
             pre = f"layer.{l}."
             # MLP: x_out = x_mid + fc2(gelu(fc1(ln2(x_mid))))
-            dyf = self.dy_fc2[l]
-            if self.drop > 0:                      # the projection's own gradient is the stream's times the mask it was dropped with
-                dyf = self.dproj_fc2[l]
-                self._dropout(self.dy_fc2[l], 0, dyf, BF16, micro, 2 * l + 1)
+            dyf = self.dproj_fc2[l] if drop else self.dy_fc2[l]      # the projection's own gradient is the stream's times the mask it was dropped with
             if self.act == "gelu":
                 self._gemm(NN, dyf, self.p(pre + "mlp.fc2", True), self.dh[l], BT, Fd, Cc, Cc, Fd, Fd, BF16, ffi.EPI_MUL_AUX, self.hgrad[l])
             else:
@@ -454,23 +477,20 @@ class FusedTrainer:
                     check(lib.ah_channel_act_bwd(BF16, self.hpre[l], self._coef_handles(l, self.p), self._act_mask, self.dact, self.dh[l],
                                                  self._coef_handles(l, self.g), acc, BT, Fd))
             self._gemm(NN, self.dh[l], self.p(pre + self.w1, True), self.dlnb, BT, Cc, self.Fin, self.Fin, Cc, Cc)
-            check(lib.ah_layernorm_bwd_deferred(self.xmid[l], self.p(pre + "ln2.weight"), self.dlnb, BF16, self.dx[cur] if f32s else self.dy_fc2[l],
-                                                self.dx[cur ^ 1] if f32s else 0, self.dy_wo[l], self._ln_part[pre + "ln2"], BT, Cc, 1e-5, SD))
+            self._norm_bwd(pre + "ln2", self.xmid[l], self.dx[cur] if f32s else self.dy_fc2[l], self.dx[cur ^ 1] if f32s else 0, self.dy_wo[l],
+                           self.dproj_wo[l] if drop else 0, micro, 2 * l)
             cur ^= f32s
             # attention: x_mid = x_in + wo(attn(wqkv(ln1(x_in))))
-            dyw = self.dy_wo[l]
-            if self.drop > 0:
-                dyw = self.dproj_wo[l]
-                self._dropout(self.dy_wo[l], 0, dyw, BF16, micro, 2 * l)
+            dyw = self.dproj_wo[l] if drop else self.dy_wo[l]
             self._gemm(NN, dyw, self.p(pre + "attn.wo", True), self.datt, BT, Cc, Cc, Cc, Cc, Cc)
             self._flash(l, True)
             if self.slabs:
                 self._gemm(NN, self.dqkv[l], self.p(pre + "attn.wqkv", True), self.dlnb, BT, Cc, 3 * Cc, Cc, Cc, Cc, a_planes=(Cc, BT * Cc))
             else:
                 self._gemm(NN, self.dqkv[l], self.p(pre + "attn.wqkv", True), self.dlnb, BT, Cc, 3 * Cc, 3 * Cc, Cc, Cc)
-            check(lib.ah_layernorm_bwd_deferred(self.x[l], self.p(pre + "ln1.weight"), self.dlnb, BF16, self.dx[cur] if f32s else self.dy_wo[l],
-                                                self.dx[cur ^ 1] if f32s else (self.dx[0] if l == 0 else 0),      # the embeddings take their gradient in f32
-                                                self.dy_fc2[l - 1] if l > 0 else self.dxb0, self._ln_part[pre + "ln1"], BT, Cc, 1e-5, SD))
+            self._norm_bwd(pre + "ln1", self.x[l], self.dx[cur] if f32s else self.dy_wo[l],
+                           self.dx[cur ^ 1] if f32s else (self.dx[0] if l == 0 else 0),      # the embeddings take their gradient in f32
+                           self.dy_fc2[l - 1] if l > 0 else self.dxb0, self.dproj_fc2[l - 1] if drop and l > 0 else 0, micro, 2 * l - 1)
             cur ^= f32s
             if self.dw_groups > 1 and l in self._dw_after_layer:
                 self._weight_grads(wepi, self._dw_after_layer[l])

@@ -322,6 +322,16 @@ int64_t ah_layernorm_bwd_partials_bytes(int64_t rows, int64_t dim);
 int32_t ah_layernorm_bwd_deferred(ah_ptr x, ah_ptr w, ah_ptr grad_out, int32_t grad_dtype, ah_ptr residual_grad,
                                   ah_ptr dx, ah_ptr dx_bf16, ah_ptr partials, int64_t rows, int64_t dim, float eps,
                                   int32_t stream_dtype);
+/* ah_layernorm_bwd_deferred of a bf16 stream, and `dropped` (bf16) = dx_bf16 times the mask of ah_dropout_mask(counter, p): the gradient of the
+ * projection whose residualDropoutAdd wrote the stream (ops.ts:616-686).  Row r's mask is drawn from seeds[r / rows_per_seed] (device int32, read when
+ * the kernel runs) and counts its elements from the first of those rows; dim % 4 == 0, dim <= 2048. */
+int32_t ah_layernorm_bwd_dropout(ah_ptr x, ah_ptr w, ah_ptr grad_out, ah_ptr residual_grad, ah_ptr dx, ah_ptr dx_bf16, ah_ptr dropped,
+                                 ah_ptr partials, int64_t rows, int64_t dim, float eps, ah_ptr seeds_i32, int64_t rows_per_seed,
+                                 int32_t counter, double p);
+/* residualDropoutAdd and the layerNorm behind it, in bf16: stream = residual + x * mask, out = layerNorm(stream) with f32 gain w and bias b; the bits of
+ * ah_dropout_apply and ah_layernorm.  Masks as in ah_layernorm_bwd_dropout. */
+int32_t ah_dropout_layernorm(ah_ptr x, ah_ptr residual, ah_ptr stream, ah_ptr w, ah_ptr b, ah_ptr out, int64_t rows, int64_t dim, float eps,
+                             ah_ptr seeds_i32, int64_t rows_per_seed, int32_t counter, double p);
 int32_t ah_layernorm_colsums(const AhColsumJob *jobs, int32_t count);
 /* loss[0] = mean_i (logsumexp(logits[i,:]) - logits[i,target[i]]); lse[N] kept for backward (0 = skip) */
 int32_t ah_cross_entropy(ah_ptr logits, int32_t logits_dtype, ah_ptr targets_i32, ah_ptr loss_out, ah_ptr lse_out,
