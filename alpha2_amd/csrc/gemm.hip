@@ -185,6 +185,7 @@ struct GroupPlan {
   ah_ptr sumsq;                        // 4 floats per block of the launch, then JOIN_BLOCKS per k-split problem (ah_gemm_grouped_run_sumsq)
   int ndescs; int64_t ws_bytes;        // what ah_gemm_grouped_update checks a new descriptor list against:
   std::vector<int64_t> shape;          // m, n, k, lda, ldb, ldc of every problem
+  int bn;                              // columns of a tile
 };
 std::vector<int64_t> group_shape(const AhGemm *descs, int count) {
   std::vector<int64_t> v;
@@ -249,25 +250,40 @@ __global__ __launch_bounds__(256) void k_grouped_sumsq_final(const float *__rest
 
 constexpr int GROUP_ROUND = 256;     // tiles that run at a time: one per CU
 
-// The launch runs its 256 x 256 tiles one per CU, in rounds of 256; all tiles of a weight-gradient group take the same
+// The launch runs its tiles of 256 rows one per CU, in rounds of 256; all tiles of a weight-gradient group take the same
 // time, so a last round of t < 256 tiles costs a whole round.  Cutting the problems that make up that round in two along
 // k turns it into 2 t half-length tiles, which still run at once when t <= 128: the round then costs half.  Chooses whole
 // problems from the end of the list whose tiles add up to between t and 128 and returns their indices (ascending), or
 // nothing when no such choice exists.
-std::vector<int> split_tail(const AhGemm *descs, int count, int64_t blocks) {
+std::vector<int> split_tail(const AhGemm *descs, int count, int64_t blocks, int bn) {
   std::vector<int> chosen;
   const int64_t tail = blocks % GROUP_ROUND;
   if (descs[0].out_dtype != AH_F32 || tail == 0 || tail > GROUP_ROUND / 2) return chosen;
   int64_t sum = 0;
   for (int i = count - 1; i >= 0 && sum < tail; i--) {
     const AhGemm &q = descs[i];
-    const int64_t t = cdiv(q.m, 256) * cdiv(q.n, 256);
+    const int64_t t = cdiv(q.m, 256) * cdiv(q.n, bn);
     if (q.k % 128 != 0 || q.n % 4 != 0 || sum + t > GROUP_ROUND / 2) continue;
     chosen.insert(chosen.begin(), i);
     sum += t;
   }
   if (sum < tail) chosen.clear();
   return chosen;
+}
+// Columns of a group's tiles: 256, or 192 or 128 (weight gradients in f32 only) where edge tiles and rounds waste that much more of the wide ones.
+// A narrower tile reads more from LDS per flop: 3 % slower at 192, half as slow again at 128, and is taken from 5 % on.  us at
+// 256 / 192 / 128 columns, all the weight gradients of a model: 8 layers x 384 of 10240 tokens 389 / 303 / 337, 6 x 320 of 8192 177 / 151 / 176, 4 x 192 of
+// 8192 89 / 76 / 65, 2 x 128 of 128 14.0 / 13.1 / 12.0, 2 x 576 of 4096 95 / 79 / 107; 4 x 512 of 8192 175 / 225 / 204, 12 x 768 of 16384 3008 / 3138 / 3431.
+int group_width(const AhGemm *descs, int count) {
+  if (descs[0].layout != AH_GEMM_TN || descs[0].out_dtype != AH_F32) return 256;
+  auto cost = [&](int bn) {
+    int64_t tiles = 0;
+    for (int i = 0; i < count; i++) tiles += cdiv(descs[i].m, 256) * cdiv(descs[i].n, bn);
+    const double rounds = split_tail(descs, count, tiles, bn).empty() ? (double)cdiv(tiles, GROUP_ROUND) : (double)(tiles / GROUP_ROUND) + 0.5;
+    return rounds * bn * (bn == 256 ? 0.95 : bn == 192 ? 1.03 : 1.5);
+  };
+  const double wide = cost(256), mid = cost(192), narrow = cost(128);
+  return wide <= mid && wide <= narrow ? 256 : mid <= narrow ? 192 : 128;
 }
 }  // namespace
 
@@ -285,7 +301,7 @@ extern "C" {
 // round as two entries each at the end) and `parts` (what k_grouped_join adds to what).  The second halves write consecutive
 // pieces of a workspace that starts at ws_base (0 while only its size, *ws_bytes, is wanted).
 static int32_t grouped_tables(const char *who, const AhGemm *descs, int32_t count, ah_ptr ws_base, std::vector<GemmGroupEntry> &tab,
-                              std::vector<JoinPart> &parts, int64_t *blocks_out, int64_t *ws_bytes) {
+                              std::vector<JoinPart> &parts, int64_t *blocks_out, int64_t *ws_bytes, int *bn_out) {
   AH_ARG(descs != nullptr && count > 0 && count <= 4096, "%s: bad descriptor list (count %d)", who, count);
   tab.assign((size_t)count, GemmGroupEntry{});
   parts.clear();
@@ -315,14 +331,19 @@ static int32_t grouped_tables(const char *who, const AhGemm *descs, int32_t coun
     AH_ARG(q.ldc < (1 << 22), "%s: problem %d: ldc %lld too large (128 rows of C must span less than 2 GiB)", who, i, (long long)q.ldc);
     GemmGroupEntry &e = tab[(size_t)i];
     e.a = dp<const void>(q.a); e.b = dp<const void>(q.b); e.c = dp<void>(q.c);
-    e.M = (int)q.m; e.N = (int)q.n; e.K = (int)q.k; e.tile_start = (int)blocks;
+    e.M = (int)q.m; e.N = (int)q.n; e.K = (int)q.k;
     e.lda = q.lda; e.ldb = q.ldb; e.ldc = q.ldc;
-    blocks += cdiv(q.m, 256) * cdiv(q.n, 256);
+  }
+  const int bn = group_width(descs, count);
+  *bn_out = bn;
+  for (GemmGroupEntry &e : tab) {
+    e.tile_start = (int)blocks;
+    blocks += cdiv(e.M, 256) * cdiv(e.N, bn);
     AH_ARG(blocks < (1ll << 31), "%s: too many tiles", who);
   }
   // the problems that make up a short last round are cut in two along k: they move to the end of the table as pairs of
   // entries, the second of which writes the workspace
-  const std::vector<int> chosen = split_tail(descs, count, blocks);
+  const std::vector<int> chosen = split_tail(descs, count, blocks, bn);
   *ws_bytes = 0;
   if (!chosen.empty()) {
     for (int i : chosen) *ws_bytes += descs[i].m * descs[i].n * 4;
@@ -332,7 +353,7 @@ static int32_t grouped_tables(const char *who, const AhGemm *descs, int32_t coun
     int64_t nblocks = 0;
     auto push = [&](GemmGroupEntry e) {
       e.tile_start = (int)nblocks;
-      nblocks += cdiv(e.M, 256) * cdiv(e.N, 256);
+      nblocks += cdiv(e.M, 256) * cdiv(e.N, bn);
       cut_tab.push_back(e);
     };
     for (int i = 0; i < count; i++)
@@ -364,15 +385,16 @@ int32_t ah_gemm_grouped_plan(const AhGemm *descs, int32_t count, uint64_t *plan_
   std::vector<GemmGroupEntry> tab;
   std::vector<JoinPart> parts;
   int64_t blocks = 0, ws_bytes = 0;
-  int32_t rc = grouped_tables("ah_gemm_grouped_plan", descs, count, 0, tab, parts, &blocks, &ws_bytes);      // sizes first
+  int bn = 0;
+  int32_t rc = grouped_tables("ah_gemm_grouped_plan", descs, count, 0, tab, parts, &blocks, &ws_bytes, &bn);      // sizes first
   if (rc) return rc;
   GroupPlan plan{0, (int)tab.size(), (int)blocks, descs[0].layout, descs[0].out_dtype, true, 0, 0, (int)parts.size(), 0, count, ws_bytes,
-                 group_shape(descs, count)};
+                 group_shape(descs, count), bn};
   if (ws_bytes > 0) {
     rc = ah_alloc((size_t)ws_bytes, &plan.ws);
     if (rc) return rc;
     rc = ah_fill_f32(plan.ws, 0.f, (uint64_t)(ws_bytes / 4));           // the workspace is all zero between runs (see k_grouped_join)
-    if (rc == AH_OK) rc = grouped_tables("ah_gemm_grouped_plan", descs, count, plan.ws, tab, parts, &blocks, &ws_bytes);
+    if (rc == AH_OK) rc = grouped_tables("ah_gemm_grouped_plan", descs, count, plan.ws, tab, parts, &blocks, &ws_bytes, &bn);
     if (rc == AH_OK) rc = ah_alloc(parts.size() * sizeof(JoinPart), &plan.parts);
     if (rc == AH_OK) rc = ah_upload(plan.parts, parts.data(), parts.size() * sizeof(JoinPart));
   }
@@ -398,10 +420,11 @@ int32_t ah_gemm_grouped_update(uint64_t plan, const AhGemm *descs, int32_t count
   std::vector<GemmGroupEntry> tab;
   std::vector<JoinPart> parts;
   int64_t blocks = 0, ws_bytes = 0;
-  int32_t rc = grouped_tables("ah_gemm_grouped_update", descs, count, p.ws, tab, parts, &blocks, &ws_bytes);
+  int bn = 0;
+  int32_t rc = grouped_tables("ah_gemm_grouped_update", descs, count, p.ws, tab, parts, &blocks, &ws_bytes, &bn);
   if (rc) return rc;
   if (count != p.ndescs || descs[0].layout != p.layout || descs[0].out_dtype != p.out_dtype || (int)tab.size() != p.count ||
-      (int)blocks != p.blocks || (int)parts.size() != p.nparts || ws_bytes != p.ws_bytes || group_shape(descs, count) != p.shape)
+      (int)blocks != p.blocks || (int)parts.size() != p.nparts || ws_bytes != p.ws_bytes || bn != p.bn || group_shape(descs, count) != p.shape)
     return fail(AH_ERR_ARG, "ah_gemm_grouped_update: the problems do not have the shapes the plan was made for");
   if (!parts.empty()) {
     rc = ah_upload(p.parts, parts.data(), parts.size() * sizeof(JoinPart));
@@ -422,9 +445,9 @@ static int32_t grouped_run(const char *who, uint64_t plan, int32_t epilogue, ah_
   float *ss = sums ? dp<float>(p.sumsq) : nullptr;
   int32_t rc;
   switch (p.layout) {
-    case AH_GEMM_NT: rc = gemm_bf16_dma_nt_grouped(tab, p.count, p.blocks, epilogue, p.out_dtype, ss); break;
-    case AH_GEMM_NN: rc = gemm_bf16_dma_nn_grouped(tab, p.count, p.blocks, epilogue, p.out_dtype, ss); break;
-    default: rc = gemm_bf16_dma_tn_grouped(tab, p.count, p.blocks, epilogue, p.out_dtype, ss);
+    case AH_GEMM_NT: rc = gemm_bf16_dma_nt_grouped(tab, p.count, p.blocks, epilogue, p.out_dtype, p.bn, ss); break;
+    case AH_GEMM_NN: rc = gemm_bf16_dma_nn_grouped(tab, p.count, p.blocks, epilogue, p.out_dtype, p.bn, ss); break;
+    default: rc = gemm_bf16_dma_tn_grouped(tab, p.count, p.blocks, epilogue, p.out_dtype, p.bn, ss);
   }
   if (rc != AH_OK) return rc;
   if (p.nparts > 0) {
