@@ -11,7 +11,7 @@
 //   k_decode_attention   keys in slices of at least 64, one workgroup to a slice and head
 //   k_decode_rows<JOIN>  joins the slices (softmax weights of the slices' maxima) in LDS + wo + the residual stream
 //   k_decode_long        fc2 + the residual stream: long rows, few of them, so four waves to a row
-// 64 tokens from a 6 x 256 model 56.0 -> 11.5 ms in launches and 9.0 in one launch a token, 24 tokens behind a prompt of 480 from the GPT-2-small shape 59.9 -> 12.6 (each with
+// 64 tokens from a 6 x 256 model 56.0 -> 11.5 ms in launches and 9.0 in one launch a token, 24 tokens behind a prompt of 480 from the GPT-2-small shape 59.9 -> 11.4 (each with
 // the pass over the finished sequence that follows).  A launch takes 2.9 to 5.7 us there and the next one starts about 1 us later.
 #include "common.h"
 #include <algorithm>
@@ -64,6 +64,7 @@ template <int PRO, int NV, int R, bool DUAL>
 __global__ __launch_bounds__(256) void k_decode_rows(DecodeRows a) {
   constexpr int ROWS = DUAL ? 2 * R : R;
   __shared__ __attribute__((aligned(16))) float joined[PRO == JOIN ? 256 * NV : 4];
+  __shared__ float weights[PRO == JOIN ? MAX_SLICES * 32 * NV : 4], sums[PRO == JOIN ? 32 * NV : 4];      // heads of 8 features at least
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nv = a.K >> 2, n0 = (blockIdx.x * 4 + wave) * R;
   float4 w[ROWS][NV], x[NV];
 #pragma unroll
@@ -111,36 +112,56 @@ __global__ __launch_bounds__(256) void k_decode_rows(DecodeRows a) {
         x[i] = make_float4((x[i].x - mean) * rstd * g[i].x + b[i].x, (x[i].y - mean) * rstd * g[i].y + b[i].y,
                            (x[i].z - mean) * rstd * g[i].z + b[i].z, (x[i].w - mean) * rstd * g[i].w + b[i].w);
   } else {
-    // eight slices at a time, all asked for at once (one after the other they took 10 of 13 us at 768 wide with 8 slices)
+    // A thread to a head makes the slices' weights (eight slices asked for at once); meanwhile the slices' sums are on their way, eight at a time.  With
+    // the weights made again for every feature this launch took 6.5 us at 768 wide with 8 slices, now 5.2.
     const int head_size = a.K / a.heads;
-#pragma unroll(NV <= 4 ? NV : 1)
+    constexpr bool AHEAD = NV <= 4;
+    float y[AHEAD ? NV : 1][8];
+    auto load = [&](int i, int s0, float (&to)[8]) {
+      const int k = min(threadIdx.x + 256 * i, a.K - 1);
+#pragma unroll
+      for (int u = 0; u < 8; u++) to[u] = a.x[(int64_t)min(s0 + u, a.slices - 1) * a.K + k];
+    };
+    if (AHEAD) {
+#pragma unroll
+      for (int i = 0; i < NV; i++) load(i, 0, y[AHEAD ? i : 0]);
+    }
+    for (int h = threadIdx.x; h < a.heads; h += 256) {
+      float2 t[MAX_SLICES];
+      float top = -INFINITY, sum = 0.f;
+#pragma unroll
+      for (int s = 0; s < MAX_SLICES; s++) {
+        if (s >= 8 && a.slices <= 8) { t[s] = make_float2(-INFINITY, 0.f); continue; }
+        t[s] = a.top[min(s, a.slices - 1) * a.heads + h];
+        if (s >= a.slices) t[s] = make_float2(-INFINITY, 0.f);
+        top = fmaxf(top, t[s].x);
+      }
+#pragma unroll
+      for (int s = 0; s < MAX_SLICES; s++) {
+        if (s >= 8 && a.slices <= 8) continue;
+        const float c = slice_weight(t[s].x, top);
+        sum = __builtin_fmaf(c, t[s].y, sum);
+        weights[s * 32 * NV + h] = c;
+      }
+      sums[h] = sum;
+    }
+    __syncthreads();
+#pragma unroll(AHEAD ? NV : 1)
     for (int i = 0; i < NV; i++) {
       const int k = min(threadIdx.x + 256 * i, a.K - 1), h = k / head_size;
-      float most = -INFINITY, sum = 0.f, v = 0.f;
+      float v = 0.f;
       for (int s0 = 0; s0 < a.slices; s0 += 8) {
-        float2 t[8];
-        float y[8];
+        float z[8];
+        if (AHEAD && s0 == 0) {
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
-          const int s = min(s0 + u, a.slices - 1);
-          t[u] = a.top[s * a.heads + h];
-          y[u] = a.x[(int64_t)s * a.K + k];
+          for (int u = 0; u < 8; u++) z[u] = y[AHEAD ? i : 0][u];
+        } else {
+          load(i, s0, z);
         }
-        float top = most;
 #pragma unroll
-        for (int u = 0; u < 8; u++) top = fmaxf(top, t[u].x);
-        const float old = most == -INFINITY ? 0.f : expf(most - top);
-        sum *= old;
-        v *= old;
-        most = top;
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
-          const float c = s0 + u >= a.slices || t[u].x == -INFINITY ? 0.f : expf(t[u].x - most);
-          sum = __builtin_fmaf(c, t[u].y, sum);
-          v = s0 + u < a.slices ? __builtin_fmaf(c, y[u], v) : v;
-        }
+        for (int u = 0; u < 8; u++) v = s0 + u < a.slices ? __builtin_fmaf(weights[(s0 + u) * 32 * NV + h], z[u], v) : v;
       }
-      joined[k] = v / sum;
+      joined[k] = v / sums[h];
     }
     __syncthreads();
 #pragma unroll
@@ -191,7 +212,8 @@ __global__ __launch_bounds__(256) void k_decode_long(const float *__restrict__ w
 }
 
 // The newest row's query against the keys of one slice, for one head.  G lanes hold a head's features, four each, so a workgroup takes
-// 256 / G keys at a time; each group of lanes keeps its own running maximum, and the groups are joined at the end.
+// 256 / G keys at a time, four of them on their way, and the waves are joined at the end.  Every lane of a group has the group's scores; each takes tanh and
+// exp of one (of all, one after the other with a running maximum to a group: 12 heads x 64 behind 500 rows 5.7 -> 4.0 us).
 // qkv: the layer's rows of [q | k | v]; sums: [slices][width], not yet divided; top: [slices][heads].
 struct DecodeAttention {
   const float *qkv;
@@ -215,41 +237,40 @@ __global__ __launch_bounds__(256) void k_decode_attention(DecodeAttention a) {
   const float *ks = at + first * pitch + a.width;
   float m = -INFINITY, l = 0.f;
   float4 o = none;
-  for (int j0 = key; j0 < count; j0 += KEYS * U) {
+  for (int j0 = 0; j0 < count; j0 += KEYS * U) {
     float4 k[U], v[U];
 #pragma unroll
     for (int u = 0; u < U; u++) {
-      const float *p = ks + min(j0 + u * KEYS, count - 1) * pitch;
+      const float *p = ks + min(j0 + key + u * KEYS, count - 1) * pitch;
       k[u] = ldq(p, 0);
       v[u] = ldq(p + a.width, 0);
     }
+    // the U scores of a group of lanes, one of them to a lane for what tanh and exp take, and one maximum to a wave
+    float mine = 0.f;
 #pragma unroll
     for (int u = 0; u < U; u++) {
-      float s = in ? dot4(q, k[u], 0.f) : 0.f;
+      const float s = near_sum<G>(in ? dot4(q, k[u], 0.f) : 0.f);
+      mine = (f & (U - 1)) == u ? s : mine;
+    }
+    mine *= a.scale;
+    if (a.cap > 0.f) mine = a.cap * tanhf(mine / a.cap);
+    if (j0 + key + (f & (U - 1)) * KEYS >= count) mine = -INFINITY;
+    const float most = fmaxf(m, wave_max(mine)), old = slice_weight(m, most), p = f < U ? slice_weight(mine, most) : 0.f;
+    l = __builtin_fmaf(l, old, wave_sum(p));
+    o.x *= old; o.y *= old; o.z *= old; o.w *= old;
+    m = most;
 #pragma unroll
-      for (int d = 1; d < G; d <<= 1) s += __shfl_xor(s, d, 64);
-      s *= a.scale;
-      if (a.cap > 0.f) s = a.cap * tanhf(s / a.cap);
-      if (j0 + u * KEYS < count) {
-        const float most = s > m ? s : (m >= s ? m : s);        // NaN stays
-        const float old = m == -INFINITY ? 0.f : expf(m - most), p = s == -INFINITY ? 0.f : expf(s - most);
-        l = __builtin_fmaf(l, old, p);
-        o.x = __builtin_fmaf(o.x, old, p * v[u].x); o.y = __builtin_fmaf(o.y, old, p * v[u].y);
-        o.z = __builtin_fmaf(o.z, old, p * v[u].z); o.w = __builtin_fmaf(o.w, old, p * v[u].w);
-        m = most;
-      }
+    for (int u = 0; u < U; u++) {
+      const float pu = __shfl(p, (lane & ~(G - 1)) + u, 64);
+      o.x = __builtin_fmaf(pu, v[u].x, o.x); o.y = __builtin_fmaf(pu, v[u].y, o.y);
+      o.z = __builtin_fmaf(pu, v[u].z, o.z); o.w = __builtin_fmaf(pu, v[u].w, o.w);
     }
   }
   // the groups of a wave, then the waves
-#pragma unroll
-  for (int d = G; d < 64; d <<= 1) {
-    const float om = __shfl_xor(m, d, 64), ol = __shfl_xor(l, d, 64);
-    const float4 oo = make_float4(__shfl_xor(o.x, d, 64), __shfl_xor(o.y, d, 64), __shfl_xor(o.z, d, 64), __shfl_xor(o.w, d, 64));
-    const float most = fmaxf(m, om), c = slice_weight(m, most), e = slice_weight(om, most);
-    l = l * c + ol * e;
-    o = make_float4(o.x * c + oo.x * e, o.y * c + oo.y * e, o.z * c + oo.z * e, o.w * c + oo.w * e);
-    m = most;
-  }
+  auto far = [&](auto step) { o.x = step(o.x); o.y = step(o.y); o.z = step(o.z); o.w = step(o.w); };
+  if (G < 16) far([](float v) { return add_lane<8>(v); });
+  if (G < 32) far([](float v) { return add_lane<16>(v); });
+  far([](float v) { return add_lane<32>(v); });
   if (lane < G) {
     reinterpret_cast<float4 *>(all_o[wave])[lane] = o;
     if (lane == 0) { all_m[wave] = m; all_l[wave] = l; }
@@ -752,9 +773,7 @@ void launch_rows(const DecodeRows &a) {
 void launch_attention(const DecodeAttention &a, int slices, int heads) {
   auto go = [&](auto kfn) { ah::launch_kernel(kfn, dim3((unsigned)slices, (unsigned)heads), dim3(256), 0, a); };
   const int quads = a.head_size / 4;
-  if (quads <= 2) go(k_decode_attention<2>);
-  else if (quads <= 4) go(k_decode_attention<4>);
-  else if (quads <= 8) go(k_decode_attention<8>);
+  if (quads <= 8) go(k_decode_attention<8>);
   else if (quads <= 16) go(k_decode_attention<16>);
   else go(k_decode_attention<32>);
 }
