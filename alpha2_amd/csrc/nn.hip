@@ -687,9 +687,11 @@ __global__ __launch_bounds__(256) void k_layernorm_bwd_vec(const X *__restrict__
 constexpr float CE_LOG2E = 1.4426950408889634f;
 __device__ __forceinline__ float exp_minus(float v, float m) { return __builtin_amdgcn_exp2f((v - m) * CE_LOG2E); }
 __device__ __forceinline__ void online_merge(float &m, float &s, float m2, float s2) {
-  float nm = fmaxf(m, m2);
+  const float nm = fmaxf(m, m2);
   if (nm == -INFINITY) { m = nm; s = 0.f; return; }
-  s = s * expf(m - nm) + s2 * expf(m2 - nm);
+  // the larger one's factor is exp(0): 1, or NaN beside an infinity.  Spelled out, so that every kernel rounds it alike
+  const float d = m - nm, d2 = m2 - nm, e = expf(fminf(m, m2) - nm);
+  s = __builtin_fmaf(s2, m2 == nm ? 1.0f + d2 : e, s * (m == nm ? 1.0f + d : e));
   m = nm;
 }
 __device__ __forceinline__ void wave_merge(float &m, float &s) {
@@ -697,52 +699,83 @@ __device__ __forceinline__ void wave_merge(float &m, float &s) {
   online_merge(m, s, lane_xor<8>(m), lane_xor<8>(s)); online_merge(m, s, lane_xor<4>(m), lane_xor<4>(s));
   online_merge(m, s, lane_xor<2>(m), lane_xor<2>(s)); online_merge(m, s, lane_xor<1>(m), lane_xor<1>(s));
 }
-// Threads to a row: as many as give each a few 16-byte chunks, so that a row of few classes is a wave's (no barrier, no LDS) and a CU holds more of
-// them.  The same for the loss alone and for both passes in one, whose bits are the same.  16384 x 256 in fp32 a block to a row
-// 26 us, now 10.1, its backward pass 10.4 -> 6.6; 10240 x 4096 in bf16, both passes, 83.5 us with 512 threads (whose registers hold 53248 classes,
-// two blocks to a CU) and 40.8 with 256.
+// A row is summed in one order whatever the number of its threads: CE_FULL shares take its 16-byte chunks (what is left of it: its classes) in turns, each
+// in order; the shares are merged by 64s, and the 64s one after the other.  A thread plays V shares, TPR apart, so that a row of few classes is a
+// wave's (no barrier, no LDS) and a CU holds more of them; a 64 that has nothing to merge is left out, which changes no bit.  What bounds short rows is the
+// merges (an exponential each).  us with a thread to a share in all cases / now, with the mean behind it: fp32 16384 x 256 29.9 / 12.9, x 512 30.6 / 20.0, x 1024
+// 32.9 / 33.2; both passes in bf16, whose registers held 53248 classes at every size, 10240 x 512 62.9 / 12.1, x 2048 67.6 / 30.0, x 4096 79.6 / 48.2, x 8192
+// 101 / 67.
+template <class T> constexpr int CE_FULL = sizeof(T) == 4 ? 256 : 512;
+constexpr int ce_block(int tpr) { return tpr == 64 ? 256 : tpr; }      // four rows of a wave each, or one row
 template <class T>
-constexpr int ce_threads(int64_t c) { return sizeof(T) == 4 ? (c <= 1024 ? 64 : 256) : c <= 2048 ? 64 : c <= 8192 ? 256 : 512; }
-// single read of the row with an online (max, sum-exp) pair per thread
+__device__ __forceinline__ void ce_chunk(const uint4 &u, float &m, float &s) {
+  constexpr int VW = 16 / sizeof(T);
+  float v[VW];
+  if (sizeof(T) == 4) { v[0] = __uint_as_float(u.x); v[1] = __uint_as_float(u.y); v[2] = __uint_as_float(u.z); v[VW - 1] = __uint_as_float(u.w); }
+  else {
+    v[0] = bf16_bits_to_f32(u.x & 0xffff); v[1] = bf16_bits_to_f32(u.x >> 16); v[2] = bf16_bits_to_f32(u.y & 0xffff); v[3] = bf16_bits_to_f32(u.y >> 16);
+    v[VW - 4] = bf16_bits_to_f32(u.z & 0xffff); v[VW - 3] = bf16_bits_to_f32(u.z >> 16); v[VW - 2] = bf16_bits_to_f32(u.w & 0xffff); v[VW - 1] = bf16_bits_to_f32(u.w >> 16);
+  }
+  float vm = v[0];
+#pragma unroll
+  for (int i = 1; i < VW; i++) vm = fmaxf(vm, v[i]);
+  if (vm > m) { s *= __expf(m - vm); m = vm; }
+#pragma unroll
+  for (int i = 0; i < VW; i++) s += exp_minus(v[i], m);
+}
+// The row's maximum and sum from its shares', valid in its first thread.  units: how many shares have a part of the row at all
+template <int TPR, int V>
+__device__ __forceinline__ void ce_join(float (&m)[V], float (&s)[V], int64_t units, float *shm, float *shs) {
+  const int wv = threadIdx.x % TPR / 64;
+#pragma unroll
+  for (int v = 0; v < V; v++)
+    if (v == 0 || v * TPR + wv * 64 < units) wave_merge(m[v], s[v]);
+  if constexpr (TPR > 64) {
+    if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+      for (int v = 0; v < V; v++) { shm[v * (TPR / 64) + wv] = m[v]; shs[v * (TPR / 64) + wv] = s[v]; }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0)
+      for (int k = 1; k < V * TPR / 64; k++) online_merge(m[0], s[0], shm[k], shs[k]);
+  } else {
+#pragma unroll
+    for (int v = 1; v < V; v++)
+      if (v * TPR < units) online_merge(m[0], s[0], m[v], s[v]);
+  }
+}
+// single read of the row with an online (max, sum-exp) pair per share
 template <class T, int TPR>
-__global__ __launch_bounds__(TPR < 256 ? 256 : TPR) void k_ce_fwd(const T *__restrict__ logits, const int32_t *__restrict__ targets, float *__restrict__ row_loss,
+__global__ __launch_bounds__(ce_block(TPR)) void k_ce_fwd(const T *__restrict__ logits, const int32_t *__restrict__ targets, float *__restrict__ row_loss,
                          float *__restrict__ lse_out, int64_t n, int64_t c) {
-  __shared__ float shm[TPR / 64], shs[TPR / 64];        // one pair per wave of the row
-  const int64_t row = TPR < 256 ? blockIdx.x * (int64_t)(256 / TPR) + threadIdx.x / TPR : blockIdx.x;
+  constexpr int V = CE_FULL<T> / TPR, VW = 16 / sizeof(T);
+  __shared__ float shm[TPR > 64 ? CE_FULL<T> / 64 : 1], shs[TPR > 64 ? CE_FULL<T> / 64 : 1];
+  const int64_t row = TPR == 64 ? blockIdx.x * (int64_t)4 + threadIdx.x / 64 : blockIdx.x;
   if (row >= n) return;                                 // (a whole wave, and only where a row is one)
   const int t0 = threadIdx.x % TPR;
   const T *p = logits + row * c;
-  float m = -INFINITY, s = 0.f;
-  constexpr int VW = 16 / sizeof(T);                    // elements per 16-byte load
-  int64_t nvec = ((((uintptr_t)p) & 15u) == 0) ? c / VW : 0;
-  for (int64_t j = t0; j < nvec; j += TPR) {
-    uint4 u = reinterpret_cast<const uint4 *>(p)[j];
-    float v[VW];
-    if (sizeof(T) == 4) { v[0] = __uint_as_float(u.x); v[1] = __uint_as_float(u.y); v[2] = __uint_as_float(u.z); v[VW - 1] = __uint_as_float(u.w); }
-    else {
-      v[0] = bf16_bits_to_f32(u.x & 0xffff); v[1] = bf16_bits_to_f32(u.x >> 16); v[2] = bf16_bits_to_f32(u.y & 0xffff); v[3] = bf16_bits_to_f32(u.y >> 16);
-      v[VW - 4] = bf16_bits_to_f32(u.z & 0xffff); v[VW - 3] = bf16_bits_to_f32(u.z >> 16); v[VW - 2] = bf16_bits_to_f32(u.w & 0xffff); v[VW - 1] = bf16_bits_to_f32(u.w >> 16);
-    }
-    float vm = v[0];
+  float m[V], s[V];
 #pragma unroll
-    for (int i = 1; i < VW; i++) vm = fmaxf(vm, v[i]);
-    if (vm > m) { s *= __expf(m - vm); m = vm; }
+  for (int v = 0; v < V; v++) { m[v] = -INFINITY; s[v] = 0.f; }
+  const int64_t nvec = ((((uintptr_t)p) & 15u) == 0) ? c / VW : 0, rest = c - nvec * VW;
+  for (int64_t j0 = t0; j0 < nvec; j0 += TPR * V) {
+    uint4 u[V];
 #pragma unroll
-    for (int i = 0; i < VW; i++) s += exp_minus(v[i], m);
+    for (int v = 0; v < V; v++) if (j0 + v * TPR < nvec) u[v] = reinterpret_cast<const uint4 *>(p)[j0 + v * TPR];
+#pragma unroll
+    for (int v = 0; v < V; v++) if (j0 + v * TPR < nvec) ce_chunk<T>(u[v], m[v], s[v]);
   }
-  for (int64_t j = nvec * VW + t0; j < c; j += TPR) {
-    float v = Io<T>::ld(p, j);
-    if (v > m) { s = s * expf(m - v) + 1.0f; m = v; } else { s += expf(v - m); }
+  for (int64_t j0 = t0; j0 < rest; j0 += TPR * V) {
+#pragma unroll
+    for (int v = 0; v < V; v++)
+      if (j0 + v * TPR < rest) {
+        const float x = Io<T>::ld(p, nvec * VW + j0 + v * TPR);
+        if (x > m[v]) { s[v] = s[v] * expf(m[v] - x) + 1.0f; m[v] = x; } else { s[v] += expf(x - m[v]); }
+      }
   }
-  wave_merge(m, s);
-  if constexpr (TPR > 64) {
-    int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (lane == 0) { shm[wv] = m; shs[wv] = s; }
-    __syncthreads();
-  }
+  ce_join<TPR, V>(m, s, nvec > rest ? nvec : rest, shm, shs);
   if (t0 == 0) {
-    for (int k = 1; k < TPR / 64; k++) online_merge(m, s, shm[k], shs[k]);
-    float lse = m + logf(s);
+    const float lse = m[0] + logf(s[0]);
     int32_t t = targets[row];
     float picked = (t >= 0 && t < c) ? Io<T>::ld(p, t) : lse;     // an out-of-range target contributes 0 loss
     row_loss[row] = lse - picked;
@@ -787,7 +820,7 @@ __device__ __forceinline__ void ce_grad8(const uint4 &u, float lse, float scale,
 #pragma unroll
   for (int i = 0; i < 4; i++) o[i] = pack_bf16x2(e[2 * i] * scale, e[2 * i + 1] * scale);
 }
-// TPR threads to a row, as ce_threads says, and 8 or so elements to a thread
+// TPR threads to a row, 8 or so elements to a thread; a wave up to 1024 classes (bf16 2048): 16384 x 256 in fp32 10.4 us with a block, 6.6 with a wave
 template <class T, int TPR>
 __global__ __launch_bounds__(256) void k_ce_bwd(const T *__restrict__ logits, const int32_t *__restrict__ targets, const float *__restrict__ lse,
                          const float *__restrict__ g, float g_mul, T *__restrict__ out, int64_t rows, int64_t n, int64_t c) {
@@ -829,42 +862,36 @@ __global__ __launch_bounds__(256) void k_ce_bwd(const T *__restrict__ logits, co
 // (max, sum) updates and the same expressions as k_ce_fwd / k_ce_bwd: results are bit-identical to that pair.
 // (past 8192 classes, measured at 16384 x 50304: 636 us with 512 threads per row, 670 with 256, 793 with 1024)
 constexpr int CE_CLASSES = 53248;      // 13 chunks of 512 threads: CE_CLASSES / 8 / 512
-// CHUNKS x TPR threads x 8 classes: what a row may have
-template <int TPR, int CHUNKS>
-__global__ __launch_bounds__(TPR < 256 ? 256 : TPR) void k_ce_fwd_bwd(const uint16_t *logits, const int32_t *__restrict__ targets,
+// CHUNKS to a share, V shares to each of TPR threads (as ce_join; 512 in all, or fewer where the row has no chunk for the others)
+template <int TPR, int V, int CHUNKS>
+__global__ __launch_bounds__(ce_block(TPR)) void k_ce_fwd_bwd(const uint16_t *logits, const int32_t *__restrict__ targets,
                                                     float *__restrict__ row_loss, float *__restrict__ lse_out, const float *__restrict__ g,
                                                     float g_mul, uint16_t *out, int64_t n, int64_t c) {      // out may be logits
-  __shared__ float shm[TPR / 64], shs[TPR / 64], sh_lse;
-  const int64_t row = TPR < 256 ? blockIdx.x * (int64_t)(256 / TPR) + threadIdx.x / TPR : blockIdx.x;
+  __shared__ float shm[TPR > 64 ? V * TPR / 64 : 1], shs[TPR > 64 ? V * TPR / 64 : 1], sh_lse;
+  const int64_t row = TPR == 64 ? blockIdx.x * (int64_t)4 + threadIdx.x / 64 : blockIdx.x;
   if (row >= n) return;                                 // (a whole wave, and only where a row is one)
   const int t0 = threadIdx.x % TPR;
   const uint16_t *p = logits + row * c;
   const int nvec = (int)(c >> 3);
-  uint4 r[CHUNKS];
-  float m = -INFINITY, s = 0.f;
+  uint4 r[CHUNKS * V];                                  // chunk t0 + k TPR of the row: of share t0 + (k % V) TPR
+  float m[V], s[V];
 #pragma unroll
-  for (int k = 0; k < CHUNKS; k++) {
+  for (int v = 0; v < V; v++) { m[v] = -INFINITY; s[v] = 0.f; }
+#pragma unroll
+  for (int k = 0; k < CHUNKS * V; k++) {
     const int j = t0 + k * TPR;
     if (j < nvec) {
       typedef unsigned u4v __attribute__((ext_vector_type(4)));     // 1.65 GB read once and written once: non-temporal (-6 %)
       const u4v un = __builtin_nontemporal_load(reinterpret_cast<const u4v *>(p) + j);
-      const uint4 u = make_uint4(un.x, un.y, un.z, un.w);
-      r[k] = u;
-      float v[8] = {bf16_bits_to_f32(u.x & 0xffff), bf16_bits_to_f32(u.x >> 16), bf16_bits_to_f32(u.y & 0xffff), bf16_bits_to_f32(u.y >> 16),
-                    bf16_bits_to_f32(u.z & 0xffff), bf16_bits_to_f32(u.z >> 16), bf16_bits_to_f32(u.w & 0xffff), bf16_bits_to_f32(u.w >> 16)};
-      float vm = v[0];
-#pragma unroll
-      for (int i = 1; i < 8; i++) vm = fmaxf(vm, v[i]);
-      if (vm > m) { s *= __expf(m - vm); m = vm; }
-#pragma unroll
-      for (int i = 0; i < 8; i++) s += exp_minus(v[i], m);
+      r[k] = make_uint4(un.x, un.y, un.z, un.w);
+      ce_chunk<uint16_t>(r[k], m[k % V], s[k % V]);
     }
   }
-  wave_merge(m, s);
+  ce_join<TPR, V>(m, s, nvec, shm, shs);
   const int32_t t = targets[row];
   float l;
   auto leave = [&]() {
-    const float lse = m + logf(s);
+    const float lse = m[0] + logf(s[0]);
     const float picked = (t >= 0 && t < c) ? bf16_bits_to_f32(p[t]) : lse;     // an out-of-range target contributes 0 loss
     row_loss[row] = lse - picked;
     if (lse_out) lse_out[row] = lse;
@@ -875,20 +902,14 @@ __global__ __launch_bounds__(TPR < 256 ? 256 : TPR) void k_ce_fwd_bwd(const uint
     if (t0 == 0) lse = leave();
     l = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(lse)));
   } else {
-    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (lane == 0) { shm[wv] = m; shs[wv] = s; }
-    __syncthreads();
-    if (t0 == 0) {
-      for (int k = 1; k < TPR / 64; k++) online_merge(m, s, shm[k], shs[k]);
-      sh_lse = leave();
-    }
+    if (t0 == 0) sh_lse = leave();
     __syncthreads();
     l = sh_lse;
   }
   const float scale = (g ? g[0] : 1.0f) * g_mul / (float)n;
   uint16_t *q = out + row * c;
 #pragma unroll
-  for (int k = 0; k < CHUNKS; k++) {
+  for (int k = 0; k < CHUNKS * V; k++) {
     const int j8 = t0 + k * TPR;
     if (j8 < nvec) {
       uint32_t o[4];
@@ -1243,15 +1264,18 @@ int32_t ah_cross_entropy(ah_ptr logits, int32_t dtype, ah_ptr targets, ah_ptr lo
   float *rows = (float *)scratch(sizeof(float) * (size_t)n);
   if (!rows) return fail(AH_ERR_OOM, "ah_cross_entropy: no scratch");
   auto go = [&](auto kfn, int tpr, auto *x) {
-    ah::launch_kernel(kfn, dim3((unsigned)(tpr < 256 ? cdiv(n, 256 / tpr) : n)), dim3(tpr < 256 ? 256 : tpr), 0, x, dp<const int32_t>(targets), rows,
+    ah::launch_kernel(kfn, dim3((unsigned)(tpr == 64 ? cdiv(n, 4) : n)), dim3((unsigned)ce_block(tpr)), 0, x, dp<const int32_t>(targets), rows,
                       dp<float>(lse_out), n, c);
   };
   if (dtype == AH_F32) {
-    if (ce_threads<float>(c) == 64) go(k_ce_fwd<float, 64>, 64, dp<const float>(logits));
-    else go(k_ce_fwd<float, 256>, 256, dp<const float>(logits));
-  } else if (ce_threads<uint16_t>(c) == 64) go(k_ce_fwd<uint16_t, 64>, 64, dp<const uint16_t>(logits));
-  else if (ce_threads<uint16_t>(c) == 256) go(k_ce_fwd<uint16_t, 256>, 256, dp<const uint16_t>(logits));
-  else go(k_ce_fwd<uint16_t, 512>, 512, dp<const uint16_t>(logits));
+    const float *x = dp<const float>(logits);
+    if (c <= 1024) go(k_ce_fwd<float, 64>, 64, x); else go(k_ce_fwd<float, 256>, 256, x);
+  } else {
+    const uint16_t *x = dp<const uint16_t>(logits);
+    if (c <= 2048) go(k_ce_fwd<uint16_t, 64>, 64, x);
+    else if (c <= 8192) go(k_ce_fwd<uint16_t, 256>, 256, x);
+    else go(k_ce_fwd<uint16_t, 512>, 512, x);
+  }
   AH_LAUNCH_CHECK();
   ah::launch_kernel(k_mean_rows, dim3(1), dim3(TPB), 0, rows, n, dp<float>(loss_out));
   AH_LAUNCH_CHECK();
@@ -1265,7 +1289,7 @@ int32_t ah_cross_entropy_bwd(ah_ptr logits, int32_t dtype, ah_ptr targets, ah_pt
   if (n == 0 || c == 0) return AH_OK;
   AH_ARG(logits && targets && lse && dlogits, "ah_cross_entropy_bwd: null operand");
   AH_ARG(n <= 65535 * 1024ll, "ah_cross_entropy_bwd: too many rows");
-  const int tpr = (dtype == AH_F32 ? ce_threads<float>(c) : ce_threads<uint16_t>(c)) == 64 ? 64 : 256, per = 256 / tpr;
+  const int tpr = c <= (dtype == AH_F32 ? 1024 : 2048) ? 64 : 256, per = 256 / tpr;
   const unsigned gx = (unsigned)cdiv(c, tpr == 64 ? c : TPB * 8);
   // gridDim.y is limited to 65535: fold rows beyond that by launching in row chunks
   for (int64_t r0 = 0; r0 < n; r0 += 65535 * (int64_t)per) {
@@ -1303,14 +1327,16 @@ int32_t ah_cross_entropy_fwd_bwd(ah_ptr logits, int32_t dtype, ah_ptr targets, a
   float *rows = (float *)scratch(sizeof(float) * (size_t)n);
   if (!rows) return fail(AH_ERR_OOM, "ah_cross_entropy_fwd_bwd: no scratch");
   auto go = [&](auto kfn, int tpr) {
-    ah::launch_kernel(kfn, dim3((unsigned)(tpr < 256 ? cdiv(n, 256 / tpr) : n)), dim3(tpr < 256 ? 256 : tpr), 0, dp<const uint16_t>(logits),
+    ah::launch_kernel(kfn, dim3((unsigned)(tpr == 64 ? cdiv(n, 4) : n)), dim3((unsigned)ce_block(tpr)), 0, dp<const uint16_t>(logits),
                       dp<const int32_t>(targets), rows, dp<float>(lse_out), dp<const float>(g_scalar), g_mul, dp<uint16_t>(dlogits), n, c);
   };
-  switch (ce_threads<uint16_t>(c)) {
-    case 64: if (c <= 512) go(k_ce_fwd_bwd<64, 1>, 64); else go(k_ce_fwd_bwd<64, 4>, 64); break;
-    case 256: go(k_ce_fwd_bwd<256, 4>, 256); break;
-    default: if (c <= 16384) go(k_ce_fwd_bwd<512, 4>, 512); else go(k_ce_fwd_bwd<512, CE_CLASSES / 8 / 512>, 512);
-  }
+  if (c <= 512) go(k_ce_fwd_bwd<64, 1, 1>, 64);
+  else if (c <= 1024) go(k_ce_fwd_bwd<64, 2, 1>, 64);
+  else if (c <= 2048) go(k_ce_fwd_bwd<64, 4, 1>, 64);
+  else if (c <= 4096) go(k_ce_fwd_bwd<256, 2, 1>, 256);
+  else if (c <= 8192) go(k_ce_fwd_bwd<256, 2, 2>, 256);
+  else if (c <= 16384) go(k_ce_fwd_bwd<512, 1, 4>, 512);
+  else go(k_ce_fwd_bwd<512, 1, CE_CLASSES / 8 / 512>, 512);
   AH_LAUNCH_CHECK();
   ah::launch_kernel(k_mean_rows, dim3(1), dim3(TPB), 0, rows, n, dp<float>(loss_out));
   AH_LAUNCH_CHECK();
