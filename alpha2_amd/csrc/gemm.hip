@@ -254,32 +254,39 @@ constexpr int GROUP_ROUND = 256;     // tiles that run at a time: one per CU
 // time, so a last round of t < 256 tiles costs a whole round.  Cutting the problems that make up that round in two along
 // k turns it into 2 t half-length tiles, which still run at once when t <= 128: the round then costs half.  Chooses whole
 // problems from the end of the list whose tiles add up to between t and 128 and returns their indices (ascending), or
-// nothing when no such choice exists.
-std::vector<int> split_tail(const AhGemm *descs, int count, int64_t blocks, int bn) {
+// nothing when no such choice exists.  The tiles are counted at 256 columns whatever group_width takes: the order in which a
+// problem's products are added up depends on the shapes alone, not on a tile's width.
+std::vector<int> split_tail(const AhGemm *descs, int count) {
   std::vector<int> chosen;
+  auto tiles = [&](int i) { return cdiv(descs[i].m, 256) * cdiv(descs[i].n, 256); };
+  int64_t blocks = 0;
+  for (int i = 0; i < count; i++) blocks += tiles(i);
   const int64_t tail = blocks % GROUP_ROUND;
   if (descs[0].out_dtype != AH_F32 || tail == 0 || tail > GROUP_ROUND / 2) return chosen;
   int64_t sum = 0;
   for (int i = count - 1; i >= 0 && sum < tail; i--) {
-    const AhGemm &q = descs[i];
-    const int64_t t = cdiv(q.m, 256) * cdiv(q.n, bn);
-    if (q.k % 128 != 0 || q.n % 4 != 0 || sum + t > GROUP_ROUND / 2) continue;
+    if (descs[i].k % 128 != 0 || descs[i].n % 4 != 0 || sum + tiles(i) > GROUP_ROUND / 2) continue;
     chosen.insert(chosen.begin(), i);
-    sum += t;
+    sum += tiles(i);
   }
   if (sum < tail) chosen.clear();
   return chosen;
 }
 // Columns of a group's tiles: 256, or 192 or 128 (weight gradients in f32 only) where edge tiles and rounds waste that much more of the wide ones.
 // A narrower tile reads more from LDS per flop: 3 % slower at 192, half as slow again at 128, and is taken from 5 % on.  us at
-// 256 / 192 / 128 columns, all the weight gradients of a model: 8 layers x 384 of 10240 tokens 389 / 303 / 337, 6 x 320 of 8192 177 / 151 / 176, 4 x 192 of
-// 8192 89 / 76 / 65, 2 x 128 of 128 14.0 / 13.1 / 12.0, 2 x 576 of 4096 95 / 79 / 107; 4 x 512 of 8192 175 / 225 / 204, 12 x 768 of 16384 3008 / 3138 / 3431.
-int group_width(const AhGemm *descs, int count) {
+// 256 / 192 / 128 columns, all the weight gradients of a model: 6 layers x 320 of 8192 tokens 176 / 149 / 192, 4 x 192 of 8192 91 / 78 / 69, 2 x 128 of 128
+// 14.1 / 13.1 / 12.4, 2 x 576 of 4096 94 / 83 / 106; 8 x 384 of 10240 358 / 356 / 358, 4 x 512 of 8192 174 / 262 / 204, 12 x 768 of 16384 2982 / 3139 / 3436.
+int group_width(const AhGemm *descs, int count, const std::vector<int> &halved) {
   if (descs[0].layout != AH_GEMM_TN || descs[0].out_dtype != AH_F32) return 256;
   auto cost = [&](int bn) {
-    int64_t tiles = 0;
-    for (int i = 0; i < count; i++) tiles += cdiv(descs[i].m, 256) * cdiv(descs[i].n, bn);
-    const double rounds = split_tail(descs, count, tiles, bn).empty() ? (double)cdiv(tiles, GROUP_ROUND) : (double)(tiles / GROUP_ROUND) + 0.5;
+    int64_t whole = 0, halves = 0;
+    for (int i = 0, c = 0; i < count; i++) {
+      const int64_t tiles = cdiv(descs[i].m, 256) * cdiv(descs[i].n, bn);
+      if (c < (int)halved.size() && halved[c] == i) { halves += 2 * tiles; c++; } else whole += tiles;
+    }
+    // the half-length tiles come last: two each where the last round of whole ones leaves a CU free, then in half rounds
+    const int64_t last = whole % GROUP_ROUND, beside = last ? 2 * (GROUP_ROUND - last) : 0;
+    const double rounds = (double)cdiv(whole, GROUP_ROUND) + (halves > beside ? 0.5 * (double)cdiv(halves - beside, GROUP_ROUND) : 0.0);
     return rounds * bn * (bn == 256 ? 0.95 : bn == 192 ? 1.03 : 1.5);
   };
   const double wide = cost(256), mid = cost(192), narrow = cost(128);
@@ -334,16 +341,16 @@ static int32_t grouped_tables(const char *who, const AhGemm *descs, int32_t coun
     e.M = (int)q.m; e.N = (int)q.n; e.K = (int)q.k;
     e.lda = q.lda; e.ldb = q.ldb; e.ldc = q.ldc;
   }
-  const int bn = group_width(descs, count);
+  // the problems that make up a short last round are cut in two along k: they move to the end of the table as pairs of
+  // entries, the second of which writes the workspace
+  const std::vector<int> chosen = split_tail(descs, count);
+  const int bn = group_width(descs, count, chosen);
   *bn_out = bn;
   for (GemmGroupEntry &e : tab) {
     e.tile_start = (int)blocks;
     blocks += cdiv(e.M, 256) * cdiv(e.N, bn);
     AH_ARG(blocks < (1ll << 31), "%s: too many tiles", who);
   }
-  // the problems that make up a short last round are cut in two along k: they move to the end of the table as pairs of
-  // entries, the second of which writes the workspace
-  const std::vector<int> chosen = split_tail(descs, count, blocks, bn);
   *ws_bytes = 0;
   if (!chosen.empty()) {
     for (int i : chosen) *ws_bytes += descs[i].m * descs[i].n * 4;
