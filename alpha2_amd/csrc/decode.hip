@@ -546,9 +546,11 @@ __global__ __launch_bounds__(512, 2) void k_decode_chain(DecodeChain a) {
   const int f = threadIdx.x & (a.lanes - 1), keys = 256 / a.lanes, key = threadIdx.x / a.lanes;
   const bool has_f = 4 * f < a.head_size;
   const int64_t pitch = 3 * (int64_t)C;
-  auto load_keys = [&](int l, int unit, int j0) {                      // of keys j0 + key + u KEYS of the unit's slice; the newest comes through `fresh`
+  // of keys j0 + key + u KEYS of the unit's slice; the newest comes through `fresh`.  The first token of all has no earlier row: its
+  // loads go to the weights (3 rows of C and more), for values that are not used.
+  auto load_keys = [&](int l, int unit, int j0) {
     const int h = unit % a.heads, begin = unit / a.heads * a.slice, count = min(a.slice, a.n - begin);
-    const float *p = a.kv + l * a.layer_stride + C + h * a.head_size + 4 * (has_f ? f : 0);
+    const float *p = (a.n > 1 ? a.kv + l * a.layer_stride : at(a.layer[l].wqkv)) + C + h * a.head_size + 4 * (has_f ? f : 0);
 #pragma unroll
     for (int u = 0; u < U; u++) {
       const float *row = p + (int64_t)max(0, min(begin + min(j0 + u * keys + key, count - 1), a.n - 2)) * pitch;
@@ -601,7 +603,8 @@ __global__ __launch_bounds__(512, 2) void k_decode_chain(DecodeChain a) {
 #pragma unroll
         for (int u = 0; u < U; u++) {
           const int j = j0 + u * keys + key;
-          if (begin + j == a.n - 1) { kk[u] = ldq(fresh[1], has_f ? f : 0); vv[u] = ldq(fresh[2], has_f ? f : 0); }
+          if (j >= count) vv[u] = none;               // whatever was loaded for it: its weight is zero, and zero times an infinity is not
+          else if (begin + j == a.n - 1) { kk[u] = ldq(fresh[1], has_f ? f : 0); vv[u] = ldq(fresh[2], has_f ? f : 0); }
           const float s = group_sum(has_f ? dot4(q, kk[u], 0.f) : 0.f, a.lanes);
           mine = (f & (U - 1)) == u ? s : mine;
         }

@@ -235,3 +235,27 @@ def test_a_launch_that_gave_up_is_computed_again(B, width, heads, act):
     for n, (a, b) in enumerate(zip(rows[:20], rows[20:])):
         assert np.array_equal(a, b), n + 61
     kept.close()
+
+
+@pytest.mark.parametrize("layers,width,heads,act", [(2, 64, 8, "gelu"), (1, 256, 2, "swiglu"), (2, 512, 16, "silu"), (33, 64, 2, "gelu"), (2, 520, 5, "relu"), (1, 768, 12, "gelu")])
+def test_the_first_token_reads_no_row_of_the_cache(B, layers, width, heads, act):
+    """Position 0 on, in one launch and in launches, over a cache of NaN: rows 0 .. pos - 1 are read, and those are written before."""
+    import ctypes
+
+    from alpha2_amd import _ffi as ffi
+    from alpha2_amd.decode import KeptContext
+    from alpha2_amd.sample import _lastRow
+    cfg, params = _model(B, 90, 70, layers, width, heads, ffnActivation=act)
+    tokens = np.random.RandomState(8).randint(0, 90, 70).astype(np.int32)
+    kept, exact = KeptContext.of(cfg, params, B, 70), _logits64(cfg, params, tokens)
+    off = lambda row, n: np.linalg.norm(row.astype(np.float64) - exact[n]) / np.linalg.norm(exact[n])
+    for count in (1, 2, 70):                     # (again from position 0, over what the run before has left behind it)
+        ffi.check(B.lib.ah_fill_f32(kept.kv._buf.ptr, float("nan"), kept.kv.size))
+        ours, theirs = [], []
+        for n in range(count):
+            ffi.check(B.lib.ah_decode(ctypes.byref(kept.model), kept.layers, int(tokens[n]), n))
+            ours.append(off(B._download(kept.logits), n))
+            theirs.append(off(_lastRow(cfg, params, B, tokens[:n + 1], B.releaseGpuTensor), n))
+        ours, theirs = (math.sqrt(np.mean(np.square(e))) for e in (ours, theirs))
+        assert ours <= max(1.5 * theirs, 8 * (cfg.nLayer + 1) * 2.0 ** -24), (count, ours, theirs)      # the bound of _compare
+    kept.close()
