@@ -156,6 +156,7 @@ SIGNATURES = {
     "ah_probe_issue": [i32, i32, i32, C.POINTER(C.c_double)],
     "ah_flash_fwd": [C.POINTER(AhFlash)], "ah_flash_bwd": [C.POINTER(AhFlash)],
     "ah_decode": [C.POINTER(AhDecode), C.POINTER(AhDecodeLayer), i32, i32], "ah_decode_head": [C.POINTER(AhDecode), u64],
+    "ah_decode_stats": [p_i64, p_i64], "ah_decode_next_ticks": [i32],
     "ah_adamw": [u64, u64, u64, u64, u64, C.POINTER(AhAdamW), u64, u64, u64],
     "ah_clip_coef": [u64, f32, f32, u64],
     "ah_side_begin": [], "ah_side_end": [], "ah_side_join": [],

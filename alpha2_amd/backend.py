@@ -259,6 +259,12 @@ class HipBackend:
         s = self._stats()
         return {"recorded": s.steps_recorded, "replayed": s.steps_replayed, "fellBack": s.steps_fallback, "nodeUpdates": s.step_node_updates}
 
+    def decodeStats(self) -> dict:
+        """Tokens from kept keys and values that were one launch, and those computed again because the GPU was shared."""
+        one, again = C.c_int64(), C.c_int64()
+        check(self.lib.ah_decode_stats(C.byref(one), C.byref(again)))
+        return {"oneLaunch": one.value, "computedAgain": again.value}
+
     def syncGpu(self):
         check(self.lib.ah_sync())
 

@@ -302,18 +302,23 @@ __global__ __launch_bounds__(256) void k_decode_attention(DecodeAttention a) {
 // phases since the earlier use, and those were computed after their inputs had been read: nobody reads the old words any more.
 // All workgroups have to be on the chip at once, which the grid's size allows but nothing guarantees while other processes use the GPU.
 // So every wait ends: after SPIN_TICKS, or as soon as another workgroup has given up, a workgroup leaves `chain_gave_up` and ends, and the launch
-// behind it, of one workgroup that depends on no other, computes the token again (and otherwise ends at once).
+// behind it computes the token again (and otherwise ends at once).  That one is a single workgroup: its waits are for words that its own waves write, which
+// are on the chip when it is, so no clock ends them - time in which the queue is switched off the chip does not count - but a number of tries
+// does, that no healthy wait comes near.  Its logits are NaN until it has computed them, and `chain_again` counts it (ah_decode_stats).  The tokens
+// behind it take one launch again: sums are cut elsewhere in the launches of a layer, and what a program computes does not depend on who else uses the GPU.
 // What bounds it is that chain of trips, 1.3 us at least and 2 to 3 as polled, five a layer, and between them the one wave that has the next step
 // (350 instructions in a row are 1 us).  A token, its logits read and chosen from, 64 of them behind a prompt of 17 (with the prompt's pass and the pass
 // over the result): 6 layers x 256 186 -> 142 us, 4 x 128 112 -> 99, 2 x 64 87 -> 73; 24 behind 200: 8 x 384 327 -> 298, 8 x 512 365 -> 316.  The
 // kernel alone: 6 x 256 96 us, 16 a layer, against 23 in launches.  All rows ahead have to be asked for unconditionally: behind branches the
 // compiler waits for the newest of them before the oldest (attention 2.3 -> 1.9 us).
 constexpr int CHAIN_LAYERS = 32, CHAIN_NV = 2, CHAIN_UNITS = 4;      // at most: layers; 1024 wide, ffn 4096; keys a lane holds
-constexpr int64_t SPIN_TICKS = 5000000;                              // of 10 ns
+constexpr int64_t SPIN_TICKS = 1000000;                              // of 10 ns; computing again takes 0.7 ms (4 x 128) to 9.6 (12 x 512)
+constexpr int RESCUE_TRIES = 1 << 24;                                // 10 s and more at a microsecond a try
 enum { WORD_QKV = 0, WORD_SUMS = 3072, WORD_TOPS = WORD_SUMS + MAX_SLICES * 1024, WORD_MID = WORD_TOPS + MAX_SLICES * 128 * 2,
        WORD_HID = WORD_MID + 1024, WORD_STREAM = WORD_HID + 4096, WORDS = WORD_STREAM + 1024 };
 __device__ uint64_t chain_words[WORDS];
 __device__ uint32_t chain_gave_up;              // the first tag of the launch that did
+__device__ uint64_t chain_again;                // tokens computed again
 
 struct DecodeChain {
   AhDecodeLayer layer[CHAIN_LAYERS];
@@ -322,7 +327,8 @@ struct DecodeChain {
   float *kv, *logits;
   int vocab, width, heads, head_size, ffn, layers, mask, n, slices, slice, lanes;      // lanes: of a head's features, four each, a power of two
   int64_t layer_stride;                         // of kv
-  int64_t ticks;                                // a wait's end
+  int64_t ticks;                                // a wait's end; in the launch that computes a token again it is `tries`
+  int32_t tries;
   float scale, cap, eps;
   uint32_t tag;                                 // layer i's words bear tag + i
   uint32_t rescue;                              // 0, or the first tag of the launch that this one computes again if it gave up
@@ -335,7 +341,7 @@ __device__ __forceinline__ void put(int at, uint32_t tag, float v) {
 __device__ __forceinline__ uint64_t peek(int at) { return __hip_atomic_load(chain_words + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 // The words index(i), i < N, once all of them (of all lanes) bear the tag; false: given up
 template <int N, class Index>
-__device__ __forceinline__ bool take(uint32_t tag, uint32_t launch, int64_t ticks, Index index, float (&v)[N]) {
+__device__ __forceinline__ bool take(const DecodeChain &a, uint32_t tag, Index index, float (&v)[N]) {
   int64_t since = 0;
   for (int tries = 1;; tries++) {
     uint64_t w[N];
@@ -345,11 +351,13 @@ __device__ __forceinline__ bool take(uint32_t tag, uint32_t launch, int64_t tick
 #pragma unroll
     for (int i = 0; i < N; i++) { other |= (uint32_t)(w[i] >> 32) ^ tag; v[i] = __uint_as_float((uint32_t)w[i]); }
     if (__all(other == 0)) return true;
-    if ((tries & 63) == 0 || ticks < 0) {
+    if (a.rescue) {
+      if (tries >= a.tries) return false;
+    } else if ((tries & 63) == 0 || a.ticks < 0) {
       const int64_t now = wall_clock64();
       if (since == 0) since = now;
-      if (now - since > ticks || __hip_atomic_load(&chain_gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == launch) {
-        __hip_atomic_store(&chain_gave_up, launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (now - since > a.ticks || __hip_atomic_load(&chain_gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == a.tag) {
+        __hip_atomic_store(&chain_gave_up, a.tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return false;
       }
     }
@@ -379,6 +387,10 @@ __global__ __launch_bounds__(512, 2) void k_decode_chain(DecodeChain a) {
   const int units = a.slices * a.heads;
   const bool in_c = blockIdx.x * 4 < (unsigned)C, in_qkv = blockIdx.x * 4 < (unsigned)(3 * C), in_f = blockIdx.x * 4 < (unsigned)F;
   if (threadIdx.x == 0) quit = 0;
+  if (a.rescue) {
+    for (int i = threadIdx.x; i < a.vocab; i += 512) a.logits[i] = __builtin_nanf("");
+    if (threadIdx.x == 0) __hip_atomic_fetch_add(&chain_again, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
   __syncthreads();
 
   auto at = [](ah_ptr p) { return reinterpret_cast<const float *>(static_cast<uintptr_t>(p)); };
@@ -406,7 +418,7 @@ __global__ __launch_bounds__(512, 2) void k_decode_chain(DecodeChain a) {
       }
     };
     auto take_row = [&](int words, uint32_t tag, float (&x)[E]) {
-      if (!take<E>(tag, a.tag, a.ticks, [&](int i) { return words + min(lane + 64 * i, C - 1); }, x)) quit = 1;
+      if (!take<E>(a, tag, [&](int i) { return words + min(lane + 64 * i, C - 1); }, x)) quit = 1;
     };
     int head2[NV];
 #pragma unroll
@@ -435,7 +447,7 @@ __global__ __launch_bounds__(512, 2) void k_decode_chain(DecodeChain a) {
         if (ct < 128) {
           float x[3];
           const int from = WORD_QKV + unit % a.heads * a.head_size + min(ct, a.head_size - 1);
-          if (!take<3>(tag, a.tag, a.ticks, [&](int i) { return from + i * C; }, x)) quit = 1;
+          if (!take<3>(a, tag, [&](int i) { return from + i * C; }, x)) quit = 1;
 #pragma unroll
           for (int i = 0; i < 3; i++) fresh[i][ct] = x[i];
         }
@@ -449,11 +461,11 @@ __global__ __launch_bounds__(512, 2) void k_decode_chain(DecodeChain a) {
         const int ntops = units * 2;
         float x[NV * S + 1];
         auto sums = [&](int s0, int e) { return WORD_SUMS + min(s0 + e % S, a.slices - 1) * C + min(ct + 256 * (e / S), C - 1); };
-        if (!take<NV * S + 1>(tag, a.tag, a.ticks, [&](int e) { return e == 0 ? WORD_TOPS + min(ct, ntops - 1) : sums(0, e - 1); }, x)) quit = 1;
+        if (!take<NV * S + 1>(a, tag, [&](int e) { return e == 0 ? WORD_TOPS + min(ct, ntops - 1) : sums(0, e - 1); }, x)) quit = 1;
         if (ct < ntops) tops[ct] = x[0];
         for (int t = ct + 256; t - ct < ntops; t += 256) {
           float y[1];
-          if (!take<1>(tag, a.tag, a.ticks, [&](int) { return WORD_TOPS + min(t, ntops - 1); }, y)) quit = 1;
+          if (!take<1>(a, tag, [&](int) { return WORD_TOPS + min(t, ntops - 1); }, y)) quit = 1;
           if (t < ntops) tops[t] = y[0];
         }
         __syncthreads();
@@ -463,7 +475,7 @@ __global__ __launch_bounds__(512, 2) void k_decode_chain(DecodeChain a) {
         for (int i = 0; i < NV; i++) { most[i] = -INFINITY; sum[i] = v[i] = 0.f; }
         for (int s0 = 0; s0 < a.slices; s0 += S) {
           float y[NV * S];
-          if (s0 > 0 && !take<NV * S>(tag, a.tag, a.ticks, [&](int e) { return sums(s0, e); }, y)) { quit = 1; break; }
+          if (s0 > 0 && !take<NV * S>(a, tag, [&](int e) { return sums(s0, e); }, y)) { quit = 1; break; }
 #pragma unroll
           for (int i = 0; i < NV; i++) {
             const float *top = tops + head2[i];
@@ -502,7 +514,7 @@ __global__ __launch_bounds__(512, 2) void k_decode_chain(DecodeChain a) {
       }
       if (in_c) {
         float x[E];
-        if (!take<E>(tag, a.tag, a.ticks, [&](int i) { return WORD_HID + min(ct + 256 * i, F - 1); }, x)) quit = 1;
+        if (!take<E>(a, tag, [&](int i) { return WORD_HID + min(ct + 256 * i, F - 1); }, x)) quit = 1;
 #pragma unroll
         for (int i = 0; i < E; i++) if (ct + 256 * i < F) hid[ct + 256 * i] = x[i];
         __syncthreads();
@@ -809,7 +821,8 @@ int chain_quads(const AhDecode *d) {
   return nv <= CHAIN_NV ? (int)nv : 0;
 }
 thread_local int64_t next_ticks = SPIN_TICKS;
-int32_t launch_chain(const AhDecode *d, const AhDecodeLayer *layers, int32_t token, int32_t pos, int nv) {
+std::atomic<int64_t> chain_tokens{0};
+int32_t launch_chain(const AhDecode *d, const AhDecodeLayer *layers, int32_t token, int32_t pos, int nv, int64_t ticks) {
   static std::atomic<uint32_t> tags{1};
   const int C = d->width, H = d->heads, hs = C / H, n = pos + 1;
   const uint32_t used = 2 * (uint32_t)d->layers;
@@ -838,14 +851,15 @@ int32_t launch_chain(const AhDecode *d, const AhDecodeLayer *layers, int32_t tok
   const int rows = std::max(std::max(3 * C, d->ffn), std::max(d->vocab, 4 * a.slices * H));
   const unsigned grid = (unsigned)std::min<int64_t>(cdiv(rows, 4), ah::num_cus());
   auto go = [&](auto kfn) {
-    a.tag = tag; a.rescue = 0; a.ticks = next_ticks;
+    a.tag = tag; a.rescue = 0; a.ticks = ticks;
     ah::launch_kernel(kfn, dim3(grid), dim3(512), 0, a);
-    a.rescue = tag; a.tag = tag + (uint32_t)d->layers; a.ticks = next_ticks = SPIN_TICKS;
+    a.rescue = tag; a.tag = tag + (uint32_t)d->layers; a.tries = ticks < -1 ? 1 : RESCUE_TRIES;
     ah::launch_kernel(kfn, dim3(1), dim3(512), 0, a);
   };
   if (gated) { if (nv == 1) go(k_decode_chain<1, true>); else go(k_decode_chain<2, true>); }
   else { if (nv == 1) go(k_decode_chain<1, false>); else go(k_decode_chain<2, false>); }
   AH_LAUNCH_CHECK();
+  chain_tokens++;
   return AH_OK;
 }
 
@@ -853,10 +867,20 @@ int32_t launch_chain(const AhDecode *d, const AhDecodeLayer *layers, int32_t tok
 
 extern "C" {
 
-// For tests: when the waits of this thread's next token in one launch end (below 0: a word that is not there at once), so that the launch behind it
-// computes the token.
 int32_t ah_decode_next_ticks(int32_t ticks) {
   next_ticks = ticks;
+  return AH_OK;
+}
+
+int32_t ah_decode_stats(int64_t *one_launch, int64_t *again) {
+  AH_REQUIRE_READY();
+  AH_ARG(one_launch && again, "ah_decode_stats: null result");
+  if (ah::step_active() || ah::capturing()) return fail(AH_ERR_STATE, "ah_decode_stats: not inside a capture or a step plan");
+  AH_HIP(hipStreamSynchronize(ah::stream()));
+  uint64_t n = 0;
+  AH_HIP(hipMemcpyFromSymbol(&n, HIP_SYMBOL(chain_again), sizeof(n)));
+  *one_launch = chain_tokens.load();
+  *again = (int64_t)n;
   return AH_OK;
 }
 
@@ -873,6 +897,7 @@ int32_t ah_decode_head(const AhDecode *d, ah_ptr row) {
 }
 
 int32_t ah_decode(const AhDecode *d, const AhDecodeLayer *layers, int32_t token, int32_t pos) {
+  const int64_t ticks = std::exchange(next_ticks, SPIN_TICKS);      // (for this token, whichever way it goes)
   AH_REQUIRE_READY();
   { const int32_t rc = check_model(d); if (rc != AH_OK) return rc; }
   AH_ARG(d->layers > 0 && layers && d->wte && d->wpe && d->kv, "ah_decode: null operand");
@@ -886,7 +911,7 @@ int32_t ah_decode(const AhDecode *d, const AhDecodeLayer *layers, int32_t token,
     AH_ARG(l.ln1_w && l.ln1_b && l.wqkv && l.wo && l.ln2_w && l.ln2_b && l.fc1 && l.fc2 && (!gated || l.up), "ah_decode: null weight in layer %d", i);
     AH_ARG(aligned16(l.ln1_w | l.ln1_b | l.wqkv | l.wo | l.ln2_w | l.ln2_b | l.fc1 | l.fc2 | l.up), "ah_decode: weights of layer %d must be 16-byte aligned", i);
   }
-  if (const int nv = chain_quads(d)) return launch_chain(d, layers, token, pos, nv);
+  if (const int nv = chain_quads(d)) return launch_chain(d, layers, token, pos, nv, ticks);
   const int C = d->width, H = d->heads, n = pos + 1;
   const int slices = (int)(cdiv(n, MIN_SLICE) < MAX_SLICES ? cdiv(n, MIN_SLICE) : MAX_SLICES);
   // the residual stream, the MLP's hidden row, the slices' sums and their maxima; stream-ordered, so it may go back at once

@@ -40,6 +40,8 @@ export const lib = dlopen(process.env.ALPHA_HIP_LIB ?? "libalpha_hip.so", {
   ah_cross_entropy_fwd_bwd:        { args: [u64, i32, u64, u64, u64, u64, f32, u64, i64, i64], returns: i32 },
   ah_decode:                       { args: [ptr, ptr, i32, i32], returns: i32 },
   ah_decode_head:                  { args: [ptr, u64], returns: i32 },
+  ah_decode_next_ticks:            { args: [i32], returns: i32 },
+  ah_decode_stats:                 { args: [ptr, ptr], returns: i32 },
   ah_device_info:                  { args: [ptr], returns: i32 },
   ah_download:                     { args: [ptr, u64, u64], returns: i32 },
   ah_download_begin:               { args: [u64, u64, ptr], returns: i32 },

@@ -212,8 +212,9 @@ def test_a_token_in_one_launch(B, vocab, ctx, layers, width, heads, more):
     from alpha2_amd.decode import KeptContext
     cfg, params = _model(B, vocab, ctx, layers, width, heads, **more)
     tokens = np.random.RandomState(3).randint(0, vocab, ctx).astype(np.int32)
-    kept = KeptContext.of(cfg, params, B, ctx)
+    kept, before = KeptContext.of(cfg, params, B, ctx), B.decodeStats()["oneLaunch"]
     _compare(kept, cfg, params, B, tokens, range(1, ctx + 1), False)
+    assert B.decodeStats()["oneLaunch"] - before == (ctx - 1 if layers <= 32 else 0)
     kept.close()
 
 
@@ -224,7 +225,7 @@ def test_a_launch_that_gave_up_is_computed_again(B, width, heads, act):
     cfg, params = _model(B, 70, 80, 2, width, heads, ffnActivation=act)
     tokens = np.random.RandomState(6).randint(0, 70, 80).astype(np.int32)
     kept = KeptContext.of(cfg, params, B, 80)
-    rows = []
+    rows, before = [], B.decodeStats()
     for given_up in (False, True):
         kept.known = 0
         kept.lastRow(tokens[:60], B.releaseGpuTensor)
@@ -232,9 +233,49 @@ def test_a_launch_that_gave_up_is_computed_again(B, width, heads, act):
             if given_up and n % 3 == 0:
                 B.lib.ah_decode_next_ticks(-1)
             rows.append(kept.lastRow(tokens[:n], B.releaseGpuTensor).copy())
+    after = B.decodeStats()
+    assert after["oneLaunch"] - before["oneLaunch"] == 40 and after["computedAgain"] - before["computedAgain"] == 6
     for n, (a, b) in enumerate(zip(rows[:20], rows[20:])):
         assert np.array_equal(a, b), n + 61
     kept.close()
+
+
+def test_a_computation_that_is_given_up_twice_is_seen(B):
+    """Its logits are not those of the token before but NaN; the contexts behind it are computed as ever."""
+    from alpha2_amd.decode import KeptContext
+    cfg, params = _model(B, 70, 80, 2, 64, 2)
+    tokens = np.random.RandomState(6).randint(0, 70, 80).astype(np.int32)
+    kept = KeptContext.of(cfg, params, B, 80)
+    kept.lastRow(tokens[:60], B.releaseGpuTensor)
+    want = kept.lastRow(tokens[:61], B.releaseGpuTensor).copy()
+    B.lib.ah_decode_next_ticks(-2)
+    assert np.isnan(kept.lastRow(tokens[:62], B.releaseGpuTensor)).all()
+    kept.known = 0
+    kept.lastRow(tokens[:60], B.releaseGpuTensor)
+    assert np.array_equal(kept.lastRow(tokens[:61], B.releaseGpuTensor), want)
+    kept.close()
+
+
+def test_the_end_of_waits_is_one_tokens(B):
+    """Set for a token that takes the launches of a layer or is refused, it does not wait for a later one."""
+    import ctypes
+
+    from alpha2_amd.decode import KeptContext
+    small, wide = (KeptContext.of(*_model(B, 40, 16, 1, width, heads), B, 16) for width, heads in ((64, 2), (576, 6)))
+    tokens = np.arange(16, dtype=np.int32)
+    for kept in (small, wide):
+        kept.lastRow(tokens[:3], B.releaseGpuTensor)
+    again = B.decodeStats()["computedAgain"]
+    for token in (3, 4):
+        B.lib.ah_decode_next_ticks(-1)
+        if token == 3:
+            wide.lastRow(tokens[:4], B.releaseGpuTensor)
+        else:
+            assert B.lib.ah_decode(ctypes.byref(small.model), small.layers, 99, 4) != 0
+        small.lastRow(tokens[:token + 1], B.releaseGpuTensor)
+    assert B.decodeStats()["computedAgain"] == again
+    for kept in (small, wide):
+        kept.close()
 
 
 @pytest.mark.parametrize("layers,width,heads,act", [(2, 64, 8, "gelu"), (1, 256, 2, "swiglu"), (2, 512, 16, "silu"), (33, 64, 2, "gelu"), (2, 520, 5, "relu"), (1, 768, 12, "gelu")])
