@@ -380,18 +380,26 @@ __global__ __launch_bounds__(512, 2) void k_decode_chain(DecodeChain a) {
   __shared__ __attribute__((aligned(16))) float fresh[3][128];         // the new row's q, k, v of a head
   __shared__ __attribute__((aligned(16))) float part_o[4][128];
   __shared__ float part_m[4], part_l[4], tops[MAX_SLICES * 128 * 2];
-  __shared__ int quit;
+  __shared__ int quit[2];
   if (a.rescue && __hip_atomic_load(&chain_gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != a.rescue) return;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, C = a.width, F = a.ffn, nv = C >> 2, nf = F >> 2;
   const int G = gridDim.x, W = 4 * G, gw = blockIdx.x * 4 + wave;      // row gw + r W of a matrix is this wave's
   const int units = a.slices * a.heads;
   const bool in_c = blockIdx.x * 4 < (unsigned)C, in_qkv = blockIdx.x * 4 < (unsigned)(3 * C), in_f = blockIdx.x * 4 < (unsigned)F;
-  if (threadIdx.x == 0) quit = 0;
+  if (threadIdx.x < 2) quit[threadIdx.x] = 0;
   if (a.rescue) {
     for (int i = threadIdx.x; i < a.vocab; i += 512) a.logits[i] = __builtin_nanf("");
     if (threadIdx.x == 0) __hip_atomic_fetch_add(&chain_again, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   __syncthreads();
+  // A barrier behind which all waves see the same: has one given up before it?  Two words in turns, since a wave may have given up on the next phase
+  // before another has read what the last one left.
+  int turn = 0;
+  auto meet = [&]() {
+    __syncthreads();
+    turn ^= 1;
+    return quit[turn ^ 1] != 0;
+  };
 
   auto at = [](ah_ptr p) { return reinterpret_cast<const float *>(static_cast<uintptr_t>(p)); };
   // The two kinds of waves run loops of their own, so that neither's registers are kept through the other's code; both come to the same barriers.
@@ -418,7 +426,7 @@ __global__ __launch_bounds__(512, 2) void k_decode_chain(DecodeChain a) {
       }
     };
     auto take_row = [&](int words, uint32_t tag, float (&x)[E]) {
-      if (!take<E>(a, tag, [&](int i) { return words + min(lane + 64 * i, C - 1); }, x)) quit = 1;
+      if (!take<E>(a, tag, [&](int i) { return words + min(lane + 64 * i, C - 1); }, x)) quit[turn] = 1;
     };
     int head2[NV];
 #pragma unroll
@@ -440,19 +448,17 @@ __global__ __launch_bounds__(512, 2) void k_decode_chain(DecodeChain a) {
           norm(x, stream);
           load_norm(a.layer[l].ln2_w, a.layer[l].ln2_b);
         }
-        __syncthreads();
-        if (quit) return;
+        if (meet()) return;
       }
       for (int unit = blockIdx.x; unit < units; unit += G) {
         if (ct < 128) {
           float x[3];
           const int from = WORD_QKV + unit % a.heads * a.head_size + min(ct, a.head_size - 1);
-          if (!take<3>(a, tag, [&](int i) { return from + i * C; }, x)) quit = 1;
+          if (!take<3>(a, tag, [&](int i) { return from + i * C; }, x)) quit[turn] = 1;
 #pragma unroll
           for (int i = 0; i < 3; i++) fresh[i][ct] = x[i];
         }
-        __syncthreads();
-        if (quit) return;
+        if (meet()) return;
         __syncthreads();
       }
       if (in_c) {
@@ -461,21 +467,20 @@ __global__ __launch_bounds__(512, 2) void k_decode_chain(DecodeChain a) {
         const int ntops = units * 2;
         float x[NV * S + 1];
         auto sums = [&](int s0, int e) { return WORD_SUMS + min(s0 + e % S, a.slices - 1) * C + min(ct + 256 * (e / S), C - 1); };
-        if (!take<NV * S + 1>(a, tag, [&](int e) { return e == 0 ? WORD_TOPS + min(ct, ntops - 1) : sums(0, e - 1); }, x)) quit = 1;
+        if (!take<NV * S + 1>(a, tag, [&](int e) { return e == 0 ? WORD_TOPS + min(ct, ntops - 1) : sums(0, e - 1); }, x)) quit[turn] = 1;
         if (ct < ntops) tops[ct] = x[0];
         for (int t = ct + 256; t - ct < ntops; t += 256) {
           float y[1];
-          if (!take<1>(a, tag, [&](int) { return WORD_TOPS + min(t, ntops - 1); }, y)) quit = 1;
+          if (!take<1>(a, tag, [&](int) { return WORD_TOPS + min(t, ntops - 1); }, y)) quit[turn] = 1;
           if (t < ntops) tops[t] = y[0];
         }
-        __syncthreads();
-        if (quit) return;
+        if (meet()) return;
         float most[NV], sum[NV], v[NV];
 #pragma unroll
         for (int i = 0; i < NV; i++) { most[i] = -INFINITY; sum[i] = v[i] = 0.f; }
         for (int s0 = 0; s0 < a.slices; s0 += S) {
           float y[NV * S];
-          if (s0 > 0 && !take<NV * S>(a, tag, [&](int e) { return sums(s0, e); }, y)) { quit = 1; break; }
+          if (s0 > 0 && !take<NV * S>(a, tag, [&](int e) { return sums(s0, e); }, y)) { quit[turn] = 1; break; }
 #pragma unroll
           for (int i = 0; i < NV; i++) {
             const float *top = tops + head2[i];
@@ -497,8 +502,7 @@ __global__ __launch_bounds__(512, 2) void k_decode_chain(DecodeChain a) {
         }
 #pragma unroll
         for (int i = 0; i < NV; i++) if (ct + 256 * i < C) joined[ct + 256 * i] = v[i] / sum[i];
-        __syncthreads();
-        if (quit) return;
+        if (meet()) return;
       }
       if (in_f || in_c) {
         if (wave == 4) {
@@ -509,16 +513,14 @@ __global__ __launch_bounds__(512, 2) void k_decode_chain(DecodeChain a) {
           const bool last = l + 1 == a.layers;
           load_norm(last ? a.lnf_w : a.layer[l + 1].ln1_w, last ? a.lnf_b : a.layer[l + 1].ln1_b);
         }
-        __syncthreads();
-        if (quit) return;
+        if (meet()) return;
       }
       if (in_c) {
         float x[E];
-        if (!take<E>(a, tag, [&](int i) { return WORD_HID + min(ct + 256 * i, F - 1); }, x)) quit = 1;
+        if (!take<E>(a, tag, [&](int i) { return WORD_HID + min(ct + 256 * i, F - 1); }, x)) quit[turn] = 1;
 #pragma unroll
         for (int i = 0; i < E; i++) if (ct + 256 * i < F) hid[ct + 256 * i] = x[i];
-        __syncthreads();
-        if (quit) return;
+        if (meet()) return;
       }
     }
     if (wave == 4) {
@@ -527,7 +529,7 @@ __global__ __launch_bounds__(512, 2) void k_decode_chain(DecodeChain a) {
       take_row(WORD_STREAM, a.tag + a.layers - 1, x);
       norm(x, stream);
     }
-    __syncthreads();
+    meet();
     return;
   }
 
@@ -580,8 +582,7 @@ __global__ __launch_bounds__(512, 2) void k_decode_chain(DecodeChain a) {
     const uint32_t tag = a.tag + l;
     // ---- LayerNorm, q, k, v
     if (in_qkv) {
-      __syncthreads();
-      if (quit) return;
+      if (meet()) return;
       float4 x[NV];
       get(xn, x);
       float *row = a.kv + l * a.layer_stride + (a.n - 1) * pitch;
@@ -603,8 +604,7 @@ __global__ __launch_bounds__(512, 2) void k_decode_chain(DecodeChain a) {
     // ---- the newest query against the keys of a slice, for one head
     for (int unit = blockIdx.x; unit < units; unit += G) {
       const int h = unit % a.heads, slice = unit / a.heads, begin = slice * a.slice, count = min(a.slice, a.n - begin);
-      __syncthreads();
-      if (quit) return;
+      if (meet()) return;
       const float4 none = make_float4(0.f, 0.f, 0.f, 0.f), q = has_f ? ldq(fresh[0], f) : none;
       float m = -INFINITY, sum = 0.f;
       float4 o = none;
@@ -659,10 +659,8 @@ __global__ __launch_bounds__(512, 2) void k_decode_chain(DecodeChain a) {
     }
     // ---- the slices joined, wo, the residual stream
     if (in_c) {
-      __syncthreads();
-      if (quit) return;
-      __syncthreads();
-      if (quit) return;
+      if (meet()) return;
+      if (meet()) return;
       float4 x[NV];
       get(joined, x);
       for (int n = gw; n < C; n += W) {
@@ -674,8 +672,7 @@ __global__ __launch_bounds__(512, 2) void k_decode_chain(DecodeChain a) {
     long_row(at(w.fc2), gw);
     // ---- LayerNorm, fc1 and its activation
     if (in_f || in_c) {
-      __syncthreads();
-      if (quit) return;
+      if (meet()) return;
     }
     if (in_f) {
       float4 x[NV];
@@ -724,8 +721,7 @@ __global__ __launch_bounds__(512, 2) void k_decode_chain(DecodeChain a) {
     for (int r = 0; r < RA; r++) row_of(wa[r], next, gw + r * W, N);
     // ---- fc2, the residual stream
     if (in_c) {
-      __syncthreads();
-      if (quit) return;
+      if (meet()) return;
       for (int n = gw; n < C; n += W) {
         if (n != gw) long_row(at(w.fc2), n);
         float s[2] = {0.f, 0.f};
@@ -743,8 +739,7 @@ __global__ __launch_bounds__(512, 2) void k_decode_chain(DecodeChain a) {
     row_of(wo, at(a.layer[after].wo), gw, C);
   }
   // ---- the head
-  __syncthreads();
-  if (quit) return;
+  if (meet()) return;
   float4 x[NV];
   get(xn, x);
   for (int n = gw; n < a.vocab; n += RA * W) {
