@@ -311,11 +311,12 @@ __global__ __launch_bounds__(256) void k_decode_attention(DecodeAttention a) {
 // over the result): 6 layers x 256 186 -> 142 us, 4 x 128 112 -> 99, 2 x 64 87 -> 73; 24 behind 200: 8 x 384 327 -> 298, 8 x 512 365 -> 316.  The
 // kernel alone: 6 x 256 96 us, 16 a layer, against 23 in launches.  All rows ahead have to be asked for unconditionally: behind branches the
 // compiler waits for the newest of them before the oldest (attention 2.3 -> 1.9 us).
-constexpr int CHAIN_LAYERS = 32, CHAIN_NV = 2, CHAIN_UNITS = 4;      // at most: layers; 1024 wide, ffn 4096; keys a lane holds
+constexpr int CHAIN_LAYERS = 32, CHAIN_NV = 2, CHAIN_UNITS = 4;      // at most: layers; 256 NV wide, ffn 1024 NV; keys a lane holds
+constexpr int CHAIN_WIDTH = 256 * CHAIN_NV, CHAIN_FFN = 1024 * CHAIN_NV, CHAIN_TOPS = MAX_SLICES * (CHAIN_WIDTH / 8) * 2;      // heads of 8 features at least
 constexpr int64_t SPIN_TICKS = 1000000;                              // of 10 ns; computing again takes 0.7 ms (4 x 128) to 9.6 (12 x 512)
 constexpr int RESCUE_TRIES = 1 << 24;                                // 10 s and more at a microsecond a try
-enum { WORD_QKV = 0, WORD_SUMS = 3072, WORD_TOPS = WORD_SUMS + MAX_SLICES * 1024, WORD_MID = WORD_TOPS + MAX_SLICES * 128 * 2,
-       WORD_HID = WORD_MID + 1024, WORD_STREAM = WORD_HID + 4096, WORDS = WORD_STREAM + 1024 };
+enum { WORD_QKV = 0, WORD_SUMS = WORD_QKV + 3 * CHAIN_WIDTH, WORD_TOPS = WORD_SUMS + MAX_SLICES * CHAIN_WIDTH, WORD_MID = WORD_TOPS + CHAIN_TOPS,
+       WORD_HID = WORD_MID + CHAIN_WIDTH, WORD_STREAM = WORD_HID + CHAIN_FFN, WORDS = WORD_STREAM + CHAIN_WIDTH };
 __device__ uint64_t chain_words[WORDS];
 __device__ uint32_t chain_gave_up;              // the first tag of the launch that did
 __device__ uint64_t chain_again;                // tokens computed again
@@ -379,7 +380,7 @@ __global__ __launch_bounds__(512, 2) void k_decode_chain(DecodeChain a) {
   __shared__ float stream[256 * NV], mid[256 * NV];
   __shared__ __attribute__((aligned(16))) float fresh[3][128];         // the new row's q, k, v of a head
   __shared__ __attribute__((aligned(16))) float part_o[4][128];
-  __shared__ float part_m[4], part_l[4], tops[MAX_SLICES * 128 * 2];
+  __shared__ float part_m[4], part_l[4], tops[CHAIN_TOPS];
   __shared__ int quit[2];
   if (a.rescue && __hip_atomic_load(&chain_gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != a.rescue) return;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, C = a.width, F = a.ffn, nv = C >> 2, nf = F >> 2;
