@@ -216,7 +216,8 @@ __global__ __launch_bounds__(256) void k_emb_runs(const uint32_t *__restrict__ s
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int c = blockIdx.x * 4 + wave;
   if (c * ES_CHUNK >= npad) return;
-  const int64_t col = blockIdx.y * (int64_t)256 + lane * 4;
+  // every lane stays, also past the row's end (where it loads the row's last elements and stores nothing): es_key reads the keys of all of them
+  const int64_t mine = blockIdx.y * (int64_t)256 + lane * 4, col = mine < dim ? mine : dim - 4;
   const uint32_t mykey = sorted[c * ES_CHUNK + (lane & 31)];
   const int prev_id = c > 0 ? es_id(sorted[c * ES_CHUNK - 1]) : -1;
   const int next_id = (c + 1) * ES_CHUNK < npad ? es_id(sorted[(c + 1) * ES_CHUNK]) : -1;
@@ -225,7 +226,6 @@ __global__ __launch_bounds__(256) void k_emb_runs(const uint32_t *__restrict__ s
     if (blockIdx.y == 0 && lane == 0) meta[c] = EmbChunk{-1, -1, 0, 0};
     return;
   }
-  if (col >= dim) return;                                           // (es_key reads the other lanes' keys all the same)
   // eight rows are added, in order, while the next eight are on their way
   constexpr int HELD = 8;
   float4 rows[HELD], next[HELD];
@@ -241,6 +241,7 @@ __global__ __launch_bounds__(256) void k_emb_runs(const uint32_t *__restrict__ s
   int cur = first_id, run = 0;
   float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
   auto emit = [&](int id, int slot) {                               // slot: of the parts, -1: the row itself
+    if (mine >= dim) return;
     float4 *dst = reinterpret_cast<float4 *>((slot < 0 ? gw + (int64_t)id * dim : part + ((int64_t)c * 2 + slot) * dim) + col);
     if (accumulate && slot < 0) { float4 o = *dst; acc.x += o.x; acc.y += o.y; acc.z += o.z; acc.w += o.w; }
     *dst = acc;

@@ -83,7 +83,7 @@ def test_an_infinite_logit_is_not_a_number_in_the_loss(B, dtype, c):
     assert np.array_equal(np.isnan(ld.data), [False, False, True, False]) and np.isnan(loss.data[0])
 
 
-@pytest.mark.parametrize("dim", [4, 256, 260])
+@pytest.mark.parametrize("dim", [4, 64, 80, 256, 260, 320])
 @pytest.mark.parametrize("count", [33, 64, 63 * 32, 64 * 32, 65 * 32 + 1, 130 * 32])
 @pytest.mark.parametrize("before", [0, 5, 31])
 def test_an_id_over_many_blocks_is_summed_in_order(B, dim, count, before):
