@@ -113,12 +113,31 @@ def test_logits_behind_a_growing_context(B, vocab, ctx, layers, width, heads, mo
 
 @pytest.mark.parametrize("head_size", [16, 32, 64, 128])
 def test_slices_of_a_long_context(B, head_size):
-    """One key more than so many slices hold, and one less: 64 keys to a slice up to 1024, then 16 longer ones."""
+    """In one launch.  One key more than so many slices hold, and one less: 128 keys to a slice (64 and 32 of heads of 64 and 128 features), then, past 16
+    of those, 16 longer ones."""
     from alpha2_amd.decode import KeptContext
-    cfg, params = _model(B, 50, 1200, 1, 2 * head_size, 2)
+    cfg, params = _model(B, 50, 2100, 1, 2 * head_size, 2)
+    tokens = np.random.RandomState(2).randint(0, 50, 2100).astype(np.int32)
+    kept, before = KeptContext.of(cfg, params, B, 2100), B.decodeStats()["oneLaunch"]
+    lengths = (31, 32, 33, 62, 63, 64, 65, 127, 128, 129, 511, 512, 513, 577, 1023, 1024, 1025, 1026, 1199, 1200, 2047, 2048, 2049, 2100)
+    _compare(kept, cfg, params, B, tokens, lengths, True)
+    assert B.decodeStats()["oneLaunch"] - before == len(lengths)
+    kept.close()
+
+
+# every group width of the attention (and one between two), every count of float4s a lane of the joined row holds (1, 2, 3, 4, up to 8 and up to 16)
+@pytest.mark.parametrize("width,heads,more", [
+    (32, 2, dict(ffnDim=2052)), (64, 2, dict(ffnDim=2052)), (128, 2, dict(ffnDim=2052)), (256, 2, dict(ffnDim=2052)),
+    (480, 6, dict(ffnDim=2052)), (768, 12, dict()), (1024, 64, dict(ffnDim=64)), (1152, 9, dict(ffnDim=64)), (2304, 18, dict(ffnDim=64)),
+])
+def test_slices_of_a_long_context_in_launches(B, width, heads, more):
+    """64 keys to a slice up to 1024, then 16 longer ones; the slices are joined eight at a time."""
+    from alpha2_amd.decode import KeptContext
+    cfg, params = _model(B, 50, 1200, 1, width, heads, **more)
     tokens = np.random.RandomState(2).randint(0, 50, 1200).astype(np.int32)
-    kept = KeptContext.of(cfg, params, B, 1200)
-    _compare(kept, cfg, params, B, tokens, (62, 63, 64, 65, 127, 128, 129, 577, 1023, 1024, 1025, 1026, 1199, 1200), True)
+    kept, before = KeptContext.of(cfg, params, B, 1200), B.decodeStats()["oneLaunch"]
+    _compare(kept, cfg, params, B, tokens, (63, 64, 65, 128, 129, 512, 513, 577, 1024, 1025, 1026, 1200), True)
+    assert B.decodeStats()["oneLaunch"] == before
     kept.close()
 
 
@@ -154,7 +173,7 @@ def test_not_finite_parameters_reach_the_logits(B):
 @pytest.mark.parametrize("temperature", [0.0, 0.8])
 @pytest.mark.parametrize("act", ["gelu", "swiglu"])
 def test_the_same_tokens_with_and_without_kept_keys(B, monkeypatch, temperature, act):
-    """Over a prompt of 60 and 20 tokens behind it (a second slice from the 65th on), while flushGpu moves every parameter to another block and
+    """Over a prompt of 60 and 20 tokens behind it, while flushGpu moves every parameter to another block and
     fills the one it left with NaN.  The largest logits lie further apart than the two ways' roundings put them (1e-4 of the row; see _compare)."""
     from alpha2_amd import sample
     from alpha2_amd.decode import KeptContext
