@@ -703,10 +703,15 @@ __device__ __forceinline__ void wave_merge(float &m, float &s) {
 // A row is summed in one order whatever the number of its threads: CE_FULL shares take its 16-byte chunks (what is left of it: its classes) in turns, each
 // in order; the shares are merged by 64s, and the 64s one after the other.  A thread plays V shares, TPR apart, so that a row of few classes is a
 // wave's (no barrier, no LDS) and a CU holds more of them; a 64 that has nothing to merge is left out, which changes no bit.  What bounds short rows is the
-// merges (an exponential each).  us with a thread to a share in all cases / now, with the mean behind it: fp32 16384 x 256 29.9 / 12.9, x 512 30.6 / 20.0, x 1024
-// 32.9 / 33.2; both passes in bf16, whose registers held 53248 classes at every size, 10240 x 512 62.9 / 12.1, x 2048 67.6 / 30.0, x 4096 79.6 / 48.2, x 8192
-// 101 / 67.
+// merges (an exponential each).  us with a thread to a share in all cases / now, with the mean behind it: fp32 10240 x 256 20.7 / 9.6, x 512 21.6 / 14.1; both
+// passes in bf16, whose registers held 53248 classes at every size, 10240 x 512 62.6 / 11.7, x 1024 63.2 / 17.5, x 2048 67.0 / 28.5, x 4096 80.6 / 48.4, x 8192
+// 101 / 68.
 template <class T> constexpr int CE_FULL = sizeof(T) == 4 ? 256 : 512;
+// A wave to a row where that leaves a lane two chunks (of rows that are no whole chunks: two classes) at most: with four to eight, few rows wait for them
+// (in bf16 64 x 2047 took 17.1 us with a wave and 6.7 with 512 threads, 64 x 2048 7.7 and 5.9), and many rows that are no whole chunks gain nothing either
+// (10240 x 511 40.3 and 40.3)
+static bool ce_whole(int64_t c, int32_t dtype, ah_ptr operands) { return c % (dtype == AH_F32 ? 4 : 8) == 0 && aligned16(operands); }
+static bool ce_wave(int64_t c, int32_t dtype, ah_ptr operands) { return c <= (!ce_whole(c, dtype, operands) ? 128 : dtype == AH_F32 ? 512 : 1024); }
 constexpr int ce_block(int tpr) { return tpr == 64 ? 256 : tpr; }      // four rows of a wave each, or one row
 template <class T>
 __device__ __forceinline__ void ce_chunk(const uint4 &u, float &m, float &s) {
@@ -821,7 +826,7 @@ __device__ __forceinline__ void ce_grad8(const uint4 &u, float lse, float scale,
 #pragma unroll
   for (int i = 0; i < 4; i++) o[i] = pack_bf16x2(e[2 * i] * scale, e[2 * i + 1] * scale);
 }
-// TPR threads to a row, 8 or so elements to a thread; a wave up to 1024 classes (bf16 2048): 16384 x 256 in fp32 10.4 us with a block, 6.6 with a wave
+// TPR threads to a row, 8 or so elements to a thread; a wave where ce_wave says: 16384 x 256 in fp32 10.4 us with a block, 6.6 with a wave
 template <class T, int TPR>
 __global__ __launch_bounds__(256) void k_ce_bwd(const T *__restrict__ logits, const int32_t *__restrict__ targets, const float *__restrict__ lse,
                          const float *__restrict__ g, float g_mul, T *__restrict__ out, int64_t rows, int64_t n, int64_t c) {
@@ -1268,13 +1273,14 @@ int32_t ah_cross_entropy(ah_ptr logits, int32_t dtype, ah_ptr targets, ah_ptr lo
     ah::launch_kernel(kfn, dim3((unsigned)(tpr == 64 ? cdiv(n, 4) : n)), dim3((unsigned)ce_block(tpr)), 0, x, dp<const int32_t>(targets), rows,
                       dp<float>(lse_out), n, c);
   };
+  const bool wave = ce_wave(c, dtype, logits);
   if (dtype == AH_F32) {
     const float *x = dp<const float>(logits);
-    if (c <= 1024) go(k_ce_fwd<float, 64>, 64, x); else go(k_ce_fwd<float, 256>, 256, x);
+    if (wave) go(k_ce_fwd<float, 64>, 64, x); else go(k_ce_fwd<float, 256>, 256, x);
   } else {
     const uint16_t *x = dp<const uint16_t>(logits);
-    if (c <= 2048) go(k_ce_fwd<uint16_t, 64>, 64, x);
-    else if (c <= 8192) go(k_ce_fwd<uint16_t, 256>, 256, x);
+    if (wave) go(k_ce_fwd<uint16_t, 64>, 64, x);
+    else if (c <= 8192 && ce_whole(c, dtype, logits)) go(k_ce_fwd<uint16_t, 256>, 256, x);
     else go(k_ce_fwd<uint16_t, 512>, 512, x);
   }
   AH_LAUNCH_CHECK();
@@ -1290,7 +1296,7 @@ int32_t ah_cross_entropy_bwd(ah_ptr logits, int32_t dtype, ah_ptr targets, ah_pt
   if (n == 0 || c == 0) return AH_OK;
   AH_ARG(logits && targets && lse && dlogits, "ah_cross_entropy_bwd: null operand");
   AH_ARG(n <= 65535 * 1024ll, "ah_cross_entropy_bwd: too many rows");
-  const int tpr = c <= (dtype == AH_F32 ? 1024 : 2048) ? 64 : 256, per = 256 / tpr;
+  const int tpr = ce_wave(c, dtype, logits | dlogits) ? 64 : 256, per = 256 / tpr;
   const unsigned gx = (unsigned)cdiv(c, tpr == 64 ? c : TPB * 8);
   // gridDim.y is limited to 65535: fold rows beyond that by launching in row chunks
   for (int64_t r0 = 0; r0 < n; r0 += 65535 * (int64_t)per) {
@@ -1333,7 +1339,7 @@ int32_t ah_cross_entropy_fwd_bwd(ah_ptr logits, int32_t dtype, ah_ptr targets, a
   };
   if (c <= 512) go(k_ce_fwd_bwd<64, 1, 1>, 64);
   else if (c <= 1024) go(k_ce_fwd_bwd<64, 2, 1>, 64);
-  else if (c <= 2048) go(k_ce_fwd_bwd<64, 4, 1>, 64);
+  else if (c <= 2048) go(k_ce_fwd_bwd<256, 1, 1>, 256);
   else if (c <= 4096) go(k_ce_fwd_bwd<256, 2, 1>, 256);
   else if (c <= 8192) go(k_ce_fwd_bwd<256, 2, 2>, 256);
   else if (c <= 16384) go(k_ce_fwd_bwd<512, 1, 4>, 512);

@@ -13,8 +13,8 @@ def B():
     return HipBackend(0)
 
 
-@pytest.mark.parametrize("dtype,c", [("f32", c) for c in (1, 3, 4, 255, 256, 1023, 1024, 1025, 1028, 2048)] +
-                         [("bf16", c) for c in (1, 8, 504, 512, 520, 2040, 2047, 2048, 2049, 2056, 8184, 8192, 8200, 16384, 16392)])
+@pytest.mark.parametrize("dtype,c", [("f32", c) for c in (1, 3, 4, 127, 129, 255, 256, 1023, 1024, 1025, 1028, 2048)] +
+                         [("bf16", c) for c in (1, 8, 127, 129, 504, 512, 520, 1023, 1024, 1032, 2040, 2047, 2048, 2049, 2056, 8184, 8192, 8200, 16384, 16392)])
 @pytest.mark.parametrize("n", [1, 3, 4, 70])
 def test_rows_of_every_number_of_threads(B, dtype, c, n):
     """Against 64 bits on the logits as stored.  A thread adds up to 40 terms after one another, thirteen more join them with three roundings each, and
