@@ -4,7 +4,7 @@
 // A single row makes every product a matrix times a vector: nothing is used twice, so there is no tile to share and the bound is the
 // weights read once (4 bytes for 2 operations) - where a launch is long enough to feel it.  At the sizes sampled in earnest (256 to
 // 1024 wide) a matrix is 0.3 to 12 MB, a microsecond or two of the chip, and what a token takes is the chain of dependent launches.
-// So the launches are few, one for the whole token up to 512 wide (k_decode_chain) and otherwise five a layer, each does the small work in front of its product itself, and each asks for its weights before
+// So the launches are few, one for the whole token of small models (k_decode_chain) and otherwise five a layer, each does the small work in front of its product itself, and each asks for its weights before
 // anything it has to wait for:
 //   k_decode_rows<NORM>  LayerNorm (the first one of all adds the two embeddings) + q, k, v into the row of the cache; + fc1 and its
 //                        activation (gate and up together); + the head.  Every wave normalises the row again, in registers.
@@ -307,9 +307,9 @@ __global__ __launch_bounds__(256) void k_decode_attention(DecodeAttention a) {
 // does, that no healthy wait comes near.  Its logits are NaN until it has computed them, and `chain_again` counts it (ah_decode_stats).  The tokens
 // behind it take one launch again: sums are cut elsewhere in the launches of a layer, and what a program computes does not depend on who else uses the GPU.
 // What bounds it is that chain of trips, 1.3 us at least and 2 to 3 as polled, five a layer, and between them the one wave that has the next step
-// (350 instructions in a row are 1 us).  A token, its logits read and chosen from, 64 of them behind a prompt of 17 (with the prompt's pass and the pass
-// over the result): 6 layers x 256 186 -> 142 us, 4 x 128 112 -> 99, 2 x 64 87 -> 73; 24 behind 200: 8 x 384 327 -> 298, 8 x 512 365 -> 316.  The
-// kernel alone: 6 x 256 96 us, 16 a layer, against 23 in launches.  All rows ahead have to be asked for unconditionally: behind branches the
+// (350 instructions in a row are 1 us).  A token, its logits read and chosen from, in launches (whose host work differs that much between processes) and in
+// one: 2 x 64 behind 17 rows 64 to 110 / 56 us, 4 x 128 89 to 149 / 86, 32 x 128 behind 100 486 to 608 / 456, 6 x 256 116 to 175 / 121, 8 x 384 153 to
+// 198 / 175, behind 200 195 to 253 / 221, 8 x 512 behind 17 163 to 213 / 185.  The kernel alone: 6 x 256 96 us, 16 a layer.  All rows ahead have to be asked for unconditionally: behind branches the
 // compiler waits for the newest of them before the oldest (attention 2.3 -> 1.9 us).
 constexpr int CHAIN_LAYERS = 32, CHAIN_NV = 2, CHAIN_UNITS = 4;      // at most: layers; 256 NV wide, ffn 1024 NV; keys a lane holds
 constexpr int CHAIN_WIDTH = 256 * CHAIN_NV, CHAIN_FFN = 1024 * CHAIN_NV, CHAIN_TOPS = MAX_SLICES * (CHAIN_WIDTH / 8) * 2;      // heads of 8 features at least
@@ -807,14 +807,26 @@ DecodeRows rows_of(const AhDecode *d, ah_ptr gain, ah_ptr bias, ah_ptr w, int n)
   return a;
 }
 
-
 // Where the token runs in one launch: up to 512 wide (ffn 2048), and with the layers that fit the kernel's arguments.  Wider, every phase's words
 // are asked for by every workgroup at 3 to 24 KB a time, their trips through memory take 5 to 7 us instead of 2 to 3, and the rows ahead no longer
-// fit the registers: 768 wide in 12 layers 430 us a token against 400 in launches.  Not inside a captured graph or a step plan, whose replays would bring the same tags again, nor on the side stream, where the launches of a layer are refused too.
-int chain_quads(const AhDecode *d) {
+// fit the registers: 768 wide in 12 layers 430 us a token against 400 in launches.  Past 256 wide (ffn 1024) that grows with the slices of the keys,
+// whose sums every workgroup joins, and up to four are taken (us a token as sampled, five launches a layer / one launch; the launches' host work
+// differs that much between processes: 8 x 512 behind 17 rows 163 to 213 / 186, behind 200 165 to 207 / 195, behind 500 181 to 213 / 221, behind 900 197 to
+// 224 / 237; at 256 wide 6 layers behind 900 123 to 175 / 132).  A single layer gains less than the phases of a long head lose, whose rows have few waves
+// here: 1 x 256 with a vocabulary of 8000 129 / 135, 2 x 256 153 to 185 / 150.  Not inside a captured graph or a step plan, whose replays would
+// bring the same tags again, nor on the side stream, where the launches of a layer are refused too.
+int chain_lanes(int head_size) {
+  int lanes = 8;
+  while (4 * lanes < head_size) lanes *= 2;
+  return lanes;
+}
+// keys to a slice: what the lanes hold at a time, at most 128
+int chain_slice(int head_size) { return std::min(256 / chain_lanes(head_size) * CHAIN_UNITS, 128); }
+int chain_quads(const AhDecode *d, int n) {
   if (d->layers > CHAIN_LAYERS || ah::step_active() || ah::capturing() || ah::on_side()) return 0;
-  const int64_t nv = cdiv(d->width, 256) > cdiv(d->ffn, 1024) ? cdiv(d->width, 256) : cdiv(d->ffn, 1024);
-  return nv <= CHAIN_NV ? (int)nv : 0;
+  const int64_t nv = std::max(cdiv(d->width, 256), cdiv(d->ffn, 1024));
+  if (nv > CHAIN_NV || (nv > 1 && n > 4 * chain_slice(d->width / d->heads)) || (d->layers == 1 && d->vocab > 2048)) return 0;
+  return (int)nv;
 }
 thread_local int64_t next_ticks = SPIN_TICKS;
 std::atomic<int64_t> chain_tokens{0};
@@ -837,9 +849,9 @@ int32_t launch_chain(const AhDecode *d, const AhDecodeLayer *layers, int32_t tok
   const bool gated = (d->act & AH_DECODE_GATED) != 0;
   a.mask = gated ? 0 : d->act;
   a.n = n; a.layer_stride = (int64_t)d->rows * 3 * C;
-  for (a.lanes = 8; 4 * a.lanes < hs;) a.lanes *= 2;
-  // a slice: what the lanes hold at a time, at most 128 keys; longer ones where there would be too many
-  const int most = 256 / a.lanes * CHAIN_UNITS, held = most < 128 ? most : 128;
+  // slices are longer where there would be too many
+  a.lanes = chain_lanes(hs);
+  const int held = chain_slice(hs);
   a.slices = (int)(cdiv(n, held) < MAX_SLICES ? cdiv(n, held) : MAX_SLICES);
   a.slice = (int)cdiv(n, a.slices);
   a.slices = (int)cdiv(n, a.slice);
@@ -907,7 +919,7 @@ int32_t ah_decode(const AhDecode *d, const AhDecodeLayer *layers, int32_t token,
     AH_ARG(l.ln1_w && l.ln1_b && l.wqkv && l.wo && l.ln2_w && l.ln2_b && l.fc1 && l.fc2 && (!gated || l.up), "ah_decode: null weight in layer %d", i);
     AH_ARG(aligned16(l.ln1_w | l.ln1_b | l.wqkv | l.wo | l.ln2_w | l.ln2_b | l.fc1 | l.fc2 | l.up), "ah_decode: weights of layer %d must be 16-byte aligned", i);
   }
-  if (const int nv = chain_quads(d)) return launch_chain(d, layers, token, pos, nv, ticks);
+  if (const int nv = chain_quads(d, pos + 1)) return launch_chain(d, layers, token, pos, nv, ticks);
   const int C = d->width, H = d->heads, n = pos + 1;
   const int slices = (int)(cdiv(n, MIN_SLICE) < MAX_SLICES ? cdiv(n, MIN_SLICE) : MAX_SLICES);
   // the residual stream, the MLP's hidden row, the slices' sums and their maxima; stream-ordered, so it may go back at once

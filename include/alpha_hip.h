@@ -482,7 +482,7 @@ typedef struct {
 int32_t ah_decode(const AhDecode *d, const AhDecodeLayer *layers, int32_t token, int32_t pos);
 /* The logits of one row that has been through all layers: the last LayerNorm and the head. */
 int32_t ah_decode_head(const AhDecode *d, ah_ptr row);
-/* Tokens so far that were one launch (up to 512 wide, outside captures and step plans), and those of them that were computed again because their
+/* Tokens so far that were one launch (small models and short contexts, outside captures and step plans), and those of them that were computed again because their
  * workgroups waited too long for each other, 10 ms: the GPU is shared, and such a token is that much late.  Waits for the stream. */
 int32_t ah_decode_stats(int64_t *one_launch, int64_t *again);
 /* For tests: when the waits of the next ah_decode of this thread end, in 10 ns.  -1: at the first word that is not there yet, so that the token is

@@ -237,6 +237,25 @@ def test_a_token_in_one_launch(B, vocab, ctx, layers, width, heads, more):
     kept.close()
 
 
+@pytest.mark.parametrize("vocab,layers,width,heads,more,last", [
+    (60, 2, 512, 4, dict(), 128), (60, 2, 272, 17, dict(), 512), (60, 2, 64, 2, dict(ffnDim=1028), 512), (60, 2, 256, 2, dict(), 1100),
+    (2048, 1, 64, 2, dict(), 1100), (2049, 1, 64, 2, dict(), 0), (2049, 2, 64, 2, dict(), 1100),
+])
+def test_where_a_context_leaves_the_one_launch(B, vocab, layers, width, heads, more, last):
+    """Past four slices of keys (32 to a slice for heads of 128 features, 128 for small ones) of a model wider than 256 or an MLP than 1024, and for one
+    layer with a long head: the rows that a launch left are those the launches go on from."""
+    from alpha2_amd.decode import KeptContext
+    cfg, params = _model(B, vocab, 1100, layers, width, heads, **more)
+    tokens = np.random.RandomState(4).randint(0, vocab, 1100).astype(np.int32)
+    kept, before = KeptContext.of(cfg, params, B, 1100), B.decodeStats()["oneLaunch"]
+    first = max(min(last, 1090) - 5, 20)
+    kept.lastRow(tokens[:first - 1], B.releaseGpuTensor)
+    _compare(kept, cfg, params, B, tokens, range(first, first + 12 if last < 1100 else 1101), False)
+    taken = B.decodeStats()["oneLaunch"] - before
+    assert taken == (0 if last == 0 else 6 if last < 1100 else 1101 - first), taken
+    kept.close()
+
+
 @pytest.mark.parametrize("width,heads,act", [(64, 2, "gelu"), (256, 8, "swiglu"), (512, 4, "kan_spline")])
 def test_a_launch_that_gave_up_is_computed_again(B, width, heads, act):
     """Its waits end at the first word that is not there yet; the one workgroup behind it sums the same terms in the same order."""
