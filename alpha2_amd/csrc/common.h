@@ -89,8 +89,8 @@ template <> struct Io<uint16_t> {   // bf16 storage
 
 // What lane ^ O holds; every lane of the wave takes part.  Rows of 16 and halves are exchanged by v_permlane16/32_swap, the rest is moved by DPP: a step
 // of a reduction is one or two vector instructions, where __shfl_xor is a trip through LDS (ds_bpermute, 100 cycles and more), and reductions
-// along a row are what a short row kernel waits for (same bits; the step of 2 layers x 128 at 2 x 64 tokens 294 -> 289 us, of 24 x 1024 at
-// 4 x 8 x 1024 96.4 -> 95.7 ms, 24 tokens sampled from 12 x 768 12.3 -> 11.9).
+// along a row are what a short row kernel waits for (same bits; the step of 2 layers x 128 at 2 x 64 tokens 294 -> 289 us, of
+// 24 x 1024 at 4 x 8 x 1024 no more than two runs differ).
 template <int CTRL>
 __device__ __forceinline__ uint32_t dpp_moved(uint32_t v) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true); }
 template <int O>
